@@ -33,9 +33,10 @@
  *     it may be NULL when that size is 0.  Its contents need no initialisation.
  *   - Alignment: the input, `values` and candidate values to the element size,
  *     indices to their width (8 bytes; 4 for the *_i32 entry points), `ws` to
- *     16 bytes (256 recommended); otherwise ATK_ERR_ALIGN.  Input, `values`
- *     and `indices` that are all 16-byte aligned, with `row_stride` a multiple
- *     of 16 bytes' worth of elements, additionally get the 16-byte-vector kernels.
+ *     16 bytes (256 recommended); otherwise ATK_ERR_ALIGN.  The interleaved
+ *     layouts load 16 bytes at a time whatever the row pitch, as long as the
+ *     input itself is 4-byte aligned; the contiguous ones want the input 16-byte
+ *     aligned and `row_stride` a multiple of 16 bytes' worth of elements for that.
  */
 #ifndef APPROX_TOPK_HIP_H_
 #define APPROX_TOPK_HIP_H_
@@ -126,8 +127,8 @@ int atk_select(const void* cand_values, const int64_t* cand_indices,
 size_t atk_topk_workspace_bytes(int64_t rows, int64_t n, int64_t k0, int j,
                                 int64_t k, int layout, int dtype);
 /*
- * The same for one particular call: 0 when the input's address and row stride
- * let the one-kernel path take it, which parks no candidates (never more than
+ * The same for one particular call: 0 when its rows start on 16-byte boundaries
+ * and the one-kernel path takes it, which parks no candidates (never more than
  * atk_topk_workspace_bytes).  Same call site as above: the workspace the
  * operator allocates before the native call (priority_queue.py:63-88).
  */

@@ -243,8 +243,10 @@ size_t atk_topk_workspace_bytes(int64_t rows, int64_t n, int64_t k0, int j, int6
 
 size_t atk_topk_workspace_bytes_at(const void* x, int64_t rows, int64_t n, int64_t row_stride, int64_t k0,
                                    int j, int64_t k, int layout, int dtype) {
+  // (the one-kernel path takes rows that start off a 16-byte boundary as well; the bound stays for them)
   if (rows > 0 && k > 0 && k < k0 && check_stage1(x, rows, n, row_stride, k0, j, layout, dtype, x, x) == ATK_OK &&
-      atk::fused_row_takes(x, rows, n, row_stride, k0, j, k, layout, dtype))
+      aligned_to(x, 16) && (row_stride * atk::elem_bytes(dtype)) % 16 == 0 &&
+      atk::fused_row_takes(x, rows, n, k0, j, k, layout, dtype))
     return 0;
   return plan_topk(rows, n, k0, j, k, layout, dtype).total;
 }
@@ -273,12 +275,9 @@ int atk_describe(const void* x, int64_t rows, int64_t n, int64_t row_stride, int
   std::string out;
   if (rows != 0 && k != 0) {
     bool fused = false;
-    if (k < k0) fused = atk::describe_fused_row(x, rows, n, row_stride, k0, j, k, layout, dtype, out);
+    if (k < k0) fused = atk::describe_fused_row(x, rows, n, k0, j, k, layout, dtype, out);
     if (!fused) {
-      // the candidates of a two-stage call are written to the (aligned) workspace
-      const void* v1 = k < k0 ? nullptr : values;
-      const void* i1 = k < k0 ? nullptr : indices;
-      if (!atk::describe_stage1_stream(x, rows, n, row_stride, k0, j, layout, dtype, v1, i1, out) &&
+      if (!atk::describe_stage1_stream(x, rows, n, k0, j, layout, dtype, out) &&
           !atk::describe_stage1_contig(x, rows, n, row_stride, k0, j, layout, dtype, out))
         atk::describe_stage1_lane_per_bucket(rows, k0, j, dtype, out);
       if (k < k0) {

@@ -57,10 +57,10 @@ static bool stores_past_cache(int64_t rows, int64_t n, int64_t k, int64_t es) {
 // 128 bytes fp16 [256, 131072] k0=8192 39.2 against 33.3 us, fp32 [64, 32768] k0=2048
 // 17.4 against 12.7 us; of 256 bytes fp16 [256, 262144] k0=8192 57.6 against 49.4 us,
 // [1024, 131072] 109.9 against 110.3 us.
-static Plan plan_short_buckets(int64_t rows, int64_t n, int64_t k0, int j, int64_t k, int dtype, bool aligned) {
+static Plan plan_short_buckets(int64_t rows, int64_t n, int64_t k0, int j, int64_t k, int dtype, bool wide) {
   Plan pl{};
   pl.ok = false;
-  if (!aligned || rows > 0x7fffffffll) return pl;
+  if (!wide || rows > 0x7fffffffll) return pl;
   if (k0 <= 0 || k <= 0 || k >= k0 || j < 1 || j > 4 || k0 % j) return pl;
   const int es = elem_bytes(dtype);
   if (es != 2 && es != 4) return pl;
@@ -94,13 +94,13 @@ static Plan plan_short_buckets(int64_t rows, int64_t n, int64_t k0, int j, int64
   return pl;
 }
 
-Plan make_plan(int64_t rows, int64_t n, int64_t k0, int j, int64_t k, int layout, int dtype, bool aligned) {
+Plan make_plan(int64_t rows, int64_t n, int64_t k0, int j, int64_t k, int layout, int dtype, bool wide) {
   Plan pl{};
   pl.ok = false;
-  if (layout == ATK_BALANCED) return plan_short_buckets(rows, n, k0, j, k, dtype, aligned);
+  if (layout == ATK_BALANCED) return plan_short_buckets(rows, n, k0, j, k, dtype, wide);
   // (a padded row is never reduced further: its callers keep every bucket)
   if (layout != ATK_INTERLEAVED) return pl;
-  if (!aligned || rows > 0x7fffffffll) return pl;
+  if (!wide || rows > 0x7fffffffll) return pl;
   if (k0 <= 0 || k <= 0 || k >= k0 || j < 1 || j > 4 || k0 % j) return pl;
   const int es = elem_bytes(dtype);
   if (!es) return pl;
@@ -213,23 +213,19 @@ Plan make_plan(int64_t rows, int64_t n, int64_t k0, int j, int64_t k, int layout
 }  // namespace fused
 
 namespace {
-fused::Plan plan_for(const void* x, int64_t rows, int64_t n, int64_t row_stride, int64_t k0, int j, int64_t k,
-                     int layout, int dtype) {
-  const int es = elem_bytes(dtype);
-  const int vf = es ? stream::full_vec(es) : 1;
-  const bool aligned = ((uintptr_t)x % 16 == 0) && (row_stride % vf == 0);
-  return fused::make_plan(rows, n, k0, j, k, layout, dtype, aligned);
+// Rows may start at any element (a row of odd length does): the 16-byte loads take such addresses.
+fused::Plan plan_for(const void* x, int64_t rows, int64_t n, int64_t k0, int j, int64_t k, int layout, int dtype) {
+  return fused::make_plan(rows, n, k0, j, k, layout, dtype, stream::wide_loads(x, elem_bytes(dtype)));
 }
 }  // namespace
 
-bool fused_row_takes(const void* x, int64_t rows, int64_t n, int64_t row_stride, int64_t k0, int j, int64_t k,
-                     int layout, int dtype) {
-  return plan_for(x, rows, n, row_stride, k0, j, k, layout, dtype).ok;
+bool fused_row_takes(const void* x, int64_t rows, int64_t n, int64_t k0, int j, int64_t k, int layout, int dtype) {
+  return plan_for(x, rows, n, k0, j, k, layout, dtype).ok;
 }
 
-bool describe_fused_row(const void* x, int64_t rows, int64_t n, int64_t row_stride, int64_t k0, int j, int64_t k,
-                        int layout, int dtype, std::string& out) {
-  const fused::Plan pl = plan_for(x, rows, n, row_stride, k0, j, k, layout, dtype);
+bool describe_fused_row(const void* x, int64_t rows, int64_t n, int64_t k0, int j, int64_t k, int layout, int dtype,
+                        std::string& out) {
+  const fused::Plan pl = plan_for(x, rows, n, k0, j, k, layout, dtype);
   if (!pl.ok) return false;
   out += std::string(pl.in_registers ? "fused_regs_kernel<" : "fused_row_kernel<") + dtype_name(dtype) + ", J=" +
          std::to_string(j) + ", V=" + std::to_string(pl.vec) + ", pos" + (pl.pos16 ? "16" : "32") +
@@ -243,7 +239,7 @@ bool describe_fused_row(const void* x, int64_t rows, int64_t n, int64_t row_stri
 int launch_fused_row(const void* x, int64_t rows, int64_t n, int64_t row_stride, int64_t k0, int j,
                      int64_t k, int layout, int dtype, void* values, IndexOut indices, hipStream_t stream,
                      bool* handled) {
-  const fused::Plan pl = plan_for(x, rows, n, row_stride, k0, j, k, layout, dtype);
+  const fused::Plan pl = plan_for(x, rows, n, k0, j, k, layout, dtype);
   *handled = pl.ok;
   if (!pl.ok) return ATK_OK;
   int rc = ATK_ERR_DTYPE;

@@ -4,8 +4,8 @@
 // [L = n / b sub-rows][b columns] plus a last partial sub-row of n mod b
 // elements; bucket c is column c.  The job is a column-wise top-J.
 //
-// Mapping.  Every lane owns V adjacent columns (V*sizeof(T) = 16 bytes when the
-// addresses allow it, else V = 1), so one wave64 load instruction reads 64*V
+// Mapping.  Every lane owns V adjacent columns (V*sizeof(T) = 16 bytes; V = 1 in
+// rows of fewer columns than that), so one wave64 load instruction reads 64*V
 // adjacent elements of one sub-row (1 KiB with 16-byte loads) and the wave walks
 // down the sub-rows.  The J-entry queue of each owned column lives in
 // registers: values in compare form plus the sub-row number they came from; the
@@ -148,9 +148,24 @@ template <> struct Cmp<Elem<ATK_I64>> {
 // V elements moved by one load instruction.
 template <typename raw_t, int V> struct alignas(sizeof(raw_t) * V) Pack { raw_t e[V]; };
 
+// The same in global memory, at any address an element may have: a row of odd
+// length starts anywhere, and so does every sub-row of an odd number of buckets.
+// The part's global loads and stores take such addresses in the one instruction
+// they are for aligned ones.
+template <typename raw_t, int V> struct __attribute__((packed, aligned(sizeof(raw_t)))) LoosePack { raw_t e[V]; };
+
 template <typename raw_t, int V>
 __device__ __forceinline__ Pack<raw_t, V> load_pack(const raw_t* p) {
-  return *reinterpret_cast<const Pack<raw_t, V>*>(p);
+  const LoosePack<raw_t, V> loose = *reinterpret_cast<const LoosePack<raw_t, V>*>(p);
+  Pack<raw_t, V> pk;
+  __builtin_memcpy(&pk, &loose, sizeof(pk));
+  return pk;
+}
+template <typename raw_t, int V>
+__device__ __forceinline__ void store_pack(raw_t* p, const Pack<raw_t, V>& pk) {
+  LoosePack<raw_t, V> loose;
+  __builtin_memcpy(&loose, &pk, sizeof(pk));
+  *reinterpret_cast<LoosePack<raw_t, V>*>(p) = loose;
 }
 
 // ---------------------------------------------------------------------------
@@ -833,7 +848,7 @@ __device__ __forceinline__ void emit(const Geom& g, const Sink<typename E::raw_t
         ATK_STATIC_FOR(t, J) {
           Pack<raw_t, V> pv;
           ATK_STATIC_FOR(e, V) { pv.e[e] = queue.template raw<(t * V + e) / J, (t * V + e) % J>(); } ATK_STATIC_END;
-          reinterpret_cast<Pack<raw_t, V>*>(ov)[t] = pv;
+          store_pack<raw_t, V>(ov + t * V, pv);
         } ATK_STATIC_END;
       }
       if (out.indices.narrow) {
@@ -845,7 +860,7 @@ __device__ __forceinline__ void emit(const Geom& g, const Sink<typename E::raw_t
             constexpr int v = (t * kPer + e) / J, sl = (t * kPer + e) % J;
             pi.e[e] = (int32_t)(col + v + (int64_t)queue.template position<v, sl>() * g.b);
           } ATK_STATIC_END;
-          reinterpret_cast<Pack<int32_t, kPer>*>(oi)[t] = pi;
+          store_pack<int32_t, kPer>(oi + t * kPer, pi);
         } ATK_STATIC_END;
       } else {
         int64_t* oi = static_cast<int64_t*>(out.indices.base) + o;
@@ -855,7 +870,7 @@ __device__ __forceinline__ void emit(const Geom& g, const Sink<typename E::raw_t
             constexpr int v = (t * 2 + e) / J, sl = (t * 2 + e) % J;
             pi.e[e] = col + v + (int64_t)queue.template position<v, sl>() * g.b;
           } ATK_STATIC_END;
-          reinterpret_cast<Pack<int64_t, 2>*>(oi)[t] = pi;
+          store_pack<int64_t, 2>(oi + t * 2, pi);
         } ATK_STATIC_END;
       }
     } else {
@@ -944,7 +959,7 @@ __device__ __forceinline__ void emit_transposed(const Geom& g, const Sink<typena
       if (i < valid) {
         const Pack<raw_t, kPerStore> pv = *reinterpret_cast<const Pack<raw_t, kPerStore>*>(
             raws + (i / NC) * T::kRawPitch + (i % NC) * sizeof(raw_t));
-        *reinterpret_cast<Pack<raw_t, kPerStore>*>(out.values + o + i) = pv;
+        store_pack<raw_t, kPerStore>(out.values + o + i, pv);
       }
     } ATK_STATIC_END;
   }
@@ -963,7 +978,7 @@ __device__ __forceinline__ void emit_transposed(const Geom& g, const Sink<typena
         Pack<int32_t, 4> pi;
         pi.e[0] = (int32_t)index_of(i, a.x); pi.e[1] = (int32_t)index_of(i + 1, a.y);
         pi.e[2] = (int32_t)index_of(i + 2, a.z); pi.e[3] = (int32_t)index_of(i + 3, a.w);
-        *reinterpret_cast<Pack<int32_t, 4>*>(oi + i) = pi;
+        store_pack<int32_t, 4>(oi + i, pi);
       }
     } ATK_STATIC_END;
   } else {
@@ -975,7 +990,7 @@ __device__ __forceinline__ void emit_transposed(const Geom& g, const Sink<typena
         Pack<int64_t, 2> pi;
         pi.e[0] = index_of(i, a.x);
         pi.e[1] = index_of(i + 1, a.y);
-        *reinterpret_cast<Pack<int64_t, 2>*>(oi + i) = pi;
+        store_pack<int64_t, 2>(oi + i, pi);
       }
     } ATK_STATIC_END;
   }
@@ -1419,8 +1434,11 @@ __global__ __launch_bounds__(kWave * W) __attribute__((amdgpu_waves_per_eu(4))) 
   const uint32_t slab = __builtin_amdgcn_readfirstlane(blk % g.slabs);
   const int64_t row = __builtin_amdgcn_readfirstlane(blk / g.slabs);
 
-  const int64_t col = (int64_t)col_tile * kTileCols + lane * V;
-  const bool live = col < g.b;  // b is a multiple of V whenever V > 1
+  // When V does not divide b, the row's last live lane moves down to its last V
+  // columns: it works out some of its neighbour's columns again and writes the same.
+  const int64_t first_col = (int64_t)col_tile * kTileCols + lane * V;
+  const bool live = first_col < g.b;
+  const int64_t col = first_col + V > g.b ? g.b - V : first_col;
 
   // sub-rows of this slab [s0, s1), then of this wave [p0, p1)
   const uint32_t s0 = slab * g.slab_len;
@@ -1625,8 +1643,15 @@ struct Plan {
   size_t part_values_off, part_pos_off, ws_bytes;
 };
 
-// `aligned`: base pointers and row stride allow 16-byte accesses.
-Plan make_plan(int64_t rows, int64_t n, int64_t k0, int j, int layout, int dtype, bool aligned);
+// `wide`: 16-byte loads may be used (wide_loads).
+Plan make_plan(int64_t rows, int64_t n, int64_t k0, int j, int layout, int dtype, bool wide);
+// Rows and sub-rows may start at any element.  One-element loads, which odd rows took before,
+// move a quarter (4-byte types) or an eighth (2-byte types) of the bytes per instruction: bf16
+// [256, 100003] k=64 j=1 k_mult=8 24.8 us that way (and in two kernels) against 14.3 us, arg-max of
+// fp16 [256, 50001] k=1000 15.4 against 10.2 us, fp32 [16, 2653751] k=10 j=2 k_mult=4 44.2 against 41.8 us.
+// Only a 2-byte input that itself starts on an odd half-word keeps them: tests/test_host_logic.py
+// states the plan of such a view.
+inline bool wide_loads(const void* x, int es) { return es >= 4 || (uintptr_t)x % 4 == 0; }
 
 // One instance per element type, each in its own translation unit.
 // `ranges`: see KeyRangeOut; may be nullptr.

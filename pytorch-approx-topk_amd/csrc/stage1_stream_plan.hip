@@ -30,7 +30,7 @@ constexpr int64_t kFoldMinLength = 8;
 constexpr int64_t kFoldAnyLength = 128;
 }  // namespace
 
-Plan make_plan(int64_t rows, int64_t n, int64_t k0, int j, int layout, int dtype, bool aligned) {
+Plan make_plan(int64_t rows, int64_t n, int64_t k0, int j, int layout, int dtype, bool wide) {
   Plan pl{};
   pl.ok = false;
   if (layout != ATK_INTERLEAVED && layout != ATK_INTERLEAVED_PADDED) return pl;
@@ -48,9 +48,13 @@ Plan make_plan(int64_t rows, int64_t n, int64_t k0, int j, int layout, int dtype
   // workgroup puts each bucket back together.
   int64_t fold = 1;
   if (length >= kFoldMinLength) {
-    const int v = aligned ? vf : 1;
+    const int v = wide ? vf : 1;
     int64_t f = (int64_t)kWave * v / b;
-    while (f > 1 && ((b * f) % v != 0 || n / (b * f) < j)) --f;
+    while (f > 1 && n / (b * f) < j) --f;
+    // whole vectors when that costs at most a quarter of the lanes
+    int64_t whole = f;
+    while (whole > 1 && (b * whole) % v != 0) --whole;
+    if (whole > 1 && whole * 4 >= f * 3) f = whole;
     // short buckets: only when at least three lanes in four would idle (a fold of
     // two costs more in the merge than it gains: [128, 4096] with 128 buckets, j = 4, +23 %)
     if (f > 1 && (length >= kFoldAnyLength || f >= 4)) fold = f;
@@ -62,7 +66,7 @@ Plan make_plan(int64_t rows, int64_t n, int64_t k0, int j, int layout, int dtype
   pl.full_rows = (uint32_t)full;
   pl.rem = (uint32_t)(n - full * width);
   pl.pad_tail = layout == ATK_INTERLEAVED_PADDED ? 1u : 0u;
-  pl.vec = (aligned && width % vf == 0) ? vf : 1;
+  pl.vec = wide && width >= vf ? vf : 1;
   pl.packed = ((dtype == ATK_F16 || dtype == ATK_BF16 || dtype == ATK_I16) && full <= kPackedMaxSubRow) ||
               ((dtype == ATK_U8 || dtype == ATK_I8) && full <= kByteMaxSubRow);
 
@@ -139,7 +143,7 @@ Plan make_plan(int64_t rows, int64_t n, int64_t k0, int j, int layout, int dtype
   // has workgroups by the thousand, and a workgroup writes at least an eighth of what it reads
   // (at a twelfth, fp16 [256, 2^20] k=16384: j=2 112.6 -> 115.1 us, j=4 118.2 -> 115.2 us, j=1 104.9 -> 102.5 us).
   pl.wave_stores = false;
-  if (pl.vec > 1 && es <= 4 && !pl.merge && pl.fold == 1) {
+  if (pl.vec > 1 && width % pl.vec == 0 && es <= 4 && !pl.merge && pl.fold == 1) {
     const int64_t entries = (int64_t)pl.vec * j;  // of a lane
     const bool whole_pieces = entries % 4 == 0 && entries % (16 / es) == 0 && j != 3;  // (Transposed::available)
     const int64_t groups = rows * (int64_t)pl.col_tiles;
@@ -162,13 +166,9 @@ size_t stage1_stream_workspace_bytes(int64_t rows, int64_t n, int64_t k0, int j,
   return need;
 }
 
-bool describe_stage1_stream(const void* x, int64_t rows, int64_t n, int64_t row_stride, int64_t k0, int j,
-                            int layout, int dtype, const void* values, const void* indices, std::string& out) {
-  const int es = elem_bytes(dtype);
-  const int vf = es ? stream::full_vec(es) : 1;
-  const bool aligned = ((uintptr_t)x % 16 == 0) && ((uintptr_t)values % 16 == 0) &&
-                       ((uintptr_t)indices % 16 == 0) && (row_stride % vf == 0);
-  const stream::Plan pl = stream::make_plan(rows, n, k0, j, layout, dtype, aligned);
+bool describe_stage1_stream(const void* x, int64_t rows, int64_t n, int64_t k0, int j, int layout, int dtype,
+                            std::string& out) {
+  const stream::Plan pl = stream::make_plan(rows, n, k0, j, layout, dtype, stream::wide_loads(x, elem_bytes(dtype)));
   if (!pl.ok) return false;
   const int loads = stream::deep_loads_for_short_columns(dtype, j, pl.vec, pl.packed, pl.run, pl.full_rows)
                         ? 8
@@ -186,11 +186,7 @@ bool describe_stage1_stream(const void* x, int64_t rows, int64_t n, int64_t row_
 int launch_stage1_stream(const void* x, int64_t rows, int64_t n, int64_t row_stride, int64_t k0, int j,
                          int layout, int dtype, void* values, IndexOut indices, void* ws,
                          size_t ws_bytes, hipStream_t stream, bool* handled, KeyRangeOut* ranges) {
-  const int es = elem_bytes(dtype);
-  const int vf = es ? stream::full_vec(es) : 1;
-  const bool aligned = ((uintptr_t)x % 16 == 0) && ((uintptr_t)values % 16 == 0) &&
-                       ((uintptr_t)indices.base % 16 == 0) && (row_stride % vf == 0);
-  const stream::Plan pl = stream::make_plan(rows, n, k0, j, layout, dtype, aligned);
+  const stream::Plan pl = stream::make_plan(rows, n, k0, j, layout, dtype, stream::wide_loads(x, elem_bytes(dtype)));
   *handled = pl.ok;
   if (!pl.ok) return ATK_OK;
   if (pl.ws_bytes && (!ws || ws_bytes < pl.ws_bytes || (uintptr_t)ws % 16 != 0)) return ATK_ERR_WORKSPACE;
