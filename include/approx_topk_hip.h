@@ -157,6 +157,17 @@ int atk_topk_i32(const void* x, int64_t rows, int64_t n, int64_t row_stride,
                  void* ws, size_t ws_bytes, atk_stream_t stream);
 
 /*
+ * The gradient of the selected values with respect to the input: grad_x[rows][n]
+ * (dense), zero but for the positions `indices` names, which hold `grad_values`.
+ * `indices` are what atk_topk (atk_stage1 when k == k0) returned for the same
+ * rows, n, k0, j, k and layout, in that order; layouts ATK_INTERLEAVED and
+ * ATK_BALANCED, n < 2^31.  Every element of grad_x is written once.  No counterpart in
+ * the reference, whose operator has no gradient (priority_queue.py:14).
+ */
+int atk_topk_grad(const void* grad_values, const int64_t* indices, int64_t rows, int64_t n, int64_t k0, int j,
+                  int64_t k, int layout, int dtype, void* grad_x, atk_stream_t stream);
+
+/*
  * Diagnostics: which kernels atk_topk (atk_stage1 when k == k0) would enqueue
  * for these arguments, as text ("name<parameters> grid=... block=...", several
  * kernels joined by " + "), truncated to text_bytes - 1 characters.  Enqueues

@@ -51,6 +51,8 @@ _SIGNATURES = {
     "atk_topk_noalloc": (ctypes.c_int, [ctypes.c_void_p] + [ctypes.c_int64] * 4
                          + [ctypes.c_int, ctypes.c_int64, ctypes.c_int, ctypes.c_int]
                          + [ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p]),
+    "atk_topk_grad": (ctypes.c_int, [ctypes.c_void_p, ctypes.c_void_p] + [ctypes.c_int64] * 3
+                      + [ctypes.c_int, ctypes.c_int64, ctypes.c_int, ctypes.c_int, ctypes.c_void_p, ctypes.c_void_p]),
     "atk_topk_i32": (ctypes.c_int, [ctypes.c_void_p] + [ctypes.c_int64] * 4 + [ctypes.c_int, ctypes.c_int64,
                                                                                ctypes.c_int, ctypes.c_int]
                      + [ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_size_t,
@@ -247,6 +249,25 @@ def topk(xs: torch.Tensor, k0: int, j: int, k: int, layout: int, index_dtype: to
     if status != 0:
         check(status)
     return values, indices
+
+
+# Longest row topk_grad takes.
+MAX_GRAD_ROW = (1 << 31) - 1
+
+
+def topk_grad(grad_values: torch.Tensor, indices: torch.Tensor, n: int, k0: int, j: int, layout: int) -> torch.Tensor:
+    """The gradient of a call's values with respect to its input (top-k along the last dim of `n`
+    elements), given the call's indices: zero but for the selected positions."""
+    require_gpu(grad_values)
+    grad_values, indices = grad_values.contiguous(), indices.contiguous()
+    k = indices.shape[-1]
+    grad_x = torch.empty(indices.shape[:-1] + (n,), dtype=grad_values.dtype, device=grad_values.device)
+    with _on_device(grad_values.device):
+        status = lib().atk_topk_grad(grad_values.data_ptr(), indices.data_ptr(), indices.numel() // k, n, k0, j, k,
+                                     layout, dtype_code(grad_values.dtype), grad_x.data_ptr(),
+                                     _stream(grad_values.device))
+    check(status)
+    return grad_x
 
 
 def describe(xs: torch.Tensor, k0: int, j: int, k: int, layout: int = INTERLEAVED,

@@ -8,13 +8,18 @@ opt-in: same arguments, same results, and the values' gradient flows back to
 the input.  The values are a gather of the input at the returned indices, so
 their gradient scatters to those positions and every other position gets zero;
 the indices are distinct along ``dim``, so a plain scatter is exact.
+
+Along the last dim one kernel writes the gradient (``csrc/topk_grad.hip``); zeros
+and a scatter are left to double backward and to the dims the operator takes only
+when every bucket is kept whole.
 """
 from __future__ import annotations
 
 import torch
 from torch import Tensor
 
-from ..priority_queue import topk as _topk
+from .. import _native
+from ..priority_queue import topk as _topk, topk_grad as _topk_grad
 
 
 class _TopkWithGradient(torch.autograd.Function):
@@ -23,17 +28,25 @@ class _TopkWithGradient(torch.autograd.Function):
         values, indices = _topk(xs, k, dim, j, k_mult, interleaved, multithread_buckets)
         ctx.dim = dim if dim >= 0 else dim + xs.ndim
         ctx.shape = xs.shape
+        ctx.buckets = (k * k_mult, j, interleaved)
+        ctx.set_materialize_grads(False)
         ctx.save_for_backward(indices)
         ctx.mark_non_differentiable(indices)
         return values, indices
 
     @staticmethod
     def backward(ctx, grad_values, _grad_indices):
+        if grad_values is None:
+            return None, None, None, None, None, None, None
         (indices,) = ctx.saved_tensors
-        if len(ctx.shape) == 0:
+        shape = ctx.shape
+        if (len(shape) and ctx.dim == len(shape) - 1 and indices.numel() and shape[-1] <= _native.MAX_GRAD_ROW
+                and not (torch.is_grad_enabled() and grad_values.requires_grad)):
+            grad_xs = _topk_grad(grad_values, indices, shape[-1], *ctx.buckets)
+        elif len(shape) == 0:
             grad_xs = grad_values.reshape(()) if indices.numel() else grad_values.new_zeros(())
         else:
-            grad_xs = grad_values.new_zeros(ctx.shape).scatter(ctx.dim, indices, grad_values)
+            grad_xs = grad_values.new_zeros(shape).scatter(ctx.dim, indices, grad_values)
         return grad_xs, None, None, None, None, None, None
 
 

@@ -131,6 +131,32 @@ def _(
 topk = torch.ops.approx_topk.topk.default
 
 
+# The gradient of the values with respect to the input, for
+# ``approx_topk.experimental.differentiable``: an operator of its own so that
+# ``torch.compile`` traces through the wrapper's backward.
+_LIBRARY.define(
+    "topk_grad(Tensor grad_values, Tensor indices, SymInt n, SymInt k0, SymInt j, bool interleaved) -> Tensor",
+    tags=(torch.Tag.pt2_compliant_tag,))
+
+
+def _topk_grad(grad_values: Tensor, indices: Tensor, n: int, k0: int, j: int, interleaved: bool) -> Tensor:
+    """The gradient of a call with top-k along the last dim of ``n`` elements, ``k0`` candidates and
+    ``j`` of them per bucket, whose indices are ``indices``."""
+    return _native.topk_grad(grad_values, indices, n, k0, j,
+                             _native.INTERLEAVED if interleaved else _native.BALANCED)
+
+
+_LIBRARY.impl("topk_grad", _topk_grad, "CompositeExplicitAutograd")
+
+
+@torch.library.register_fake("approx_topk::topk_grad", lib=_LIBRARY)
+def _(grad_values: Tensor, indices: Tensor, n: int, k0: int, j: int, interleaved: bool) -> Tensor:
+    return grad_values.new_empty(indices.shape[:-1] + (n,))
+
+
+topk_grad = torch.ops.approx_topk.topk_grad.default
+
+
 # The reference's ``topk`` is a ``CustomOpDef`` (approx_topk/priority_queue.py:14), whose
 # ``register_fake`` (used at :91) and ``register_autograd`` methods callers may reach for; the
 # overload object carries the same two names, forwarding to ``torch.library``.

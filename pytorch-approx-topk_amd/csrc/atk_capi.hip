@@ -265,6 +265,20 @@ int atk_topk_i32(const void* x, int64_t rows, int64_t n, int64_t row_stride, int
                  ws_bytes, (hipStream_t)stream);
 }
 
+int atk_topk_grad(const void* grad_values, const int64_t* indices, int64_t rows, int64_t n, int64_t k0, int j,
+                  int64_t k, int layout, int dtype, void* grad_x, atk_stream_t stream) {
+  if (layout != ATK_INTERLEAVED && layout != ATK_BALANCED) return ATK_ERR_LAYOUT;
+  if (k < 1 || k > k0) return ATK_ERR_K;
+  const int rc = check_stage1(grad_x, rows, n, n, k0, j, layout, dtype, grad_values, indices);
+  if (rc != ATK_OK || rows == 0) return rc;
+  if (!grad_values) return ATK_ERR_ARG;
+  if (n > 0x7fffffffll) return ATK_ERR_TOO_LARGE;
+  if (const int rca = check_alignment(grad_x, grad_values, dtype, atk::IndexOut{const_cast<int64_t*>(indices), 0}, nullptr);
+      rca != ATK_OK)
+    return rca;
+  return atk::launch_topk_grad(grad_values, indices, rows, n, k0, j, k, layout, dtype, grad_x, (hipStream_t)stream);
+}
+
 int atk_describe(const void* x, int64_t rows, int64_t n, int64_t row_stride, int64_t k0, int j, int64_t k,
                  int layout, int dtype, const void* values, const void* indices, char* text,
                  size_t text_bytes) {

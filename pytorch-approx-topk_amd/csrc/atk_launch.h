@@ -96,6 +96,10 @@ int launch_multi_select(const void* cand_values, const int64_t* cand_indices, in
                         int64_t k, int64_t index_bound, int dtype, void* values, IndexOut indices, void* ws,
                         size_t ws_bytes, hipStream_t stream, bool* handled);
 
+// topk_grad.hip: the gradient of the selected values with respect to the input.
+int launch_topk_grad(const void* grad_values, const int64_t* indices, int64_t rows, int64_t n, int64_t k0, int j,
+                     int64_t k, int layout, int dtype, void* grad_x, hipStream_t stream);
+
 // The kernels each launcher above would enqueue for a call, as text appended to
 // `out` ("name<parameters> grid=... block=..."; several kernels joined by " + ").
 // The describe_* functions that return bool say whether their launcher takes

@@ -1,0 +1,64 @@
+"""The kernel behind the gradient of approx_topk.experimental.differentiable against zeros and a
+scatter in plain torch: bits are moved to distinct positions, so the two are equal."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+# (rows, n, k, j, k_mult): rows of one tile and of one element more; few entries over many tiles;
+# column tiles with every sub-row and with runs of them, all of a bucket's entries kept and
+# found by search; the last column tile, sub-row and run not full
+SHAPES = [
+    (3, 64, 16, 4, 1),
+    (3, 16384, 4096, 2, 1), (2, 16385, 4096, 2, 1), (2, 32769, 2048, 1, 4),
+    (2, 400003, 60, 2, 2), (3, 100003, 1024, 1, 1),
+    (2, 1 << 18, 16384, 2, 1), (2, 300007, 18750, 2, 1), (2, 300007, 4690, 2, 4),
+    (1, 1 << 20, 2048, 1, 1), (1, (1 << 21) + 77, 1540, 4, 1), (1, (1 << 21) + 77, 1540, 4, 2),
+    (1, 1 << 19, 2052, 2, 1),
+]
+
+
+@pytest.mark.parametrize("interleaved", [True, False])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16, torch.float64],
+                         ids=lambda d: str(d).split(".")[-1])
+def test_gradient_kernel_equals_a_scatter(dtype, interleaved):
+    from approx_topk.experimental.differentiable import topk
+    for rows, n, k, j, k_mult in SHAPES:
+        g = torch.Generator(device="cuda").manual_seed(n + k)
+        x = torch.randn(rows, n, generator=g, device="cuda").to(dtype).requires_grad_()
+        values, indices = topk(x, k, -1, j=j, k_mult=k_mult, interleaved=interleaved)
+        w = torch.randn(rows, k, generator=g, device="cuda").to(dtype)
+        (grad,) = torch.autograd.grad(values, x, w)
+        expect = torch.zeros_like(x).scatter(1, indices, w)
+        assert torch.equal(grad, expect), (rows, n, k, j, k_mult)
+
+
+def test_gradient_of_sums_of_views_and_of_unused_values():
+    from approx_topk.experimental.differentiable import topk
+    x = torch.randn(2, 3, 5000, device="cuda", requires_grad=True)
+    values, indices = topk(x, 40, -1, j=2, k_mult=2)
+    (grad,) = torch.autograd.grad(values.sum(), x)   # an expanded gradient
+    assert torch.equal(grad, torch.zeros_like(x).scatter(2, indices, 1.0))
+    values, _ = topk(x, 40, -1)
+    assert torch.autograd.grad(x.sum() + 0 * values.sum(), x)[0].shape == x.shape
+
+
+def test_gradient_of_the_gradient():
+    from approx_topk.experimental.differentiable import topk
+    x = torch.randn(2, 4096, device="cuda", requires_grad=True)
+    values, _ = topk(x, 64, -1, j=2)
+    (grad,) = torch.autograd.grad((values ** 3).sum(), x, create_graph=True)
+    (second,) = torch.autograd.grad(grad.sum(), x)
+    _, indices = topk(x.detach(), 64, -1, j=2)
+    expect = torch.zeros_like(x).scatter(1, indices, 6 * x.detach().gather(1, indices))
+    assert torch.allclose(second, expect, rtol=1e-6, atol=0)   # one rounding of a product each
+
+
+def test_gradient_operator_under_compile():
+    from approx_topk.experimental.differentiable import topk
+    x = torch.randn(3, 4096, device="cuda")
+    _, indices = topk(x, 64, -1, j=2)
+    w = torch.randn(3, 64, device="cuda")
+    op = torch.ops.approx_topk.topk_grad.default
+    torch.library.opcheck(op, (w, indices, 4096, 64, 2, True),
+                          test_utils=("test_schema", "test_faketensor"))
