@@ -2,7 +2,7 @@
 //
 // Reading a bucket front to back with one lane per bucket puts a whole bucket
 // length between the addresses of neighbouring lanes.  Here a workgroup instead
-// copies a span of whole buckets from the row into LDS with coalesced 16-byte
+// (contig_kernel) copies a span of whole buckets from the row into LDS with coalesced 16-byte
 // loads and scans it from there: each of its 256 threads walks one *piece* of a
 // bucket (at most 32 adjacent elements; 16 for 8-byte types) with a J-entry
 // queue in registers, the P = 2^k threads that share a bucket combine their
@@ -60,6 +60,9 @@ struct Geom {
   uint32_t slab_chunks;  // least chunks per slab: slab s takes chunks [s * chunks / slabs, (s + 1) * chunks / slabs)
   uint32_t fast;         // the shape allows scan_even (see there)
   uint32_t whole;        // the shape allows whole_bucket_kernel (see there)
+  uint32_t split;        // the shape allows split_bucket_kernel (see there)
+  uint32_t split_log2;   // split: log2 of the pieces per bucket
+  uint32_t split_trip;   // split: the longest piece (the others hold as many elements or one less)
   uint32_t wide_out;     // the outputs allow 16-byte stores (filled in at launch)
 };
 
@@ -436,6 +439,9 @@ __global__ __launch_bounds__(kThreads) void contig_kernel(const typename E::raw_
 // order keys.  Buckets are numbered row after row: lane t of workgroup w takes
 // bucket w * kThreads + t of the rows * b there are.
 constexpr uint32_t kWholeBucket = 64;
+// Longest piece (bytes) a lane of split_bucket_kernel takes at a time, and longest bucket.
+constexpr uint32_t kSplitBytes = 64;
+constexpr uint32_t kSplitBucket = 64 * 1024;
 
 template <typename E, int J, bool PACKED>
 __global__ __launch_bounds__(kThreads) void whole_bucket_kernel(const typename E::raw_t* __restrict__ x,
@@ -549,6 +555,131 @@ __global__ __launch_bounds__(kThreads) void whole_bucket_kernel(const typename E
   } ATK_STATIC_END;
 }
 
+// Buckets of any length up to kSplitBucket bytes, elements of two or four bytes: a bucket is cut
+// into 2^pieces pieces of at most kSplitBytes, which adjacent lanes take, and in turn when there are more
+// than a wave has lanes.  A lane loads its piece whole (16 bytes a load, all of them issued together;
+// the last one moves down so that it ends with the piece, and what it repeats is left out) and
+// feeds it to a one-column register queue; the lanes of a bucket then put their queues together by
+// shuffles, under the full order.  Pieces start anywhere, nothing goes through LDS and no wave waits for
+// another.  Buckets are numbered row after row, as in whole_bucket_kernel.
+//
+// Bound: HBM.  Against contig_kernel, whose workgroups each copy, wait, scan, wait and write (and of
+// whose loads of one element, in rows off 16 bytes, four or eight make one of these):
+// fp32 [512, 40001] k=1000 j=2 28.6 -> 19.5 us (4.5 TB/s), fp16 23.2 -> 15.6, [128, 300007] with buckets
+// of 6000 elements, j=4 53.4 -> 23.6, fp32 [16, 2000003] of 10000 elements 51.6 -> 26.2.  Pieces of 128 bytes:
+// 22.4 us for the first; a line's second half is asked for long after its first.
+template <typename E, int J, bool PACKED>
+__global__ __launch_bounds__(kThreads) void split_bucket_kernel(const typename E::raw_t* __restrict__ x,
+                                                                typename E::raw_t* __restrict__ values,
+                                                                const IndexOut indices, const Geom g,
+                                                                int64_t buckets) {
+  using raw_t = typename E::raw_t;
+  using M = MergeWord<E>;
+  using word_t = typename M::word_t;
+  using Queue = stream::QueueFor<E, J, 1, PACKED>;
+  constexpr int N = J == 3 ? 4 : J;
+  constexpr int EPL = 16 / (int)sizeof(raw_t);      // elements per load
+  constexpr int kMaxLoads = (int)kSplitBytes / 16;  // loads of a piece
+  static_assert(EPL >= J && EPL % 2 == 0, "the first load of a piece fills its queue");
+  using Load = Pack<raw_t, EPL>;
+
+  const uint32_t lane = threadIdx.x % stream::kWave;
+  const uint32_t lanes_log2 = g.split_log2 < 6 ? g.split_log2 : 6u, lanes = 1u << lanes_log2;  // per bucket
+  const uint32_t turns = 1u << (g.split_log2 - lanes_log2);
+  const int64_t at = ((int64_t)blockIdx.x * kThreads + threadIdx.x) >> lanes_log2;
+  const bool has = at < buckets;
+  const int64_t mine = has ? at : buckets - 1;  // idle lanes go through the last bucket and write nothing
+  const uint32_t share = threadIdx.x & (lanes - 1);
+  int64_t row;
+  uint32_t c;
+  if (buckets <= 0xffffffffll) {
+    const uint32_t row32 = (uint32_t)mine / g.b;
+    row = row32;
+    c = (uint32_t)mine - row32 * g.b;
+  } else {
+    row = mine / g.b;
+    c = (uint32_t)(mine - row * g.b);
+  }
+  const raw_t* xr = x + row * g.row_stride;
+  const uint32_t start = c * g.m + (c < g.r ? c : g.r), len = g.m + (c < g.r ? 1u : 0u);
+  const raw_t* bucket = xr + start;
+  const uint32_t loads = __builtin_amdgcn_readfirstlane((g.split_trip + EPL - 1) / EPL);
+  // piece q of the bucket: its first element; pieces hold split_trip elements or one less, EPL or more
+  auto first_of = [&](uint32_t q) __attribute__((always_inline)) { return (len * q) >> g.split_log2; };
+
+  Queue queue;
+  queue.reset();
+  auto scan_piece = [&](auto first_c, uint32_t q) __attribute__((always_inline)) {
+    constexpr bool kFillsQueue = decltype(first_c)::value;
+    const uint32_t lo = first_of(q);
+    const uint32_t tail = first_of(q + 1) - lo - EPL;  // where the last load starts
+    Load buf[kMaxLoads - 1], last;
+#pragma unroll
+    for (int l = 0; l < kMaxLoads - 1; ++l) {
+      if ((uint32_t)l + 1 < loads) buf[l] = stream::load_pack<raw_t, EPL>(bucket + lo + l * EPL);
+    }
+    last = stream::load_pack<raw_t, EPL>(bucket + lo + tail);
+    auto feed = [&](auto fills_c, const Load& got, uint32_t p) __attribute__((always_inline)) {
+      constexpr bool kFills = decltype(fills_c)::value;
+      ATK_STATIC_FOR(d, EPL / 2) {
+        constexpr int kFilled = (kFills && 2 * d < J) ? 2 * d : J;
+        if constexpr (PACKED) {
+          uint32_t pair;
+          __builtin_memcpy(&pair, &got.e[2 * d], 4);
+          queue.template take_two<0, kFilled>(pair, p + 2 * d);
+        } else {
+          queue.template take_two<0, kFilled>(got.e[2 * d], got.e[2 * d + 1], p + 2 * d);
+        }
+      } ATK_STATIC_END;
+    };
+    using Fills = std::integral_constant<bool, kFillsQueue>;
+    if (loads == 1) {  // (every piece is one load then)
+      feed(Fills{}, last, lo);
+      return;
+    }
+    feed(Fills{}, buf[0], lo);
+#pragma unroll
+    for (int l = 1; l < kMaxLoads - 1; ++l) {
+      if ((uint32_t)l + 1 < loads) feed(std::false_type{}, buf[l], lo + l * EPL);
+    }
+    const uint32_t fed = (loads - 1) * EPL;
+    ATK_STATIC_FOR(e, EPL) {
+      queue.template take_one<0>(last.e[e], lo + tail + e, tail + e >= fed);
+    } ATK_STATIC_END;
+  };
+  scan_piece(std::true_type{}, share);
+#pragma nounroll
+  for (uint32_t turn = 1; turn < turns; ++turn) scan_piece(std::false_type{}, turn * lanes + share);
+
+  word_t acc[N], in[N];
+  ATK_STATIC_FOR(sl, N) { acc[sl] = M::empty(); in[sl] = M::empty(); } ATK_STATIC_END;
+  if (queue.poisoned()) {  // (wave-uniform) a NaN: the pieces again, with order keys
+    raw_t qv[J];
+    uint32_t qp[J];
+    stream::clear_exact<E, J>(qv, qp);
+    for (uint32_t turn = 0; turn < turns; ++turn) {
+      const uint32_t q = turn * lanes + share, end = first_of(q + 1);
+      for (uint32_t p = first_of(q); p < end; ++p) stream::push_exact<E, J>(qv, qp, bucket[p], p);
+    }
+    ATK_STATIC_FOR(sl, J) { acc[N - J + sl] = M::make(qv[sl], qp[sl]); } ATK_STATIC_END;
+  } else {
+    ATK_STATIC_FOR(sl, J) {
+      acc[N - J + sl] = M::from_key(queue.template key<0, sl>(), queue.template position<0, sl>());
+    } ATK_STATIC_END;
+  }
+  for (uint32_t half = lanes / 2; half >= 1; half /= 2) {
+    ATK_STATIC_FOR(sl, N) { in[sl] = M::from_lane(acc[sl], (int)(lane + half)); } ATK_STATIC_END;
+    stream::merge_best<M, N>(acc, in);  // meaningful in the lanes with share < half, which are the ones read next
+  }
+  if (!has || share != 0) return;
+  const int64_t o = (row * g.b + c) * J;
+  ATK_STATIC_FOR(sl, J) {  // (adjacent stores: the compiler makes wide ones of them)
+    const uint32_t p = start + M::pos(acc[N - J + sl]);
+    if (values != nullptr) values[o + sl] = stream::element_of<E>(acc[N - J + sl], xr, p);
+    indices.put(o + sl, p);
+  } ATK_STATIC_END;
+}
+
 // Combines the `slabs` partial results of every bucket: one wave per bucket,
 // lane l folding slabs l, l + 64, ..., then pairwise by lane shuffles.
 template <typename E, int J>
@@ -595,8 +726,14 @@ struct Plan {
   size_t ws_bytes;   // workspace for the slabs' partial results
 };
 
-// `aligned`: base pointer and row stride allow 16-byte loads.
-Plan make_plan(int64_t rows, int64_t n, int64_t k0, int j, int layout, int dtype, bool aligned);
+// Workgroups of whole_bucket_kernel or split_bucket_kernel.
+inline int64_t bucket_groups(const Geom& g, int64_t rows) {
+  const uint32_t lanes_log2 = g.whole != 0 ? 0u : (g.split_log2 < 6 ? g.split_log2 : 6u);
+  return (((rows * (int64_t)g.b) << lanes_log2) + kThreads - 1) / kThreads;
+}
+
+// `aligned`: every row starts on 16 bytes; `wide`: 16-byte loads may be used (stream::wide_loads).
+Plan make_plan(int64_t rows, int64_t n, int64_t k0, int j, int layout, int dtype, bool aligned, bool wide);
 
 template <typename E>
 int launch_typed(const Plan& pl, const void* x, int64_t rows, int64_t row_stride, int j, void* values,

@@ -24,15 +24,15 @@ template <typename E, int J>
 static int launch_j(const Plan& pl, const Geom& g, const typename E::raw_t* x, int64_t rows,
                     typename E::raw_t* values, IndexOut indices, void* ws, hipStream_t stream) {
   constexpr int VF = stream::full_vec((int)sizeof(typename E::raw_t));
-  if (g.whole != 0) {
+  if (g.whole != 0 || g.split != 0) {
     constexpr int ES = (int)sizeof(typename E::raw_t);
     if constexpr (ES == 2 || ES == 4) {
       const int64_t buckets = rows * (int64_t)g.b;
-      const int64_t groups = (buckets + kThreads - 1) / kThreads;
+      const int64_t groups = bucket_groups(g, rows);
       if (groups > 0x7fffffffll) return ATK_ERR_TOO_LARGE;
       constexpr bool kPacked = ES == 2 && stream::PackedKey<E>::available;
-      hipLaunchKernelGGL((whole_bucket_kernel<E, J, kPacked>), dim3((unsigned)groups), dim3(kThreads), 0, stream, x,
-                         values, indices, g, buckets);
+      auto kern = g.whole != 0 ? whole_bucket_kernel<E, J, kPacked> : split_bucket_kernel<E, J, kPacked>;
+      hipLaunchKernelGGL(kern, dim3((unsigned)groups), dim3(kThreads), 0, stream, x, values, indices, g, buckets);
       return hipGetLastError() == hipSuccess ? ATK_OK : ATK_ERR_LAUNCH;
     } else {
       return ATK_ERR_ARG;  // the planner never asks for it

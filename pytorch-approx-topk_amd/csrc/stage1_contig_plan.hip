@@ -7,9 +7,13 @@ namespace contig {
 namespace {
 // Workgroups wanted in the grid before long buckets are left whole.
 constexpr int64_t kTargetGroups = 1024;
+// split_bucket_kernel: buckets of a launch from which on a wave may take more than kFewTurns turns
+// at its bucket, and from which on buckets shorter than one piece go there.
+constexpr int64_t kManyWaves = 512, kFewTurns = 8, kManyBuckets = 16384;
 }  // namespace
 
-Plan make_plan(int64_t rows, int64_t n, int64_t k0, int j, int layout, int dtype, bool aligned) {
+Plan make_plan(int64_t rows, int64_t n, int64_t k0, int j, int layout, int dtype, bool aligned,
+               bool wide) {
   Plan pl{};
   pl.ok = false;
   if (layout != ATK_BALANCED && layout != ATK_CEIL_CHUNK) return pl;
@@ -63,7 +67,10 @@ Plan make_plan(int64_t rows, int64_t n, int64_t k0, int j, int layout, int dtype
   }
   if (rows * (int64_t)g.groups > 0x7fffffffll) return pl;
 
-  pl.vec = aligned ? stream::full_vec(es) : 1;
+  // 16-byte loads in rows off 16 bytes: they pay for elements of four bytes and more (fp32 [16, 2000003] with
+  // buckets of 40 KB 51.6 -> 48.0 us; fp16 41.2 -> 43.3, and [512, 100003] k=50000 j=4 115 -> 155, where
+  // the eight elements of a load are parked in LDS a word at a time)
+  pl.vec = aligned || (wide && es >= 4) ? stream::full_vec(es) : 1;
   // LDS: the longest span (whole packs, one element of slack) with its padding, or the queues
   const int64_t span = (g.chunks > 1 ? kThreads * piece : per_group * longest) + 2 * pl.vec + 2;
   const size_t data_bytes = (size_t)(span + ((span >> 5) + 1) * pad_elems(es)) * es;
@@ -91,6 +98,30 @@ Plan make_plan(int64_t rows, int64_t n, int64_t k0, int j, int layout, int dtype
     pl.ws_bytes = 0;
     pl.lds_bytes = 0;
   }
+  // split_bucket_kernel: adjacent lanes share a bucket, no LDS.  (A padded row's last bucket may
+  // reach past the row: not here.)  contig_kernel keeps:
+  //   the even shapes, whose packs it copies and scans whole (fp32 [128, 2^20] with buckets of 256 bytes
+  //   99 against 111 us, fp16 of 512 bytes 84 against 90);
+  //   buckets of which more than a quarter is kept, three or four elements each (fp32 [256, 100003] k=50000 j=4
+  //   68.6 against 76.2 us; with j=2 and buckets of 16 bytes 64.4 against 46.5);
+  //   few buckets that a wave would need many turns for (200 of 40 KB in one row 11.9 against 13.4 us, but 800 in
+  //   four rows 17.3 against 13.9);
+  //   small launches of short buckets, which take the same either way (fp32 [64, 8200] k=1024 j=2 11.7 against 11.5).
+  g.split = 0;
+  if (wide && (es == 2 || es == 4) && !g.whole && !g.fast && (layout == ATK_BALANCED || b * m == n) &&
+      longest * es <= (int64_t)kSplitBucket && (j <= 2 || m >= 4 * j) &&
+      (m * es >= (int64_t)kSplitBytes || rows * b >= kManyBuckets)) {
+    uint32_t pieces_log2 = 0;
+    while (((longest + (1ll << pieces_log2) - 1) >> pieces_log2) * es > (int64_t)kSplitBytes) ++pieces_log2;
+    if ((m >> pieces_log2) * es >= 16 && ((1 << pieces_log2) <= kFewTurns * stream::kWave || rows * b >= kManyWaves)) {
+      g.split = 1;
+      g.split_log2 = pieces_log2;
+      g.split_trip = (uint32_t)((longest + (1ll << pieces_log2) - 1) >> pieces_log2);
+      g.slabs = 1;
+      pl.ws_bytes = 0;
+      pl.lds_bytes = 0;
+    }
+  }
   if (pl.lds_bytes > 64 * 1024) return pl;
   pl.ok = true;
   return pl;
@@ -98,9 +129,18 @@ Plan make_plan(int64_t rows, int64_t n, int64_t k0, int j, int layout, int dtype
 
 }  // namespace contig
 
+namespace {
+contig::Plan plan_for(const void* x, int64_t rows, int64_t n, int64_t row_stride, int64_t k0, int j, int layout,
+                      int dtype) {
+  const int es = elem_bytes(dtype);
+  const bool aligned = (uintptr_t)x % 16 == 0 && row_stride % (es ? stream::full_vec(es) : 1) == 0;
+  return contig::make_plan(rows, n, k0, j, layout, dtype, aligned, stream::wide_loads(x, es));
+}
+}  // namespace
+
 size_t stage1_contig_workspace_bytes(int64_t rows, int64_t n, int64_t k0, int j, int layout, int dtype) {
-  const contig::Plan a = contig::make_plan(rows, n, k0, j, layout, dtype, true);
-  const contig::Plan u = contig::make_plan(rows, n, k0, j, layout, dtype, false);
+  const contig::Plan a = contig::make_plan(rows, n, k0, j, layout, dtype, true, true);
+  const contig::Plan u = contig::make_plan(rows, n, k0, j, layout, dtype, false, false);
   size_t need = 0;
   if (a.ok && a.ws_bytes > need) need = a.ws_bytes;
   if (u.ok && u.ws_bytes > need) need = u.ws_bytes;
@@ -109,14 +149,17 @@ size_t stage1_contig_workspace_bytes(int64_t rows, int64_t n, int64_t k0, int j,
 
 bool describe_stage1_contig(const void* x, int64_t rows, int64_t n, int64_t row_stride, int64_t k0, int j,
                             int layout, int dtype, std::string& out) {
-  const int es = elem_bytes(dtype);
-  const int vf = es ? stream::full_vec(es) : 1;
-  const bool aligned = ((uintptr_t)x % 16 == 0) && (row_stride % vf == 0);
-  const contig::Plan pl = contig::make_plan(rows, n, k0, j, layout, dtype, aligned);
+  const contig::Plan pl = plan_for(x, rows, n, row_stride, k0, j, layout, dtype);
   if (!pl.ok) return false;
   if (pl.geom.whole) {
     out += "whole_bucket_kernel<" + std::string(dtype_name(dtype)) + ", J=" + std::to_string(j) + "> grid=" +
-           std::to_string((rows * (int64_t)pl.geom.b + contig::kThreads - 1) / contig::kThreads) + " block=256";
+           std::to_string(contig::bucket_groups(pl.geom, rows)) + " block=256";
+    return true;
+  }
+  if (pl.geom.split) {
+    out += "split_bucket_kernel<" + std::string(dtype_name(dtype)) + ", J=" + std::to_string(j) + "> grid=" +
+           std::to_string(contig::bucket_groups(pl.geom, rows)) + " block=256 pieces=" +
+           std::to_string(1 << pl.geom.split_log2);
     return true;
   }
   out += "contig_kernel<" + std::string(dtype_name(dtype)) + ", J=" + std::to_string(j) + ", V=" +
@@ -130,10 +173,7 @@ bool describe_stage1_contig(const void* x, int64_t rows, int64_t n, int64_t row_
 int launch_stage1_contig(const void* x, int64_t rows, int64_t n, int64_t row_stride, int64_t k0, int j,
                          int layout, int dtype, void* values, IndexOut indices, void* ws, size_t ws_bytes,
                          hipStream_t stream, bool* handled) {
-  const int es = elem_bytes(dtype);
-  const int vf = es ? stream::full_vec(es) : 1;
-  const bool aligned = ((uintptr_t)x % 16 == 0) && (row_stride % vf == 0);
-  const contig::Plan pl = contig::make_plan(rows, n, k0, j, layout, dtype, aligned);
+  const contig::Plan pl = plan_for(x, rows, n, row_stride, k0, j, layout, dtype);
   *handled = pl.ok;
   if (!pl.ok) return ATK_OK;
   if (pl.ws_bytes && (!ws || ws_bytes < pl.ws_bytes || (uintptr_t)ws % 16 != 0)) return ATK_ERR_WORKSPACE;
