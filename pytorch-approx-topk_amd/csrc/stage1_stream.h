@@ -1106,8 +1106,15 @@ __device__ __forceinline__ void scan_partial_sub_row(const typename E::raw_t* __
 // `with_rem`.  `xr` is the row; lanes that are not `live` load column 0 and are
 // ignored by the caller.  RUN > 0 promises p1 - p0 == RUN (J <= RUN): all loads
 // are issued at once and the code is one straight line.  RUN == 0 takes any
-// length: the first J sub-rows, then the rest as scan_rest does.
-template <typename E, int J, int V, int U, int RUN, typename Queue>
+// length: the first J sub-rows, then the rest as scan_rest does.  AHEAD (kernels of
+// short columns, see deep_loads_for_short_columns, in launches of thousands of workgroups):
+// those J, the odd batch and the first whole one are all issued before the first of them is used.  A
+// run of a few dozen sub-rows at most waits for memory three times otherwise: bf16 [256, 2^20]
+// k=65536 j=4 134.6 -> 128.4 us, [200, 500000] k=20000 j=2 54.8 -> 52.6, fp16 [16, 2^22] k=2^18 j=4
+// 40.4 -> 37.5.  It costs registers (fp32 j=2 82 -> 106), for which longer columns and smaller launches get
+// nothing: fp16 [128, 65536] k=2048 j=4 10.7 -> 11.4 us, [500, 20000] k=1600 j=4 11.2 -> 11.8, fp32
+// [1, 2^23] k=4096 j=2 k_mult=2 24.7 -> 27.0.
+template <typename E, int J, int V, int U, int RUN, bool AHEAD = false, typename Queue>
 __device__ __forceinline__ void scan_run(const typename E::raw_t* __restrict__ xr, const Geom& g, int64_t col,
                                 bool live, uint32_t p0, uint32_t p1, bool with_rem, Queue& queue) {
   using raw_t = typename E::raw_t;
@@ -1126,6 +1133,40 @@ __device__ __forceinline__ void scan_run(const typename E::raw_t* __restrict__ x
 #pragma unroll
     for (int u = 0; u < RUN; ++u) buf[u] = load_next();
     ATK_STATIC_FOR(u, RUN) { queue.template take<(u < J ? u : J)>(buf[u], p0 + u); } ATK_STATIC_END;
+  } else if constexpr (AHEAD) {
+    uint32_t p = p0 + J;
+    const uint32_t odd = (p1 - p) % U;
+    uint32_t batches = (p1 - p) / U;
+    Pack<raw_t, V> first[J], rest[U - 1], buf[U];
+#pragma unroll
+    for (int u = 0; u < J; ++u) first[u] = load_next();
+#pragma unroll
+    for (int u = 0; u < U - 1; ++u) {
+      if ((uint32_t)u < odd) rest[u] = load_next();
+    }
+    if (batches != 0) {
+#pragma unroll
+      for (int u = 0; u < U; ++u) buf[u] = load_next();
+    }
+    ATK_STATIC_FOR(u, J) { queue.template take<u>(first[u], p0 + u); } ATK_STATIC_END;
+#pragma unroll
+    for (int u = 0; u < U - 1; ++u) {
+      if ((uint32_t)u < odd) queue.template take<J>(rest[u], p + u);
+    }
+    p += odd;
+    if (batches != 0) {
+      for (; batches > 1; --batches) {
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+          const Pack<raw_t, V> cur = buf[u];
+          buf[u] = load_next();
+          queue.template take<J>(cur, p + u);
+        }
+        p += U;
+      }
+#pragma unroll
+      for (int u = 0; u < U; ++u) queue.template take<J>(buf[u], p + u);
+    }
   } else {
     {  // the first J sub-rows fill the queues
       Pack<raw_t, V> buf[J];
@@ -1450,7 +1491,9 @@ __global__ __launch_bounds__(kWave * W) __attribute__((amdgpu_waves_per_eu(4))) 
   const raw_t* xr = x + row * g.row_stride;
   Queue queue;
   ATK_TRACE_WAVE((int)wave * 2);  // slots 2w, 2w + 1: wave w's scan; 16: the workgroup's end
-  scan_run<E, J, V, U, RUN>(xr, g, col, live, p0, p1, last_slab && wave == W - 1, queue);
+  constexpr bool kAhead = WAVE_STORES && U == 8 &&
+                          deep_loads_for_short_columns(DtypeOf<E>::value, J, V, PACKED, RUN, 0);
+  scan_run<E, J, V, U, RUN, kAhead>(xr, g, col, live, p0, p1, last_slab && wave == W - 1, queue);
   ATK_TRACE_WAVE((int)wave * 2 + 1);
 
   bool redo = queue.poisoned();
