@@ -91,10 +91,10 @@ TopkPlan plan_topk(int64_t rows, int64_t n, int64_t k0, int j, int64_t k, int la
 // general kernel.
 int run_stage1(const void* x, int64_t rows, int64_t n, int64_t row_stride, int64_t k0, int j,
                int layout, int dtype, void* values, atk::IndexOut indices, void* ws, size_t ws_bytes,
-               hipStream_t stream, atk::KeyRangeOut* ranges = nullptr) {
+               hipStream_t stream, atk::KeyRangeOut* ranges = nullptr, atk::SelectOut* last = nullptr) {
   bool handled = false;
   const int rc = atk::launch_stage1_stream(x, rows, n, row_stride, k0, j, layout, dtype, values,
-                                           indices, ws, ws_bytes, stream, &handled, ranges);
+                                           indices, ws, ws_bytes, stream, &handled, ranges, last);
   if (handled || rc != ATK_OK) return rc;
   const int rc2 = atk::launch_stage1_contig(x, rows, n, row_stride, k0, j, layout, dtype, values, indices,
                                             ws, ws_bytes, stream, &handled);
@@ -161,10 +161,13 @@ int do_topk(const void* x, int64_t rows, int64_t n, int64_t row_stride, int64_t 
   // a chained select can take the key ranges of the candidates from stage 1's last kernel
   atk::KeyRangeOut ranges = atk::chain_select_ranges(rows, k0, k, index_bound_of(n, k0, layout), dtype,
                                                       base + p.select_off, p.select_bytes);
+  // rows cut into slabs may leave their merge with the second stage done
+  atk::SelectOut last{k, index_bound_of(n, k0, layout), 1, values, indices, false, false};
+  while (last.index_bits < 63 && (1ll << last.index_bits) < last.index_bound) ++last.index_bits;
   // the candidates keep int64 indices whatever the output's width
   const int rc1 = run_stage1(x, rows, n, row_stride, k0, j, layout, dtype, cand_values,
-                             atk::IndexOut{cand_indices, 0}, base + p.stage1_off, p.stage1_bytes, stream, &ranges);
-  if (rc1 != ATK_OK) return rc1;
+                             atk::IndexOut{cand_indices, 0}, base + p.stage1_off, p.stage1_bytes, stream, &ranges, &last);
+  if (rc1 != ATK_OK || last.done) return rc1;
   return run_select(cand_values, cand_indices, rows, k0, k, index_bound_of(n, k0, layout), dtype, values,
                     indices, base + p.select_off, p.select_bytes, stream, ranges.entries, ranges.hist_done != 0);
 }
@@ -291,10 +294,12 @@ int atk_describe(const void* x, int64_t rows, int64_t n, int64_t row_stride, int
     bool fused = false;
     if (k < k0) fused = atk::describe_fused_row(x, rows, n, k0, j, k, layout, dtype, out);
     if (!fused) {
-      if (!atk::describe_stage1_stream(x, rows, n, k0, j, layout, dtype, out) &&
+      bool selected = false;
+      if (!atk::describe_stage1_stream(x, rows, n, k0, j, k, layout, dtype, index_bound_of(n, k0, layout), &selected,
+                                       out) &&
           !atk::describe_stage1_contig(x, rows, n, row_stride, k0, j, layout, dtype, out))
         atk::describe_stage1_lane_per_bucket(rows, k0, j, dtype, out);
-      if (k < k0) {
+      if (k < k0 && !selected) {
         out += " + ";
         if (!atk::describe_chain_select(rows, k0, k, index_bound_of(n, k0, layout), dtype, out) &&
             !atk::describe_multi_select(rows, k0, k, index_bound_of(n, k0, layout), dtype, out))

@@ -39,13 +39,24 @@ struct KeyRangeOut {
   uint32_t hist_done;
 };
 
+// Where the second stage's results go, for a stage-1 launcher whose last kernel may take that
+// stage along: it sets `wanted` (the call's plan does) and `done` (the results are written).
+struct SelectOut {
+  int64_t k, index_bound;
+  int index_bits;           // of index_bound
+  void* values;             // (may be NULL)
+  IndexOut indices;
+  bool wanted, done;
+};
+
 // stage1_stream_plan.hip: interleaved layouts with at least j full sub-rows.
 // `*handled` tells whether the shape was accepted; if not, nothing was enqueued.
 size_t stage1_stream_workspace_bytes(int64_t rows, int64_t n, int64_t k0, int j, int layout,
                                      int dtype);
 int launch_stage1_stream(const void* x, int64_t rows, int64_t n, int64_t row_stride, int64_t k0,
                          int j, int layout, int dtype, void* values, IndexOut indices, void* ws,
-                         size_t ws_bytes, hipStream_t stream, bool* handled, KeyRangeOut* ranges = nullptr);
+                         size_t ws_bytes, hipStream_t stream, bool* handled, KeyRangeOut* ranges = nullptr,
+                         SelectOut* last = nullptr);
 
 // stage1_contig_plan.hip: the contiguous layouts, through LDS.  `*handled` as above.
 size_t stage1_contig_workspace_bytes(int64_t rows, int64_t n, int64_t k0, int j, int layout, int dtype);
@@ -105,8 +116,9 @@ int launch_topk_grad(const void* grad_values, const int64_t* indices, int64_t ro
 // The describe_* functions that return bool say whether their launcher takes
 // the call; they enqueue nothing.
 const char* dtype_name(int dtype);
-bool describe_stage1_stream(const void* x, int64_t rows, int64_t n, int64_t k0, int j, int layout, int dtype,
-                            std::string& out);
+// `*selected`: the second stage is among the kernels named.
+bool describe_stage1_stream(const void* x, int64_t rows, int64_t n, int64_t k0, int j, int64_t k, int layout,
+                            int dtype, int64_t index_bound, bool* selected, std::string& out);
 bool describe_stage1_contig(const void* x, int64_t rows, int64_t n, int64_t row_stride, int64_t k0, int j,
                             int layout, int dtype, std::string& out);
 void describe_stage1_lane_per_bucket(int64_t rows, int64_t k0, int j, int dtype, std::string& out);

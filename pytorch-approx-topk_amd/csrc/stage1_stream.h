@@ -1667,6 +1667,130 @@ __global__ __launch_bounds__(kMergeThreads) void stream_merge_kernel(
   }
 }
 
+// The same merge and the second stage behind it, for rows of few candidates: one workgroup
+// folds the partial queues of all of its row's buckets, parks the candidates in LDS as words of
+// key and inverted index, and writes the k best in candidate order.  Up to kRankMax
+// candidates are ranked by counting the better words (all of them are different), more go
+// through the block-wide radix select.
+//
+// Bound: latency, of two launches as of one: merging and selecting took 4.6 and 4.8 us behind a
+// launch each, whatever the candidates, and a row's partial queues are a few ten KB.
+// In one launch: fp32 [16, 2653751] k=10 j=2 k_mult=4 41.3 -> 36.9 us per call, [4, 2^20] 17.7 -> 14.6,
+// [64, 2^20] k=64 j=4 k_mult=2 62.6 -> 58.2, [1, 2^24] k=10 31.2 -> 26.9.
+constexpr uint32_t kRankMax = 256;
+
+template <typename E, int J>
+__global__ __launch_bounds__(1024) void stream_merge_select_kernel(
+    const typename E::raw_t* __restrict__ x, int64_t row_stride,
+    const typename E::raw_t* __restrict__ part_values, const uint32_t* __restrict__ part_pos, uint32_t b,
+    uint32_t slabs, uint32_t cb, uint32_t k, int index_bits, typename E::raw_t* __restrict__ values,
+    const IndexOut indices) {
+  using M = MergeWord<E>;
+  using word_t = typename M::word_t;
+  using key_t = typename E::key_t;
+  static_assert(std::is_same<word_t, uint64_t>::value, "keys of at most 32 bits");
+  constexpr int N = J == 3 ? 4 : J;
+  extern __shared__ __align__(16) unsigned char dyn_lds[];
+  __shared__ select::SharedT<2> sh;
+  const uint32_t t = threadIdx.x, nt = blockDim.x, lane = t % kWave;
+  const uint32_t wave = __builtin_amdgcn_readfirstlane(t / kWave);
+  const int64_t row = blockIdx.x;
+  const typename E::raw_t* xr = x + row * row_stride;
+  const uint32_t k0 = b * J;
+  uint64_t* cand = reinterpret_cast<uint64_t*>(dyn_lds);  // [k0, rounded up to even]
+  word_t* lists = cand + ((k0 + 1) & ~1u);                // [N][nt]
+
+  // cb buckets at a time, nt / cb threads each: first lists are put together within a wave, then
+  // one list per wave (or per share of whole waves) by the bucket's first thread
+  const uint32_t share = t / cb, shares = nt / cb;
+  const uint32_t per_wave = cb < (uint32_t)kWave ? kWave / cb : 1u;
+  for (uint32_t c0 = 0; c0 < b; c0 += cb) {
+    const uint32_t c = c0 + t % cb;
+    word_t acc[N], in[N];
+    ATK_STATIC_FOR(s, N) { acc[s] = M::empty(); in[s] = M::empty(); } ATK_STATIC_END;
+    if (c < b) {
+      constexpr int kBatch = 4;  // slabs per round, their loads issued together
+      for (uint32_t slab0 = share; slab0 < slabs; slab0 += shares * kBatch) {
+        typename E::raw_t got[kBatch][J];
+        uint32_t at[kBatch][J];
+        bool real[kBatch];
+        ATK_STATIC_FOR(u, kBatch) {
+          const uint32_t slab = slab0 + u * shares;
+          real[u] = slab < slabs;
+          const int64_t o = ((row * slabs + (real[u] ? slab : share)) * b + c) * J;  // a slab that exists
+          ATK_STATIC_FOR(s, J) { got[u][s] = part_values[o + s]; at[u][s] = part_pos[o + s]; } ATK_STATIC_END;
+        } ATK_STATIC_END;
+        ATK_STATIC_FOR(u, kBatch) {
+          if (real[u]) {
+            ATK_STATIC_FOR(s, J) { in[N - J + s] = M::make(got[u][s], at[u][s]); } ATK_STATIC_END;
+            merge_best<M, N>(acc, in);
+          }
+        } ATK_STATIC_END;
+      }
+    }
+    for (uint32_t half = per_wave / 2; half >= 1; half /= 2) {
+      ATK_STATIC_FOR(s, N) { in[s] = M::from_lane(acc[s], (int)(lane + half * cb)); } ATK_STATIC_END;
+      merge_best<M, N>(acc, in);  // meaningful in the lanes whose share within the wave is < half
+    }
+    const uint32_t groups = shares / per_wave;  // lists per bucket that are left
+    if (groups > 1) {
+      // (only when all buckets are covered at once: cb < nt)
+      ATK_STATIC_FOR(s, N) { lists[s * nt + t] = acc[s]; } ATK_STATIC_END;
+      __syncthreads();
+    }
+    if (t < cb && c < b) {
+      for (uint32_t g = 1; g < groups; ++g) {
+        ATK_STATIC_FOR(s, N) { in[s] = lists[s * nt + t + g * per_wave * cb]; } ATK_STATIC_END;
+        merge_best<M, N>(acc, in);
+      }
+      ATK_STATIC_FOR(s, J) {
+        const uint32_t index = c + M::pos(acc[N - J + s]) * b;
+        cand[c * J + s] = ((uint64_t)M::key(acc[N - J + s]) << 32) | (uint32_t)~index;
+      } ATK_STATIC_END;
+    }
+  }
+  if (t == 0 && k0 % 2 != 0) cand[k0] = 0;  // below every candidate
+  __syncthreads();
+
+  auto index_at = [&](uint32_t i) -> uint64_t { return (uint64_t)(~(uint32_t)cand[i]); };
+  auto write = [&](uint32_t i, uint32_t o) __attribute__((always_inline)) {
+    const key_t key = (key_t)(cand[i] >> 32);
+    const int64_t index = (int64_t)index_at(i);
+    if (values != nullptr) {
+      typename E::raw_t value = E::unkey(key);
+      if (!E::key_is_exact(key)) value = xr[index];
+      values[row * k + o] = value;
+    }
+    indices.put(row * k + o, index);
+  };
+  if (k0 <= kRankMax) {  // a candidate per thread
+    const uint64_t mine = t < k0 ? cand[t] : 0;
+    uint32_t better = 0;
+    for (uint32_t i = 0; i < k0; i += 2) {
+      const ulonglong2 two = *reinterpret_cast<const ulonglong2*>(&cand[i]);
+      better += (two.x > mine ? 1u : 0u) + (two.y > mine ? 1u : 0u);
+    }
+    const bool kept = t < k0 && better < k;
+    const uint64_t mask = __ballot(kept);
+    if (lane == 0) sh.wave_total[wave] = (uint32_t)__popcll(mask);
+    __syncthreads();
+    uint32_t o = select::rank_in(mask);
+    for (uint32_t w = 0; w < wave; ++w) o += sh.wave_total[w];
+    if (kept) write(t, o);
+    return;
+  }
+  auto key_at = [&](uint32_t i) -> key_t { return (key_t)(cand[i] >> 32); };
+  const select::Cut<key_t> cut = select::find_cut<key_t, E::key_bits>(sh, k0, k, index_bits, key_at, index_at);
+  auto survives = [&](uint32_t i) -> bool {
+    const key_t key = key_at(i);
+    if (key != cut.T) return key > cut.T;
+    return cut.index_cut == ~0ull || index_at(i) <= cut.index_cut;
+  };
+  select::compact(
+      sh, k0, k, survives, [](uint32_t i) { return i; },
+      [&](uint32_t, uint32_t o, uint32_t i) { write(i, o); });
+}
+
 // ---------------------------------------------------------------------------
 // Host side: the plan (pure arithmetic, shared with the workspace query) and
 // the launch.
@@ -1698,9 +1822,13 @@ inline bool wide_loads(const void* x, int es) { return es >= 4 || (uintptr_t)x %
 
 // One instance per element type, each in its own translation unit.
 // `ranges`: see KeyRangeOut; may be nullptr.
+// `last`: see SelectOut; may be nullptr.
 template <typename E>
 int launch_typed(const Plan& pl, const void* x, int64_t rows, int64_t row_stride, int j, void* values,
-                 IndexOut indices, void* ws, hipStream_t stream, KeyRangeOut* ranges);
+                 IndexOut indices, void* ws, hipStream_t stream, KeyRangeOut* ranges, SelectOut* last);
+
+// Whether the merge of a row cut into slabs takes the second stage along (stream_merge_select_kernel).
+bool selects_in_merge(const Plan& pl, int64_t k0, int64_t index_bound, int dtype);
 
 }  // namespace stream
 }  // namespace atk

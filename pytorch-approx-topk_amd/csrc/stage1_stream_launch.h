@@ -83,7 +83,7 @@ static int launch_w(const Plan& pl, const typename E::raw_t* x, const Sink<typen
 
 template <typename E, int J>
 static int launch_j(const Plan& pl, const typename E::raw_t* x, const Sink<typename E::raw_t>& out,
-                    const Geom& g, int64_t rows, hipStream_t stream, KeyRangeOut* ranges) {
+                    const Geom& g, int64_t rows, hipStream_t stream, KeyRangeOut* ranges, SelectOut* last) {
   using raw_t = typename E::raw_t;
   constexpr int VF = full_vec((int)sizeof(raw_t));
   // Kernels that end in the merge of slabs can leave a chained select its key
@@ -103,6 +103,29 @@ static int launch_j(const Plan& pl, const typename E::raw_t* x, const Sink<typen
                             : launch_w<E, J, 1>(pl, x, out, g, rows, stream, left);
   if (rc != ATK_OK || !pl.merge) return rc;
   const int64_t b = pl.width / pl.fold;  // buckets
+  if constexpr (E::key_bits <= 32) {
+    if (last != nullptr && last->wanted) {
+      const uint32_t k0 = (uint32_t)b * J;
+      // threads: those that rank, or as many as there are when a bucket's partial queues would go
+      // through too few of them (fp16 [1, 2^22] k=50 j=1 k_mult=4 21.5 -> 30.9 us with one thread per bucket)
+      auto buckets_at_once = [&](uint32_t threads) {
+        uint32_t at_once = threads;
+        while (at_once > 1 && (int64_t)(at_once / 2) >= b) at_once /= 2;
+        return at_once;
+      };
+      uint32_t nt = kRankMax;
+      if (k0 > kRankMax || pl.slabs > 8 * (nt / buckets_at_once(nt))) nt = 1024;
+      const uint32_t cb = buckets_at_once(nt);
+      constexpr int N = J == 3 ? 4 : J;
+      const size_t lds = (((size_t)k0 + 1) / 2 * 2 + (size_t)N * nt) * sizeof(uint64_t);
+      hipLaunchKernelGGL((stream_merge_select_kernel<E, J>), dim3((unsigned)rows), dim3(nt), lds, stream, x,
+                         g.row_stride, (const raw_t*)out.part_values, (const uint32_t*)out.part_pos, (uint32_t)b,
+                         pl.slabs, cb, (uint32_t)last->k, last->index_bits, static_cast<raw_t*>(last->values),
+                         last->indices);
+      last->done = true;
+      return hipGetLastError() == hipSuccess ? ATK_OK : ATK_ERR_LAUNCH;
+    }
+  }
   // buckets per workgroup: a power of two, no more than there are, and few
   // enough that a thread folds at most about 32 of a bucket's partial queues
   uint32_t cb = kWave;
@@ -118,7 +141,7 @@ static int launch_j(const Plan& pl, const typename E::raw_t* x, const Sink<typen
 
 template <typename E>
 int launch_typed(const Plan& pl, const void* x, int64_t rows, int64_t row_stride, int j,
-                 void* values, IndexOut indices, void* ws, hipStream_t stream, KeyRangeOut* ranges) {
+                 void* values, IndexOut indices, void* ws, hipStream_t stream, KeyRangeOut* ranges, SelectOut* last) {
   using raw_t = typename E::raw_t;
   Geom g;
   g.row_stride = row_stride; g.b = pl.width;
@@ -132,17 +155,17 @@ int launch_typed(const Plan& pl, const void* x, int64_t rows, int64_t row_stride
   out.part_pos = pl.merge ? reinterpret_cast<uint32_t*>(base + pl.part_pos_off) : nullptr;
   const raw_t* xs = static_cast<const raw_t*>(x);
   switch (j) {
-    case 1: return launch_j<E, 1>(pl, xs, out, g, rows, stream, ranges);
-    case 2: return launch_j<E, 2>(pl, xs, out, g, rows, stream, ranges);
-    case 3: return launch_j<E, 3>(pl, xs, out, g, rows, stream, ranges);
-    case 4: return launch_j<E, 4>(pl, xs, out, g, rows, stream, ranges);
+    case 1: return launch_j<E, 1>(pl, xs, out, g, rows, stream, ranges, last);
+    case 2: return launch_j<E, 2>(pl, xs, out, g, rows, stream, ranges, last);
+    case 3: return launch_j<E, 3>(pl, xs, out, g, rows, stream, ranges, last);
+    case 4: return launch_j<E, 4>(pl, xs, out, g, rows, stream, ranges, last);
   }
   return ATK_ERR_J;
 }
 
 #define ATK_INSTANTIATE_STREAM(DT)                                                          \
   template int launch_typed<Elem<DT>>(const Plan&, const void*, int64_t, int64_t, int, void*, \
-                                      IndexOut, void*, hipStream_t, KeyRangeOut*);
+                                      IndexOut, void*, hipStream_t, KeyRangeOut*, SelectOut*);
 
 }  // namespace stream
 }  // namespace atk

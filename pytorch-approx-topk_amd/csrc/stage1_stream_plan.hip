@@ -26,6 +26,11 @@ constexpr int64_t kLongWaveRun = 16;
 // (measured down to 8: fp32 [32768, 1024] with 16 buckets 104 -> 22 us, bf16
 // 193 -> 32 us; [65536, 256] with 16 buckets 70 -> 31 us).
 constexpr int64_t kFoldMinLength = 8;
+// Candidates, and entries of all their partial queues, up to which the merge of a row takes the second
+// stage along.  One workgroup reads these entries: up to 16384 it saves 1-5 us in rows of 2^20 to 2^24, beyond
+// that it wins and loses (fp32 [1, 2^22] k=64 j=4 k_mult=2, 32768 entries, 27.4 -> 24.1 us; k=500 j=2 k_mult=4,
+// 64000 entries, 19.9 -> 26.5; k=256 j=4 k_mult=4, 262144, 30.7 -> 58.0).
+constexpr int64_t kMergeSelectMax = 2048, kMergeSelectEntries = 16384;
 // Buckets from this length on are folded whatever the fold.
 constexpr int64_t kFoldAnyLength = 128;
 }  // namespace
@@ -155,6 +160,11 @@ Plan make_plan(int64_t rows, int64_t n, int64_t k0, int j, int layout, int dtype
   return pl;
 }
 
+bool selects_in_merge(const Plan& pl, int64_t k0, int64_t index_bound, int dtype) {
+  return pl.ok && pl.merge && elem_bytes(dtype) <= 4 && index_bound <= 0xffffffffll && k0 <= kMergeSelectMax &&
+         k0 * (int64_t)pl.slabs <= kMergeSelectEntries;
+}
+
 }  // namespace stream
 
 size_t stage1_stream_workspace_bytes(int64_t rows, int64_t n, int64_t k0, int j, int layout, int dtype) {
@@ -166,8 +176,9 @@ size_t stage1_stream_workspace_bytes(int64_t rows, int64_t n, int64_t k0, int j,
   return need;
 }
 
-bool describe_stage1_stream(const void* x, int64_t rows, int64_t n, int64_t k0, int j, int layout, int dtype,
-                            std::string& out) {
+bool describe_stage1_stream(const void* x, int64_t rows, int64_t n, int64_t k0, int j, int64_t k, int layout,
+                            int dtype, int64_t index_bound, bool* selected, std::string& out) {
+  *selected = false;
   const stream::Plan pl = stream::make_plan(rows, n, k0, j, layout, dtype, stream::wide_loads(x, elem_bytes(dtype)));
   if (!pl.ok) return false;
   const int loads = stream::deep_loads_for_short_columns(dtype, j, pl.vec, pl.packed, pl.run, pl.full_rows)
@@ -179,21 +190,26 @@ bool describe_stage1_stream(const void* x, int64_t rows, int64_t n, int64_t k0, 
          std::to_string(rows * (int64_t)pl.slabs * pl.col_tiles) + " block=" + std::to_string(64 * pl.waves) +
          " fold=" + std::to_string(pl.fold) + " slabs=" + std::to_string(pl.slabs) +
          (pl.wave_stores ? " wave-stores" : "");
-  if (pl.merge) out += " + stream_merge_kernel<" + std::string(dtype_name(dtype)) + ", J=" + std::to_string(j) + ">";
+  if (pl.merge) {
+    *selected = k < k0 && stream::selects_in_merge(pl, k0, index_bound, dtype);
+    out += std::string(" + stream_merge_") + (*selected ? "select_" : "") + "kernel<" + dtype_name(dtype) + ", J=" +
+           std::to_string(j) + ">";
+  }
   return true;
 }
 
 int launch_stage1_stream(const void* x, int64_t rows, int64_t n, int64_t row_stride, int64_t k0, int j,
                          int layout, int dtype, void* values, IndexOut indices, void* ws,
-                         size_t ws_bytes, hipStream_t stream, bool* handled, KeyRangeOut* ranges) {
+                         size_t ws_bytes, hipStream_t stream, bool* handled, KeyRangeOut* ranges, SelectOut* last) {
   const stream::Plan pl = stream::make_plan(rows, n, k0, j, layout, dtype, stream::wide_loads(x, elem_bytes(dtype)));
   *handled = pl.ok;
   if (!pl.ok) return ATK_OK;
   if (pl.ws_bytes && (!ws || ws_bytes < pl.ws_bytes || (uintptr_t)ws % 16 != 0)) return ATK_ERR_WORKSPACE;
+  if (last != nullptr) last->wanted = stream::selects_in_merge(pl, k0, last->index_bound, dtype);
   int rc = ATK_ERR_DTYPE;
   ATK_DTYPE_SWITCH(dtype, E, rc = ATK_ERR_DTYPE,
                    rc = stream::launch_typed<E>(pl, x, rows, row_stride, j, values, indices, ws,
-                                                stream, ranges));
+                                                stream, ranges, last));
   return rc;
 }
 
