@@ -1477,9 +1477,10 @@ __global__ __launch_bounds__(kWave * W) __attribute__((amdgpu_waves_per_eu(4))) 
 
   // When V does not divide b, the row's last live lane moves down to its last V
   // columns: it works out some of its neighbour's columns again and writes the same.
-  const int64_t first_col = (int64_t)col_tile * kTileCols + lane * V;
-  const bool live = first_col < g.b;
-  const int64_t col = first_col + V > g.b ? g.b - V : first_col;
+  // (In 32 bits, which a row's columns fit: the 64-bit form cost fp32 j=2 a wave per SIMD, 78 -> 82 registers.)
+  const uint32_t width = (uint32_t)g.b, first_col = col_tile * kTileCols + lane * V;
+  const bool live = first_col < width;
+  const int64_t col = first_col < width - V ? first_col : width - V;
 
   // sub-rows of this slab [s0, s1), then of this wave [p0, p1)
   const uint32_t s0 = slab * g.slab_len;

@@ -31,11 +31,14 @@ constexpr int64_t kFoldMinLength = 8;
 // that it wins and loses (fp32 [1, 2^22] k=64 j=4 k_mult=2, 32768 entries, 27.4 -> 24.1 us; k=500 j=2 k_mult=4,
 // 64000 entries, 19.9 -> 26.5; k=256 j=4 k_mult=4, 262144, 30.7 -> 58.0).
 constexpr int64_t kMergeSelectMax = 2048, kMergeSelectEntries = 16384;
+// Most workgroups (with 16-byte loads) and bytes of a launch that may take one-element loads instead.
+constexpr int64_t kFewGroups = 3000;
+constexpr int64_t kFewBytes = 100 << 20;
 // Buckets from this length on are folded whatever the fold.
 constexpr int64_t kFoldAnyLength = 128;
-}  // namespace
 
-Plan make_plan(int64_t rows, int64_t n, int64_t k0, int j, int layout, int dtype, bool wide) {
+// The plan with 16-byte loads (`wide`) or with one-element loads.
+Plan plan_with(int64_t rows, int64_t n, int64_t k0, int j, int layout, int dtype, bool wide) {
   Plan pl{};
   pl.ok = false;
   if (layout != ATK_INTERLEAVED && layout != ATK_INTERLEAVED_PADDED) return pl;
@@ -159,6 +162,60 @@ Plan make_plan(int64_t rows, int64_t n, int64_t k0, int j, int layout, int dtype
   pl.ok = true;
   return pl;
 }
+}  // namespace
+
+namespace {
+// Whether one-element loads are faster where 16-byte loads are possible.  A lane then owns one
+// column instead of four or eight: launches of few rows and few buckets have that many times the
+// workgroups, and where rows are cut into slabs fewer of those, so fewer partial queues for the
+// merge, or no merge at all.  What is lost is bytes in flight, so the batch and a wave's run have
+// limits.  Each line from 220 batches of 1-512 rows (fp32 and fp16, rows of 2^15 to 2^24, j 1, 2, 4, k_mult
+// 1-8, a launch of at most 1500 workgroups with 16-byte loads), timed both ways, and 260 calls drawn at
+// random; of the 220 about a hundred are picked, 16 % faster in the geometric mean and at most 1.68 times; one of
+// them is slower (fp32 [4, 1487193] b=766 j=2 13.4 -> 14.6 us).
+// Beyond the lines one-element loads lose up to a quarter (fp32 [91, 262144] b=4096 j=1 29.0 -> 36.5 us).
+bool narrow_is_faster(const Plan& w, const Plan& v, int64_t rows, int64_t n, int64_t b, int j, int es) {
+  const int64_t bytes = rows * n * es, mib = 1 << 20;
+  const int64_t groups = rows * (int64_t)w.slabs * w.col_tiles;
+  const int64_t waves_w = groups * w.waves, waves_v = rows * (int64_t)v.slabs * v.col_tiles * v.waves;
+  const int64_t run = (int64_t)v.full_rows / v.slabs / v.waves;  // sub-rows a wave scans
+  if (w.slabs > 1) {
+    // no merge: fp16 [4, 2^20] b=4096 j=4 23.6 -> 14.9 us, fp32 [14, 2^19] b=1024 j=4 25.2 -> 17.7
+    if (v.slabs == 1 && run <= 160 && bytes <= kFewBytes) return true;
+    // long lists of partial queues: fp16 [1, 5527026] b=176 j=2 24.4 -> 15.5, fp32 [3, 2^21] b=128 j=4 30.2 -> 17.9
+    // (longer ones where the columns get too long for packed queues: bf16 [1, 16001820] b=74 j=2 30.0 -> 26.8,
+    // but fp16 [1, 2^23] b=32 j=4 22.6 -> 30.1)
+    if (v.slabs > 1 && (int64_t)w.slabs * b * j > (v.packed == w.packed ? 16000 : 32000) && run <= 226 &&
+        bytes <= 64 * mib)
+      return true;
+    // half the slabs or fewer: fp32 [5, 1767589] b=136 j=2 23.3 -> 20.1
+    if (w.slabs >= 2 * v.slabs && run <= 128 && w.fold == 1 && bytes <= kFewBytes) return true;
+  } else if (v.slabs == 1) {
+    // CUs left idle: fp16 [4, 746849] b=3912 j=4 25.8 -> 15.9, [32, 936425] b=1556 j=2 54.1 -> 33.5, bf16 [20, 2395075]
+    // b=5200 j=2 (91 MiB) 61.5 -> 55.8, but [98, 2^19] b=1024 j=2 (98 MiB) 41.5 -> 44.2
+    if (j >= 2 && groups <= (es == 2 ? 256 : 64) && bytes <= (es == 2 ? 96 : 64) * mib) return true;
+    if (es == 2 && groups <= 128 && bytes <= 32 * mib) return true;  // [4, 2439482] b=12992 j=1 22.2 -> 20.5
+    // long queues of many folded columns per bucket: fp16 [451, 11857] b=17 j=4 12.8 -> 9.6, [2912, 15278] b=5
+    // 39.2 -> 33.0, [205, 32768] b=128 18.5 -> 14.6
+    if (es == 2 && j >= 3 && w.fold > 1) return true;
+  }
+  // small batches of 16-bit elements, whose waves have twice the columns to go through: fp16 [8, 301240] b=79 j=4
+  // 19.4 -> 14.9, [3, 2^20] b=256 j=2 17.9 -> 14.9, [4, 1618720] b=105 j=4 21.1 -> 13.3 (but no merge is worth
+  // having for it: [1, 65536] b=16 j=1 13.7 -> 16.8)
+  return es == 2 && (w.slabs > 1 || v.slabs == 1) && 2 * waves_v >= 3 * waves_w && groups <= 256 &&
+         bytes <= (j >= 2 && v.packed == w.packed ? 16 : 8) * mib;
+}
+}  // namespace
+
+Plan make_plan(int64_t rows, int64_t n, int64_t k0, int j, int layout, int dtype, bool wide) {
+  const Plan w = plan_with(rows, n, k0, j, layout, dtype, wide);
+  const int es = elem_bytes(dtype);
+  if (!w.ok || w.vec == 1 || (es != 2 && es != 4) || rows * (int64_t)w.slabs * w.col_tiles > kFewGroups ||
+      rows * n * es > kFewBytes)
+    return w;
+  const Plan v = plan_with(rows, n, k0, j, layout, dtype, false);
+  return v.ok && narrow_is_faster(w, v, rows, n, k0 / j, j, es) ? v : w;
+}
 
 bool selects_in_merge(const Plan& pl, int64_t k0, int64_t index_bound, int dtype) {
   return pl.ok && pl.merge && elem_bytes(dtype) <= 4 && index_bound <= 0xffffffffll && k0 <= kMergeSelectMax &&
@@ -168,8 +225,9 @@ bool selects_in_merge(const Plan& pl, int64_t k0, int64_t index_bound, int dtype
 }  // namespace stream
 
 size_t stage1_stream_workspace_bytes(int64_t rows, int64_t n, int64_t k0, int j, int layout, int dtype) {
-  const stream::Plan a = stream::make_plan(rows, n, k0, j, layout, dtype, true);
-  const stream::Plan u = stream::make_plan(rows, n, k0, j, layout, dtype, false);
+  // (make_plan picks one of these)
+  const stream::Plan a = stream::plan_with(rows, n, k0, j, layout, dtype, true);
+  const stream::Plan u = stream::plan_with(rows, n, k0, j, layout, dtype, false);
   size_t need = 0;
   if (a.ok && a.ws_bytes > need) need = a.ws_bytes;
   if (u.ok && u.ws_bytes > need) need = u.ws_bytes;
