@@ -180,9 +180,9 @@ bool narrow_is_faster(const Plan& w, const Plan& v, int64_t rows, int64_t n, int
   const int64_t waves_w = groups * w.waves, waves_v = rows * (int64_t)v.slabs * v.col_tiles * v.waves;
   const int64_t run = (int64_t)v.full_rows / v.slabs / v.waves;  // sub-rows a wave scans
   if (w.slabs > 1) {
-    // no merge: fp16 [4, 2^20] b=4096 j=4 23.6 -> 14.9 us, fp32 [14, 2^19] b=1024 j=4 25.2 -> 17.7
+    // no merge: fp16 [4, 2^20] b=4096 j=4 23.4 -> 15.1 us, fp32 [14, 2^19] b=1024 j=4 25.2 -> 17.7
     if (v.slabs == 1 && run <= 160 && bytes <= kFewBytes) return true;
-    // long lists of partial queues: fp16 [1, 5527026] b=176 j=2 24.4 -> 15.5, fp32 [3, 2^21] b=128 j=4 30.2 -> 17.9
+    // long lists of partial queues: fp16 [1, 5527026] b=176 j=2 22.1 -> 15.5, fp32 [3, 2^21] b=128 j=4 30.2 -> 17.9
     // (longer ones where the columns get too long for packed queues: bf16 [1, 16001820] b=74 j=2 30.0 -> 26.8,
     // but fp16 [1, 2^23] b=32 j=4 22.6 -> 30.1)
     if (v.slabs > 1 && (int64_t)w.slabs * b * j > (v.packed == w.packed ? 16000 : 32000) && run <= 226 &&
@@ -191,16 +191,16 @@ bool narrow_is_faster(const Plan& w, const Plan& v, int64_t rows, int64_t n, int
     // half the slabs or fewer: fp32 [5, 1767589] b=136 j=2 23.3 -> 20.1
     if (w.slabs >= 2 * v.slabs && run <= 128 && w.fold == 1 && bytes <= kFewBytes) return true;
   } else if (v.slabs == 1) {
-    // CUs left idle: fp16 [4, 746849] b=3912 j=4 25.8 -> 15.9, [32, 936425] b=1556 j=2 54.1 -> 33.5, bf16 [20, 2395075]
-    // b=5200 j=2 (91 MiB) 61.5 -> 55.8, but [98, 2^19] b=1024 j=2 (98 MiB) 41.5 -> 44.2
-    if (j >= 2 && groups <= (es == 2 ? 256 : 64) && bytes <= (es == 2 ? 96 : 64) * mib) return true;
+    // CUs left idle: fp16 [4, 746849] b=3912 j=4 23.0 -> 15.8, [32, 936425] b=1556 j=2 (57 MiB) 39.9 -> 33.8, but bf16
+    // [20, 2395075] b=5200 j=2 (91 MiB) 50.7 -> 55.2, [98, 2^19] b=1024 j=2 32.0 -> 44.2
+    if (j >= 2 && groups <= (es == 2 ? 256 : 64) && bytes <= 64 * mib) return true;
     if (es == 2 && groups <= 128 && bytes <= 32 * mib) return true;  // [4, 2439482] b=12992 j=1 22.2 -> 20.5
-    // long queues of many folded columns per bucket: fp16 [451, 11857] b=17 j=4 12.8 -> 9.6, [2912, 15278] b=5
-    // 39.2 -> 33.0, [205, 32768] b=128 18.5 -> 14.6
+    // long queues of many folded columns per bucket: fp16 [451, 11857] b=17 j=4 12.4 -> 9.5, [2912, 15278] b=5
+    // 40.4 -> 33.8, [205, 32768] b=128 18.6 -> 14.7
     if (es == 2 && j >= 3 && w.fold > 1) return true;
   }
   // small batches of 16-bit elements, whose waves have twice the columns to go through: fp16 [8, 301240] b=79 j=4
-  // 19.4 -> 14.9, [3, 2^20] b=256 j=2 17.9 -> 14.9, [4, 1618720] b=105 j=4 21.1 -> 13.3 (but no merge is worth
+  // 19.1 -> 15.3, [3, 2^20] b=256 j=2 16.6 -> 15.3, [4, 1618720] b=105 j=4 20.7 -> 13.7 (but no merge is worth
   // having for it: [1, 65536] b=16 j=1 13.7 -> 16.8)
   return es == 2 && (w.slabs > 1 || v.slabs == 1) && 2 * waves_v >= 3 * waves_w && groups <= 256 &&
          bytes <= (j >= 2 && v.packed == w.packed ? 16 : 8) * mib;
