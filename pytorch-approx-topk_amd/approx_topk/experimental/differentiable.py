@@ -10,16 +10,24 @@ their gradient scatters to those positions and every other position gets zero;
 the indices are distinct along ``dim``, so a plain scatter is exact.
 
 Along the last dim one kernel writes the gradient (``csrc/topk_grad.hip``); zeros
-and a scatter are left to double backward and to the dims the operator takes only
+and a scatter are left to derivatives of the gradient and to the dims the operator takes only
 when every bucket is kept whole.
 """
 from __future__ import annotations
 
 import torch
 from torch import Tensor
+from torch.autograd import forward_ad
 
 from .. import _native
 from ..priority_queue import topk as _topk, topk_grad as _topk_grad
+
+
+def _autograd_has_work(grad_values: Tensor) -> bool:
+    """Whether the gradient may itself be differentiated or traced: reverse mode, forward mode (both kinds enter
+    a level), a functorch transform, or ``torch.compile``, which does not look into dispatcher guards."""
+    return ((torch.is_grad_enabled() and grad_values.requires_grad) or forward_ad._current_level >= 0
+            or torch._C._functorch.peek_interpreter_stack() is not None or torch.compiler.is_compiling())
 
 
 class _TopkWithGradient(torch.autograd.Function):
@@ -40,9 +48,12 @@ class _TopkWithGradient(torch.autograd.Function):
             return None, None, None, None, None, None, None
         (indices,) = ctx.saved_tensors
         shape = ctx.shape
-        if (len(shape) and ctx.dim == len(shape) - 1 and indices.numel() and shape[-1] <= _native.MAX_GRAD_ROW
-                and not (torch.is_grad_enabled() and grad_values.requires_grad)):
-            grad_xs = _topk_grad(grad_values, indices, shape[-1], *ctx.buckets)
+        if len(shape) and ctx.dim == len(shape) - 1 and indices.numel() and shape[-1] <= _native.MAX_GRAD_ROW:
+            if _autograd_has_work(grad_values):
+                grad_xs = _topk_grad(grad_values, indices, shape[-1], *ctx.buckets)
+            else:  # the operator's autograd kernel would find nothing to do, in 6 us of host time
+                with torch._C._AutoDispatchBelowAutograd():
+                    grad_xs = _topk_grad(grad_values, indices, shape[-1], *ctx.buckets)
         elif len(shape) == 0:
             grad_xs = grad_values.reshape(()) if indices.numel() else grad_values.new_zeros(())
         else:

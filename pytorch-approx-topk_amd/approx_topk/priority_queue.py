@@ -133,7 +133,9 @@ topk = torch.ops.approx_topk.topk.default
 
 # The gradient of the values with respect to the input, for
 # ``approx_topk.experimental.differentiable``: an operator of its own so that
-# ``torch.compile`` traces through the wrapper's backward.
+# ``torch.compile`` traces through the wrapper's backward.  It is linear in ``grad_values``:
+# where its result has a derivative or a tangent, zeros and a scatter, for which every
+# transform has its rule, take the native kernel's place.
 _LIBRARY.define(
     "topk_grad(Tensor grad_values, Tensor indices, SymInt n, SymInt k0, SymInt j, bool interleaved) -> Tensor",
     tags=(torch.Tag.pt2_compliant_tag,))
@@ -147,6 +149,26 @@ def _topk_grad(grad_values: Tensor, indices: Tensor, n: int, k0: int, j: int, in
 
 
 _LIBRARY.impl("topk_grad", _topk_grad, "CompositeExplicitAutograd")
+
+
+def _topk_grad_autograd(grad_values: Tensor, indices: Tensor, n: int, k0: int, j: int, interleaved: bool) -> Tensor:
+    if ((grad_values.requires_grad and torch.is_grad_enabled())
+            or torch.autograd.forward_ad.unpack_dual(grad_values).tangent is not None):
+        return grad_values.new_zeros(indices.shape[:-1] + (n,)).scatter(-1, indices, grad_values)
+    with torch._C._AutoDispatchBelowAutograd():
+        return topk_grad(grad_values, indices, n, k0, j, interleaved)
+
+
+_LIBRARY.impl("topk_grad", _topk_grad_autograd, "Autograd")
+
+
+@torch.library.register_vmap("approx_topk::topk_grad", lib=_LIBRARY)
+def _(info, in_dims, grad_values, indices, n, k0, j, interleaved):
+    # rows are independent: a batch is more of them
+    def batch_first(t, dim):
+        return t.movedim(dim, 0) if dim is not None else t.expand((info.batch_size,) + t.shape)
+
+    return topk_grad(batch_first(grad_values, in_dims[0]), batch_first(indices, in_dims[1]), n, k0, j, interleaved), 0
 
 
 @torch.library.register_fake("approx_topk::topk_grad", lib=_LIBRARY)

@@ -54,6 +54,33 @@ def test_gradient_of_the_gradient():
     assert torch.allclose(second, expect, rtol=1e-6, atol=0)   # one rounding of a product each
 
 
+def test_transforms_of_the_backward():
+    # forward mode of both kinds, batches and both together, next to zeros and a scatter (autograd runs the
+    # backward in a thread of its own on a GPU)
+    from torch.autograd import forward_ad
+    from approx_topk.experimental.differentiable import topk
+    x = torch.randn(3, 5000, device="cuda", requires_grad=True)
+    values, indices = topk(x, 40, -1, j=2, k_mult=2)
+    w, t = torch.randn(2, 3, 40, device="cuda")
+    many = torch.randn(5, 3, 40, device="cuda")
+
+    def backward(g):
+        return torch.autograd.grad(values, x, g, retain_graph=True)[0]
+
+    def expect(g):
+        return g.new_zeros(g.shape[:-1] + (5000,)).scatter(-1, indices.expand(g.shape), g)
+
+    primal, tangent = torch.func.jvp(backward, (w,), (t,))
+    assert torch.equal(primal, expect(w)) and torch.equal(tangent, expect(t))
+    with forward_ad.dual_level():
+        primal, tangent = forward_ad.unpack_dual(backward(forward_ad.make_dual(w, t)))
+        assert torch.equal(primal, expect(w)) and torch.equal(tangent, expect(t))
+    assert torch.equal(torch.autograd.grad(values, x, many, is_grads_batched=True, retain_graph=True)[0], expect(many))
+    assert torch.equal(torch.func.vmap(backward)(many), expect(many))
+    assert torch.equal(torch.func.vmap(lambda g: torch.func.jvp(backward, (g,), (g,))[1])(many), expect(many))
+    assert torch.equal(torch.func.jvp(torch.func.vmap(backward), (many,), (many,))[1], expect(many))
+
+
 def test_gradient_operator_under_compile():
     from approx_topk.experimental.differentiable import topk
     x = torch.randn(3, 4096, device="cuda")
