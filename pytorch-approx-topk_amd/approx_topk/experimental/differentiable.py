@@ -35,7 +35,7 @@ class _TopkWithGradient(torch.autograd.Function):
     def forward(ctx, xs, k, dim, j, k_mult, interleaved, multithread_buckets):
         values, indices = _topk(xs, k, dim, j, k_mult, interleaved, multithread_buckets)
         ctx.dim = dim if dim >= 0 else dim + xs.ndim
-        ctx.shape = xs.shape
+        ctx.shape, ctx.dtype = xs.shape, xs.dtype
         ctx.buckets = (k * k_mult, j, interleaved)
         ctx.set_materialize_grads(False)
         ctx.save_for_backward(indices)
@@ -44,10 +44,10 @@ class _TopkWithGradient(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, grad_values, _grad_indices):
-        if grad_values is None:
-            return None, None, None, None, None, None, None
         (indices,) = ctx.saved_tensors
         shape = ctx.shape
+        if grad_values is None:  # (not materialized: that would fill an int64 gradient of the indices as well)
+            return indices.new_zeros(shape, dtype=ctx.dtype), None, None, None, None, None, None
         if len(shape) and ctx.dim == len(shape) - 1 and indices.numel() and shape[-1] <= _native.MAX_GRAD_ROW:
             if _autograd_has_work(grad_values):
                 grad_xs = _topk_grad(grad_values, indices, shape[-1], *ctx.buckets)

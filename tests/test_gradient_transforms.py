@@ -153,3 +153,26 @@ def test_direct_calls_of_the_operator_are_differentiable():
     assert torch.equal(got, torch.stack([torch.zeros(3, 64).scatter(1, i, w.detach()) for i in many]))
     assert torch.equal(torch.func.jacrev(lambda v: op(v, indices, 64, 8, 2, True))(w.detach()),
                        torch.func.jacfwd(lambda v: op(v, indices, 64, 8, 2, True))(w.detach()))
+
+
+class _Drops(torch.autograd.Function):
+    """Sums its input and hands no gradient back."""
+    @staticmethod
+    def forward(ctx, values):
+        return values.sum()
+
+    @staticmethod
+    def backward(ctx, g):
+        return None
+
+
+def test_a_missing_gradient_of_the_values_counts_as_zeros():
+    pairs, _ = _both()
+    for values, x in pairs:
+        (grad,) = torch.autograd.grad(_Drops.apply(values), x)
+        assert grad.shape == x.shape and grad.dtype == x.dtype and not grad.any()
+    from approx_topk.experimental.differentiable import topk
+    for dtype in (torch.float16, torch.float64):
+        x = torch.randn(2, 64).to(dtype).requires_grad_()
+        _Drops.apply(topk(x, 8, -1)[0]).backward()
+        assert x.grad.dtype == dtype and x.grad.shape == x.shape and not x.grad.any()
