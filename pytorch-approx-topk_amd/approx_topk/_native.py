@@ -255,13 +255,26 @@ def topk(xs: torch.Tensor, k0: int, j: int, k: int, layout: int, index_dtype: to
 MAX_GRAD_ROW = (1 << 31) - 1
 
 
+def check_grad_tensors(grad_values: torch.Tensor, indices: torch.Tensor) -> None:
+    """What the gradient's kernel takes for granted: it reads as many gradients as indices, of eight bytes."""
+    if (indices.dtype != torch.int64 or grad_values.shape != indices.shape or grad_values.device != indices.device
+            or indices.ndim == 0):
+        raise RuntimeError(
+            "topk_grad: expected int64 indices and gradients of the same shape on one device, got "
+            f"{indices.dtype} {tuple(indices.shape)} on {indices.device} and {tuple(grad_values.shape)} on "
+            f"{grad_values.device}")
+
+
 def topk_grad(grad_values: torch.Tensor, indices: torch.Tensor, n: int, k0: int, j: int, layout: int) -> torch.Tensor:
     """The gradient of a call's values with respect to its input (top-k along the last dim of `n`
     elements), given the call's indices: zero but for the selected positions."""
+    check_grad_tensors(grad_values, indices)
     require_gpu(grad_values)
     grad_values, indices = grad_values.contiguous(), indices.contiguous()
     k = indices.shape[-1]
     grad_x = torch.empty(indices.shape[:-1] + (n,), dtype=grad_values.dtype, device=grad_values.device)
+    if indices.numel() == 0:
+        return grad_x.zero_()
     with _on_device(grad_values.device):
         status = lib().atk_topk_grad(grad_values.data_ptr(), indices.data_ptr(), indices.numel() // k, n, k0, j, k,
                                      layout, dtype_code(grad_values.dtype), grad_x.data_ptr(),

@@ -173,6 +173,7 @@ def _(info, in_dims, grad_values, indices, n, k0, j, interleaved):
 
 @torch.library.register_fake("approx_topk::topk_grad", lib=_LIBRARY)
 def _(grad_values: Tensor, indices: Tensor, n: int, k0: int, j: int, interleaved: bool) -> Tensor:
+    _native.check_grad_tensors(grad_values, indices)
     return grad_values.new_empty(indices.shape[:-1] + (n,))
 
 

@@ -250,3 +250,16 @@ def test_operator_object_offers_register_fake_and_register_autograd():
     """) % os.path.join(ROOT, "pytorch-approx-topk_amd")
     out = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, timeout=300)
     assert out.returncode == 0 and "registered" in out.stdout, out.stderr[-2000:]
+
+
+def test_gradient_operator_checks_its_tensors_before_any_native_call():
+    # the kernel reads rows * k entries of both tensors, the indices eight bytes each: what does not
+    # match must not reach it
+    op = torch.ops.approx_topk.topk_grad.default
+    w, i = torch.randn(3, 8), torch.zeros(3, 8, dtype=torch.int64)
+    with pytest.raises(RuntimeError, match="GPU"):
+        op(w, i, 64, 8, 1, True)                       # valid arguments, but no CPU path exists
+    for grad_values, indices in ((w, i.int()), (w, i.double()), (w[:2], i), (w[:, :4], i), (w[0], i), (w, i[0]),
+                                 (w.reshape(8, 3), i), (w, i.to("meta")), (w[0, 0], i[0, 0])):
+        with pytest.raises(RuntimeError, match="topk_grad"):
+            op(grad_values, indices, 64, 8, 1, True)
