@@ -33,6 +33,27 @@ def test_gradient_kernel_equals_a_scatter(dtype, interleaved):
         assert torch.equal(grad, expect), (rows, n, k, j, k_mult)
 
 
+# batches whose tiles hold several rows: two of them and a last tile of one; as many as a tile has room for, and
+# a last tile of fewer; rows of one element; two rows to a tile of 64 KiB in four-byte types, then only one
+SHORT = [
+    (1025, 7, 3, 1, 1), (5003, 64, 16, 4, 1), (40003, 1001, 20, 2, 2), (2049, 1, 1, 1, 1),
+    (2101, 8192, 60, 2, 2), (2101, 8193, 60, 2, 2), (1024, 64, 16, 4, 2),
+]
+
+
+@pytest.mark.parametrize("interleaved", [True, False])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.float64], ids=lambda d: str(d).split(".")[-1])
+def test_short_rows_share_a_tile(dtype, interleaved):
+    from approx_topk.experimental.differentiable import topk
+    for rows, n, k, j, k_mult in SHORT:
+        g = torch.Generator(device="cuda").manual_seed(n + k)
+        x = torch.randn(rows, n, generator=g, device="cuda").to(dtype).requires_grad_()
+        values, indices = topk(x, k, -1, j=j, k_mult=k_mult, interleaved=interleaved)
+        w = torch.randn(rows, k, generator=g, device="cuda").to(dtype)
+        (grad,) = torch.autograd.grad(values, x, w)
+        assert torch.equal(grad, torch.zeros_like(x).scatter(1, indices, w)), (rows, n, k, j, k_mult)
+
+
 def test_gradient_of_sums_of_views_and_of_unused_values():
     from approx_topk.experimental.differentiable import topk
     x = torch.randn(2, 3, 5000, device="cuda", requires_grad=True)
