@@ -10,6 +10,8 @@ constexpr int64_t kTargetGroups = 1024;
 // split_bucket_kernel: buckets of a launch from which on a wave may take more than kFewTurns turns
 // at its bucket, and from which on buckets shorter than one piece go there.
 constexpr int64_t kManyWaves = 512, kFewTurns = 8, kManyBuckets = 16384;
+// Workgroups whose threads a launch can count (in 32 bits); contig_kernel gives a short bucket fewer lanes.
+constexpr int64_t kMostGroups = 0xffffffffll / kThreads;
 }  // namespace
 
 Plan make_plan(int64_t rows, int64_t n, int64_t k0, int j, int layout, int dtype, bool aligned,
@@ -113,9 +115,10 @@ Plan make_plan(int64_t rows, int64_t n, int64_t k0, int j, int layout, int dtype
       (m * es >= (int64_t)kSplitBytes || rows * b >= kManyBuckets)) {
     uint32_t pieces_log2 = 0;
     while (((longest + (1ll << pieces_log2) - 1) >> pieces_log2) * es > (int64_t)kSplitBytes) ++pieces_log2;
-    if ((m >> pieces_log2) * es >= 16 && ((1 << pieces_log2) <= kFewTurns * stream::kWave || rows * b >= kManyWaves)) {
+    g.split_log2 = pieces_log2;
+    if ((m >> pieces_log2) * es >= 16 && ((1 << pieces_log2) <= kFewTurns * stream::kWave || rows * b >= kManyWaves) &&
+        bucket_groups(g, rows) <= kMostGroups) {
       g.split = 1;
-      g.split_log2 = pieces_log2;
       g.split_trip = (uint32_t)((longest + (1ll << pieces_log2) - 1) >> pieces_log2);
       g.slabs = 1;
       pl.ws_bytes = 0;

@@ -263,3 +263,23 @@ def test_gradient_operator_checks_its_tensors_before_any_native_call():
                                  (w.reshape(8, 3), i), (w, i.to("meta")), (w[0, 0], i[0, 0])):
         with pytest.raises(RuntimeError, match="topk_grad"):
             op(grad_values, indices, 64, 8, 1, True)
+
+
+def test_no_kernel_of_a_contiguous_call_has_more_threads_than_a_launch_takes():
+    # 32 bits count them; batches beyond that many lanes keep the kernel that needs fewer
+    from approx_topk import _native
+    L = _native.lib()
+
+    def describe(rows, n, code, k, j):
+        buf = ctypes.create_string_buffer(1024)
+        assert L.atk_describe(4096, rows, n, n, k, j, k, 1, code, 4096, 4096, buf, 1024) == 0
+        return buf.value.decode()
+
+    for rows, n, code, k, j in ((16260510, 2803, 0, 292, 2), (12075969, 3677, 0, 106, 1), (16275156, 2318, 7, 54, 3),
+                                (1 << 22, 20001, 1, 1500, 1)):
+        text = describe(rows, n, code, k, j)
+        grid, block = (int(re.search(f"{key}=(\\d+)", text).group(1)) for key in ("grid", "block"))
+        assert grid * block < 1 << 32, text
+    # two lanes to each of 146 buckets: 2^24 - 1 workgroups of 256 are the most
+    assert describe(14708791, 2803, 0, 292, 2).startswith("split_bucket_kernel<f32")
+    assert describe(14708792, 2803, 0, 292, 2).startswith("contig_kernel<f32")
