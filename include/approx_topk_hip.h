@@ -128,13 +128,20 @@ int atk_select(const void* cand_values, const int64_t* cand_indices,
 size_t atk_topk_workspace_bytes(int64_t rows, int64_t n, int64_t k0, int j,
                                 int64_t k, int layout, int dtype);
 /*
- * The same for one particular call: 0 when its rows start on 16-byte boundaries
- * and the one-kernel path takes it, which parks no candidates (never more than
- * atk_topk_workspace_bytes).  Same call site as above: the workspace the
- * operator allocates before the native call (priority_queue.py:63-88).
+ * A bound for one particular call, which atk_topk_noalloc goes by: 0 when all rows
+ * start on 16-byte boundaries and the one-kernel path takes the call, which parks no
+ * candidates, else atk_topk_workspace_bytes, also for rows of other starts that
+ * the one-kernel path takes as well.
  */
 size_t atk_topk_workspace_bytes_at(const void* x, int64_t rows, int64_t n, int64_t row_stride,
                                    int64_t k0, int j, int64_t k, int layout, int dtype);
+/*
+ * What that call's kernels use: 0 whenever the one-kernel path takes it (never more
+ * than the bound above).  Same call site as above: the workspace the operator
+ * allocates before the native call (priority_queue.py:63-88).
+ */
+size_t atk_topk_workspace_bytes_used(const void* x, int64_t rows, int64_t n, int64_t row_stride,
+                                     int64_t k0, int j, int64_t k, int layout, int dtype);
 int atk_topk(const void* x, int64_t rows, int64_t n, int64_t row_stride,
              int64_t k0, int j, int64_t k, int layout, int dtype,
              void* values, int64_t* indices,

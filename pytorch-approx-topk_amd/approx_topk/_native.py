@@ -41,6 +41,8 @@ _SIGNATURES = {
                                                                           ctypes.c_int, ctypes.c_int]),
     "atk_topk_workspace_bytes_at": (ctypes.c_size_t, [ctypes.c_void_p] + [ctypes.c_int64] * 4
                                     + [ctypes.c_int, ctypes.c_int64, ctypes.c_int, ctypes.c_int]),
+    "atk_topk_workspace_bytes_used": (ctypes.c_size_t, [ctypes.c_void_p] + [ctypes.c_int64] * 4
+                                      + [ctypes.c_int, ctypes.c_int64, ctypes.c_int, ctypes.c_int]),
     "atk_topk": (ctypes.c_int, [ctypes.c_void_p] + [ctypes.c_int64] * 4 + [ctypes.c_int, ctypes.c_int64,
                                                                            ctypes.c_int, ctypes.c_int]
                  + [ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_size_t,
@@ -130,7 +132,7 @@ def _stage1_workspace(rows: int, n: int, k0: int, j: int, layout: int, code: int
 def _topk_workspace(misalign: int, rows: int, n: int, step: int, k0: int, j: int, k: int, layout: int,
                     code: int) -> int:
     # the library only looks at the address's alignment: any address with the same one stands for it
-    return lib().atk_topk_workspace_bytes_at(4096 + misalign, rows, n, step, k0, j, k, layout, code)
+    return lib().atk_topk_workspace_bytes_used(4096 + misalign, rows, n, step, k0, j, k, layout, code)
 
 
 def rows_view(xs: torch.Tensor) -> tuple[torch.Tensor, int, int, int]:

@@ -244,13 +244,20 @@ size_t atk_topk_workspace_bytes(int64_t rows, int64_t n, int64_t k0, int j, int6
   return plan_topk(rows, n, k0, j, k, layout, dtype).total;
 }
 
-size_t atk_topk_workspace_bytes_at(const void* x, int64_t rows, int64_t n, int64_t row_stride, int64_t k0,
-                                   int j, int64_t k, int layout, int dtype) {
-  // (the one-kernel path takes rows that start off a 16-byte boundary as well; the bound stays for them)
+size_t atk_topk_workspace_bytes_used(const void* x, int64_t rows, int64_t n, int64_t row_stride, int64_t k0,
+                                     int j, int64_t k, int layout, int dtype) {
   if (rows > 0 && k > 0 && k < k0 && check_stage1(x, rows, n, row_stride, k0, j, layout, dtype, x, x) == ATK_OK &&
-      aligned_to(x, 16) && (row_stride * atk::elem_bytes(dtype)) % 16 == 0 &&
       atk::fused_row_takes(x, rows, n, k0, j, k, layout, dtype))
     return 0;
+  return plan_topk(rows, n, k0, j, k, layout, dtype).total;
+}
+
+size_t atk_topk_workspace_bytes_at(const void* x, int64_t rows, int64_t n, int64_t row_stride, int64_t k0,
+                                   int j, int64_t k, int layout, int dtype) {
+  // Callers that size buffers by this figure, and atk_topk_noalloc's limit, have relied on it since only rows on
+  // 16 bytes went through one kernel: calls it calls too large stay refused.
+  if (aligned_to(x, 16) && (row_stride * atk::elem_bytes(dtype)) % 16 == 0)
+    return atk_topk_workspace_bytes_used(x, rows, n, row_stride, k0, j, k, layout, dtype);
   return plan_topk(rows, n, k0, j, k, layout, dtype).total;
 }
 

@@ -37,7 +37,7 @@ def test_workspace_of_one_call_depends_on_the_address():
     general = L.atk_topk_workspace_bytes(512, 32768, 1024, 1, 256, 0, 1)
     assert general >= 512 * 1024 * (2 + 8)
     assert L.atk_topk_workspace_bytes_at(4096, 512, 32768, 32768, 1024, 1, 256, 0, 1) == 0
-    # a misaligned input or an odd row stride goes through two kernels
+    # a misaligned input goes through two kernels; an odd row stride keeps their bound, whatever takes it
     assert L.atk_topk_workspace_bytes_at(4098, 512, 32768, 32768, 1024, 1, 256, 0, 1) == general
     assert L.atk_topk_workspace_bytes_at(4096, 512, 32768, 32769, 1024, 1, 256, 0, 1) == general
     # k == k0: stage 1 alone
@@ -47,6 +47,33 @@ def test_workspace_of_one_call_depends_on_the_address():
     assert L.atk_topk_workspace_bytes_at(4096, 512, 32768, 32768, 1024, 1, 256, 1, 1) == 0
     assert L.atk_topk_workspace_bytes_at(4096, 512, 1 << 18, 1 << 18, 1024, 1, 256, 1, 1) == \
         L.atk_topk_workspace_bytes(512, 1 << 18, 1024, 1, 256, 1, 1) > 0
+
+
+def test_workspace_a_call_uses_follows_the_kernels_it_takes():
+    from approx_topk import _native
+    L = _native.lib()
+
+    def used(x, n, stride, k0, j, k, layout=0, code=1):
+        args = (512, n, stride, k0, j, k, layout, code)
+        buf = ctypes.create_string_buffer(1024)
+        assert L.atk_describe(x, *args, 4096, 4096, buf, 1024) == 0
+        need = L.atk_topk_workspace_bytes_used(x, *args)
+        assert need <= L.atk_topk_workspace_bytes_at(x, *args) <= L.atk_topk_workspace_bytes(512, n, *args[3:])
+        one_kernel = buf.value.startswith(b"fused_")
+        assert (need == 0) == one_kernel and need in (0, L.atk_topk_workspace_bytes(512, n, *args[3:]))
+        return one_kernel
+
+    assert used(4096, 32768, 32768, 1024, 1, 256)
+    for n, stride in ((32768, 32769), (32768, 32775), (32767, 32767), (32761, 32768)):   # rows that start anywhere
+        assert used(4096, n, stride, 1024, 1, 256) and used(4100, n, stride, 1024, 1, 256)
+    assert not used(4098, 32768, 32768, 1024, 1, 256)         # an input that starts on an odd half-word
+    assert not used(4096, 32768, 32768, 1022, 2, 511)         # a number of buckets off the load width
+    assert used(4096, 32768, 32768, 1024, 1, 256, layout=1) and not used(4096, 1 << 18, 1 << 18, 1024, 1, 256, layout=1)
+    # what no kernel takes needs none of its own: the bound, as for every invalid call
+    assert L.atk_topk_workspace_bytes_used(4096, 0, 32768, 32768, 1024, 1, 256, 0, 1) == 0
+    # the operator's wrapper allocates by it
+    assert _native._topk_workspace(0, 512, 32768, 32769, 1024, 1, 256, 0, 1) == 0
+    assert _native._topk_workspace(2, 512, 32768, 32768, 1024, 1, 256, 0, 1) > 0
 
 
 def test_native_argument_checks_need_no_gpu():

@@ -52,10 +52,12 @@ CASES = [
     [(1, 1 << 22, torch.float32, 8192, 4, 4096), (1, 1 << 20, torch.float32, 2048, 4, 1024)],
     # stage 1 alone (k == k0) on a row cut into slabs, then a smaller one
     [(2, 1 << 21, torch.float32, 64, 2, 64), (1, 1 << 19, torch.float32, 16, 1, 16)],
-    # a batch through stage 1 + select with parked candidates (rows spaced so that one kernel declines), then fewer rows
+    # rows spaced by an odd pitch, for which the bound counts candidates whether one kernel takes them or two, then fewer
     [(48, 40000, torch.float16, 1024, 2, 256), (5, 9000, torch.float16, 512, 1, 64)],
     # contiguous buckets shared out over workgroups, then interleaved in one kernel (no scratch at all)
     [(1, 1 << 22, torch.bfloat16, 8, 2, 4), (130, 4096, torch.bfloat16, 256, 4, 64)],
+    # a batch through stage 1 + select with parked candidates (511 and 255 buckets, off the load width), then fewer rows
+    [(48, 40000, torch.float16, 1022, 2, 511), (5, 9000, torch.float16, 510, 2, 255)],
 ]
 
 
@@ -65,7 +67,7 @@ def test_noalloc_equals_workspace_version_on_consecutive_calls(pair):
     for call, (rows, n, dtype, k0, j, k) in enumerate(CASES[pair]):
         layout = 1 if (pair == 3 and call == 0) else 0
         x_cpu = (torch.randint(-60, 61, (rows, n), generator=g).float() / 8).to(dtype)   # many ties
-        stride_pad = 7 if pair == 2 else 0   # odd row pitch: the one-kernel path declines
+        stride_pad = 7 if pair == 2 else 0
         holder = torch.empty(rows, n + stride_pad, dtype=dtype, device="cuda")
         x = holder[:, :n]
         x.copy_(x_cpu)
@@ -88,7 +90,7 @@ def test_noalloc_equals_workspace_version_on_consecutive_calls(pair):
 def test_noalloc_rejects_what_does_not_fit_and_bad_arguments():
     from approx_topk import _native
     L = _native.lib()
-    x = torch.zeros(4096, 16385, dtype=torch.float32, device="cuda")[:, :16384]   # odd row pitch: two kernels
+    x = torch.zeros(4096, 16385, dtype=torch.float32, device="cuda")[:, :16384]   # odd row pitch
     need = L.atk_topk_workspace_bytes_at(x.data_ptr(), 4096, 16384, x.stride(0), 4096, 1, 1024, 0, 0)
     assert need > SCRATCH_BYTES
     rc, _, _ = _call_noalloc(x, 4096, 1, 1024)
