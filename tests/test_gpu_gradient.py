@@ -61,7 +61,9 @@ def test_gradient_of_sums_of_views_and_of_unused_values():
     (grad,) = torch.autograd.grad(values.sum(), x)   # an expanded gradient
     assert torch.equal(grad, torch.zeros_like(x).scatter(2, indices, 1.0))
     values, _ = topk(x, 40, -1)
-    assert torch.autograd.grad(x.sum() + 0 * values.sum(), x)[0].shape == x.shape
+    assert torch.equal(torch.autograd.grad(x.sum() + 0 * values.sum(), x)[0], torch.ones_like(x))
+    topk(x, 40, -1)   # nothing of it used
+    assert torch.equal(torch.autograd.grad(x.sum(), x)[0], torch.ones_like(x))
 
 
 def test_gradient_of_the_gradient():
@@ -110,3 +112,22 @@ def test_gradient_operator_under_compile():
     op = torch.ops.approx_topk.topk_grad.default
     torch.library.opcheck(op, (w, indices, 4096, 64, 2, True),
                           test_utils=("test_schema", "test_faketensor"))
+
+    # a function compiled whole, its backward through the operator
+    def loss(x, w):
+        values, _ = topk(2 * x, 64, -1, j=2, k_mult=2)
+        return (values * w).sum()
+
+    x.requires_grad_()
+    (eager,) = torch.autograd.grad(loss(x, w), x)
+    graphs = []
+
+    def backend(graph, example_inputs):
+        graphs.append(graph.print_readable(print_output=False))
+        return make_boxed_func(graph)
+
+    from functorch.compile import make_boxed_func
+    from torch._dynamo.backends.common import aot_autograd
+    compiled = torch.compile(loss, fullgraph=True, backend=aot_autograd(fw_compiler=backend, bw_compiler=backend))
+    (grad,) = torch.autograd.grad(compiled(x, w), x)
+    assert torch.equal(grad, eager) and len(graphs) == 2 and "approx_topk.topk_grad" in graphs[1], graphs
