@@ -4,8 +4,9 @@
 // [L = n / b sub-rows][b columns] plus a last partial sub-row of n mod b
 // elements; bucket c is column c.  The job is a column-wise top-J.
 //
-// Mapping.  Every lane owns V adjacent columns (V*sizeof(T) = 16 bytes; V = 1 in
-// rows of fewer columns than that), so one wave64 load instruction reads 64*V
+// Mapping.  Every lane owns V adjacent columns (V*sizeof(T) = 16 bytes, 8 for 1-byte types;
+// V = 1 in rows of fewer columns than that and where the planner finds that faster), so
+// one wave64 load instruction reads 64*V
 // adjacent elements of one sub-row (1 KiB with 16-byte loads) and the wave walks
 // down the sub-rows.  The J-entry queue of each owned column lives in
 // registers: values in compare form plus the sub-row number they came from; the
@@ -1821,8 +1822,9 @@ struct Plan {
   size_t part_values_off, part_pos_off, ws_bytes;
 };
 
-// `wide`: 16-byte loads may be used (wide_loads).
-Plan make_plan(int64_t rows, int64_t n, int64_t k0, int j, int layout, int dtype, bool wide);
+// `wide`: 16-byte loads may be used (wide_loads).  `select_bound`: the index bound of a second stage behind
+// the candidates, 0 for none.
+Plan make_plan(int64_t rows, int64_t n, int64_t k0, int j, int layout, int dtype, bool wide, int64_t select_bound);
 // Rows and sub-rows may start at any element.  One-element loads, which odd rows took before,
 // move a quarter (4-byte types) or an eighth (2-byte types) of the bytes per instruction: bf16
 // [256, 100003] k=64 j=1 k_mult=8 24.8 us that way (and in two kernels) against 14.3 us, arg-max of

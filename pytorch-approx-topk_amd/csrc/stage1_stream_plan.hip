@@ -1,4 +1,6 @@
 // Host-side planning and dispatch of the streaming stage-1 kernels.
+#include <cmath>
+
 #include "stage1_stream.h"
 
 namespace atk {
@@ -31,9 +33,9 @@ constexpr int64_t kFoldMinLength = 8;
 // that it wins and loses (fp32 [1, 2^22] k=64 j=4 k_mult=2, 32768 entries, 27.4 -> 24.1 us; k=500 j=2 k_mult=4,
 // 64000 entries, 19.9 -> 26.5; k=256 j=4 k_mult=4, 262144, 30.7 -> 58.0).
 constexpr int64_t kMergeSelectMax = 2048, kMergeSelectEntries = 16384;
-// Most workgroups (with 16-byte loads) and bytes of a launch that may take one-element loads instead.
-constexpr int64_t kFewGroups = 3000;
-constexpr int64_t kFewBytes = 100 << 20;
+// Most bytes of a call that may take one-element loads where 16-byte loads are possible (see estimate): as far as
+// both were timed.
+constexpr int64_t kFewBytes = 128 << 20;
 // Buckets from this length on are folded whatever the fold.
 constexpr int64_t kFoldAnyLength = 128;
 
@@ -165,56 +167,78 @@ Plan plan_with(int64_t rows, int64_t n, int64_t k0, int j, int layout, int dtype
 }  // namespace
 
 namespace {
-// Whether one-element loads are faster where 16-byte loads are possible.  A lane then owns one
-// column instead of four or eight: launches of few rows and few buckets have that many times the
-// workgroups, and where rows are cut into slabs fewer of those, so fewer partial queues for the
-// merge, or no merge at all.  What is lost is bytes in flight, so the batch and a wave's run have
-// limits.  Each line from 220 batches of 1-512 rows (fp32 and fp16, rows of 2^15 to 2^24, j 1, 2, 4, k_mult
-// 1-8, a launch of at most 1500 workgroups with 16-byte loads), timed both ways, and 260 calls drawn at
-// random; of the 220 about a hundred are picked, 16 % faster in the geometric mean and at most 1.68 times; one of
-// them is slower (fp32 [4, 1487193] b=766 j=2 13.4 -> 14.6 us).
-// Beyond the lines one-element loads lose up to a quarter (fp32 [91, 262144] b=4096 j=1 29.0 -> 36.5 us).
-bool narrow_is_faster(const Plan& w, const Plan& v, int64_t rows, int64_t n, int64_t b, int j, int es) {
-  const int64_t bytes = rows * n * es, mib = 1 << 20;
-  const int64_t groups = rows * (int64_t)w.slabs * w.col_tiles;
-  const int64_t waves_w = groups * w.waves, waves_v = rows * (int64_t)v.slabs * v.col_tiles * v.waves;
-  const int64_t run = (int64_t)v.full_rows / v.slabs / v.waves;  // sub-rows a wave scans
-  if (w.slabs > 1) {
-    // no merge: fp16 [4, 2^20] b=4096 j=4 23.4 -> 15.1 us, fp32 [14, 2^19] b=1024 j=4 25.2 -> 17.7
-    if (v.slabs == 1 && run <= 160 && bytes <= kFewBytes) return true;
-    // long lists of partial queues: fp16 [1, 5527026] b=176 j=2 22.1 -> 15.5, fp32 [3, 2^21] b=128 j=4 30.2 -> 17.9
-    // (longer ones where the columns get too long for packed queues: bf16 [1, 16001820] b=74 j=2 30.0 -> 26.8,
-    // but fp16 [1, 2^23] b=32 j=4 22.6 -> 30.1)
-    if (v.slabs > 1 && (int64_t)w.slabs * b * j > (v.packed == w.packed ? 16000 : 32000) && run <= 226 &&
-        bytes <= 64 * mib)
-      return true;
-    // half the slabs or fewer: fp32 [5, 1767589] b=136 j=2 23.3 -> 20.1
-    if (w.slabs >= 2 * v.slabs && run <= 128 && w.fold == 1 && bytes <= kFewBytes) return true;
-  } else if (v.slabs == 1) {
-    // CUs left idle: fp16 [4, 746849] b=3912 j=4 23.0 -> 15.8, [32, 936425] b=1556 j=2 (57 MiB) 39.9 -> 33.8, but bf16
-    // [20, 2395075] b=5200 j=2 (91 MiB) 50.7 -> 55.2, [98, 2^19] b=1024 j=2 32.0 -> 44.2
-    if (j >= 2 && groups <= (es == 2 ? 256 : 64) && bytes <= 64 * mib) return true;
-    if (es == 2 && groups <= 128 && bytes <= 32 * mib) return true;  // [4, 2439482] b=12992 j=1 22.2 -> 20.5
-    // long queues of many folded columns per bucket: fp16 [451, 11857] b=17 j=4 12.4 -> 9.5, [2912, 15278] b=5
-    // 40.4 -> 33.8, [205, 32768] b=128 18.6 -> 14.7
-    if (es == 2 && j >= 3 && w.fold > 1) return true;
+// Estimated microseconds of a plan (less what all plans of a call share), for the choice between 16-byte and
+// one-element loads where both are possible.  With one-element loads a lane owns one column instead of two to eight:
+// more workgroups, in rows cut into slabs fewer partial queues, and a shorter end of every workgroup, against fewer bytes
+// in flight, a load for every element and more waves to launch.  What a plan takes is
+//   the scan: memory, instructions, the launch of the waves and the round trips of a wave's loads, which overlap
+//     (the root of the sum of their squares);
+//   a workgroup's end: the other waves' queues folded into the leading wave's, folded columns put together, and a
+//     lane's entries written, side by side with other workgroups on the CU;
+//   the launches behind it: the merge of the slabs, with or without the second stage, or the stand-alone select.
+// The constants are a least-squares fit to 2070 calls timed both ways (all nine types, 1-20000 rows of 37 to 2^24
+// elements, up to 128 MiB, j 1-4, k_mult 1-8, half of them few rows, most of them off 16 bytes).  Its choice is
+// 1.0 % slower than the better one of the two in the geometric mean (10 % and more in one call of 22), 16-byte loads
+// throughout 14 %, one-element loads throughout 6 %: fp32 [3, 2^21] b=128 j=4 k_mult=8 30.2 us wide, 17.9 narrow, int8
+// [1, 172601] b=1310 j=4 8.5 and 4.0, uint8 [39, 152696] b=201 j=4 14.7 and 8.6, fp64 [2, 310384] b=799 j=4 13.6 and
+// 11.1, fp16 [168, 298475] b=544 j=4 67.9 and 42.1, but int8 [51, 507136] b=2391 j=3 11.5 and 17.4, fp16 [21, 1426304]
+// b=8338 j=2 17.1 and 24.1.
+double estimate(const Plan& pl, int64_t rows, int64_t n, int64_t k0, int j, int dtype, bool second_stage,
+                bool selects) {
+  constexpr double kBytes = 5.1e6, kSlowFolds = 1.2, kWaveLaunch = 3.6e-4;  // per us; us
+  constexpr double kTrip = 0.34, kLoad = 0.0087;          // us: a batch of loads, issuing one (a wave per SIMD)
+  constexpr double kHandOver = 0.008, kEntry = 0.067;     // us an entry of a lane: handed over, written
+  constexpr double kFold = 0.4, kFoldStep = 0.039;
+  constexpr double kSharedEnd = 0.18;                     // of a workgroup's end, where a CU has several
+  constexpr double kMerge = 2.8, kMergeStep = 0.097;
+  constexpr double kMergeSelect = 4.5, kMergeSelectEntry = 3.1e-4, kSelect = 6.0, kSelectEntry = 6.6e-4;
+  struct Push { double column, entry; };                  // us per sub-row (a wave per SIMD): a column, and per entry kept
+  const int es = elem_bytes(dtype);
+  const Push push = es == 1 ? Push{0.0067, 0.001} : es == 8 ? Push{0.0026, 0.029} : es == 4 ? Push{0.021, 0.0036}
+                    : pl.packed ? Push{0.019, 0.0} : Push{0.011, 0.0068};
+  const int loads = deep_loads_for_short_columns(dtype, j, pl.vec, pl.packed, pl.run, pl.full_rows)
+                        ? 8
+                        : loads_in_flight(dtype, j, pl.vec, pl.packed);
+  const double b = (double)(k0 / j), groups = (double)rows * pl.slabs * pl.col_tiles, waves = groups * pl.waves;
+  const double run = (double)pl.full_rows / pl.slabs / pl.waves;  // sub-rows a wave scans
+  const double bytes = (double)rows * (double)n * es + (double)rows * pl.slabs * (double)k0 * (es + 8);
+  // folded sub-rows of four-byte elements in rows cut into slabs: short queues wait for memory longer with 16-byte loads
+  // (20 such calls of 12 MiB and more: 9 % slower than one-element loads, where this estimate saw 2 % the other way)
+  const bool slow_folds = es == 4 && j <= 2 && pl.vec > 1 && pl.fold > 1 && pl.slabs > 1;
+  const double memory = bytes / kBytes * (slow_folds ? kSlowFolds : 1.0), launch = waves * kWaveLaunch;
+  const double trips = kTrip * (1 + (run > loads ? run / loads : 1.0));
+  const double pushes = run * (kLoad + pl.vec * (push.column + j * push.entry)) * (waves > 1024 ? waves / 1024 : 1.0);
+  double us = std::sqrt(memory * memory + launch * launch + trips * trips + pushes * pushes);
+  double end = (kHandOver * (pl.waves - 1) + kEntry) * j * pl.vec;
+  if (pl.fold > 1) {
+    uint32_t at_once = kWave;  // buckets (see fold_columns)
+    while (at_once > 1 && at_once / 2 >= b) at_once /= 2;
+    const double shares = (double)kWave / at_once;
+    end += kFold + kFoldStep * j * std::ceil(pl.fold / shares) * std::ceil(b / at_once);
   }
-  // small batches of 16-bit elements, whose waves have twice the columns to go through: fp16 [8, 301240] b=79 j=4
-  // 19.1 -> 15.3, [3, 2^20] b=256 j=2 16.6 -> 15.3, [4, 1618720] b=105 j=4 20.7 -> 13.7 (but no merge is worth
-  // having for it: [1, 65536] b=16 j=1 13.7 -> 16.8)
-  return es == 2 && (w.slabs > 1 || v.slabs == 1) && 2 * waves_v >= 3 * waves_w && groups <= 256 &&
-         bytes <= (j >= 2 && v.packed == w.packed ? 16 : 8) * mib;
+  us += end * (kSharedEnd * groups > 256 ? kSharedEnd * groups / 256 : 1.0);
+  if (pl.merge && selects) {
+    us += kMergeSelect + kMergeSelectEntry * (double)pl.slabs * (double)k0;
+  } else if (pl.merge) {
+    uint32_t at_once = kWave;  // buckets (as the launch chooses them)
+    while (at_once > 1 && (at_once / 2 >= b || (int64_t)pl.slabs * at_once > 32 * kMergeThreads)) at_once /= 2;
+    us += kMerge + kMergeStep * j * std::ceil((double)pl.slabs * at_once / kMergeThreads);
+  }
+  if (second_stage && !selects) us += kSelect + kSelectEntry * (double)k0 * (rows > 256 ? rows / 256.0 : 1.0);
+  return us;
 }
 }  // namespace
 
-Plan make_plan(int64_t rows, int64_t n, int64_t k0, int j, int layout, int dtype, bool wide) {
+Plan make_plan(int64_t rows, int64_t n, int64_t k0, int j, int layout, int dtype, bool wide, int64_t select_bound) {
   const Plan w = plan_with(rows, n, k0, j, layout, dtype, wide);
-  const int es = elem_bytes(dtype);
-  if (!w.ok || w.vec == 1 || (es != 2 && es != 4) || rows * (int64_t)w.slabs * w.col_tiles > kFewGroups ||
-      rows * n * es > kFewBytes)
-    return w;
+  if (!w.ok || w.vec == 1 || rows * n * elem_bytes(dtype) > kFewBytes) return w;
   const Plan v = plan_with(rows, n, k0, j, layout, dtype, false);
-  return v.ok && narrow_is_faster(w, v, rows, n, k0 / j, j, es) ? v : w;
+  if (!v.ok) return w;
+  auto us = [&](const Plan& pl) {
+    const bool second = select_bound > 0;
+    return estimate(pl, rows, n, k0, j, dtype, second, second && selects_in_merge(pl, k0, select_bound, dtype));
+  };
+  return us(v) < us(w) ? v : w;
 }
 
 bool selects_in_merge(const Plan& pl, int64_t k0, int64_t index_bound, int dtype) {
@@ -237,7 +261,8 @@ size_t stage1_stream_workspace_bytes(int64_t rows, int64_t n, int64_t k0, int j,
 bool describe_stage1_stream(const void* x, int64_t rows, int64_t n, int64_t k0, int j, int64_t k, int layout,
                             int dtype, int64_t index_bound, bool* selected, std::string& out) {
   *selected = false;
-  const stream::Plan pl = stream::make_plan(rows, n, k0, j, layout, dtype, stream::wide_loads(x, elem_bytes(dtype)));
+  const stream::Plan pl = stream::make_plan(rows, n, k0, j, layout, dtype, stream::wide_loads(x, elem_bytes(dtype)),
+                                            k < k0 ? index_bound : 0);
   if (!pl.ok) return false;
   const int loads = stream::deep_loads_for_short_columns(dtype, j, pl.vec, pl.packed, pl.run, pl.full_rows)
                         ? 8
@@ -259,7 +284,8 @@ bool describe_stage1_stream(const void* x, int64_t rows, int64_t n, int64_t k0, 
 int launch_stage1_stream(const void* x, int64_t rows, int64_t n, int64_t row_stride, int64_t k0, int j,
                          int layout, int dtype, void* values, IndexOut indices, void* ws,
                          size_t ws_bytes, hipStream_t stream, bool* handled, KeyRangeOut* ranges, SelectOut* last) {
-  const stream::Plan pl = stream::make_plan(rows, n, k0, j, layout, dtype, stream::wide_loads(x, elem_bytes(dtype)));
+  const stream::Plan pl = stream::make_plan(rows, n, k0, j, layout, dtype, stream::wide_loads(x, elem_bytes(dtype)),
+                                            last != nullptr ? last->index_bound : 0);
   *handled = pl.ok;
   if (!pl.ok) return ATK_OK;
   if (pl.ws_bytes && (!ws || ws_bytes < pl.ws_bytes || (uintptr_t)ws % 16 != 0)) return ATK_ERR_WORKSPACE;

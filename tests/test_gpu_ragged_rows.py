@@ -39,10 +39,9 @@ def test_bucket_counts_off_the_load_width(dtype, j):
             x = _data(3, n, dtype, 10 * b + j)
             want = oracle.topk(x, b * j, -1, j=j)
             assert_same(*topk(x.cuda(), b * j, -1, j=j), *want, f"b={b} n={n}")
-            # the same rows in a batch that keeps the 16-byte loads (small ones of 2- and 4-byte elements may not)
-            xd = x.cuda().repeat(90, 1)
-            if b >= 64 or j <= 2:   # (three and more of few buckets take narrow loads in batches of any size)
-                assert f"V={v}," in _native.describe(xd, b * j, j, b * j)
+            # the same rows in a batch that keeps the 16-byte loads: beyond 128 MiB all do
+            xd = x.cuda().repeat((1 << 27) // (3 * n * x.element_size()) + 1, 1)
+            assert f"V={v}," in _native.describe(xd, b * j, j, b * j)
             values, indices = topk(xd, b * j, -1, j=j)
             assert_same(values[-3:], indices[-3:], *want, f"many rows, b={b} n={n}")
 

@@ -309,3 +309,34 @@ def test_no_kernel_of_a_contiguous_call_has_more_threads_than_a_launch_takes():
     # two lanes to each of 146 buckets: 2^24 - 1 workgroups of 256 are the most
     assert describe(14708791, 2803, 0, 292, 2).startswith("split_bucket_kernel<f32")
     assert describe(14708792, 2803, 0, 292, 2).startswith("contig_kernel<f32")
+
+
+# (type code, rows, n, k, j, k_mult): calls timed with 16-byte and with one-element loads in one-stage and two-stage
+# kernels, at least 15 % apart: the planner takes the faster one
+NARROW = [
+    (0, 39, 761703, 40, 2, 1), (0, 16, 110067, 112, 2, 1), (0, 5, 119152, 572, 2, 1), (0, 5, 432090, 108, 3, 2),
+    (7, 17, 56249, 388, 4, 1), (7, 2, 1096704, 1764, 2, 1), (7, 1, 1896432, 64458, 2, 1),
+    (1, 5, 41786, 592, 4, 1), (2, 14, 75102, 424, 4, 1), (1, 10, 98448, 154, 2, 2), (2, 11, 3395763, 1088, 2, 1),
+    (1, 3, 15355401, 572, 4, 2),
+    (5, 1, 172601, 5240, 4, 1), (5, 1, 2514382, 20604, 4, 1), (5, 33, 511713, 1845, 3, 1), (5, 85, 84195, 520, 2, 1),
+    (4, 39, 152696, 804, 4, 1), (4, 26, 379453, 2120, 2, 1), (4, 5, 1954268, 525, 3, 1),
+    (3, 6, 108793, 1833, 3, 1), (3, 2, 310384, 3196, 4, 1), (8, 1, 112815, 1752, 4, 1), (8, 14, 71905, 112, 2, 1),
+]
+WIDE = [
+    (0, 71, 276112, 4172, 2, 1), (0, 128, 1 << 20, 65536, 2, 1),
+    (2, 3011, 15788, 1500, 3, 1), (1, 21, 1426304, 16676, 2, 1), (1, 65, 303684, 2924, 2, 1), (2, 17, 847929, 82694, 1, 1),
+    (6, 4, 12701536, 102288, 4, 1), (6, 26, 602919, 495, 1, 1), (2, 98, 1 << 19, 1024, 2, 2),
+    (5, 51, 507136, 7173, 3, 1), (4, 236, 122243, 220, 2, 4), (4, 51, 2066190, 7404, 3, 2),
+]
+
+
+@pytest.mark.parametrize("vec,calls", [("V=1,", NARROW), ("wide", WIDE)], ids=["narrow", "wide"])
+def test_the_width_of_loads_follows_the_faster_plan(vec, calls):
+    from approx_topk import _native
+    L = _native.lib()
+    for code, rows, n, k, j, k_mult in calls:
+        buf = ctypes.create_string_buffer(1024)
+        assert L.atk_describe(4096, rows, n, n, k * k_mult, j, k, 0, code, 4096, 4096, buf, 1024) == 0
+        text = buf.value.decode()
+        want = vec if vec != "wide" else f"V={min(8, 16 // [4, 2, 2, 8, 1, 1, 2, 4, 8][code])},"
+        assert text.startswith("stream_kernel<") and want in text, (rows, n, k, j, k_mult, text)
