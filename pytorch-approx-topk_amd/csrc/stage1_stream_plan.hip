@@ -33,9 +33,12 @@ constexpr int64_t kFoldMinLength = 8;
 // that it wins and loses (fp32 [1, 2^22] k=64 j=4 k_mult=2, 32768 entries, 27.4 -> 24.1 us; k=500 j=2 k_mult=4,
 // 64000 entries, 19.9 -> 26.5; k=256 j=4 k_mult=4, 262144, 30.7 -> 58.0).
 constexpr int64_t kMergeSelectMax = 2048, kMergeSelectEntries = 16384;
-// Most bytes of a call that may take one-element loads where 16-byte loads are possible (see estimate): as far as
-// both were timed.
-constexpr int64_t kFewBytes = 128 << 20;
+// Calls of more bytes than this (kLargeEight: of eight-byte elements) take one-element loads only where their estimate
+// is that share of the other (see estimate): what counts there is memory, of which the estimate sees little.
+// 150 calls of 128 to 640 MiB: 1.6 % slower than the better one in the mean, 16-byte loads throughout 3.4 %,
+// one-element loads 27 % (fp16 [136579, 2311] b=4 j=4 679 us wide, 425 narrow, fp32 [17703, 2921] b=66 j=4 112 and 82).
+constexpr int64_t kLargeBytes = 128 << 20, kLargeEight = 48 << 20;
+constexpr double kLargeShare = 0.92;
 // Buckets from this length on are folded whatever the fold.
 constexpr int64_t kFoldAnyLength = 128;
 
@@ -231,14 +234,16 @@ double estimate(const Plan& pl, int64_t rows, int64_t n, int64_t k0, int j, int 
 
 Plan make_plan(int64_t rows, int64_t n, int64_t k0, int j, int layout, int dtype, bool wide, int64_t select_bound) {
   const Plan w = plan_with(rows, n, k0, j, layout, dtype, wide);
-  if (!w.ok || w.vec == 1 || rows * n * elem_bytes(dtype) > kFewBytes) return w;
+  if (!w.ok || w.vec == 1) return w;
   const Plan v = plan_with(rows, n, k0, j, layout, dtype, false);
   if (!v.ok) return w;
   auto us = [&](const Plan& pl) {
     const bool second = select_bound > 0;
     return estimate(pl, rows, n, k0, j, dtype, second, second && selects_in_merge(pl, k0, select_bound, dtype));
   };
-  return us(v) < us(w) ? v : w;
+  const int es = elem_bytes(dtype);
+  const bool large = rows * n * es > (es == 8 ? kLargeEight : kLargeBytes);
+  return us(v) < us(w) * (large ? kLargeShare : 1.0) ? v : w;
 }
 
 bool selects_in_merge(const Plan& pl, int64_t k0, int64_t index_bound, int dtype) {
