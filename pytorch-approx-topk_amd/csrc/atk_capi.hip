@@ -247,7 +247,7 @@ size_t atk_topk_workspace_bytes(int64_t rows, int64_t n, int64_t k0, int j, int6
 size_t atk_topk_workspace_bytes_used(const void* x, int64_t rows, int64_t n, int64_t row_stride, int64_t k0,
                                      int j, int64_t k, int layout, int dtype) {
   if (rows > 0 && k > 0 && k < k0 && check_stage1(x, rows, n, row_stride, k0, j, layout, dtype, x, x) == ATK_OK &&
-      atk::fused_row_takes(x, rows, n, k0, j, k, layout, dtype))
+      atk::fused_row_takes(x, rows, n, row_stride, k0, j, k, layout, dtype))
     return 0;
   return plan_topk(rows, n, k0, j, k, layout, dtype).total;
 }
@@ -299,7 +299,7 @@ int atk_describe(const void* x, int64_t rows, int64_t n, int64_t row_stride, int
   std::string out;
   if (rows != 0 && k != 0) {
     bool fused = false;
-    if (k < k0) fused = atk::describe_fused_row(x, rows, n, k0, j, k, layout, dtype, out);
+    if (k < k0) fused = atk::describe_fused_row(x, rows, n, row_stride, k0, j, k, layout, dtype, out);
     if (!fused) {
       bool selected = false;
       if (!atk::describe_stage1_stream(x, rows, n, k0, j, k, layout, dtype, index_bound_of(n, k0, layout), &selected,

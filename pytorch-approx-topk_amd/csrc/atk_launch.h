@@ -64,8 +64,9 @@ int launch_stage1_contig(const void* x, int64_t rows, int64_t n, int64_t row_str
                          int layout, int dtype, void* values, IndexOut indices, void* ws, size_t ws_bytes,
                          hipStream_t stream, bool* handled);
 
-// Whether launch_fused_row takes this very call (the input's address decides with the shape).
-bool fused_row_takes(const void* x, int64_t rows, int64_t n, int64_t k0, int j, int64_t k, int layout, int dtype);
+// Whether launch_fused_row takes this very call (where its rows start decides with the shape).
+bool fused_row_takes(const void* x, int64_t rows, int64_t n, int64_t row_stride, int64_t k0, int j, int64_t k,
+                     int layout, int dtype);
 // fused_row_plan.hip: both stages in one kernel, one workgroup per row, for
 // batches of many rows whose candidates fit in LDS.  `*handled` as above.
 int launch_fused_row(const void* x, int64_t rows, int64_t n, int64_t row_stride, int64_t k0, int j,
@@ -122,8 +123,8 @@ bool describe_stage1_stream(const void* x, int64_t rows, int64_t n, int64_t k0, 
 bool describe_stage1_contig(const void* x, int64_t rows, int64_t n, int64_t row_stride, int64_t k0, int j,
                             int layout, int dtype, std::string& out);
 void describe_stage1_lane_per_bucket(int64_t rows, int64_t k0, int j, int dtype, std::string& out);
-bool describe_fused_row(const void* x, int64_t rows, int64_t n, int64_t k0, int j, int64_t k, int layout, int dtype,
-                        std::string& out);
+bool describe_fused_row(const void* x, int64_t rows, int64_t n, int64_t row_stride, int64_t k0, int j, int64_t k,
+                        int layout, int dtype, std::string& out);
 bool describe_multi_select(int64_t rows, int64_t k0, int64_t k, int64_t index_bound, int dtype, std::string& out);
 bool describe_chain_select(int64_t rows, int64_t k0, int64_t k, int64_t index_bound, int dtype, std::string& out);
 void describe_select(int64_t rows, int64_t k0, int64_t k, int64_t index_bound, int dtype, bool with_workspace,

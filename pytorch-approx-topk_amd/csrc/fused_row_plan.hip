@@ -32,6 +32,25 @@ constexpr int64_t kManyRows = 1024, kAllCus = 256;
 // Longest contiguous bucket (bytes) the register kernel takes.
 constexpr int64_t kShortBucket = 256;
 constexpr size_t kShortRow = 128 * 1024, kLongRow = 512 * 1024;
+
+// Whether rows that do not all start on 16 bytes are faster in one kernel.  256 calls of such rows timed against the
+// two kernels (with the width of loads that the planner takes there): what decides is how many sub-rows a wave
+// goes through (`run`, over all its tiles), for which the two kernels have any number of workgroups.
+//   Fewer rows than kMinRows: runs of up to 40 sub-rows with queues of one or two entries, of up to 20 with more, and
+//   sub-rows of 256 bytes (fp16 [75, 42783] b=952 j=2, run 22, 15.6 -> 11.0 us, [16, 45917] b=1276, run 36, 10.9 -> 8.1, but
+//   [5, 104575] b=392 j=2, run 67, 10.2 -> 15.7, bf16 [4, 118981] b=1072 j=3, run 111, 13.5 -> 19.9, [7, 2193] b=16 j=4
+//   9.0 -> 11.8); longer queues of eight-byte elements lose throughout (fp64 [14, 3303] b=32 j=4 13.6 -> 25.2).
+//   Fewer rows than CUs: runs of up to 256 (fp32 [193, 82525] b=680 j=3, run 60, 29.1 -> 23.0; fp16 [183, 340470] b=304
+//   j=4, run 280, 49.7 -> 59, i16 [152, 394615] b=1140 j=4, run 346, 49.9 -> 60.3).
+//   More rows: all (fp16 [742, 9559] b=264 15.4 -> 11.0, bf16 [552, 6915] b=132 j=4 17.4 -> 12.4, i16 [759, 57865]
+//   b=448 j=4 48.4 -> 42.1).
+//   One-byte elements, whose packed queues this kernel lacks: batches with queues of one or two entries (uint8 [1354, 66483]
+//   j=1 67.0 -> 50.5, [374, 23585] j=2 23.4 -> 19.2, but [1538, 37707] j=4 74 -> 214, [11, 10433] j=4 10.6 -> 40.7).
+bool loose_rows_gain(int64_t rows, int64_t sub_row_bytes, int64_t run, int j, int es) {
+  if (es == 1) return rows >= kMinRows && j <= 2;
+  if (rows >= kMinRows) return rows >= kAllCus || run <= 256;
+  return run <= (j <= 2 ? 40 : es == 8 ? 0 : 20) && sub_row_bytes >= 256;
+}
 }  // namespace
 
 // Staged results leave in non-temporal stores when the launch is one round of workgroups
@@ -94,7 +113,7 @@ static Plan plan_short_buckets(int64_t rows, int64_t n, int64_t k0, int j, int64
   return pl;
 }
 
-Plan make_plan(int64_t rows, int64_t n, int64_t k0, int j, int64_t k, int layout, int dtype, bool wide) {
+Plan make_plan(int64_t rows, int64_t n, int64_t k0, int j, int64_t k, int layout, int dtype, bool wide, bool aligned) {
   Plan pl{};
   pl.ok = false;
   if (layout == ATK_BALANCED) return plan_short_buckets(rows, n, k0, j, k, dtype, wide);
@@ -195,6 +214,8 @@ Plan make_plan(int64_t rows, int64_t n, int64_t k0, int j, int64_t k, int layout
   }
   pl.split = split;
   pl.waves = pl.tiles * split <= max_waves ? pl.tiles * split : max_waves;
+  const int64_t turns = ((int64_t)pl.tiles * split + pl.waves - 1) / pl.waves;
+  if (!aligned && !loose_rows_gain(rows, b * es, full / split * turns, j, es)) return pl;
   const bool one_round = pl.tiles * split <= max_waves;
   pl.hand_off = (split > 1 && !one_round) ? (uint32_t)cand_bytes : 0u;
   pl.lds_bytes = lds_need(split);
@@ -214,18 +235,22 @@ Plan make_plan(int64_t rows, int64_t n, int64_t k0, int j, int64_t k, int layout
 
 namespace {
 // Rows may start at any element (a row of odd length does): the 16-byte loads take such addresses.
-fused::Plan plan_for(const void* x, int64_t rows, int64_t n, int64_t k0, int j, int64_t k, int layout, int dtype) {
-  return fused::make_plan(rows, n, k0, j, k, layout, dtype, stream::wide_loads(x, elem_bytes(dtype)));
+fused::Plan plan_for(const void* x, int64_t rows, int64_t n, int64_t row_stride, int64_t k0, int j, int64_t k,
+                     int layout, int dtype) {
+  const int es = elem_bytes(dtype);
+  const bool aligned = (uintptr_t)x % 16 == 0 && (row_stride * es) % 16 == 0;
+  return fused::make_plan(rows, n, k0, j, k, layout, dtype, stream::wide_loads(x, es), aligned);
 }
 }  // namespace
 
-bool fused_row_takes(const void* x, int64_t rows, int64_t n, int64_t k0, int j, int64_t k, int layout, int dtype) {
-  return plan_for(x, rows, n, k0, j, k, layout, dtype).ok;
+bool fused_row_takes(const void* x, int64_t rows, int64_t n, int64_t row_stride, int64_t k0, int j, int64_t k,
+                     int layout, int dtype) {
+  return plan_for(x, rows, n, row_stride, k0, j, k, layout, dtype).ok;
 }
 
-bool describe_fused_row(const void* x, int64_t rows, int64_t n, int64_t k0, int j, int64_t k, int layout, int dtype,
-                        std::string& out) {
-  const fused::Plan pl = plan_for(x, rows, n, k0, j, k, layout, dtype);
+bool describe_fused_row(const void* x, int64_t rows, int64_t n, int64_t row_stride, int64_t k0, int j, int64_t k,
+                        int layout, int dtype, std::string& out) {
+  const fused::Plan pl = plan_for(x, rows, n, row_stride, k0, j, k, layout, dtype);
   if (!pl.ok) return false;
   out += std::string(pl.in_registers ? "fused_regs_kernel<" : "fused_row_kernel<") + dtype_name(dtype) + ", J=" +
          std::to_string(j) + ", V=" + std::to_string(pl.vec) + ", pos" + (pl.pos16 ? "16" : "32") +
@@ -239,7 +264,7 @@ bool describe_fused_row(const void* x, int64_t rows, int64_t n, int64_t k0, int 
 int launch_fused_row(const void* x, int64_t rows, int64_t n, int64_t row_stride, int64_t k0, int j,
                      int64_t k, int layout, int dtype, void* values, IndexOut indices, hipStream_t stream,
                      bool* handled) {
-  const fused::Plan pl = plan_for(x, rows, n, k0, j, k, layout, dtype);
+  const fused::Plan pl = plan_for(x, rows, n, row_stride, k0, j, k, layout, dtype);
   *handled = pl.ok;
   if (!pl.ok) return ATK_OK;
   int rc = ATK_ERR_DTYPE;

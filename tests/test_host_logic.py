@@ -340,3 +340,31 @@ def test_the_width_of_loads_follows_the_faster_plan(vec, calls):
         text = buf.value.decode()
         want = vec if vec != "wide" else f"V={min(8, 16 // [4, 2, 2, 8, 1, 1, 2, 4, 8][code])},"
         assert text.startswith("stream_kernel<") and want in text, (rows, n, k, j, k_mult, text)
+
+
+# the same for rows off 16 bytes with a second stage, timed in one kernel and in two
+ONE_KERNEL = [
+    (8, 254, 2501, 36, 2, 8), (8, 3, 24169, 358, 1, 2), (3, 206, 5521, 116, 1, 2), (6, 760, 2813, 41, 1, 4),
+    (6, 100, 7861, 184, 4, 4), (8, 137, 10039, 452, 4, 2), (1, 288, 15375, 60, 2, 8), (1, 75, 42783, 476, 2, 4),
+    (1, 742, 9559, 33, 1, 8), (7, 3312, 2349, 126, 1, 2), (0, 307, 18439, 304, 2, 2), (4, 1354, 66483, 286, 1, 8),
+    (7, 171, 121527, 3366, 3, 4), (3, 170, 93177, 560, 2, 8), (2, 256, 100003, 64, 1, 8),
+]
+TWO_KERNELS = [
+    (4, 11, 10433, 128, 4, 4), (4, 1538, 37707, 400, 4, 8), (7, 33, 2131, 56, 4, 2), (3, 14, 3303, 16, 4, 8),
+    (5, 2, 92341, 784, 4, 8), (1, 5, 104575, 196, 2, 4), (7, 3, 35717, 196, 4, 8), (2, 4, 118981, 402, 3, 8),
+    (1, 2, 122721, 2580, 1, 2), (2, 7, 2193, 16, 4, 4), (1, 168, 298475, 544, 4, 4), (1, 9, 6995, 32, 2, 2),
+    (0, 37, 2557, 24, 3, 2), (6, 152, 394615, 2280, 4, 2), (1, 183, 340470, 152, 4, 8),
+]
+
+
+@pytest.mark.parametrize("kernel,calls", [("fused_", ONE_KERNEL), ("stream_kernel<", TWO_KERNELS)], ids=["one", "two"])
+def test_rows_off_16_bytes_take_one_kernel_where_that_is_faster(kernel, calls):
+    from approx_topk import _native
+    L = _native.lib()
+    for code, rows, n, k, j, k_mult in calls:
+        buf = ctypes.create_string_buffer(1024)
+        args = (rows, n, n, k * k_mult, j, k, 0, code)
+        assert L.atk_describe(4096, *args, 4096, 4096, buf, 1024) == 0
+        assert buf.value.decode().startswith(kernel), (args, buf.value)
+        # the workspace follows, also where the rows are those of a wider matrix
+        assert (L.atk_topk_workspace_bytes_used(4096, *args) == 0) == (kernel == "fused_")
