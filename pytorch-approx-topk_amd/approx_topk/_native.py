@@ -259,8 +259,8 @@ MAX_GRAD_ROW = (1 << 31) - 1
 
 def check_grad_tensors(grad_values: torch.Tensor, indices: torch.Tensor) -> None:
     """What the gradient's kernel takes for granted: it reads as many gradients as indices, of eight bytes."""
-    if (indices.dtype != torch.int64 or grad_values.shape != indices.shape or grad_values.device != indices.device
-            or indices.ndim == 0):
+    if (indices.dtype is not torch.int64 or grad_values.shape != indices.shape or indices.ndim == 0
+            or grad_values.device != indices.device):
         raise RuntimeError(
             "topk_grad: expected int64 indices and gradients of the same shape on one device, got "
             f"{indices.dtype} {tuple(indices.shape)} on {indices.device} and {tuple(grad_values.shape)} on "
@@ -273,15 +273,17 @@ def topk_grad(grad_values: torch.Tensor, indices: torch.Tensor, n: int, k0: int,
     check_grad_tensors(grad_values, indices)
     require_gpu(grad_values)
     grad_values, indices = grad_values.contiguous(), indices.contiguous()
-    k = indices.shape[-1]
-    grad_x = torch.empty(indices.shape[:-1] + (n,), dtype=grad_values.dtype, device=grad_values.device)
-    if indices.numel() == 0:
+    shape = indices.shape
+    grad_x = grad_values.new_empty((*shape[:-1], n))
+    entries, k = indices.numel(), shape[-1]
+    if entries == 0:
         return grad_x.zero_()
-    with _on_device(grad_values.device):
-        status = lib().atk_topk_grad(grad_values.data_ptr(), indices.data_ptr(), indices.numel() // k, n, k0, j, k,
-                                     layout, dtype_code(grad_values.dtype), grad_x.data_ptr(),
-                                     _stream(grad_values.device))
-    check(status)
+    device = grad_values.device
+    with _on_device(device):
+        status = lib().atk_topk_grad(grad_values.data_ptr(), indices.data_ptr(), entries // k, n, k0, j, k, layout,
+                                     dtype_code(grad_values.dtype), grad_x.data_ptr(), _stream(device))
+    if status != 0:
+        check(status)
     return grad_x
 
 

@@ -16,8 +16,11 @@ when every bucket is kept whole.
 from __future__ import annotations
 
 import torch
-from torch import Tensor
+from torch import Tensor, is_grad_enabled
+from torch._C import _AutoDispatchBelowAutograd
+from torch._C._functorch import peek_interpreter_stack
 from torch.autograd import forward_ad
+from torch.compiler import is_compiling
 
 from .. import _native
 from ..priority_queue import topk as _topk, topk_grad as _topk_grad
@@ -26,8 +29,8 @@ from ..priority_queue import topk as _topk, topk_grad as _topk_grad
 def _autograd_has_work(grad_values: Tensor) -> bool:
     """Whether the gradient may itself be differentiated or traced: reverse mode, forward mode (both kinds enter
     a level), a functorch transform, or ``torch.compile``, which does not look into dispatcher guards."""
-    return ((torch.is_grad_enabled() and grad_values.requires_grad) or forward_ad._current_level >= 0
-            or torch._C._functorch.peek_interpreter_stack() is not None or torch.compiler.is_compiling())
+    return ((is_grad_enabled() and grad_values.requires_grad) or forward_ad._current_level >= 0
+            or peek_interpreter_stack() is not None or is_compiling())
 
 
 class _TopkWithGradient(torch.autograd.Function):
@@ -52,7 +55,7 @@ class _TopkWithGradient(torch.autograd.Function):
             if _autograd_has_work(grad_values):
                 grad_xs = _topk_grad(grad_values, indices, shape[-1], *ctx.buckets)
             else:  # the operator's autograd kernel would find nothing to do, in 6 us of host time
-                with torch._C._AutoDispatchBelowAutograd():
+                with _AutoDispatchBelowAutograd():
                     grad_xs = _topk_grad(grad_values, indices, shape[-1], *ctx.buckets)
         elif len(shape) == 0:
             grad_xs = grad_values.reshape(()) if indices.numel() else grad_values.new_zeros(())
