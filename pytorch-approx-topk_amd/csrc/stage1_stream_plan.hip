@@ -35,10 +35,10 @@ constexpr int64_t kFoldMinLength = 8;
 constexpr int64_t kMergeSelectMax = 2048, kMergeSelectEntries = 16384;
 // Calls of more bytes than this (kLargeEight: of eight-byte elements) take one-element loads only where their estimate
 // is that share of the other (see estimate): what counts there is memory, of which the estimate sees little.
-// 150 calls of 128 to 640 MiB: 1.6 % slower than the better one in the mean, 16-byte loads throughout 3.4 %,
+// 150 calls of 128 to 640 MiB: 1.4 % slower than the better one in the mean, 16-byte loads throughout 3.4 %,
 // one-element loads 27 % (fp16 [136579, 2311] b=4 j=4 679 us wide, 425 narrow, fp32 [17703, 2921] b=66 j=4 112 and 82).
 constexpr int64_t kLargeBytes = 128 << 20, kLargeEight = 48 << 20;
-constexpr double kLargeShare = 0.92;
+constexpr double kLargeShare = 0.95;
 // Buckets from this length on are folded whatever the fold.
 constexpr int64_t kFoldAnyLength = 128;
 
@@ -177,11 +177,11 @@ namespace {
 //   the scan: memory, instructions, the launch of the waves and the round trips of a wave's loads, which overlap
 //     (the root of the sum of their squares);
 //   a workgroup's end: the other waves' queues folded into the leading wave's, folded columns put together, and a
-//     lane's entries written, side by side with other workgroups on the CU;
+//     lane's entries written, by one wave, next to the ends and scans of the workgroups that the CU holds with it;
 //   the launches behind it: the merge of the slabs, with or without the second stage, or the stand-alone select.
 // The constants are a least-squares fit to 2070 calls timed both ways (all nine types, 1-20000 rows of 37 to 2^24
 // elements, up to 128 MiB, j 1-4, k_mult 1-8, half of them few rows, most of them off 16 bytes).  Its choice is
-// 1.0 % slower than the better one of the two in the geometric mean (10 % and more in one call of 22), 16-byte loads
+// 1.0 % slower than the better one of the two in the geometric mean (10 % and more in one call of 24), 16-byte loads
 // throughout 14 %, one-element loads throughout 6 %: fp32 [3, 2^21] b=128 j=4 k_mult=8 30.2 us wide, 17.9 narrow, int8
 // [1, 172601] b=1310 j=4 8.5 and 4.0, uint8 [39, 152696] b=201 j=4 14.7 and 8.6, fp64 [2, 310384] b=799 j=4 13.6 and
 // 11.1, fp16 [168, 298475] b=544 j=4 67.9 and 42.1, but int8 [51, 507136] b=2391 j=3 11.5 and 17.4, fp16 [21, 1426304]
@@ -192,7 +192,6 @@ double estimate(const Plan& pl, int64_t rows, int64_t n, int64_t k0, int j, int 
   constexpr double kTrip = 0.34, kLoad = 0.0087;          // us: a batch of loads, issuing one (a wave per SIMD)
   constexpr double kHandOver = 0.008, kEntry = 0.067;     // us an entry of a lane: handed over, written
   constexpr double kFold = 0.4, kFoldStep = 0.039;
-  constexpr double kSharedEnd = 0.18;                     // of a workgroup's end, where a CU has several
   constexpr double kMerge = 2.8, kMergeStep = 0.097;
   constexpr double kMergeSelect = 4.5, kMergeSelectEntry = 3.1e-4, kSelect = 6.0, kSelectEntry = 6.6e-4;
   struct Push { double column, entry; };                  // us per sub-row (a wave per SIMD): a column, and per entry kept
@@ -219,7 +218,13 @@ double estimate(const Plan& pl, int64_t rows, int64_t n, int64_t k0, int j, int 
     const double shares = (double)kWave / at_once;
     end += kFold + kFoldStep * j * std::ceil(pl.fold / shares) * std::ceil(b / at_once);
   }
-  us += end * (kSharedEnd * groups > 256 ? kSharedEnd * groups / 256 : 1.0);
+  // workgroups that a CU holds: by their LDS, and sixteen waves with 16-byte loads, twice as many with one-element loads
+  const int entry_bytes = pl.packed ? 4 : (es > 4 ? 8 : 4) + 4;
+  const double hand = (double)merge_lds_bytes(pl.vec, j, pl.waves, entry_bytes);
+  const double words = (double)kWave * pl.vec * j * (es == 8 ? 16 : 8);
+  const double by_lds = 160 * 1024 / (hand > words ? hand : words), by_waves = (pl.vec > 1 ? 16.0 : 32.0) / pl.waves;
+  const double held = by_lds < by_waves ? (by_lds > 1 ? by_lds : 1.0) : by_waves;
+  us += end * (groups > 256 * held ? groups / (256 * held) : 1.0);
   if (pl.merge && selects) {
     us += kMergeSelect + kMergeSelectEntry * (double)pl.slabs * (double)k0;
   } else if (pl.merge) {
@@ -235,6 +240,9 @@ double estimate(const Plan& pl, int64_t rows, int64_t n, int64_t k0, int j, int 
 Plan make_plan(int64_t rows, int64_t n, int64_t k0, int j, int layout, int dtype, bool wide, int64_t select_bound) {
   const Plan w = plan_with(rows, n, k0, j, layout, dtype, wide);
   if (!w.ok || w.vec == 1) return w;
+  // whole-wave stores spare the lanes' entries most of what the estimate takes for them; with half of the lanes at work
+  // they stay ahead (i8 [4475, 6579] b=320 j=2 42.8 us, 56.5 with one-element loads; bf16 [10470, 6399] b=136 j=4 163 and 114)
+  if (w.wave_stores && 2 * w.width >= (int64_t)w.col_tiles * kWave * w.vec) return w;
   const Plan v = plan_with(rows, n, k0, j, layout, dtype, false);
   if (!v.ok) return w;
   auto us = [&](const Plan& pl) {
