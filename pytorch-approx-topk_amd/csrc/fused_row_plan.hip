@@ -39,7 +39,9 @@ constexpr size_t kShortRow = 128 * 1024, kLongRow = 512 * 1024;
 //   Fewer rows than kMinRows: runs of up to 40 sub-rows with queues of one or two entries, of up to 20 with more, and
 //   sub-rows of 256 bytes (fp16 [75, 42783] b=952 j=2, run 22, 15.6 -> 11.0 us, [16, 45917] b=1276, run 36, 10.9 -> 8.1, but
 //   [5, 104575] b=392 j=2, run 67, 10.2 -> 15.7, bf16 [4, 118981] b=1072 j=3, run 111, 13.5 -> 19.9, [7, 2193] b=16 j=4
-//   9.0 -> 11.8); longer queues of eight-byte elements lose throughout (fp64 [14, 3303] b=32 j=4 13.6 -> 25.2).
+//   9.0 -> 11.8); longer queues with sub-rows of 2.5 KB and more, runs of up to 64 (i16 [46, 72589] b=1428 j=4, run 50,
+//   17.3 -> 14.0; f32 [14, 51519] b=344 j=4, run 37, 13.5 -> 16.8); of eight-byte elements they lose throughout (fp64
+//   [14, 3303] b=32 j=4 13.6 -> 25.2).
 //   Fewer rows than CUs: runs of up to 256 (fp32 [193, 82525] b=680 j=3, run 60, 29.1 -> 23.0; fp16 [183, 340470] b=304
 //   j=4, run 280, 49.7 -> 59, i16 [152, 394615] b=1140 j=4, run 346, 49.9 -> 60.3).
 //   More rows: all (fp16 [742, 9559] b=264 15.4 -> 11.0, bf16 [552, 6915] b=132 j=4 17.4 -> 12.4, i16 [759, 57865]
@@ -49,7 +51,7 @@ constexpr size_t kShortRow = 128 * 1024, kLongRow = 512 * 1024;
 bool loose_rows_gain(int64_t rows, int64_t sub_row_bytes, int64_t run, int j, int es) {
   if (es == 1) return rows >= kMinRows && j <= 2;
   if (rows >= kMinRows) return rows >= kAllCus || run <= 256;
-  return run <= (j <= 2 ? 40 : es == 8 ? 0 : 20) && sub_row_bytes >= 256;
+  return run <= (j <= 2 ? 40 : es == 8 ? 0 : sub_row_bytes >= 2560 ? 64 : 20) && sub_row_bytes >= 256;
 }
 }  // namespace
 

@@ -347,7 +347,7 @@ ONE_KERNEL = [
     (8, 254, 2501, 36, 2, 8), (8, 3, 24169, 358, 1, 2), (3, 206, 5521, 116, 1, 2), (6, 760, 2813, 41, 1, 4),
     (6, 100, 7861, 184, 4, 4), (8, 137, 10039, 452, 4, 2), (1, 288, 15375, 60, 2, 8), (1, 75, 42783, 476, 2, 4),
     (1, 742, 9559, 33, 1, 8), (7, 3312, 2349, 126, 1, 2), (0, 307, 18439, 304, 2, 2), (4, 1354, 66483, 286, 1, 8),
-    (7, 171, 121527, 3366, 3, 4), (3, 170, 93177, 560, 2, 8), (2, 256, 100003, 64, 1, 8),
+    (7, 171, 121527, 3366, 3, 4), (3, 170, 93177, 560, 2, 8), (2, 256, 100003, 64, 1, 8), (6, 46, 72589, 714, 4, 8),
 ]
 TWO_KERNELS = [
     (4, 11, 10433, 128, 4, 4), (4, 1538, 37707, 400, 4, 8), (7, 33, 2131, 56, 4, 2), (3, 14, 3303, 16, 4, 8),
