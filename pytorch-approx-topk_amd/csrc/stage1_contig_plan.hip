@@ -10,6 +10,8 @@ constexpr int64_t kTargetGroups = 1024;
 // split_bucket_kernel: buckets of a launch from which on a wave may take more than kFewTurns turns
 // at its bucket, and from which on buckets shorter than one piece go there.
 constexpr int64_t kManyWaves = 512, kFewTurns = 8, kManyBuckets = 16384;
+// The same for queues of three or four entries of four bytes, from kFewTurns turns on.
+constexpr int64_t kManyLong = 1024;
 // Workgroups whose threads a launch can count (in 32 bits); contig_kernel gives a short bucket fewer lanes.
 constexpr int64_t kMostGroups = 0xffffffffll / kThreads;
 }  // namespace
@@ -107,7 +109,8 @@ Plan make_plan(int64_t rows, int64_t n, int64_t k0, int j, int layout, int dtype
   //   buckets of which more than a quarter is kept, three or four elements each (fp32 [256, 100003] k=50000 j=4
   //   68.6 against 76.2 us; with j=2 and buckets of 16 bytes 64.4 against 46.5);
   //   few buckets that a wave would need many turns for (200 of 40 KB in one row 11.9 against 13.4 us, but 800 in
-  //   four rows 17.3 against 13.9);
+  //   four rows 17.3 against 13.9), and with queues of three or four four-byte entries up to twice as many (128 of 28 KB,
+  //   j=4 7.5 against 10.4 us, 512 of 50 KB 16.0 against 20.8; 1024 of 63 KB 25.1 against 25.4, 2048 of 28 KB 23.9 against 17.2);
   //   small launches of short buckets, which take the same either way (fp32 [64, 8200] k=1024 j=2 11.7 against 11.5).
   g.split = 0;
   if (wide && (es == 2 || es == 4) && !g.whole && !g.fast && (layout == ATK_BALANCED || b * m == n) &&
@@ -116,8 +119,10 @@ Plan make_plan(int64_t rows, int64_t n, int64_t k0, int j, int layout, int dtype
     uint32_t pieces_log2 = 0;
     while (((longest + (1ll << pieces_log2) - 1) >> pieces_log2) * es > (int64_t)kSplitBytes) ++pieces_log2;
     g.split_log2 = pieces_log2;
-    if ((m >> pieces_log2) * es >= 16 && ((1 << pieces_log2) <= kFewTurns * stream::kWave || rows * b >= kManyWaves) &&
-        bucket_groups(g, rows) <= kMostGroups) {
+    const int64_t turns = (1ll << pieces_log2) / stream::kWave;
+    const bool long_queues = es == 4 && j >= 3 && turns >= kFewTurns;
+    if ((m >> pieces_log2) * es >= 16 && (turns <= kFewTurns || rows * b >= kManyWaves) &&
+        (!long_queues || rows * b >= kManyLong) && bucket_groups(g, rows) <= kMostGroups) {
       g.split = 1;
       g.split_trip = (uint32_t)((longest + (1ll << pieces_log2) - 1) >> pieces_log2);
       g.slabs = 1;

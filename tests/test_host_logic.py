@@ -368,3 +368,22 @@ def test_rows_off_16_bytes_take_one_kernel_where_that_is_faster(kernel, calls):
         assert buf.value.decode().startswith(kernel), (args, buf.value)
         # the workspace follows, also where the rows are those of a wider matrix
         assert (L.atk_topk_workspace_bytes_used(4096, *args) == 0) == (kernel == "fused_")
+
+
+def test_few_long_contiguous_buckets_with_long_queues_keep_workgroups_of_their_own():
+    # (a lane of split_bucket_kernel goes through eight pieces and more of such a bucket, queue and all)
+    from approx_topk import _native
+    L = _native.lib()
+
+    def kernel(rows, m, b, j, code):
+        n = b * m + b // 2
+        buf = ctypes.create_string_buffer(1024)
+        assert L.atk_describe(4096, rows, n, n, b * j, j, b * j, 1, code, 4096, 4096, buf, 1024) == 0
+        return buf.value.decode().split("_kernel")[0]
+
+    for code in (0, 7):
+        assert kernel(4, 7169, 32, 4, code) == kernel(1, 4353, 32, 3, code) == kernel(512, 16129, 1, 4, code) == "contig"
+        assert kernel(32, 7169, 32, 4, code) == kernel(4, 4001, 32, 4, code) == "split_bucket"     # many; fewer pieces
+        assert kernel(4, 7169, 32, 2, code) == "split_bucket"                                       # short queues
+    for code in (1, 2, 6):
+        assert kernel(4, 14337, 32, 4, code) == kernel(1, 8705, 32, 3, code) == "split_bucket"      # 16-bit elements
