@@ -302,7 +302,7 @@ int atk_describe(const void* x, int64_t rows, int64_t n, int64_t row_stride, int
     if (k < k0) fused = atk::describe_fused_row(x, rows, n, row_stride, k0, j, k, layout, dtype, out);
     if (!fused) {
       bool selected = false;
-      if (!atk::describe_stage1_stream(x, rows, n, k0, j, k, layout, dtype, index_bound_of(n, k0, layout), &selected,
+      if (!atk::describe_stage1_stream(rows, n, k0, j, k, layout, dtype, index_bound_of(n, k0, layout), &selected,
                                        out) &&
           !atk::describe_stage1_contig(x, rows, n, row_stride, k0, j, layout, dtype, out))
         atk::describe_stage1_lane_per_bucket(rows, k0, j, dtype, out);

@@ -118,7 +118,7 @@ int launch_topk_grad(const void* grad_values, const int64_t* indices, int64_t ro
 // the call; they enqueue nothing.
 const char* dtype_name(int dtype);
 // `*selected`: the second stage is among the kernels named.
-bool describe_stage1_stream(const void* x, int64_t rows, int64_t n, int64_t k0, int j, int64_t k, int layout,
+bool describe_stage1_stream(int64_t rows, int64_t n, int64_t k0, int j, int64_t k, int layout,
                             int dtype, int64_t index_bound, bool* selected, std::string& out);
 bool describe_stage1_contig(const void* x, int64_t rows, int64_t n, int64_t row_stride, int64_t k0, int j,
                             int layout, int dtype, std::string& out);

@@ -713,8 +713,8 @@ struct Plan {
   bool past_cache;      // staged: ... in non-temporal stores (one round of workgroups with a sizeable output)
 };
 
-// `wide`: 16-byte loads may be used (stream::wide_loads); `aligned`: every row starts on 16 bytes.
-Plan make_plan(int64_t rows, int64_t n, int64_t k0, int j, int64_t k, int layout, int dtype, bool wide, bool aligned);
+// `aligned`: every row starts on 16 bytes.
+Plan make_plan(int64_t rows, int64_t n, int64_t k0, int j, int64_t k, int layout, int dtype, bool aligned);
 
 template <typename E>
 int launch_typed(const Plan& pl, const void* x, int64_t rows, int64_t row_stride, int64_t k0, int j,

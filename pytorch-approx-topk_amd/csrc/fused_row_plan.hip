@@ -78,10 +78,10 @@ static bool stores_past_cache(int64_t rows, int64_t n, int64_t k, int64_t es) {
 // 128 bytes fp16 [256, 131072] k0=8192 39.2 against 33.3 us, fp32 [64, 32768] k0=2048
 // 17.4 against 12.7 us; of 256 bytes fp16 [256, 262144] k0=8192 57.6 against 49.4 us,
 // [1024, 131072] 109.9 against 110.3 us.
-static Plan plan_short_buckets(int64_t rows, int64_t n, int64_t k0, int j, int64_t k, int dtype, bool wide) {
+static Plan plan_short_buckets(int64_t rows, int64_t n, int64_t k0, int j, int64_t k, int dtype) {
   Plan pl{};
   pl.ok = false;
-  if (!wide || rows > 0x7fffffffll) return pl;
+  if (rows > 0x7fffffffll) return pl;
   if (k0 <= 0 || k <= 0 || k >= k0 || j < 1 || j > 4 || k0 % j) return pl;
   const int es = elem_bytes(dtype);
   if (es != 2 && es != 4) return pl;
@@ -115,13 +115,13 @@ static Plan plan_short_buckets(int64_t rows, int64_t n, int64_t k0, int j, int64
   return pl;
 }
 
-Plan make_plan(int64_t rows, int64_t n, int64_t k0, int j, int64_t k, int layout, int dtype, bool wide, bool aligned) {
+Plan make_plan(int64_t rows, int64_t n, int64_t k0, int j, int64_t k, int layout, int dtype, bool aligned) {
   Plan pl{};
   pl.ok = false;
-  if (layout == ATK_BALANCED) return plan_short_buckets(rows, n, k0, j, k, dtype, wide);
+  if (layout == ATK_BALANCED) return plan_short_buckets(rows, n, k0, j, k, dtype);
   // (a padded row is never reduced further: its callers keep every bucket)
   if (layout != ATK_INTERLEAVED) return pl;
-  if (!wide || rows > 0x7fffffffll) return pl;
+  if (rows > 0x7fffffffll) return pl;
   if (k0 <= 0 || k <= 0 || k >= k0 || j < 1 || j > 4 || k0 % j) return pl;
   const int es = elem_bytes(dtype);
   if (!es) return pl;
@@ -236,12 +236,11 @@ Plan make_plan(int64_t rows, int64_t n, int64_t k0, int j, int64_t k, int layout
 }  // namespace fused
 
 namespace {
-// Rows may start at any element (a row of odd length does): the 16-byte loads take such addresses.
+// Rows may start at any element (rows of odd length do, and views): the 16-byte loads take such addresses.
 fused::Plan plan_for(const void* x, int64_t rows, int64_t n, int64_t row_stride, int64_t k0, int j, int64_t k,
                      int layout, int dtype) {
-  const int es = elem_bytes(dtype);
-  const bool aligned = (uintptr_t)x % 16 == 0 && (row_stride * es) % 16 == 0;
-  return fused::make_plan(rows, n, k0, j, k, layout, dtype, stream::wide_loads(x, es), aligned);
+  const bool aligned = (uintptr_t)x % 16 == 0 && (row_stride * elem_bytes(dtype)) % 16 == 0;
+  return fused::make_plan(rows, n, k0, j, k, layout, dtype, aligned);
 }
 }  // namespace
 

@@ -732,8 +732,8 @@ inline int64_t bucket_groups(const Geom& g, int64_t rows) {
   return (((rows * (int64_t)g.b) << lanes_log2) + kThreads - 1) / kThreads;
 }
 
-// `aligned`: every row starts on 16 bytes; `wide`: 16-byte loads may be used (stream::wide_loads).
-Plan make_plan(int64_t rows, int64_t n, int64_t k0, int j, int layout, int dtype, bool aligned, bool wide);
+// `aligned`: every row starts on 16 bytes.
+Plan make_plan(int64_t rows, int64_t n, int64_t k0, int j, int layout, int dtype, bool aligned);
 
 template <typename E>
 int launch_typed(const Plan& pl, const void* x, int64_t rows, int64_t row_stride, int j, void* values,

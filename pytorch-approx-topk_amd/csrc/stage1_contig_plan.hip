@@ -16,8 +16,7 @@ constexpr int64_t kManyLong = 1024;
 constexpr int64_t kMostGroups = 0xffffffffll / kThreads;
 }  // namespace
 
-Plan make_plan(int64_t rows, int64_t n, int64_t k0, int j, int layout, int dtype, bool aligned,
-               bool wide) {
+Plan make_plan(int64_t rows, int64_t n, int64_t k0, int j, int layout, int dtype, bool aligned) {
   Plan pl{};
   pl.ok = false;
   if (layout != ATK_BALANCED && layout != ATK_CEIL_CHUNK) return pl;
@@ -74,7 +73,7 @@ Plan make_plan(int64_t rows, int64_t n, int64_t k0, int j, int layout, int dtype
   // 16-byte loads in rows off 16 bytes: they pay for elements of four bytes and more (fp32 [16, 2000003] with
   // buckets of 40 KB 51.6 -> 48.0 us; fp16 41.2 -> 43.3, and [512, 100003] k=50000 j=4 115 -> 155, where
   // the eight elements of a load are parked in LDS a word at a time)
-  pl.vec = aligned || (wide && es >= 4) ? stream::full_vec(es) : 1;
+  pl.vec = aligned || es >= 4 ? stream::full_vec(es) : 1;
   // LDS: the longest span (whole packs, one element of slack) with its padding, or the queues
   const int64_t span = (g.chunks > 1 ? kThreads * piece : per_group * longest) + 2 * pl.vec + 2;
   const size_t data_bytes = (size_t)(span + ((span >> 5) + 1) * pad_elems(es)) * es;
@@ -113,7 +112,7 @@ Plan make_plan(int64_t rows, int64_t n, int64_t k0, int j, int layout, int dtype
   //   j=4 7.5 against 10.4 us, 512 of 50 KB 16.0 against 20.8; 1024 of 63 KB 25.1 against 25.4, 2048 of 28 KB 23.9 against 17.2);
   //   small launches of short buckets, which take the same either way (fp32 [64, 8200] k=1024 j=2 11.7 against 11.5).
   g.split = 0;
-  if (wide && (es == 2 || es == 4) && !g.whole && !g.fast && (layout == ATK_BALANCED || b * m == n) &&
+  if ((es == 2 || es == 4) && !g.whole && !g.fast && (layout == ATK_BALANCED || b * m == n) &&
       longest * es <= (int64_t)kSplitBucket && (j <= 2 || m >= 4 * j) &&
       (m * es >= (int64_t)kSplitBytes || rows * b >= kManyBuckets)) {
     uint32_t pieces_log2 = 0;
@@ -142,13 +141,13 @@ contig::Plan plan_for(const void* x, int64_t rows, int64_t n, int64_t row_stride
                       int dtype) {
   const int es = elem_bytes(dtype);
   const bool aligned = (uintptr_t)x % 16 == 0 && row_stride % (es ? stream::full_vec(es) : 1) == 0;
-  return contig::make_plan(rows, n, k0, j, layout, dtype, aligned, stream::wide_loads(x, es));
+  return contig::make_plan(rows, n, k0, j, layout, dtype, aligned);
 }
 }  // namespace
 
 size_t stage1_contig_workspace_bytes(int64_t rows, int64_t n, int64_t k0, int j, int layout, int dtype) {
-  const contig::Plan a = contig::make_plan(rows, n, k0, j, layout, dtype, true, true);
-  const contig::Plan u = contig::make_plan(rows, n, k0, j, layout, dtype, false, false);
+  const contig::Plan a = contig::make_plan(rows, n, k0, j, layout, dtype, true);
+  const contig::Plan u = contig::make_plan(rows, n, k0, j, layout, dtype, false);
   size_t need = 0;
   if (a.ok && a.ws_bytes > need) need = a.ws_bytes;
   if (u.ok && u.ws_bytes > need) need = u.ws_bytes;

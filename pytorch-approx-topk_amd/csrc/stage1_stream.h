@@ -1822,16 +1822,14 @@ struct Plan {
   size_t part_values_off, part_pos_off, ws_bytes;
 };
 
-// `wide`: 16-byte loads may be used (wide_loads).  `select_bound`: the index bound of a second stage behind
-// the candidates, 0 for none.
-Plan make_plan(int64_t rows, int64_t n, int64_t k0, int j, int layout, int dtype, bool wide, int64_t select_bound);
-// Rows and sub-rows may start at any element.  One-element loads, which odd rows took before,
-// move a quarter (4-byte types) or an eighth (2-byte types) of the bytes per instruction: bf16
-// [256, 100003] k=64 j=1 k_mult=8 24.8 us that way (and in two kernels) against 14.3 us, arg-max of
-// fp16 [256, 50001] k=1000 15.4 against 10.2 us, fp32 [16, 2653751] k=10 j=2 k_mult=4 44.2 against 41.8 us.
-// Only a 2-byte input that itself starts on an odd half-word keeps them: tests/test_host_logic.py
-// states the plan of such a view.
-inline bool wide_loads(const void* x, int es) { return es >= 4 || (uintptr_t)x % 4 == 0; }
+// `select_bound`: the index bound of a second stage behind the candidates, 0 for none.
+// Rows and sub-rows may start at any element, of the input as of a row within it: the loads of several elements take
+// every address.  One-element loads, which odd rows took before, move a quarter (4-byte types) or an eighth (2-byte types)
+// of the bytes per instruction: bf16 [256, 100003] k=64 j=1 k_mult=8 24.8 us that way (and in two kernels) against 14.3 us,
+// arg-max of fp16 [256, 50001] k=1000 15.4 against 10.2 us, fp32 [16, 2653751] k=10 j=2 k_mult=4 44.2 against 41.8 us; views
+// that start two bytes into a line, fp16 [1024, 32768] k=2048 j=4 k_mult=4 76.1 against 25.0, [128, 2^20] k=65536 j=2 225
+// against 67, one byte, uint8 [1024, 32768] k=2048 j=2 45.0 against 13.1.
+Plan make_plan(int64_t rows, int64_t n, int64_t k0, int j, int layout, int dtype, int64_t select_bound);
 
 // One instance per element type, each in its own translation unit.
 // `ranges`: see KeyRangeOut; may be nullptr.

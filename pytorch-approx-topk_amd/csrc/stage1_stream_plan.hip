@@ -237,8 +237,8 @@ double estimate(const Plan& pl, int64_t rows, int64_t n, int64_t k0, int j, int 
 }
 }  // namespace
 
-Plan make_plan(int64_t rows, int64_t n, int64_t k0, int j, int layout, int dtype, bool wide, int64_t select_bound) {
-  const Plan w = plan_with(rows, n, k0, j, layout, dtype, wide);
+Plan make_plan(int64_t rows, int64_t n, int64_t k0, int j, int layout, int dtype, int64_t select_bound) {
+  const Plan w = plan_with(rows, n, k0, j, layout, dtype, true);
   if (!w.ok || w.vec == 1) return w;
   // whole-wave stores spare the lanes' entries most of what the estimate takes for them; with half of the lanes at work
   // they stay ahead (i8 [4475, 6579] b=320 j=2 42.8 us, 56.5 with one-element loads; bf16 [10470, 6399] b=136 j=4 163 and 114)
@@ -271,11 +271,10 @@ size_t stage1_stream_workspace_bytes(int64_t rows, int64_t n, int64_t k0, int j,
   return need;
 }
 
-bool describe_stage1_stream(const void* x, int64_t rows, int64_t n, int64_t k0, int j, int64_t k, int layout,
+bool describe_stage1_stream(int64_t rows, int64_t n, int64_t k0, int j, int64_t k, int layout,
                             int dtype, int64_t index_bound, bool* selected, std::string& out) {
   *selected = false;
-  const stream::Plan pl = stream::make_plan(rows, n, k0, j, layout, dtype, stream::wide_loads(x, elem_bytes(dtype)),
-                                            k < k0 ? index_bound : 0);
+  const stream::Plan pl = stream::make_plan(rows, n, k0, j, layout, dtype, k < k0 ? index_bound : 0);
   if (!pl.ok) return false;
   const int loads = stream::deep_loads_for_short_columns(dtype, j, pl.vec, pl.packed, pl.run, pl.full_rows)
                         ? 8
@@ -297,8 +296,7 @@ bool describe_stage1_stream(const void* x, int64_t rows, int64_t n, int64_t k0, 
 int launch_stage1_stream(const void* x, int64_t rows, int64_t n, int64_t row_stride, int64_t k0, int j,
                          int layout, int dtype, void* values, IndexOut indices, void* ws,
                          size_t ws_bytes, hipStream_t stream, bool* handled, KeyRangeOut* ranges, SelectOut* last) {
-  const stream::Plan pl = stream::make_plan(rows, n, k0, j, layout, dtype, stream::wide_loads(x, elem_bytes(dtype)),
-                                            last != nullptr ? last->index_bound : 0);
+  const stream::Plan pl = stream::make_plan(rows, n, k0, j, layout, dtype, last != nullptr ? last->index_bound : 0);
   *handled = pl.ok;
   if (!pl.ok) return ATK_OK;
   if (pl.ws_bytes && (!ws || ws_bytes < pl.ws_bytes || (uintptr_t)ws % 16 != 0)) return ATK_ERR_WORKSPACE;

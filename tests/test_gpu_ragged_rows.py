@@ -88,3 +88,37 @@ def test_nan_rows_off_the_load_width():
             x[1::2, ::97] = float("nan")
             x[0, 1::3] = -0.0
             assert_same(*topk(x.cuda(), b * j, -1, j=j), *oracle.topk(x, b * j, -1, j=j), f"b={b}")
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.int16, torch.uint8, torch.int8],
+                         ids=lambda d: str(d).split(".")[-1])
+def test_views_that_start_off_four_bytes(dtype):
+    """Two bytes into a line (16-bit elements), one and three (8-bit ones), with even and odd pitches: the kernels
+    with loads of several elements take the address as they take the start of a row."""
+    from approx_topk import _native, topk
+    two_bytes = dtype.itemsize == 2
+    v = 8
+    cases = [  # rows, n, k, j, k_mult, interleaved, the kernel
+        (256, 50003, 1001, 1, 1, True, f"J=1, V={v},"),                    # the last lane moves down
+        (64, 1 << 17, 4096, 2, 1, True, f"J=2, V={v},"),
+        (128, 70001, 4002, 2, 1, True, f"J=2, V={v},"),
+        (2, 1 << 19, 50, 1, 2, True, "slabs"),
+        (300, 4096, 256, 2, 2, True, "fused_"),                            # both stages in one kernel
+        (300, 4099, 256, 1, 4, True, "fused_"),
+        (7, 30011, 200, 2, 1, False, "split_bucket_kernel" if two_bytes else "contig_kernel"),
+        (300, 8192, 256, 2, 4, False, "short contiguous" if two_bytes else "contig_kernel"),
+    ]
+    for rows, n, k, j, k_mult, interleaved, kernel in cases:
+        x = _data(rows, n, dtype, n + j)
+        if dtype.is_floating_point:
+            x[0, ::97] = float("nan")
+            x[1, ::3] = -0.0
+        want = oracle.topk(x, k, -1, j=j, k_mult=k_mult, interleaved=interleaved)
+        for pad, off in ((8, 1), (5, 1), (16, 3)):
+            whole = torch.zeros(rows, n + pad, dtype=dtype, device="cuda")
+            view = whole[:, off:off + n]
+            view.copy_(x)
+            assert view.data_ptr() % 4 != 0
+            plan = _native.describe(view, k * k_mult, j, k, _native.INTERLEAVED if interleaved else _native.BALANCED)
+            assert kernel in plan, plan
+            assert_same(*topk(view, k, -1, j=j, k_mult=k_mult, interleaved=interleaved), *want, f"{plan} pad={pad} off={off}")

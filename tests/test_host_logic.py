@@ -37,7 +37,7 @@ def test_workspace_of_one_call_depends_on_the_address():
     general = L.atk_topk_workspace_bytes(512, 32768, 1024, 1, 256, 0, 1)
     assert general >= 512 * 1024 * (2 + 8)
     assert L.atk_topk_workspace_bytes_at(4096, 512, 32768, 32768, 1024, 1, 256, 0, 1) == 0
-    # a misaligned input goes through two kernels; an odd row stride keeps their bound, whatever takes it
+    # rows off 16 bytes keep the bound of two kernels, whatever takes them
     assert L.atk_topk_workspace_bytes_at(4098, 512, 32768, 32768, 1024, 1, 256, 0, 1) == general
     assert L.atk_topk_workspace_bytes_at(4096, 512, 32768, 32769, 1024, 1, 256, 0, 1) == general
     # k == k0: stage 1 alone
@@ -66,14 +66,16 @@ def test_workspace_a_call_uses_follows_the_kernels_it_takes():
     assert used(4096, 32768, 32768, 1024, 1, 256)
     for n, stride in ((32768, 32769), (32768, 32775), (32767, 32767), (32761, 32768)):   # rows that start anywhere
         assert used(4096, n, stride, 1024, 1, 256) and used(4100, n, stride, 1024, 1, 256)
-    assert not used(4098, 32768, 32768, 1024, 1, 256)         # an input that starts on an odd half-word
+        assert used(4098, n, stride, 1024, 1, 256)            # ... on an odd half-word as well
+    assert used(4098, 32768, 32768, 1024, 1, 256)
     assert not used(4096, 32768, 32768, 1022, 2, 511)         # a number of buckets off the load width
     assert used(4096, 32768, 32768, 1024, 1, 256, layout=1) and not used(4096, 1 << 18, 1 << 18, 1024, 1, 256, layout=1)
     # what no kernel takes needs none of its own: the bound, as for every invalid call
     assert L.atk_topk_workspace_bytes_used(4096, 0, 32768, 32768, 1024, 1, 256, 0, 1) == 0
     # the operator's wrapper allocates by it
     assert _native._topk_workspace(0, 512, 32768, 32769, 1024, 1, 256, 0, 1) == 0
-    assert _native._topk_workspace(2, 512, 32768, 32768, 1024, 1, 256, 0, 1) > 0
+    assert _native._topk_workspace(2, 512, 32768, 32768, 1024, 1, 256, 0, 1) == 0
+    assert _native._topk_workspace(0, 512, 32768, 32768, 1022, 2, 511, 0, 1) > 0
 
 
 def test_native_argument_checks_need_no_gpu():
@@ -137,9 +139,8 @@ def test_describe_names_the_planned_kernels():
     assert "chain_emit_kernel<f32> grid=2048 block=256 per_thread=16" in describe(64, 1 << 18, 0, 16384, 2, 8)
     assert "chain_" not in describe(65, 1 << 18, 0, 16384, 2, 8)
     assert "chain_" not in describe(17, 1 << 20, 0, 16384, 1, 2)
-    # a misaligned input: scalar loads, and two kernels instead of the fused one
-    odd = describe(1024, 32768, 1, 2048, 4, 4, x=4098)
-    assert odd.startswith("stream_kernel<f16, J=4, V=1") and "select_kernel<f16" in odd
+    # an input that starts on an odd half-word is loaded like rows that do
+    assert describe(1024, 32768, 1, 2048, 4, 4, x=4098) == c3
     # contiguous buckets of 16-256 bytes with a second stage: one kernel too; longer buckets, a bucket
     # count that does not fill whole column tiles, or a row with a remainder: two kernels
     def contiguous(rows, n, code, k, j, k_mult):
