@@ -33,11 +33,11 @@
  *     it may be NULL when that size is 0.  Its contents need no initialisation.
  *   - Alignment: the input, `values` and candidate values to the element size,
  *     indices to their width (8 bytes; 4 for the *_i32 entry points), `ws` to
- *     16 bytes (256 recommended); otherwise ATK_ERR_ALIGN.  Loads are 16
- *     bytes wide whatever the row pitch, as long as the input itself is 4-byte
- *     aligned; only elements of up to two bytes in contiguous buckets that neither
- *     whole_bucket_kernel nor split_bucket_kernel (stage1_contig.h) takes want
- *     rows that start on 16-byte boundaries for that.
+ *     16 bytes (256 recommended); otherwise ATK_ERR_ALIGN.  The input and its
+ *     rows may start at any element: 16-byte loads take every address, and whether
+ *     a call uses them goes by its sizes.  Only elements of up to two bytes in
+ *     contiguous buckets that neither whole_bucket_kernel nor split_bucket_kernel
+ *     (stage1_contig.h) takes want rows that start on 16-byte boundaries for them.
  */
 #ifndef APPROX_TOPK_HIP_H_
 #define APPROX_TOPK_HIP_H_

@@ -291,9 +291,8 @@ def describe(xs: torch.Tensor, k0: int, j: int, k: int, layout: int = INTERLEAVE
              values: torch.Tensor | None = None, indices: torch.Tensor | None = None) -> str:
     """The kernels a call on `xs` (top-k along the last dim) would launch, as text.
 
-    The plan depends on the alignment of the output buffers as well: pass the ones the call
-    will write (slices of larger buffers may be misaligned); without them the outputs are taken
-    to be fresh `torch.empty` tensors, which are at least 256-byte aligned."""
+    `values` and `indices`: the buffers the call will write, checked like the call's; the plan does not
+    depend on them."""
     xs, rows, n, step = rows_view(xs)
     buf = ctypes.create_string_buffer(1024)
     check(lib().atk_describe(xs.data_ptr() if xs.numel() else 4096, rows, n, step, k0, j, k, layout,

@@ -565,9 +565,9 @@ __global__ __launch_bounds__(kThreads) void whole_bucket_kernel(const typename E
 //
 // Bound: HBM.  Against contig_kernel, whose workgroups each copy, wait, scan, wait and write (and of
 // whose loads of one element, in rows off 16 bytes, four or eight make one of these):
-// fp32 [512, 40001] k=1000 j=2 28.6 -> 19.5 us (4.5 TB/s), fp16 23.2 -> 15.6, [128, 300007] with buckets
+// fp32 [512, 40001] k=1000 j=2 25.1 -> 17.0 us (5.2 TB/s), fp16 23.2 -> 15.6, [128, 300007] with buckets
 // of 6000 elements, j=4 53.4 -> 23.6, fp32 [16, 2000003] of 10000 elements 51.6 -> 26.2.  Pieces of 128 bytes:
-// 22.4 us for the first; a line's second half is asked for long after its first.
+// 15 % more for the first; a line's second half is asked for long after its first.
 template <typename E, int J, bool PACKED>
 __global__ __launch_bounds__(kThreads) void split_bucket_kernel(const typename E::raw_t* __restrict__ x,
                                                                 typename E::raw_t* __restrict__ values,

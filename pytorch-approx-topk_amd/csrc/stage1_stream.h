@@ -1122,9 +1122,9 @@ __device__ __forceinline__ void scan_partial_sub_row(const typename E::raw_t* __
 // those J, the odd batch and the first whole one are all issued before the first of them is used.  A
 // run of a few dozen sub-rows at most waits for memory three times otherwise: bf16 [256, 2^20]
 // k=65536 j=4 134.6 -> 128.4 us, [200, 500000] k=20000 j=2 54.8 -> 52.6, fp16 [16, 2^22] k=2^18 j=4
-// 40.4 -> 37.5.  It costs registers (fp32 j=2 82 -> 106), for which longer columns and smaller launches get
-// nothing: fp16 [128, 65536] k=2048 j=4 10.7 -> 11.4 us, [500, 20000] k=1600 j=4 11.2 -> 11.8, fp32
-// [1, 2^23] k=4096 j=2 k_mult=2 24.7 -> 27.0.
+// 40.4 -> 37.5.  It costs registers, for which smaller launches get nothing (fp16 [128, 65536] k=2048 j=4 10.7 -> 11.4
+// us, [500, 20000] k=1600 j=4 11.2 -> 11.8), nor do longer columns and other types, for which no such kernel is
+// built (tried with one, fp32 j=2 takes 106 registers instead of 82, [1, 2^23] k=4096 j=2 k_mult=2 24.7 -> 27.0 us).
 template <typename E, int J, int V, int U, int RUN, bool AHEAD = false, typename Queue>
 __device__ __forceinline__ void scan_run(const typename E::raw_t* __restrict__ xr, const Geom& g, int64_t col,
                                 bool live, uint32_t p0, uint32_t p1, bool with_rem, Queue& queue) {
@@ -1688,7 +1688,8 @@ __global__ __launch_bounds__(kMergeThreads) void stream_merge_kernel(
 // Bound: latency, of two launches as of one: merging and selecting took 4.6 and 4.8 us behind a
 // launch each, whatever the candidates, and a row's partial queues are a few ten KB.
 // In one launch: fp32 [16, 2653751] k=10 j=2 k_mult=4 41.3 -> 36.9 us per call, [4, 2^20] 17.7 -> 14.6,
-// [64, 2^20] k=64 j=4 k_mult=2 62.6 -> 58.2, [1, 2^24] k=10 31.2 -> 26.9.
+// [64, 2^20] k=64 j=4 k_mult=2 62.6 -> 58.2, [1, 2^24] k=10 31.2 -> 26.9 (with 16-byte loads throughout; the second
+// and the last take one-element loads now, 11.7 and 23.4 us).
 constexpr uint32_t kRankMax = 256;
 
 template <typename E, int J>
