@@ -244,7 +244,8 @@ Plan make_plan(int64_t rows, int64_t n, int64_t k0, int j, int layout, int dtype
   // they stay ahead (i8 [4475, 6579] b=320 j=2 42.8 us, 56.5 with one-element loads; bf16 [10470, 6399] b=136 j=4 163 and 114)
   if (w.wave_stores && 2 * w.width >= (int64_t)w.col_tiles * kWave * w.vec) return w;
   const Plan v = plan_with(rows, n, k0, j, layout, dtype, false);
-  if (!v.ok) return w;
+  // (a launch's threads are counted in 32 bits)
+  if (!v.ok || rows * (int64_t)v.slabs * v.col_tiles > 0xffffffffll / (kWave * v.waves)) return w;
   auto us = [&](const Plan& pl) {
     const bool second = select_bound > 0;
     return estimate(pl, rows, n, k0, j, dtype, second, second && selects_in_merge(pl, k0, select_bound, dtype));

@@ -388,3 +388,17 @@ def test_few_long_contiguous_buckets_with_long_queues_keep_workgroups_of_their_o
         assert kernel(4, 7169, 32, 2, code) == "split_bucket"                                       # short queues
     for code in (1, 2, 6):
         assert kernel(4, 14337, 32, 4, code) == kernel(1, 8705, 32, 3, code) == "split_bucket"      # 16-bit elements
+
+
+def test_no_narrow_plan_has_more_threads_than_a_launch_takes():
+    # one-element loads take several times the workgroups: batches of very many short rows, which 16-byte
+    # loads can do in one launch, keep them
+    from approx_topk import _native
+    L = _native.lib()
+    for rows, n, k0, j, k, code in ((21017715, 2076, 496, 4, 248, 5), (23423180, 1131, 339, 3, 339, 2),
+                                    (47186238, 768, 12, 3, 3, 4), (52139250, 653, 96, 4, 24, 6),
+                                    (28117324, 1242, 104, 4, 104, 6), (50756832, 223, 54, 3, 27, 1)):
+        buf = ctypes.create_string_buffer(1024)
+        assert L.atk_describe(4096, rows, n, n, k0, j, k, 0, code, 4096, 4096, buf, 1024) == 0
+        for grid, block in re.findall(r"grid=(\d+) block=(\d+)", buf.value.decode()):
+            assert int(grid) * int(block) < 1 << 32, buf.value
