@@ -128,10 +128,11 @@ int atk_select(const void* cand_values, const int64_t* cand_indices,
 size_t atk_topk_workspace_bytes(int64_t rows, int64_t n, int64_t k0, int j,
                                 int64_t k, int layout, int dtype);
 /*
- * A bound for one particular call, which atk_topk_noalloc goes by: 0 when all rows
- * start on 16-byte boundaries and the one-kernel path takes the call, which parks no
- * candidates, else atk_topk_workspace_bytes, also for rows of other starts that
- * the one-kernel path takes as well.
+ * A bound for one particular call, which atk_topk_noalloc goes by: 0 when the input
+ * starts on 16 bytes, its rows are a multiple of 16 bytes apart (8 for one-byte
+ * elements) and the one-kernel path takes the call, which parks no candidates, else
+ * atk_topk_workspace_bytes, also for rows of other starts that the one-kernel path
+ * takes as well.
  */
 size_t atk_topk_workspace_bytes_at(const void* x, int64_t rows, int64_t n, int64_t row_stride,
                                    int64_t k0, int j, int64_t k, int layout, int dtype);

@@ -255,8 +255,8 @@ size_t atk_topk_workspace_bytes_used(const void* x, int64_t rows, int64_t n, int
 size_t atk_topk_workspace_bytes_at(const void* x, int64_t rows, int64_t n, int64_t row_stride, int64_t k0,
                                    int j, int64_t k, int layout, int dtype) {
   // Callers that size buffers by this figure, and atk_topk_noalloc's limit, have relied on it since only rows on
-  // 16 bytes went through one kernel: calls it calls too large stay refused.
-  if (aligned_to(x, 16) && (row_stride * atk::elem_bytes(dtype)) % 16 == 0)
+  // the width of a load went through one kernel: calls it calls too large stay refused.
+  if (atk::rows_on_load_width(x, row_stride, dtype))
     return atk_topk_workspace_bytes_used(x, rows, n, row_stride, k0, j, k, layout, dtype);
   return plan_topk(rows, n, k0, j, k, layout, dtype).total;
 }

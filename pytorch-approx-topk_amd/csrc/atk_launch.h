@@ -64,6 +64,11 @@ int launch_stage1_contig(const void* x, int64_t rows, int64_t n, int64_t row_str
                          int layout, int dtype, void* values, IndexOut indices, void* ws, size_t ws_bytes,
                          hipStream_t stream, bool* handled);
 
+// Whether every row starts where loads of several elements are aligned: the input on 16 bytes and its rows 16 bytes
+// apart, 8 for one-byte elements, whose loads are that wide.  The plans of both stages in one kernel and of contiguous
+// buckets go by it, and the workspace bound of calls that cannot allocate.
+bool rows_on_load_width(const void* x, int64_t row_stride, int dtype);
+
 // Whether launch_fused_row takes this very call (where its rows start decides with the shape).
 bool fused_row_takes(const void* x, int64_t rows, int64_t n, int64_t row_stride, int64_t k0, int j, int64_t k,
                      int layout, int dtype);

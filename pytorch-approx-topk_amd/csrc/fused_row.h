@@ -713,7 +713,7 @@ struct Plan {
   bool past_cache;      // staged: ... in non-temporal stores (one round of workgroups with a sizeable output)
 };
 
-// `aligned`: every row starts on 16 bytes.
+// `aligned`: every row starts on 16 bytes (8 for one-byte elements).
 Plan make_plan(int64_t rows, int64_t n, int64_t k0, int j, int64_t k, int layout, int dtype, bool aligned);
 
 template <typename E>

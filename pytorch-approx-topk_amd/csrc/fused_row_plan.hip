@@ -33,7 +33,7 @@ constexpr int64_t kManyRows = 1024, kAllCus = 256;
 constexpr int64_t kShortBucket = 256;
 constexpr size_t kShortRow = 128 * 1024, kLongRow = 512 * 1024;
 
-// Whether rows that do not all start on 16 bytes are faster in one kernel.  256 calls of such rows timed against the
+// Whether rows that do not all start on 16 bytes (8 for one-byte elements) are faster in one kernel.  256 calls of such rows timed against the
 // two kernels (with the width of loads that the planner takes there): what decides is how many sub-rows a wave
 // goes through (`run`, over all its tiles), for which the two kernels have any number of workgroups.
 //   Fewer rows than kMinRows: runs of up to 40 sub-rows with queues of one or two entries, of up to 20 with more, and
@@ -235,12 +235,16 @@ Plan make_plan(int64_t rows, int64_t n, int64_t k0, int j, int64_t k, int layout
 
 }  // namespace fused
 
+bool rows_on_load_width(const void* x, int64_t row_stride, int dtype) {
+  const int es = elem_bytes(dtype);
+  return es && (uintptr_t)x % 16 == 0 && row_stride % stream::full_vec(es) == 0;
+}
+
 namespace {
 // Rows may start at any element (rows of odd length do, and views): the 16-byte loads take such addresses.
 fused::Plan plan_for(const void* x, int64_t rows, int64_t n, int64_t row_stride, int64_t k0, int j, int64_t k,
                      int layout, int dtype) {
-  const bool aligned = (uintptr_t)x % 16 == 0 && (row_stride * elem_bytes(dtype)) % 16 == 0;
-  return fused::make_plan(rows, n, k0, j, k, layout, dtype, aligned);
+  return fused::make_plan(rows, n, k0, j, k, layout, dtype, rows_on_load_width(x, row_stride, dtype));
 }
 }  // namespace
 

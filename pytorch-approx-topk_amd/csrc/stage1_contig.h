@@ -732,7 +732,7 @@ inline int64_t bucket_groups(const Geom& g, int64_t rows) {
   return (((rows * (int64_t)g.b) << lanes_log2) + kThreads - 1) / kThreads;
 }
 
-// `aligned`: every row starts on 16 bytes.
+// `aligned`: every row starts on 16 bytes (8 for one-byte elements).
 Plan make_plan(int64_t rows, int64_t n, int64_t k0, int j, int layout, int dtype, bool aligned);
 
 template <typename E>

@@ -139,9 +139,7 @@ Plan make_plan(int64_t rows, int64_t n, int64_t k0, int j, int layout, int dtype
 namespace {
 contig::Plan plan_for(const void* x, int64_t rows, int64_t n, int64_t row_stride, int64_t k0, int j, int layout,
                       int dtype) {
-  const int es = elem_bytes(dtype);
-  const bool aligned = (uintptr_t)x % 16 == 0 && row_stride % (es ? stream::full_vec(es) : 1) == 0;
-  return contig::make_plan(rows, n, k0, j, layout, dtype, aligned);
+  return contig::make_plan(rows, n, k0, j, layout, dtype, rows_on_load_width(x, row_stride, dtype));
 }
 }  // namespace
 

@@ -343,6 +343,24 @@ def test_the_width_of_loads_follows_the_faster_plan(vec, calls):
         assert text.startswith("stream_kernel<") and want in text, (rows, n, k, j, k_mult, text)
 
 
+def test_rows_of_one_byte_elements_on_8_bytes_are_rows_on_their_load_width():
+    # (a load of theirs is 8 bytes: they were accepted by the one-kernel path, and by the call that cannot
+    # allocate, before rows of any start were)
+    from approx_topk import _native
+    L = _native.lib()
+    limit = 8 << 20
+    for args in ((362, 18608, 18616, 4416, 3, 1104, 0, 5), (960, 16248, 16248, 3144, 3, 1572, 0, 5),
+                 (154, 239560, 239576, 22304, 4, 11152, 0, 4), (4096, 8200, 8200, 1024, 1, 256, 0, 4)):
+        rows, n, _, k0, j, k, layout, code = args
+        assert L.atk_topk_workspace_bytes(rows, n, k0, j, k, layout, code) > limit
+        buf = ctypes.create_string_buffer(1024)
+        assert L.atk_describe(4096, *args, 4096, 4096, buf, 1024) == 0 and buf.value.startswith(b"fused_"), buf.value
+        assert L.atk_topk_workspace_bytes_at(4096, *args) == 0 == L.atk_topk_workspace_bytes_used(4096, *args)
+        # rows on 4 bytes, and an input off 16, keep the bound of two kernels
+        off = (rows, n, n + 12, *args[3:])
+        assert L.atk_topk_workspace_bytes_at(4096, *off) > limit and L.atk_topk_workspace_bytes_at(4104, *args) > limit
+
+
 # the same for rows off 16 bytes with a second stage, timed in one kernel and in two
 ONE_KERNEL = [
     (8, 254, 2501, 36, 2, 8), (8, 3, 24169, 358, 1, 2), (3, 206, 5521, 116, 1, 2), (6, 760, 2813, 41, 1, 4),
