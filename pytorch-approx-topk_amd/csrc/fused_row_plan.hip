@@ -47,9 +47,10 @@ constexpr size_t kShortRow = 128 * 1024, kLongRow = 512 * 1024;
 //   More rows: all (fp16 [742, 9559] b=264 15.4 -> 11.0, bf16 [552, 6915] b=132 j=4 17.4 -> 12.4, i16 [759, 57865]
 //   b=448 j=4 48.4 -> 42.1).
 //   One-byte elements, whose packed queues this kernel lacks: batches with queues of one or two entries (uint8 [1354, 66483]
-//   j=1 67.0 -> 50.5, [374, 23585] j=2 23.4 -> 19.2, but [1538, 37707] j=4 74 -> 214, [11, 10433] j=4 10.6 -> 40.7).
+//   j=1 67.0 -> 50.5, [374, 23585] j=2 23.4 -> 19.2, but [1538, 37707] j=4 74 -> 214, [11, 10433] j=4 10.6 -> 40.7), and those of more
+//   rows than the second stage's workgroups of up to 1024 threads have launches for (threads are counted in 32 bits).
 bool loose_rows_gain(int64_t rows, int64_t sub_row_bytes, int64_t run, int j, int es) {
-  if (es == 1) return rows >= kMinRows && j <= 2;
+  if (es == 1) return (rows >= kMinRows && j <= 2) || rows > 0xffffffffll / 1024;
   if (rows >= kMinRows) return rows >= kAllCus || run <= 256;
   return run <= (j <= 2 ? 40 : es == 8 ? 0 : sub_row_bytes >= 2560 ? 64 : 20) && sub_row_bytes >= 256;
 }

@@ -408,14 +408,15 @@ def test_few_long_contiguous_buckets_with_long_queues_keep_workgroups_of_their_o
         assert kernel(4, 14337, 32, 4, code) == kernel(1, 8705, 32, 3, code) == "split_bucket"      # 16-bit elements
 
 
-def test_no_narrow_plan_has_more_threads_than_a_launch_takes():
-    # one-element loads take several times the workgroups: batches of very many short rows, which 16-byte
-    # loads can do in one launch, keep them
+def test_no_plan_has_more_threads_than_a_launch_takes():
+    # batches of very many short rows: one-element loads would take several times the workgroups, and the
+    # second stage's of their own several times the threads of one kernel for both
     from approx_topk import _native
     L = _native.lib()
     for rows, n, k0, j, k, code in ((21017715, 2076, 496, 4, 248, 5), (23423180, 1131, 339, 3, 339, 2),
                                     (47186238, 768, 12, 3, 3, 4), (52139250, 653, 96, 4, 24, 6),
-                                    (28117324, 1242, 104, 4, 104, 6), (50756832, 223, 54, 3, 27, 1)):
+                                    (28117324, 1242, 104, 4, 104, 6), (50756832, 223, 54, 3, 27, 1),
+                                    (5099261, 3822, 3720, 3, 1860, 4), (16484397, 3913, 1752, 3, 438, 5)):
         buf = ctypes.create_string_buffer(1024)
         assert L.atk_describe(4096, rows, n, n, k0, j, k, 0, code, 4096, 4096, buf, 1024) == 0
         for grid, block in re.findall(r"grid=(\d+) block=(\d+)", buf.value.decode()):
