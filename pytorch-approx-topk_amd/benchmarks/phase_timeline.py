@@ -81,7 +81,7 @@ def main():
         d = np.diff(t[:, cols], axis=1)
         print("median time between them:", " ".join("%.2f" % v for v in np.median(d, axis=0)))
         first, last = 0, cols[-1]
-        for x in range(8):
+        for x in range(min(8, groups)):
             s = t[x::8] - t0
             print("XCD %d: start %s | scan done %s | written %s" % (x, three(s[:, first]), three(s[:, 1]), three(s[:, last])))
         end = t[:, last] - t0

@@ -8,6 +8,19 @@
 
 namespace atk {
 
+// Barrier of a workgroup of `waves` waves of 64 threads that tells every thread whether
+// `flag` is set in any of them: a word of LDS per wave, written before the barrier and read
+// behind it (the words may be written again after the caller's next barrier).
+// HIP's __syncthreads_or comes out as three barriers with lane exchanges and an
+// atomic between them.
+__device__ __forceinline__ bool any_in_group(bool flag, uint32_t* words, uint32_t waves) {
+  const uint32_t lane = threadIdx.x % 64;
+  const bool mine = __ballot(flag) != 0;
+  if (lane == 0) words[threadIdx.x / 64] = mine ? 1u : 0u;
+  __syncthreads();
+  return __ballot(lane < waves && words[lane] != 0) != 0;
+}
+
 // ---------------------------------------------------------------------------
 // Element traits.  Kernels move elements as raw bit patterns (`raw_t`) so that
 // outputs are bit-identical to inputs, and compare them through `key_t`, an

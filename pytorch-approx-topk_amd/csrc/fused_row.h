@@ -119,6 +119,7 @@ __global__ __launch_bounds__(kWave * MAXW) __attribute__((amdgpu_num_sgpr(80))) 
 
   extern __shared__ __align__(16) unsigned char dyn_lds[];
   __shared__ select::SharedT<4> sh;  // four histogram copies: four workgroups of C3's shape fit one CU's LDS
+  __shared__ uint32_t nan_waves[MAXW];
   // Candidates, and the hand-over area of the waves that share a tile: behind
   // the candidates, or (hand_off == 0, single round only) on top of them, in
   // which case a barrier separates the last fold from the first candidate.
@@ -170,7 +171,7 @@ __global__ __launch_bounds__(kWave * MAXW) __attribute__((amdgpu_num_sgpr(80))) 
     if (split > 1 && hand_off != 0) __syncthreads();  // the hand-over area is reused by the next round
   }
 
-  if (__syncthreads_or(any_nan)) redo_exact_into_lds<E, J, false>(xr, g, cand_key, cand_pos);
+  if (any_in_group(any_nan, nan_waves, nwaves)) redo_exact_into_lds<E, J, false>(xr, g, cand_key, cand_pos);
   // (the select's first pass starts with a barrier, which also publishes the candidates)
   select_from_lds<E, J, false>(sh, xr, g, cand_key, cand_pos, k0, k, index_bits, row, values, indices);
 }
@@ -343,27 +344,39 @@ __attribute__((amdgpu_waves_per_eu(PACKED && V * J <= 16 && !(CONTIG && V * J > 
   // packed entries: sub-row numbers 0..full_rows at the top of the low half, so
   // that the bits in which entries differ are the leading ones
   queue.set_position_shift(sizeof(pos_t) == 2 ? (uint32_t)__builtin_clz(g.full_rows | 1u) - 16u : 0u);
-  // The first radix pass over sel_key (below) takes its leading `bits0` bits.  With a wave per
-  // tile (split == 1) nothing else uses the LDS while the row is scanned, so the histograms are
-  // cleared before the scan and a wave counts its candidates' digits as soon as its own scan is
-  // done, rather than after the workgroup's slowest wave: one barrier phase less in the chain that
-  // every workgroup goes through after its scan.
+  // The first radix pass over sel_key (below) takes its leading `bits0` bits.  Its histogram is cleared before the
+  // scan and lies apart from the hand-over area, so that a wave counts its candidates' digits as soon as it
+  // holds them: after its own scan, or, where waves share a tile, after the fold.  What follows the scan is a
+  // chain of barrier phases of 0.3-0.8 us that every workgroup goes through, and in small launches a
+  // third of the call: fp16 [32, 20480] k=512 j=2 k_mult=2 (indices) 8.5 -> 7.45 us per launch with the clearing
+  // and its barriers out of that chain, the list below entered by one atomic add a wave instead of one an entry, its ranking
+  // shared out over the waves, and the barrier that tells of NaNs a plain one; [4, 32768] k=512 j=1 k_mult=2 7.8 -> 6.7,
+  // [256, 65536] k=512 j=2 12.7 -> 11.8, [1024, 65536] 31.7 -> 30.6, fp32 [2048, 16384] k=1024 j=2 46.8 -> 43.0.
   constexpr bool kKeyHalf = CONTIG && PACKED;
   const int shift_end = kKeyHalf ? 16 : queue.sel_constant_bits();
   const int bits0 = Queue::sel_bits - shift_end < regs::kDigitBits ? Queue::sel_bits - shift_end : regs::kDigitBits;
-  const bool early = (CONTIG || split == 1) && k != k0 && k0 > regs::kListMax && bits0 > 0;
-  if (early) {
-    for (uint32_t i = tid * 4; i < 2 * regs::kHistWords; i += nt * 4)
-      *reinterpret_cast<uint4*>(&hist[i]) = make_uint4(0, 0, 0, 0);
-    if (tid == 0) rs.list_count = 0;
-    __syncthreads();
-  }
-  bool any_nan = false;
+  const bool early = k != k0 && k0 > regs::kListMax && bits0 > 0;
+  for (uint32_t i = tid * 4; i < regs::kHistWords; i += nt * 4)
+    *reinterpret_cast<uint4*>(&hist[i]) = make_uint4(0, 0, 0, 0);
+  if (tid < regs::kListMax) rs.rank[tid] = 0;
+  if (tid == 0) rs.list_count = 0;
+  if (CONTIG || split == 1) __syncthreads();
+  bool any_nan = false, nan_row = false;
   if (has_tile) {
     if constexpr (CONTIG) scan_short_buckets<E, J, V, PACKED, !PACKED>(xr, g.full_rows, col, queue);
     else if (split > 1) stream::scan_windows<E, J, V, U>(xr, g, col, live, part, split, part == split - 1, queue);
     else stream::scan_run<E, J, V, U, 0>(xr, g, col, live, p0, p1, true, queue);
     any_nan = queue.poisoned();
+  }
+  if constexpr (!CONTIG) {
+    if (split > 1) {
+      if (part > 0) queue.hand_over(hand + (size_t)(tile * (split - 1) + (part - 1)) * Queue::kHandBytes, lane);
+      nan_row = any_in_group(any_nan, rs.nan_waves, nt / kWave);
+      if (part == 0) {
+        for (uint32_t w = 0; w + 1 < split; ++w)
+          queue.fold_in_interleaved(hand + (size_t)(tile * (split - 1) + w) * Queue::kHandBytes, lane);
+      }
+    }
   }
   if (early && mine) {  // (a wave that met a NaN counts keys that mean nothing: the row leaves the fast path anyway)
     const int shift0 = Queue::sel_bits - bits0;
@@ -374,27 +387,9 @@ __attribute__((amdgpu_waves_per_eu(PACKED && V * J <= 16 && !(CONTIG && V * J > 
       atomicAdd(&hist[regs::hist_slot((uint32_t)(key >> shift0) & dmask0)], 1u);
     } ATK_STATIC_END;
   }
-  if constexpr (!CONTIG) {
-    if (split > 1) {
-      if (has_tile && part > 0)
-        queue.hand_over(hand + (size_t)(tile * (split - 1) + (part - 1)) * Queue::kHandBytes, lane);
-      __syncthreads();
-      if (has_tile && part == 0) {
-        for (uint32_t w = 0; w + 1 < split; ++w)
-          queue.fold_in_interleaved(hand + (size_t)(tile * (split - 1) + w) * Queue::kHandBytes, lane);
-      }
-    }
-    // Both histograms start at zero.  Waves that shared a tile must first be done
-    // with the hand-over area, which may lie in the same place.
-    if (split > 1) __syncthreads();
-  }
   ATK_TRACE_GROUP(1);
-  if (!early) {
-    for (uint32_t i = tid * 4; i < 2 * regs::kHistWords; i += nt * 4)
-      *reinterpret_cast<uint4*>(&hist[i]) = make_uint4(0, 0, 0, 0);
-    if (tid == 0) rs.list_count = 0;
-  }
-  const bool nan_row = __syncthreads_or(any_nan);
+  if (CONTIG || split == 1) nan_row = any_in_group(any_nan, rs.nan_waves, nt / kWave);
+  else __syncthreads();
   ATK_TRACE_GROUP(2);
 
   // (keys are taken from the queues where they are used rather than kept: registers)
@@ -416,8 +411,8 @@ __attribute__((amdgpu_waves_per_eu(PACKED && V * J <= 16 && !(CONTIG && V * J > 
   // to the result.  The race ends when all of them do (the cut is then the
   // prefix itself), when they are few enough to be listed and ranked, or, with
   // no bits left, when they are too many equal keys for that (the LDS path then
-  // cuts them by index).  Pass p counts into histogram p % 2, which the pass
-  // before last left cleared; wave 0 reads it.
+  // cuts them by index).  Pass p counts into histogram p % 2, which is cleared while
+  // wave 0 reads the other one in the pass before.
   sel_t prefix = 0, mask = 0;
   uint32_t need = k, count = k0;
   enum { kByPrefix, kByList, kGiveUp } how = kGiveUp;
@@ -431,21 +426,13 @@ __attribute__((amdgpu_waves_per_eu(PACKED && V * J <= 16 && !(CONTIG && V * J > 
       shift -= bits;
       const uint32_t dmask = (1u << bits) - 1u;
       uint32_t* h = hist + (pass & 1u) * regs::kHistWords;
-      if (pass == 0 && early) {
-        // counted already, and the barrier that told of NaNs has published the counts
-      } else {
+      // (pass 0 is counted already, and the barrier above has published the counts)
+      if (pass != 0) {
         if (mine) {
-          if (pass == 0) {  // every candidate counts
-            ATK_STATIC_FOR(e, NC) {
-              const sel_t key = key_of(std::integral_constant<int, e>{});
-              atomicAdd(&h[regs::hist_slot((uint32_t)(key >> shift) & dmask)], 1u);
-            } ATK_STATIC_END;
-          } else {
-            ATK_STATIC_FOR(e, NC) {
-              const sel_t key = key_of(std::integral_constant<int, e>{});
-              if ((key & mask) == prefix) atomicAdd(&h[regs::hist_slot((uint32_t)(key >> shift) & dmask)], 1u);
-            } ATK_STATIC_END;
-          }
+          ATK_STATIC_FOR(e, NC) {
+            const sel_t key = key_of(std::integral_constant<int, e>{});
+            if ((key & mask) == prefix) atomicAdd(&h[regs::hist_slot((uint32_t)(key >> shift) & dmask)], 1u);
+          } ATK_STATIC_END;
         }
         __syncthreads();
       }
@@ -453,7 +440,7 @@ __attribute__((amdgpu_waves_per_eu(PACKED && V * J <= 16 && !(CONTIG && V * J > 
         const regs::Found f = regs::find_bin_wave(h, need, count, lane);
         if (lane == 0) { rs.digit = f.digit; rs.need = f.need; rs.count = f.count; }
       }
-      if (pass >= 1) {  // the other histogram, for the pass after this one
+      {  // the other histogram, for the pass after this one
         uint32_t* other = hist + ((pass & 1u) ^ 1u) * regs::kHistWords;
         for (uint32_t i = tid * 4; i < regs::kHistWords; i += nt * 4)
           *reinterpret_cast<uint4*>(&other[i]) = make_uint4(0, 0, 0, 0);
@@ -492,64 +479,67 @@ __attribute__((amdgpu_waves_per_eu(PACKED && V * J <= 16 && !(CONTIG && V * J > 
     cut_key = prefix - 1;
     cut_below = 0;
   } else {
-    // List the candidates that share the prefix; wave 0 ranks them (lane t takes
-    // entry t and counts the better ones): the need-th best is the cut.  An entry
-    // is one 64-bit word when key and index fit 32 bits each (key above inverted
-    // index: a larger word is a better candidate), else two.  The list is read
-    // four entries at a time; its last group is filled up with entries that
-    // beat nothing.
+    // List the candidates that share the prefix and rank them under the full order: the
+    // need-th best is the cut.  An entry is one 64-bit word when key and index fit 32 bits each (key above
+    // inverted index: a larger word is a better candidate), else two.  The waves share the ranking out: lane t
+    // of every wave holds entry t and counts the better ones among a share of the entries, which reach it through
+    // scalar registers; the counts are added up in LDS and every wave finds the cut for itself.
     constexpr bool kOneWord = sizeof(sel_t) == 4 && sizeof(idx_t) == 4;
-    if (tid < 8u) {
-      list_key[count + tid] = 0;
-      list_index[count + tid] = ~0ull;
-    }
-    if (mine) {
+    if (part == 0) {
+      // one add to the list's length per wave that has members
+      uint32_t members = 0;  // bit e: candidate e shares the prefix
       ATK_STATIC_FOR(e, NC) {
-        const sel_t key = key_of(std::integral_constant<int, e>{});
-        if ((key & mask) == prefix) {
-          const uint32_t slot = atomicAdd(&rs.list_count, 1u);
-          const idx_t index = index_of(std::integral_constant<int, e>{});
-          if constexpr (kOneWord) {
-            list_key[slot] = ((uint64_t)key << 32) | (uint64_t)(0xffffffffu - (uint32_t)index);
-          } else {
-            list_key[slot] = (uint64_t)key;
-            list_index[slot] = (uint64_t)index;
-          }
-        }
+        members |= mine && (key_of(std::integral_constant<int, e>{}) & mask) == prefix ? (1u << e) : 0u;
       } ATK_STATIC_END;
+      uint32_t slot = regs::wave_scan((uint32_t)__popc(members));
+      uint32_t base = 0;
+      if (lane == kWave - 1 && slot != 0) base = atomicAdd(&rs.list_count, slot);
+      slot += (uint32_t)__builtin_amdgcn_readlane((int)base, kWave - 1);
+      if (members != 0) {
+        uint32_t at = slot - (uint32_t)__popc(members);
+        ATK_STATIC_FOR(e, NC) {
+          if ((members >> e) & 1u) {
+            const sel_t key = key_of(std::integral_constant<int, e>{});
+            const idx_t index = index_of(std::integral_constant<int, e>{});
+            if constexpr (kOneWord) {
+              list_key[at] = ((uint64_t)key << 32) | (uint64_t)(0xffffffffu - (uint32_t)index);
+            } else {
+              list_key[at] = (uint64_t)key;
+              list_index[at] = (uint64_t)index;
+            }
+            ++at;
+          }
+        } ATK_STATIC_END;
+      }
     }
     __syncthreads();
-    if (wave == 0) {
-      const uint32_t t = lane < count ? lane : 0u;
-      const uint64_t my_key = list_key[t];
-      const uint64_t my_index = kOneWord ? 0ull : list_index[t];
+    const bool listed = lane < count;
+    const uint64_t my_key = listed ? list_key[lane] : 0ull;
+    const uint64_t my_index = kOneWord || !listed ? 0ull : list_index[lane];
+    {
+      const uint32_t entries = __builtin_amdgcn_readfirstlane(count);
       uint32_t better = 0;
-      // (four entries per trip and no unrolling: with eight, the sixteen registers of a trip were
-      // what made the compiler spill part of the lane's candidates to scratch memory in the
-      // kernels held to 64 registers -- 9 to 24 registers, 13 to 35 MB of HBM traffic per launch
-      // of fp16 [1024, 32768] k=2048 j=4 k_mult=4, which takes 24.2 us without them against 25.9)
-      constexpr int kGroup = 4;
-#pragma nounroll
-      for (uint32_t m = 0; m < count; m += kGroup) {
-        uint64_t key[kGroup], index[kGroup];
-#pragma unroll
-        for (int u = 0; u < kGroup; ++u) { key[u] = list_key[m + u]; index[u] = kOneWord ? 0ull : list_index[m + u]; }
-#pragma unroll
-        for (int u = 0; u < kGroup; ++u)
-          better += (key[u] > my_key || (!kOneWord && key[u] == my_key && index[u] < my_index)) ? 1u : 0u;
+      for (uint32_t m = wave; m < entries; m += nt / kWave) {
+        const uint64_t key = regs::from_lane(my_key, m);
+        if constexpr (kOneWord) {
+          better += key > my_key ? 1u : 0u;
+        } else {
+          const uint64_t index = regs::from_lane(my_index, m);
+          better += (key > my_key || (key == my_key && index < my_index)) ? 1u : 0u;
+        }
       }
-      if (lane < count && better + 1 == need) {  // one lane
-        rs.cut_key = my_key;
-        rs.cut_index = my_index;
-      }
+      if (listed && better != 0) atomicAdd(&rs.rank[lane], better);
     }
     __syncthreads();
+    const uint64_t hit = __ballot(listed && rs.rank[lane] + 1 == need);  // one lane
+    const uint32_t at = (uint32_t)__builtin_amdgcn_readfirstlane((int)__ffsll((unsigned long long)hit) - 1);
+    const uint64_t key = regs::from_lane(my_key, at);
     if constexpr (kOneWord) {
-      cut_key = (sel_t)(rs.cut_key >> 32);
-      cut_below = (idx_t)(0xffffffffu - (uint32_t)rs.cut_key) + 1u;
+      cut_key = (sel_t)(key >> 32);
+      cut_below = (idx_t)(0xffffffffu - (uint32_t)key) + 1u;
     } else {
-      cut_key = (sel_t)rs.cut_key;
-      cut_below = (idx_t)rs.cut_index + 1u;
+      cut_key = (sel_t)key;
+      cut_below = (idx_t)regs::from_lane(my_index, at) + 1u;
     }
   }
 

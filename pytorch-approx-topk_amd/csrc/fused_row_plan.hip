@@ -225,7 +225,14 @@ Plan make_plan(int64_t rows, int64_t n, int64_t k0, int j, int64_t k, int layout
   // every tile has its waves: stage 2 runs on the candidates where they are, in
   // registers, and needs the histogram's room in LDS
   pl.in_registers = one_round && pl.waves <= kMaxWaves;  // (the register kernel is built for eight waves)
-  if (pl.in_registers && pl.lds_bytes < regs::kLdsBytes) pl.lds_bytes = regs::kLdsBytes;
+  if (pl.in_registers) {
+    // the hand-over area lies behind the first digits' histogram, which is counted while it is in use
+    pl.hand_off = split > 1 ? (uint32_t)(regs::kHistWords * sizeof(uint32_t)) : 0u;
+    const size_t hand = pl.hand_off + (size_t)(pl.waves - pl.waves / split) * pl.vec * j * stream::kWave *
+                                          (pl.packed ? 4 : cmp_size + 4);
+    pl.lds_bytes = hand > cand_bytes ? hand : cand_bytes;
+    if (pl.lds_bytes < regs::kLdsBytes) pl.lds_bytes = regs::kLdsBytes;
+  }
   // survivors staged in LDS, eight bytes each (element, 32-bit index), when that fits
   pl.staged = pl.in_registers && pl.pos16 && es <= 4 && (size_t)k * 8 <= kLdsBudget;
   if (pl.staged && pl.lds_bytes < (size_t)k * 8) pl.lds_bytes = (size_t)k * 8;

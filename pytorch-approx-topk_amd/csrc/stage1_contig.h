@@ -176,7 +176,8 @@ __device__ __forceinline__ bool scan_buckets(const typename E::raw_t* __restrict
       park(pk, got);
     }
     if constexpr (kScreen) {
-      if (__syncthreads_or(nan)) return false;
+      __shared__ uint32_t nan_waves[kThreads / 64];
+      if (any_in_group(nan, nan_waves, kThreads / 64)) return false;
     } else {
       __syncthreads();
     }
@@ -337,7 +338,8 @@ __device__ __forceinline__ bool scan_even(const typename E::raw_t* __restrict__ 
       ATK_STATIC_FOR(e, V) { queue.template take<J>(Pack<raw_t, 1>{{cur.e[e]}}, first + i * kPer + e); } ATK_STATIC_END;
     }
   }
-  if (__syncthreads_or(queue.poisoned())) return false;  // (also: the span is no longer read)
+  __shared__ uint32_t nan_waves[kThreads / 64];
+  if (any_in_group(queue.poisoned(), nan_waves, kThreads / 64)) return false;  // (also: the span is no longer read)
 
   // combine the pieces of every bucket
   const uint32_t start = c * g.m;

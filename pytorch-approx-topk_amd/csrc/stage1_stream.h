@@ -1523,7 +1523,8 @@ __global__ __launch_bounds__(kWave * W) __attribute__((amdgpu_waves_per_eu(4))) 
   if constexpr (W > 1) {
     // waves 1.. hand their queues to wave 0 through LDS
     if (wave > 0) queue.hand_over(lds + (size_t)(wave - 1) * Queue::kHandBytes, lane);
-    redo = __syncthreads_or(redo);
+    __shared__ uint32_t redo_waves[W];
+    redo = any_in_group(redo, redo_waves, W);
     if (wave > 0) return;
     if (!redo) {
 #pragma nounroll

@@ -296,15 +296,16 @@ __device__ __forceinline__ uint32_t hist_slot(uint32_t digit) { return digit + (
 // alternate, so that two barriers per pass are enough), then the listed
 // candidates.
 constexpr size_t kListOff = 2 * (size_t)kHistWords * sizeof(uint32_t);
-constexpr size_t kListWords = kListMax + 8;  // rounded up to whole groups of eight when ranking
+constexpr size_t kListWords = kListMax;
 constexpr size_t kLdsBytes = kListOff + 2 * kListWords * sizeof(uint64_t);
 
 struct Shared {
   uint32_t wave_total[kMaxWaves];
   uint32_t wave_low[kMaxWaves], wave_high[kMaxWaves];  // per-wave smallest and largest key
+  uint32_t nan_waves[kMaxWaves];     // waves that met a NaN
   uint32_t list_count;
   uint32_t digit, need, count;       // what wave 0 found in the last pass
-  uint64_t cut_key, cut_index;       // the cut, when wave 0 ranked a list
+  uint32_t rank[kListMax];           // better entries of the list, per entry
 };
 
 // Inclusive prefix sum over the 64 lanes of a wave, in registers.
@@ -344,6 +345,13 @@ __device__ __forceinline__ uint32_t wave_max(uint32_t v) {
   ATK_WAVE_STEP(0x142, 0xa) ATK_WAVE_STEP(0x143, 0xc)
 #undef ATK_WAVE_STEP
   return (uint32_t)__builtin_amdgcn_readlane((int)v, kWave - 1);
+}
+
+// The value of lane `lane` (wave-uniform) in every lane.
+__device__ __forceinline__ uint64_t from_lane(uint64_t v, uint32_t lane) {
+  const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)v, (int)lane);
+  const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(v >> 32), (int)lane);
+  return ((uint64_t)hi << 32) | lo;
 }
 
 struct Found { uint32_t digit, need, count; };  // wave-uniform
