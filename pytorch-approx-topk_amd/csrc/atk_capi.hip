@@ -256,8 +256,10 @@ size_t atk_topk_workspace_bytes_at(const void* x, int64_t rows, int64_t n, int64
                                    int j, int64_t k, int layout, int dtype) {
   // Callers that size buffers by this figure, and atk_topk_noalloc's limit, have relied on it since only rows on
   // the width of a load went through one kernel: calls it calls too large stay refused.
-  if (atk::rows_on_load_width(x, row_stride, dtype))
-    return atk_topk_workspace_bytes_used(x, rows, n, row_stride, k0, j, k, layout, dtype);
+  if (rows > 0 && k > 0 && k < k0 && check_stage1(x, rows, n, row_stride, k0, j, layout, dtype, x, x) == ATK_OK &&
+      atk::rows_on_load_width(x, row_stride, dtype) &&
+      atk::fused_row_taken_by_size(x, rows, n, row_stride, k0, j, k, layout, dtype))
+    return 0;
   return plan_topk(rows, n, k0, j, k, layout, dtype).total;
 }
 

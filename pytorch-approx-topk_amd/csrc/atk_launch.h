@@ -69,6 +69,10 @@ int launch_stage1_contig(const void* x, int64_t rows, int64_t n, int64_t row_str
 // buckets go by it, and the workspace bound of calls that cannot allocate.
 bool rows_on_load_width(const void* x, int64_t row_stride, int dtype);
 
+// Whether the rules of size alone would give this call to launch_fused_row (it takes more: see fused::make_plan).
+bool fused_row_taken_by_size(const void* x, int64_t rows, int64_t n, int64_t row_stride, int64_t k0, int j, int64_t k,
+                             int layout, int dtype);
+
 // Whether launch_fused_row takes this very call (where its rows start decides with the shape).
 bool fused_row_takes(const void* x, int64_t rows, int64_t n, int64_t row_stride, int64_t k0, int j, int64_t k,
                      int layout, int dtype);

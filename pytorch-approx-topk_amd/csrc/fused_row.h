@@ -193,6 +193,18 @@ __global__ __launch_bounds__(kWave * MAXW) __attribute__((amdgpu_num_sgpr(80))) 
 // ---------------------------------------------------------------------------
 namespace regs = select::regs;
 
+// Loads of less than half the usual width: two 2-byte, one or two 4-byte elements.  Only the register kernel is built
+// for them, with eight waves per SIMD.  A lane then owns half or a quarter of the columns: a row's candidates sit in more
+// waves with fewer each, fewer waves share a tile (their queues are folded by one of them, an entry after the other),
+// and four-byte elements take 61 or 64 registers where 16-byte loads take 89 to 120, so that four workgroups
+// share a CU instead of two.  fp32 [2048, 16384] k=1024 j=2 k_mult=2 43.0 -> 32.8 us with two columns a lane, [4096, 16384]
+// k=256 j=4 k_mult=8 104 -> 64, [256, 131072] k=64 j=1 k_mult=8 27.8 -> 26.5, [512, 8192] k=64 j=4 k_mult=4 19.5 -> 12.8 (and 10.0
+// with one); fp16 [1024, 8192] k=64 j=4 k_mult=4 22.1 -> 13.4, [32, 20480] k=512 j=2 k_mult=2 7.45 -> 6.95, but [2048, 32768]
+// k=512 j=1 k_mult=2 31.8 -> 34.5, bound by the load instructions (see `estimate`, fused_row_plan.hip).
+constexpr bool registers_only(int elem_bytes, int vec) {
+  return (elem_bytes == 4 && vec <= 2) || (elem_bytes == 2 && vec == 2);
+}
+
 // Stage 1 of a row whose buckets are runs of `m` adjacent elements of 16 to 256
 // bytes each (contiguous layout, every bucket as long).  A lane takes V buckets
 // kWave apart, `first` the first of them, so that the lanes of a wave load from
@@ -295,7 +307,8 @@ __device__ __forceinline__ void scan_short_buckets(const typename E::raw_t* __re
 // of every lane's first bucket, then of every lane's second, ...
 template <typename E, int J, int V, int MAXW, typename pos_t, bool PACKED, bool CONTIG = false, bool PAST_CACHE = false>
 __global__ __launch_bounds__(kWave * MAXW)
-__attribute__((amdgpu_waves_per_eu(PACKED && V * J <= 16 && !(CONTIG && V * J > 8) ? 8 : 1))) void fused_regs_kernel(
+__attribute__((amdgpu_waves_per_eu(registers_only((int)sizeof(typename E::raw_t), V) ||
+                                   (PACKED && V * J <= 16 && !(CONTIG && V * J > 8)) ? 8 : 1))) void fused_regs_kernel(
     const typename E::raw_t* __restrict__ x, typename E::raw_t* __restrict__ values,
     const IndexOut indices, const Geom g, uint32_t tiles, uint32_t split, uint32_t hand_off,
     uint32_t k0, uint32_t k, int index_bits, int staged) {

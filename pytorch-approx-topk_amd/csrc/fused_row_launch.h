@@ -39,15 +39,19 @@ static int launch_packed(const Plan& pl, const typename E::raw_t* x, int64_t row
                        indices, g, pl.tiles, pl.split, pl.hand_off, k0, k, pl.index_bits, staged);
     return hipGetLastError() == hipSuccess ? ATK_OK : ATK_ERR_LAUNCH;
   }
-  auto kern = fused_row_kernel<E, J, V, MAXW, pos_t, PACKED>;
-  if (pl.lds_bytes > 48 * 1024) {
-    if (hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
-                            (int)pl.lds_bytes) != hipSuccess)
-      return ATK_ERR_LAUNCH;
+  if constexpr (registers_only((int)sizeof(typename E::raw_t), V)) {
+    return ATK_ERR_ARG;  // the planner never asks for it
+  } else {
+    auto kern = fused_row_kernel<E, J, V, MAXW, pos_t, PACKED>;
+    if (pl.lds_bytes > 48 * 1024) {
+      if (hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
+                              (int)pl.lds_bytes) != hipSuccess)
+        return ATK_ERR_LAUNCH;
+    }
+    hipLaunchKernelGGL(kern, dim3((unsigned)rows), dim3(kWave * pl.waves), pl.lds_bytes, stream, x, values,
+                       indices, g, pl.tiles, pl.split, pl.hand_off, k0, k, pl.index_bits);
+    return hipGetLastError() == hipSuccess ? ATK_OK : ATK_ERR_LAUNCH;
   }
-  hipLaunchKernelGGL(kern, dim3((unsigned)rows), dim3(kWave * pl.waves), pl.lds_bytes, stream, x, values,
-                     indices, g, pl.tiles, pl.split, pl.hand_off, k0, k, pl.index_bits);
-  return hipGetLastError() == hipSuccess ? ATK_OK : ATK_ERR_LAUNCH;
 }
 
 template <typename E, int J, int V, int MAXW, typename pos_t>
@@ -85,6 +89,19 @@ static int launch_j(const Plan& pl, const typename E::raw_t* x, int64_t rows, co
   if constexpr (stream::PackedKey<E>::available && sizeof(typename E::raw_t) == 2) {
     // packed queues may run at half the load width (fewer registers, more workgroups per CU)
     if (pl.vec == VF / 2) return launch_v<E, J, VF / 2>(pl, x, rows, g, k0, k, values, indices, stream);
+  }
+  // narrower loads yet: the register kernel's, with 16-bit sub-row numbers and (16-bit elements) packed queues
+  constexpr int ES = (int)sizeof(typename E::raw_t);
+  constexpr bool kPacked = stream::PackedKey<E>::available && ES == 2;
+  if constexpr (ES == 4 || kPacked) {
+    if (pl.vec < VF) {
+      if (!pl.in_registers || !pl.pos16 || pl.packed != kPacked || pl.contig) return ATK_ERR_ARG;  // (never planned)
+      if (pl.vec == 2) return launch_packed<E, J, 2, 8, uint16_t, kPacked>(pl, x, rows, g, k0, k, values, indices, stream);
+      if constexpr (ES == 4) {
+        if (pl.vec == 1) return launch_packed<E, J, 1, 8, uint16_t, false>(pl, x, rows, g, k0, k, values, indices, stream);
+      }
+      return ATK_ERR_ARG;
+    }
   }
   return launch_v<E, J, VF>(pl, x, rows, g, k0, k, values, indices, stream);
 }

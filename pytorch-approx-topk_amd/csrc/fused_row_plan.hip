@@ -1,4 +1,6 @@
 // Host-side planning and dispatch of the fused one-workgroup-per-row kernel.
+#include <cmath>
+
 #include "fused_row.h"
 
 namespace atk {
@@ -116,17 +118,17 @@ static Plan plan_short_buckets(int64_t rows, int64_t n, int64_t k0, int j, int64
   return pl;
 }
 
-Plan make_plan(int64_t rows, int64_t n, int64_t k0, int j, int64_t k, int layout, int dtype, bool aligned) {
+// Interleaved buckets, loads of `vec` elements.  `by_size`: only where the rules of size below call this path the faster one
+// (they were measured with loads of the usual width); else wherever the kernels take the call.
+static Plan plan_interleaved(int64_t rows, int64_t n, int64_t k0, int j, int64_t k, int dtype, bool aligned, int vec,
+                             bool by_size) {
   Plan pl{};
   pl.ok = false;
-  if (layout == ATK_BALANCED) return plan_short_buckets(rows, n, k0, j, k, dtype);
-  // (a padded row is never reduced further: its callers keep every bucket)
-  if (layout != ATK_INTERLEAVED) return pl;
   if (rows > 0x7fffffffll) return pl;
   if (k0 <= 0 || k <= 0 || k >= k0 || j < 1 || j > 4 || k0 % j) return pl;
   const int es = elem_bytes(dtype);
   if (!es) return pl;
-  if (rows < kMinRows && (size_t)n * es > kSoloRow) return pl;
+  if (by_size && rows < kMinRows && (size_t)n * es > kSoloRow) return pl;
   const int64_t b = k0 / j;
   const int64_t full = n / b;
   if (full < j || full > 0x7fffffffll) return pl;
@@ -135,10 +137,10 @@ Plan make_plan(int64_t rows, int64_t n, int64_t k0, int j, int64_t k, int layout
   pl.pad_tail = 0;
   pl.pos16 = full + 1 <= 0xffff;
   pl.packed = (dtype == ATK_F16 || dtype == ATK_BF16 || dtype == ATK_I16) && full <= stream::kPackedMaxSubRow;
-  pl.vec = stream::full_vec(es);
+  pl.vec = vec;
   // packed queues at half the load width need about 50 VGPRs instead of 127:
   // twice the workgroups per CU, which is worth more here than 16-byte loads
-  if (pl.packed) pl.vec /= 2;
+  if (pl.packed && pl.vec == stream::full_vec(es)) pl.vec /= 2;
   if (b % pl.vec) return pl;
   const int64_t bound = (full + 1) * b;  // indices are < this
   pl.index_bits = 1;
@@ -164,7 +166,7 @@ Plan make_plan(int64_t rows, int64_t n, int64_t k0, int j, int64_t k, int layout
     if (row_bytes_ > 16 * 1024) least = 256;
     if (row_bytes_ > 32 * 1024 || rows >= 2048) least = 512;
     const bool small_batch = (size_t)rows * row_bytes_ <= (1u << 20);
-    if (sub_row_bytes < least && (!small_batch || full >= 256)) return pl;
+    if (by_size && sub_row_bytes < least && (!small_batch || full >= 256)) return pl;
   }
   // One launch instead of two, and no candidates parked in HBM: measured over
   // 128-4096 rows of 8192-262144 elements with 256-4096 candidates, this kernel
@@ -179,7 +181,7 @@ Plan make_plan(int64_t rows, int64_t n, int64_t k0, int j, int64_t k, int layout
   const size_t row_bytes = (size_t)n * es;
   const bool corner = es == 1 || (!pl.packed && ((rows >= kManyRows && row_bytes < kShortRow) ||
                                                  (rows < kAllCus && j >= 3 && row_bytes >= kLongRow)));
-  if (corner && (size_t)k0 * (es + 8) * 4 < row_bytes) return pl;
+  if (by_size && corner && (size_t)k0 * (es + 8) * 4 < row_bytes) return pl;
   const int skey = (dtype == ATK_U8 || dtype == ATK_I8) ? 2 : es;  // stored key width
   const size_t cand_bytes = (((size_t)k0 * skey + 15) & ~(size_t)15) +
                             (((size_t)k0 * (pl.pos16 ? 2 : 4) + 15) & ~(size_t)15);
@@ -218,7 +220,7 @@ Plan make_plan(int64_t rows, int64_t n, int64_t k0, int j, int64_t k, int layout
   pl.split = split;
   pl.waves = pl.tiles * split <= max_waves ? pl.tiles * split : max_waves;
   const int64_t turns = ((int64_t)pl.tiles * split + pl.waves - 1) / pl.waves;
-  if (!aligned && !loose_rows_gain(rows, b * es, full / split * turns, j, es)) return pl;
+  if (by_size && !aligned && !loose_rows_gain(rows, b * es, full / split * turns, j, es)) return pl;
   const bool one_round = pl.tiles * split <= max_waves;
   pl.hand_off = (split > 1 && !one_round) ? (uint32_t)cand_bytes : 0u;
   pl.lds_bytes = lds_need(split);
@@ -241,6 +243,84 @@ Plan make_plan(int64_t rows, int64_t n, int64_t k0, int j, int64_t k, int layout
   return pl;
 }
 
+// Whether the rules of size alone, which the figure of atk_topk_workspace_bytes_at follows, choose one kernel.
+bool taken_by_size(int64_t rows, int64_t n, int64_t k0, int j, int64_t k, int layout, int dtype, bool aligned) {
+  if (layout == ATK_BALANCED) return plan_short_buckets(rows, n, k0, j, k, dtype).ok;
+  const int es = elem_bytes(dtype);
+  return layout == ATK_INTERLEAVED && es != 0 &&
+         plan_interleaved(rows, n, k0, j, k, dtype, aligned, stream::full_vec(es), true).ok;
+}
+
+namespace {
+// Rows and candidates up to which the estimates below were fitted.
+constexpr int64_t kEstimatedRow = 1 << 20, kEstimatedCandidates = 8192;
+// A call that the rules of size leave to two kernels takes one where its estimate is this share of theirs.
+constexpr double kOneKernelShare = 0.92;
+
+// Estimated microseconds of the register kernel under a plan of elements of two or four bytes: the scan (memory, instructions
+// and the round trips of a wave's loads, which overlap: the root of the sum of their squares), and what every
+// round of workgroups that the GPU holds at once goes through behind it, the fold of the waves that share a tile and the
+// selection, by the candidates of a lane and the waves that wait for one another.
+// The constants are a least-squares fit to 1415 launches of 620 calls (fp32 and fp16, 1-8192 rows of 2048-2^18 elements,
+// half of them of no round length, 32-8192 candidates, j 1, 2, 4, k_mult 2-8, up to 160 MiB; every width of load): off by
+// 10 % in the root mean square.  Among those calls, the choice by these estimates is 1.4 % slower than the best of two kernels
+// and one with each width; the rules of size with the usual width, which stood before, are 16 %.  (float32 [859, 2048]
+// k=64 j=4 k_mult=2 29.0 us by the rules, 10.4 with one column a lane; [1053, 19352] k=152 j=1 k_mult=2 35.5 in two kernels, 21.1
+// in one; fp16 [2048, 8192] k=100 j=2 k_mult=4 37.1 in two kernels, 18 in one.)
+double estimate(const Plan& pl, int64_t rows, int64_t n, int j, int es) {
+  constexpr double kBytes = 5.2e6;                                      // per us
+  constexpr double kLaunch = 1.45, kTrip = 0.14, kShare = 0.51;         // us; kShare: a SIMD's wave beside others
+  constexpr double kLoad = 0.0225, kPush = 0.0128, kPushEntry = 0.0056; // us per sub-row, column, entry: 4-byte elements
+  constexpr double kLoad2 = 0.0206, kPush2 = 0.0142, kPushEntry2 = 0.003;  // ... 2-byte elements
+  constexpr double kChain = 2.32, kChainWave = 0.081, kChainEntry = 0.298, kFoldEntry = 0.002;
+  const int entries = pl.vec * j;  // of a lane
+  const double run = (double)pl.full_rows / pl.split;
+  const int loads = es == 2 ? (entries <= 8 ? 8 : 4) : (j <= 2 ? 8 : 4);  // in flight
+  const double sub_row = es == 2 ? kLoad2 + pl.vec * (kPush2 + kPushEntry2 * j) : kLoad + pl.vec * (kPush + kPushEntry * j);
+  // workgroups a CU holds: by registers (waves per SIMD) and by LDS, the kernel's own 5.6 KB included
+  const int waves_per_simd = es == 4 && pl.vec == 4 ? (j == 1 ? 5 : 4) : 8;
+  const int by_waves = waves_per_simd * 4 / (int)pl.waves, by_lds = (int)(160 * 1024 / (pl.lds_bytes + 5600));
+  const double held = by_waves < by_lds ? by_waves : by_lds;
+  const double rounds = (double)rows > 256 * held ? (double)rows / (256 * held) : 1.0;
+  const double on_cu = std::ceil((double)rows / 256);
+  const double on_simd = pl.waves * (on_cu < held ? on_cu : held) / 4;
+  const double share = on_simd > 1 ? on_simd * kShare : kShare;
+  const double memory = (double)rows * (double)n * es / kBytes;
+  const double issue = run * sub_row * (share > 1 ? share : 1.0) * rounds;
+  const double trips = kTrip * (run > loads ? run / loads : 1.0) * rounds;
+  return kLaunch + std::sqrt(memory * memory + issue * issue + trips * trips) +
+         rounds * (kChain + kChainWave * pl.waves + kChainEntry * entries + kFoldEntry * (pl.split - 1) * entries);
+}
+}  // namespace
+
+Plan make_plan(int64_t rows, int64_t n, int64_t k0, int j, int64_t k, int layout, int dtype, bool aligned) {
+  if (layout == ATK_BALANCED) return plan_short_buckets(rows, n, k0, j, k, dtype);
+  Plan pl{};
+  pl.ok = false;
+  const int es = elem_bytes(dtype);
+  // (a padded row is never reduced further: its callers keep every bucket)
+  if (layout != ATK_INTERLEAVED || es == 0) return pl;
+  pl = plan_interleaved(rows, n, k0, j, k, dtype, aligned, stream::full_vec(es), true);
+  if ((es != 2 && es != 4) || n * es > kEstimatedRow || k0 > kEstimatedCandidates || (pl.ok && !pl.in_registers)) return pl;
+  // the register kernel with every width of load that it takes here
+  Plan best = pl;
+  double least = pl.ok ? estimate(pl, rows, n, j, es)
+                       : kOneKernelShare * stream::estimate_two_kernels(rows, n, k0, j, dtype);
+  for (int vec = stream::full_vec(es) / (es == 2 ? 2 : 1); vec >= 4 / es; vec /= 2) {
+    if (pl.ok && vec == pl.vec) continue;
+    const Plan other = plan_interleaved(rows, n, k0, j, k, dtype, aligned, vec, false);
+    if (!other.ok || !other.in_registers || !other.pos16 || other.packed != (es == 2)) continue;
+    // Few rows off 16 bytes whose sub-rows leave more than half of a wave's lanes idle stay with two kernels: short ones
+    // would gain (fp32 [22, 3603] b=24 j=4 9.0 -> 5.6 us), long ones lose many times over, and of 40 such calls the
+    // estimate is off most (fp16 [14, 15031] b=40 j=2 7.7 -> 8.9).
+    if (!pl.ok && !aligned && rows < kMinRows && k0 / j * 2 < (int64_t)stream::kWave * vec) continue;
+    if (rows > 0xffffffffll / (64 * (int64_t)other.waves)) continue;  // (a launch's threads are counted in 32 bits)
+    const double us = estimate(other, rows, n, j, es);
+    if (us < least) { best = other; least = us; }
+  }
+  return best;
+}
+
 }  // namespace fused
 
 bool rows_on_load_width(const void* x, int64_t row_stride, int dtype) {
@@ -250,11 +330,30 @@ bool rows_on_load_width(const void* x, int64_t row_stride, int dtype) {
 
 namespace {
 // Rows may start at any element (rows of odd length do, and views): the 16-byte loads take such addresses.
+// The plans of a thread's last shapes are kept: every call asks for its plan, and a program repeats few shapes.
 fused::Plan plan_for(const void* x, int64_t rows, int64_t n, int64_t row_stride, int64_t k0, int j, int64_t k,
                      int layout, int dtype) {
-  return fused::make_plan(rows, n, k0, j, k, layout, dtype, rows_on_load_width(x, row_stride, dtype));
+  struct Made {
+    int64_t rows, n, k0, k;  // rows == 0: nothing made yet (such calls have no plan)
+    int j, layout, dtype, aligned;
+    fused::Plan plan;
+  };
+  constexpr uint64_t kMade = 16;
+  static thread_local Made made[kMade];
+  const int aligned = rows_on_load_width(x, row_stride, dtype) ? 1 : 0;
+  const uint64_t h = ((uint64_t)rows * 31 + (uint64_t)n) * 31 + (uint64_t)k0 * 7 + (uint64_t)k;
+  Made& m = made[(h ^ (h >> 17)) % kMade];
+  if (rows <= 0 || m.rows != rows || m.n != n || m.k0 != k0 || m.k != k || m.j != j || m.layout != layout ||
+      m.dtype != dtype || m.aligned != aligned)
+    m = Made{rows, n, k0, k, j, layout, dtype, aligned, fused::make_plan(rows, n, k0, j, k, layout, dtype, aligned != 0)};
+  return m.plan;
 }
 }  // namespace
+
+bool fused_row_taken_by_size(const void* x, int64_t rows, int64_t n, int64_t row_stride, int64_t k0, int j, int64_t k,
+                             int layout, int dtype) {
+  return fused::taken_by_size(rows, n, k0, j, k, layout, dtype, rows_on_load_width(x, row_stride, dtype));
+}
 
 bool fused_row_takes(const void* x, int64_t rows, int64_t n, int64_t row_stride, int64_t k0, int j, int64_t k,
                      int layout, int dtype) {

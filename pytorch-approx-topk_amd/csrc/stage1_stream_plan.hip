@@ -255,6 +255,14 @@ Plan make_plan(int64_t rows, int64_t n, int64_t k0, int j, int layout, int dtype
   return us(v) < us(w) * (large ? kLargeShare : 1.0) ? v : w;
 }
 
+double estimate_two_kernels(int64_t rows, int64_t n, int64_t k0, int j, int dtype) {
+  const Plan pl = make_plan(rows, n, k0, j, ATK_INTERLEAVED, dtype, n);
+  if (!pl.ok) return INFINITY;
+  const bool selects = selects_in_merge(pl, k0, n, dtype);
+  const double us = estimate(pl, rows, n, k0, j, dtype, true, selects);
+  return selects ? 2.66 + 0.962 * us : 1.68 + us;
+}
+
 bool selects_in_merge(const Plan& pl, int64_t k0, int64_t index_bound, int dtype) {
   return pl.ok && pl.merge && elem_bytes(dtype) <= 4 && index_bound <= 0xffffffffll && k0 <= kMergeSelectMax &&
          k0 * (int64_t)pl.slabs <= kMergeSelectEntries;

@@ -421,3 +421,25 @@ def test_no_plan_has_more_threads_than_a_launch_takes():
         assert L.atk_describe(4096, rows, n, n, k0, j, k, 0, code, 4096, 4096, buf, 1024) == 0
         for grid, block in re.findall(r"grid=(\d+) block=(\d+)", buf.value.decode()):
             assert int(grid) * int(block) < 1 << 32, buf.value
+
+
+def test_the_workspace_a_call_uses_stays_within_the_figure_at_its_address():
+    # (more calls go through one kernel than that figure tells: it stays what callers have sized buffers by)
+    import random
+    from approx_topk import _native
+    L = _native.lib()
+    rng = random.Random(7)
+    for _ in range(4000):
+        code, j, k_mult = rng.choice((0, 1, 2, 6, 7)), rng.randint(1, 4), rng.choice((2, 3, 4, 8))
+        n = int(2 ** rng.uniform(6, 19))
+        k = max(1, int(2 ** rng.uniform(2, 13)) // k_mult) * j
+        if k * k_mult > n:
+            continue
+        rows = int(2 ** rng.uniform(0, 14))
+        args = (rows, n, n + rng.choice((0, 0, 1, 8)), k * k_mult, j, k, 0, code)
+        at = L.atk_topk_workspace_bytes_at(4096, *args)
+        used = L.atk_topk_workspace_bytes_used(4096, *args)
+        assert used in (0, L.atk_topk_workspace_bytes(rows, n, k * k_mult, j, k, 0, code)) and used <= at, args
+        buf = ctypes.create_string_buffer(1024)
+        assert L.atk_describe(4096, *args, 4096, 4096, buf, 1024) == 0
+        assert (used == 0) == buf.value.startswith(b"fused_"), (args, buf.value)
