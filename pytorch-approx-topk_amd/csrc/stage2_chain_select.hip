@@ -596,25 +596,48 @@ __global__ __launch_bounds__(kSoloThreads) void chain_solo_kernel(
   const bool own_valid = FULL || own < k0;
   // survivors above the cut digit (or in it, when it belongs whole) in the
   // segments before this one, and the members of a cut digit: listed, or flagged for the
-  // look at their indices below
+  // look at their indices below.
+  // (Sixteen waves go through every key here, and an operation on each of a thread's 32 keys is 0.2 us.  So: two comparisons
+  // with keys at the digit's ends, whose outcomes are shifted into two words; no branch, no wave-wide mask (the
+  // kernel with 32 keys has no scalar registers for 32 of them) and no atomic per key.  The few members leave their
+  // places in the list, and their keys are read again with their indices.  32768 fp32 candidates, k = 16384: this step
+  // 3.6 -> 1.9 us, the launch 12.4 -> 10.1.)
+  const uint32_t first = low + (f.digit << shift), width1 = (1u << shift) - 1u;  // the digit's keys: first .. first + width1
+  // keys above it are survivors (first > 0 where the digit belongs whole: something is cut)
+  const uint32_t above = cut_digit ? (first > ~0u - width1 ? ~0u : first + width1) : first - 1u;
   uint32_t before = 0;
-  uint32_t own_key = 0;
-  [[maybe_unused]] uint32_t members = 0;
+  uint32_t members = 0;  // bit u: candidate u is a member
+  {
+    uint32_t better = 0;
 #pragma unroll
-  for (int u = 0; u < NPT; ++u) {
-    const uint32_t d = (key[u] - low) >> shift;
-    const bool ok = valid(u);
-    if ((uint32_t)u < g) before += (ok && (d > f.digit || (d == f.digit && !cut_digit))) ? 1u : 0u;
-    if ((uint32_t)u == g) own_key = key[u];
-    if (ok && cut_digit && d == f.digit) {
-      if constexpr (TIES) members |= 1u << u;
-      if (list_it) {
-        const uint32_t at = (uint32_t)u * kSoloThreads + tid;
-        const uint32_t slot = atomicAdd(&list_count, 1u);
-        words[slot] = (uint64_t)key[u] << 32;  // (the index follows below, for all members in one trip to memory)
-        ats[slot] = at;
-      }
+    for (int u = NPT - 1; u >= 0; --u) {
+      // better = 2 * better + (key > above), members = 2 * members + (key - first <= width1), an add with carry each
+      // (a comparison's mask is read two issue slots after it is written, at the earliest)
+      uint64_t mask;
+      asm("v_cmp_lt_u32_e64 %2, %4, %3\n\t"
+          "v_cmp_ge_u32_e32 vcc, %6, %5\n\t"
+          "s_nop 0\n\t"
+          "v_addc_co_u32_e64 %0, %2, %0, %0, %2\n\t"
+          "v_addc_co_u32_e32 %1, vcc, %1, %1, vcc"
+          : "+v"(better), "+v"(members), "=&s"(mask)
+          : "v"(key[u]), "s"(above), "v"(key[u] - first), "s"(width1)
+          : "vcc");
     }
+    uint32_t exist = ~0u;
+    if constexpr (!FULL) {
+      const uint32_t mine = tid < k0 ? (k0 - tid + kSoloThreads - 1) / kSoloThreads : 0u;  // candidates of this thread
+      exist = mine >= 32u ? ~0u : (1u << mine) - 1u;
+    }
+    members &= cut_digit ? exist : 0u;
+    before = (uint32_t)__popc(better & exist & ((1u << g) - 1u));  // (g < NPT <= 32)
+  }
+  if (list_it) {
+    const uint32_t mine = (uint32_t)__popc(members), incl = regs::wave_scan(mine);
+    uint32_t slot = 0;
+    if (lane == select::kWave - 1 && incl != 0) slot = atomicAdd(&list_count, incl);
+    slot = (uint32_t)__builtin_amdgcn_readlane((int)slot, select::kWave - 1) + incl - mine;
+    for (uint32_t left = members; left != 0; left &= left - 1u)
+      ats[slot++] = (uint32_t)(__ffs((int)left) - 1) * kSoloThreads + tid;
   }
   uint32_t need = f.need, count = f.count;
   uint64_t floor_word = 0;  // tie mode, when a whole group of indices survives: its smallest word
@@ -785,10 +808,7 @@ __global__ __launch_bounds__(kSoloThreads) void chain_solo_kernel(
     return;
   }
   const uint32_t n = need != count ? count : 0u;  // (== list_count after the barrier)
-  if (tid < 8u) {  // entries past the list's end beat nothing (ranking reads it in groups of eight)
-    words[n + tid] = 0ull;
-    ats[n + tid] = ~0u;
-  }
+  if (tid < kSoloRankDirect) hist[tid] = 0;  // (read by wave 0 before the last barrier: the list's ranks from here on)
   __syncthreads();
   ATK_TRACE_GROUP(4);
   // This thread's own candidate, asked for together with the listed members'
@@ -799,21 +819,21 @@ __global__ __launch_bounds__(kSoloThreads) void chain_solo_kernel(
   uint64_t cut = floor_word;  // the weakest surviving member of B (0: all of them survive)
   if (n != 0) {
     if (!tie_mode)
-      for (uint32_t i = tid; i < n; i += kSoloThreads) words[i] |= (uint64_t)(~(uint32_t)ci[ats[i]]);
+      for (uint32_t i = tid; i < n; i += kSoloThreads)
+        words[i] = ((uint64_t)(uint32_t)E::key(cv[ats[i]]) << 32) | (uint64_t)(~(uint32_t)ci[ats[i]]);
     __syncthreads();
     if (n <= kSoloRankDirect) {
-      if (tid < n) {  // thread t counts the entries better than entry t: the need-th best is the cut
-        const uint64_t mine = words[tid];
-        uint32_t better = 0;
-        for (uint32_t m = 0; m < n; m += 8) {
-          uint64_t got[8];
-#pragma unroll
-          for (int e = 0; e < 8; ++e) got[e] = words[m + e];
-#pragma unroll
-          for (int e = 0; e < 8; ++e) better += got[e] > mine ? 1u : 0u;
-        }
-        if (better + 1 == need) cut_word = mine;
-      }
+      // The need-th best is the cut.  Whole waves take a share of the comparisons of 64 entries with all others.
+      uint32_t stretch = select::kWave;  // threads that hold all entries once
+      while (stretch < n) stretch *= 2;
+      const uint32_t e = tid & (stretch - 1u), shares = kSoloThreads / stretch;
+      const uint64_t mine = e < n ? words[e] : ~0ull;
+      uint32_t better = 0;
+#pragma unroll 4
+      for (uint32_t m = tid / stretch; m < n; m += shares) better += words[m] > mine ? 1u : 0u;
+      if (better != 0) atomicAdd(&hist[e], better);
+      __syncthreads();
+      if (tid < n && hist[tid] + 1 == need) cut_word = mine;
       __syncthreads();
       cut = cut_word;
     } else {  // a longer list: the block-wide radix select over its words (all distinct)
@@ -825,7 +845,7 @@ __global__ __launch_bounds__(kSoloThreads) void chain_solo_kernel(
   }
   ATK_TRACE_GROUP(5);
   // this thread's own candidate
-  const uint32_t own_d = (own_key - low) >> shift;
+  const uint32_t own_key = (uint32_t)E::key(own_raw), own_d = (own_key - low) >> shift;
   const bool sel = own_valid && (own_d > f.digit ||
                                  (own_d == f.digit && (((uint64_t)own_key << 32) | own_inv) >= cut));
   const uint64_t m = __ballot(sel);

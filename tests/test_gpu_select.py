@@ -230,3 +230,21 @@ def test_chain_select_after_stage1_takes_the_key_ranges_from_the_merge():
     v, i = topk(x16.cuda(), 4096, -1, j=2, k_mult=4)
     ev, ei = oracle.topk(x16, 4096, -1, j=2, k_mult=4)
     assert_same(v, i, ev, ei, "two long fp16 rows")
+
+
+@pytest.mark.parametrize("k0", [10241, 16384, 31745, 32767, 32768])
+@pytest.mark.parametrize("m", [2, 64, 65, 512, 513, 1000])
+def test_one_launch_select_of_lists_of_every_length(k0, m):
+    # m candidates share the digit that is cut (2048 digits of 1024 values each), at the end of the row,
+    # in its last segment, whole or not; up to 512 of them are ranked by comparison, more by radix passes
+    g = torch.Generator().manual_seed(k0 + m)
+    others = torch.randint(0, 2047 * 1024, (3, k0 - m), generator=g)
+    others = others + 1024 * (others >= 700 * 1024)  # none in digit 700
+    others[:, 0], others[:, 1] = 0, 2048 * 1024 - 1
+    listed = 700 * 1024 + torch.stack([torch.randperm(1024, generator=g)[:m] for _ in range(3)])
+    cv = torch.cat((others, listed), 1).to(torch.int32)
+    ci = torch.stack([torch.randperm(1 << 21, generator=g)[:k0] for _ in range(3)])
+    above = int((others[0] >= 701 * 1024).sum())
+    for k in {above + 1, above + (m + 1) // 2, above + m - 1, above + m}:
+        v, i = _select(cv, ci, k, 1 << 21)
+        assert_same(v, i, *oracle.stage2(cv, ci, k), f"k0={k0} m={m} k={k}")
