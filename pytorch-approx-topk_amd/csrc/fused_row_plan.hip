@@ -255,7 +255,7 @@ namespace {
 // Rows and candidates up to which the estimates below were fitted.
 constexpr int64_t kEstimatedRow = 1 << 20, kEstimatedCandidates = 8192;
 // A call that the rules of size leave to two kernels takes one where its estimate is this share of theirs.
-constexpr double kOneKernelShare = 0.92;
+constexpr double kOneKernelShare = 0.85;
 
 // Estimated microseconds of the register kernel under a plan of elements of two or four bytes: the scan (memory, instructions
 // and the round trips of a wave's loads, which overlap: the root of the sum of their squares), and what every
