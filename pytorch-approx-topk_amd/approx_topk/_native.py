@@ -1,13 +1,15 @@
 """ctypes binding of libapprox_topk_hip.so (the C ABI in include/approx_topk_hip.h).
 
 The library is built in-tree by ``pytorch-approx-topk_amd/build.py`` and sits
-next to this file.  There is no fallback: if it cannot be loaded, every call
-that needs it raises.
+next to this file, as does ``_host.so`` (csrc/host_binding.cpp), which makes the
+common calls without Python in between: contiguous rows of plain tensors.  There
+is no fallback: if either cannot be loaded, every call that needs them raises.
 """
 from __future__ import annotations
 
 import ctypes
 import functools
+import importlib
 import os
 
 import torch
@@ -62,6 +64,11 @@ _SIGNATURES = {
 }
 
 
+_HOST_PATH = os.path.join(os.path.dirname(os.path.abspath(__file__)), "_host.so")
+# (imported with the package: it registers the operators' kernels for the GPU)
+host = importlib.import_module("._host", __package__) if os.path.exists(_HOST_PATH) else None
+
+
 def library_path() -> str:
     return os.environ.get("APPROX_TOPK_HIP_LIB") or os.path.join(
         os.path.dirname(os.path.abspath(__file__)), LIB_NAME)
@@ -80,6 +87,11 @@ def lib() -> ctypes.CDLL:
         fn.restype, fn.argtypes = restype, argtypes
     if handle.atk_version() != ABI_VERSION:
         raise RuntimeError(f"approx_topk: {path} has ABI {handle.atk_version()}, expected {ABI_VERSION}")
+    if host is None:
+        raise RuntimeError(
+            f"approx_topk: {_HOST_PATH} is missing. Build it with `python pytorch-approx-topk_amd/build.py`; "
+            "there is no fallback path.")
+    host.bind({name: ctypes.cast(getattr(handle, name), ctypes.c_void_p).value for name in _SIGNATURES})
     return handle
 
 
@@ -191,6 +203,10 @@ def stage1(xs: torch.Tensor, k0: int, j: int, layout: int, index_dtype: torch.dt
     ``index_dtype``: torch.int64 (the operator's contract) or torch.int32.
     ``want_values=False``: only the indices are written; values is None."""
     require_gpu(xs)
+    if host is not None:
+        out = host.run(xs, k0, j, k0, layout, index_dtype != torch.int64, want_values, False)
+        if out is not None:
+            return out
     step = None
     if not xs.is_contiguous():
         xs, _, _, step = rows_view(xs)
@@ -234,6 +250,10 @@ def topk(xs: torch.Tensor, k0: int, j: int, k: int, layout: int, index_dtype: to
          want_values: bool = True) -> tuple[torch.Tensor | None, torch.Tensor]:
     """Stage 1 (k0 candidates) and stage 2 (k survivors) along the last dim."""
     require_gpu(xs)
+    if host is not None:
+        out = host.run(xs, k0, j, k, layout, index_dtype != torch.int64, want_values, True)
+        if out is not None:
+            return out
     step = None
     if not xs.is_contiguous():
         xs, _, _, step = rows_view(xs)

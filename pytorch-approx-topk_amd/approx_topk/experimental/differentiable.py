@@ -26,6 +26,9 @@ from .. import _native
 from ..priority_queue import topk as _topk, topk_grad as _topk_grad
 
 
+_PLAIN = (Tensor, torch.nn.Parameter)
+
+
 def _autograd_has_work(grad_values: Tensor) -> bool:
     """Whether the gradient may itself be differentiated or traced: reverse mode, forward mode (both kinds enter
     a level), a functorch transform, or ``torch.compile``, which does not look into dispatcher guards."""
@@ -74,4 +77,9 @@ def topk(
     multithread_buckets: bool | None = False,
 ) -> tuple[Tensor, Tensor]:
     """``approx_topk.topk`` whose values carry a gradient with respect to ``xs``."""
+    # Plain GPU tensors outside of every transform: the same node in native code (csrc/host_binding.cpp), whose
+    # backward leaves what is differentiated again to the operator's autograd kernel as the one above does.
+    if (not is_compiling() and _native.host is not None and type(xs) in _PLAIN and xs.is_cuda
+            and peek_interpreter_stack() is None and forward_ad._current_level < 0):
+        return _native.host.differentiable_topk(xs, k, dim, j, k_mult, interleaved, multithread_buckets)
     return _TopkWithGradient.apply(xs, k, dim, j, k_mult, interleaved, multithread_buckets)

@@ -3,6 +3,8 @@
 Same operator name, signature, defaults and error behaviour as the reference's
 approx_topk/priority_queue.py:14-110; the body calls hand-written HIP kernels
 through the C ABI of libapprox_topk_hip.so instead of a JIT-built CUDA module.
+On GPU tensors the operators' kernels are those of csrc/host_binding.cpp, which make
+the common calls themselves and hand everything else to the bodies below.
 
 The operator is defined on a ``torch.library.Library`` and ``topk`` is its
 overload object (callable like the reference's, accepted by
@@ -178,6 +180,9 @@ def _(grad_values: Tensor, indices: Tensor, n: int, k0: int, j: int, interleaved
 
 
 topk_grad = torch.ops.approx_topk.topk_grad.default
+
+if _native.host is not None:
+    _native.host.set_general(_topk, _topk_grad)
 
 
 # The reference's ``topk`` is a ``CustomOpDef`` (approx_topk/priority_queue.py:14), whose

@@ -4,7 +4,9 @@
 
 Every .hip file under csrc/ is compiled to an object (in parallel) and linked
 into approx_topk/libapprox_topk_hip.so, next to the Python package that loads
-it.  Nothing is linked against libtorch: the library speaks a C ABI only.
+it.  Nothing of it is linked against libtorch: the library speaks a C ABI only.
+csrc/host_binding.cpp, which calls that library with torch's tensors, becomes the
+extension module approx_topk/_host.so.
 
 --trace builds a second library, approx_topk/libapprox_topk_hip_trace.so, whose long
 kernels stamp a clock at their phase boundaries (csrc/atk_trace.h); it is what
@@ -14,14 +16,17 @@ from __future__ import annotations
 
 import concurrent.futures
 import glob
+import importlib.util
 import os
 import subprocess
 import sys
+import sysconfig
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 OBJ = os.path.join(HERE, "build")
 LIB = os.path.join(HERE, "approx_topk", "libapprox_topk_hip.so")
+HOST = os.path.join(HERE, "approx_topk", "_host.so")
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 
 FLAGS = [
@@ -39,6 +44,18 @@ def _newer(target: str, deps: list[str]) -> bool:
         return False
     t = os.path.getmtime(target)
     return all(os.path.getmtime(d) <= t for d in deps)
+
+
+def _host_command(source: str) -> list[str]:
+    torch_dir = importlib.util.find_spec("torch").submodule_search_locations[0]
+    include, lib = os.path.join(torch_dir, "include"), os.path.join(torch_dir, "lib")
+    rocm = os.path.join(os.path.dirname(os.path.dirname(HIPCC)), "include")
+    return [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden", "-Wall",
+            "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1", "-DTORCH_API_INCLUDE_EXTENSION_H", "-DTORCH_EXTENSION_NAME=_host",
+            # (the headers of others, whose warnings are theirs)
+            "-isystem", include, "-isystem", os.path.join(include, "torch", "csrc", "api", "include"), "-isystem", rocm,
+            "-isystem", sysconfig.get_paths()["include"], source, "-L" + lib, "-Wl,-rpath," + lib,
+            "-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch_hip", "-ltorch", "-ltorch_python", "-o", HOST]
 
 
 def build(force: bool = False, verbose: bool = True, trace: bool = False) -> str:
@@ -74,6 +91,9 @@ def build(force: bool = False, verbose: bool = True, trace: bool = False) -> str
                 return rank
         return len(heavy)
     jobs.sort(key=weight)
+    host = os.path.join(CSRC, "host_binding.cpp")
+    if not trace and (force or not _newer(HOST, [host, headers[-1]])):
+        jobs.append(_host_command(host))
     with concurrent.futures.ThreadPoolExecutor(max_workers=min(8, max(1, len(jobs)))) as ex:
         for cmd, r in ex.map(run, jobs):
             # hipcc's host pass warns that it does not know the packed-fp32 feature.
@@ -82,7 +102,7 @@ def build(force: bool = False, verbose: bool = True, trace: bool = False) -> str
                 raise RuntimeError(f"{' '.join(cmd)}\n{r.stdout}\n{r.stderr}")
             if verbose and err.strip():
                 print(err, file=sys.stderr)
-    if force or jobs or not _newer(lib, objects):
+    if force or not _newer(lib, objects):
         cmd, r = run([HIPCC, "--offload-arch=gfx950", "-shared", "-fPIC", "-o", lib, *objects])
         if r.returncode != 0:
             raise RuntimeError(f"{' '.join(cmd)}\n{r.stdout}\n{r.stderr}")
