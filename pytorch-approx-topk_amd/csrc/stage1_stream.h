@@ -1590,6 +1590,10 @@ __global__ __launch_bounds__(kWave * W) __attribute__((amdgpu_waves_per_eu(4))) 
 // ascending, so combining two is a merge network, not J insertions.  The
 // winners' values are the input's bit patterns (`element_of`).
 constexpr int kMergeThreads = 256;
+// Partial queues of a bucket that a thread folds at most: one round trip to memory (they were 32, eight round trips:
+// fp32 [1, 5065506] k=152 j=4, 256 slabs, 30.7 -> 20.7 us per call, arg-max of fp16 [1, 2^23] k=64 15.5 -> 10.6; more
+// workgroups and a step or two more in the tree that follows).
+constexpr int kMergeQueues = 4;
 
 template <typename E, int J>
 __global__ __launch_bounds__(kMergeThreads) void stream_merge_kernel(

@@ -127,9 +127,9 @@ static int launch_j(const Plan& pl, const typename E::raw_t* x, const Sink<typen
     }
   }
   // buckets per workgroup: a power of two, no more than there are, and few
-  // enough that a thread folds at most about 32 of a bucket's partial queues
+  // enough that a thread folds at most kMergeQueues of a bucket's partial queues
   uint32_t cb = kWave;
-  while (cb > 1 && ((int64_t)(cb / 2) >= b || (int64_t)pl.slabs * cb > 32 * kMergeThreads)) cb /= 2;
+  while (cb > 1 && ((int64_t)(cb / 2) >= b || (int64_t)pl.slabs * cb > kMergeQueues * kMergeThreads)) cb /= 2;
   const int64_t blocks_per_row = (b + cb - 1) / cb;
   if (blocks_per_row * rows > 0x7fffffffll) return ATK_ERR_TOO_LARGE;
   hipLaunchKernelGGL((stream_merge_kernel<E, J>), dim3((unsigned)(blocks_per_row * rows)),

@@ -12,6 +12,9 @@ inline size_t align_up(size_t v, size_t a) { return (v + a - 1) / a * a; }
 // Waves wanted in the grid before a row is cut into slabs: one per SIMD of the
 // 256 CUs x 4 SIMDs (each keeps 8 KiB of loads in flight).
 constexpr int64_t kTargetWaves = 1024;
+constexpr int64_t kCus = 256;
+// Fewest bytes a wave reads, and most bytes of partial queues, of slabs that are cut to have a workgroup on every CU.
+constexpr int64_t kWaveBytes = 8 << 10, kRaisedBytes = 2 << 20;
 // Sub-rows worth giving to one wave before a row is also cut into slabs.
 constexpr int64_t kSlabRun = 16;
 // Fewest workgroups of a launch whose results take the trip through LDS.
@@ -135,6 +138,26 @@ Plan plan_with(int64_t rows, int64_t n, int64_t k0, int j, int layout, int dtype
     if (slabs > longest) slabs = longest;
     if (slabs > (int64_t)pl.slabs) pl.slabs = (uint32_t)slabs;
   }
+  // A launch of a few workgroups more than CUs gives those few CUs twice the work, with the others waiting: down to no
+  // more workgroups than CUs (264 -> 242 workgroups bf16 [22, 546918] k=60 j=4 18.0 -> 14.2 us, 294 -> 252 fp32 [42, 632917]
+  // k=484 j=2 30.1 -> 24.6, 266 -> 252 fp16 [14, 4194304] k=16 j=2 k_mult=4 37.4 -> 29.1; of 24 such shapes 20 are up to a fifth
+  // faster, none with 240 workgroups and more left is slower by over 3 %; with one slab left, and no merge, some lose a third).
+  const int64_t per_slab = rows * pl.col_tiles;  // workgroups
+  if (pl.slabs > 1 && pl.slabs * per_slab > kCus && kCus / per_slab > 1) pl.slabs = (uint32_t)(kCus / per_slab);
+  // CUs left idle while every wave has a long way to go: up to a workgroup each, with what a wave reads at kWaveBytes or
+  // more, and the second stage left in the merge where it is (132 -> 252 workgroups fp16 [7, 2^22] k=32 j=4 k_mult=2 28.8 ->
+  // 24.0 us, 144 -> 252 bf16 [9, 2^22] k=512 j=4 32.9 -> 24.7, fp32 [2, 2^23] k=1024 j=4 k_mult=4 128 -> 256 37.2 -> 29.3; with 2-4 KB
+  // a wave, f16 [3, 346950] k=324 j=2, 7.7 -> 8.3).  Small partial queues only: the workspace stays within what the call
+  // that cannot allocate has taken.
+  if (pl.slabs > 1 && pl.slabs * per_slab < kCus && rows * k0 * (es + 8) <= kRaisedBytes) {
+    int64_t slabs = kCus / per_slab;
+    const int64_t by_wave = full * kWave * pl.vec * es / (w * kWaveBytes), by_queues = kRaisedBytes / (rows * k0 * (es + 4));
+    if (slabs > by_wave) slabs = by_wave;
+    if (slabs > by_queues) slabs = by_queues;
+    if (k0 <= kMergeSelectMax && k0 * (int64_t)pl.slabs <= kMergeSelectEntries && slabs > kMergeSelectEntries / k0)
+      slabs = kMergeSelectEntries / k0;
+    if (slabs > (int64_t)pl.slabs) pl.slabs = (uint32_t)slabs;
+  }
   pl.slab_len = (uint32_t)(full / pl.slabs);
   // every wave scans exactly 4 or 8 sub-rows: straight-line kernels exist for that
   pl.run = 0;
@@ -229,7 +252,7 @@ double estimate(const Plan& pl, int64_t rows, int64_t n, int64_t k0, int j, int 
     us += kMergeSelect + kMergeSelectEntry * (double)pl.slabs * (double)k0;
   } else if (pl.merge) {
     uint32_t at_once = kWave;  // buckets (as the launch chooses them)
-    while (at_once > 1 && (at_once / 2 >= b || (int64_t)pl.slabs * at_once > 32 * kMergeThreads)) at_once /= 2;
+    while (at_once > 1 && (at_once / 2 >= b || (int64_t)pl.slabs * at_once > kMergeQueues * kMergeThreads)) at_once /= 2;
     us += kMerge + kMergeStep * j * std::ceil((double)pl.slabs * at_once / kMergeThreads);
   }
   if (second_stage && !selects) us += kSelect + kSelectEntry * (double)k0 * (rows > 256 ? rows / 256.0 : 1.0);
