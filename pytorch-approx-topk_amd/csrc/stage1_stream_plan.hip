@@ -143,6 +143,7 @@ Plan plan_with(int64_t rows, int64_t n, int64_t k0, int j, int layout, int dtype
   // k=484 j=2 30.1 -> 24.6, 266 -> 252 fp16 [14, 4194304] k=16 j=2 k_mult=4 37.4 -> 29.1; of 24 such shapes 20 are up to a fifth
   // faster, none with 240 workgroups and more left is slower by over 3 %; with one slab left, and no merge, some lose a third).
   const int64_t per_slab = rows * pl.col_tiles;  // workgroups
+  const uint32_t slabs_asked = pl.slabs;
   if (pl.slabs > 1 && pl.slabs * per_slab > kCus && kCus / per_slab > 1) pl.slabs = (uint32_t)(kCus / per_slab);
   // CUs left idle while every wave has a long way to go: up to a workgroup each, with what a wave reads at kWaveBytes or
   // more, and the second stage left in the merge where it is (132 -> 252 workgroups fp16 [7, 2^22] k=32 j=4 k_mult=2 28.8 ->
@@ -169,7 +170,8 @@ Plan plan_with(int64_t rows, int64_t n, int64_t k0, int j, int layout, int dtype
   // its slab itself) go to the workspace and the merge kernel follows
   pl.merge = pl.slabs > 1;
   if (pl.merge) {
-    const size_t entries = (size_t)rows * pl.slabs * (size_t)b * (size_t)j;
+    // (sized for the slabs as first asked for where they are more: the figure callers size their buffers by stays)
+    const size_t entries = (size_t)rows * (pl.slabs > slabs_asked ? pl.slabs : slabs_asked) * (size_t)b * (size_t)j;
     pl.part_values_off = 0;
     pl.part_pos_off = align_up(entries * es, 256);
     pl.ws_bytes = pl.part_pos_off + align_up(entries * sizeof(uint32_t), 256);
@@ -333,6 +335,7 @@ int launch_stage1_stream(const void* x, int64_t rows, int64_t n, int64_t row_str
   if (!pl.ok) return ATK_OK;
   if (pl.ws_bytes && (!ws || ws_bytes < pl.ws_bytes || (uintptr_t)ws % 16 != 0)) return ATK_ERR_WORKSPACE;
   if (last != nullptr) last->wanted = stream::selects_in_merge(pl, k0, last->index_bound, dtype);
+  if (last != nullptr && last->wanted) ranges = nullptr;  // (no chained select follows)
   int rc = ATK_ERR_DTYPE;
   ATK_DTYPE_SWITCH(dtype, E, rc = ATK_ERR_DTYPE,
                    rc = stream::launch_typed<E>(pl, x, rows, row_stride, j, values, indices, ws,

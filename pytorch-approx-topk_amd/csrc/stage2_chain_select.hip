@@ -875,6 +875,11 @@ __global__ __launch_bounds__(kSoloThreads) void chain_solo_kernel(
 // workgroups, 8 rows 18.4 us in 256).
 // (With 64 keys per thread the kernel spills: rows of 40000-65536 candidates took
 // 28-30 us against 18 us for the chain of launches.)
+// The shortest rows: select alone behind fp32 and fp16 [rows, 2^19] j=2 k_mult=2, us per call against one workgroup per
+// row: 1 row of 4096 / 6144 / 8192 candidates 15.4 / 16.8 / 15.8 -> 12.6 / 10.8 / 10.1, 4 of 8192 16.9 -> 11.4, 16 of 2048 14.7 ->
+// 13.2, of 1536 15.5 -> 14.4, 20 of 8192 23.7 -> 18.4, 32 of 8192 29.0 -> 24.2, 64 of 4096 38.8 -> 36.5; of 1024 candidates 64 rows
+// 36.1 -> 34.6, fewer not measured (their slabs' merge takes the select along).
+constexpr int64_t kSoloMinCandidates = 1536;
 constexpr int64_t kSoloMaxCandidates = 32 * kSoloThreads;
 constexpr int64_t kSoloMaxWorkgroups = 256;
 
@@ -889,7 +894,7 @@ constexpr int64_t kSoloMaxWorkgroups = 256;
 // 64 rows of 131072: 99 / 110 against 107 / 118, 96 rows 141 / 162 against 142 / 173.
 // Segments of 4096 candidates from 1024 workgroups of the short ones on: 32 rows of
 // 131072 took 120 / 127 us with segments of 1024, 33 rows 65 / 71 us with 4096.
-constexpr int64_t kChainMinCandidates = 10240;  // (8192: 11.8 us against 10.5 for one workgroup)
+constexpr int64_t kChainMinCandidates = 10240;  // (in several launches)
 constexpr int64_t kChainMaxCandidates = 1 << 17;
 constexpr int64_t kChainMaxRows = 16;
 constexpr int64_t kChainMaxRowsLong = 64;  // rows of more than kSoloMaxCandidates candidates
@@ -900,14 +905,20 @@ ChainPlan plan_chain(int64_t rows, int64_t k0, int64_t k, int64_t index_bound, i
   pl.use = false;
   const int es = elem_bytes(dtype);
   if (es == 0 || es > 4 || rows <= 0 || k <= 0 || k >= k0) return pl;
-  if (k0 < kChainMinCandidates || k0 > kChainMaxCandidates || index_bound > 0x7fffffffll) return pl;
-  if (rows > (k0 > kSoloMaxCandidates ? kChainMaxRowsLong : kChainMaxRows)) return pl;
+  if (k0 > kChainMaxCandidates || index_bound > 0x7fffffffll) return pl;
   pl.groups = (uint32_t)((k0 + kSoloSegment - 1) / kSoloSegment);
+  pl.solo = k0 >= kSoloMinCandidates && k0 <= kSoloMaxCandidates && rows * (int64_t)pl.groups <= kSoloMaxWorkgroups;
+  if (!pl.solo && (k0 < kChainMinCandidates || rows > (k0 > kSoloMaxCandidates ? kChainMaxRowsLong : kChainMaxRows))) return pl;
   pl.per_thread = rows * (int64_t)pl.groups > kChainShortSegmentGroups ? kPerThreadMany : kPerThreadFew;
-  pl.solo = k0 <= kSoloMaxCandidates && rows * (int64_t)pl.groups <= kSoloMaxWorkgroups;
   if (!pl.solo) {
     const int64_t segment = (int64_t)kThreads * pl.per_thread;
     pl.groups = (uint32_t)((k0 + segment - 1) / segment);
+  }
+  if (pl.solo && (k0 < kChainMinCandidates || rows > kChainMaxRows)) {
+    // short rows, and more of them: the kernel works the key range out itself, and no workspace is asked for
+    // where one workgroup per row needed none
+    pl.use = true;
+    return pl;
   }
   pl.range_off = 0;
   pl.range_capacity = pl.groups > kRangeCapacity ? pl.groups : kRangeCapacity;
@@ -1033,7 +1044,7 @@ KeyRangeOut chain_select_ranges(int64_t rows, int64_t k0, int64_t k, int64_t ind
                                 size_t ws_bytes) {
   KeyRangeOut out{};
   const ChainPlan pl = plan_chain(rows, k0, k, index_bound, dtype);
-  if (!pl.use || !ws || ws_bytes < pl.total || (uintptr_t)ws % 16 != 0) return out;
+  if (!pl.use || pl.total == 0 || !ws || ws_bytes < pl.total || (uintptr_t)ws % 16 != 0) return out;
   unsigned char* base = static_cast<unsigned char*>(ws);
   out.range = reinterpret_cast<uint2*>(base + pl.range_off);
   out.capacity = pl.range_capacity;
@@ -1051,7 +1062,7 @@ int launch_chain_select(const void* cand_values, const int64_t* cand_indices, in
   const ChainPlan pl = plan_chain(rows, k0, k, index_bound, dtype);
   *handled = pl.use;
   if (!pl.use) return ATK_OK;
-  if (!ws || ws_bytes < pl.total || (uintptr_t)ws % 16 != 0) return ATK_ERR_WORKSPACE;
+  if (pl.total != 0 && (!ws || ws_bytes < pl.total || (uintptr_t)ws % 16 != 0)) return ATK_ERR_WORKSPACE;
   int index_bits = 1;
   while (index_bits < 63 && (1ll << index_bits) < index_bound) ++index_bits;
   int rc = ATK_ERR_DTYPE;

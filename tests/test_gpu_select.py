@@ -248,3 +248,11 @@ def test_one_launch_select_of_lists_of_every_length(k0, m):
     for k in {above + 1, above + (m + 1) // 2, above + m - 1, above + m}:
         v, i = _select(cv, ci, k, 1 << 21)
         assert_same(v, i, *oracle.stage2(cv, ci, k), f"k0={k0} m={m} k={k}")
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.int32, torch.uint8])
+@pytest.mark.parametrize("rows,k0,k", [(1, 1536, 700), (3, 1537, 1), (128, 2048, 1024), (127, 2047, 2046), (85, 2049, 1500),
+                                       (64, 4096, 64), (32, 8192, 4000), (25, 10240, 300)])
+def test_one_launch_select_of_short_rows(dtype, rows, k0, k):
+    kinds = ["ties", "equal", "steps"] if dtype == torch.uint8 else ["spread", "ties", "equal", "steps", "crowded"]
+    _chain_case([kinds[r % len(kinds)] for r in range(rows)], k0, k, dtype, seed=k0 + k + rows)
