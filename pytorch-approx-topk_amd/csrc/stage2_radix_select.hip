@@ -91,6 +91,72 @@ __global__ __launch_bounds__(COPIES == 8 ? 1024 : 256) void select_kernel(
       });
 }
 
+// Rows of up to kRankMax candidates, a candidate per thread: its word of key and inverted
+// index goes to LDS, every thread counts the better words of its row, and the k best leave in
+// candidate order.  WAVES waves to a row, 4 / WAVES rows to a workgroup.
+//
+// Bound: latency.  The radix select takes up to four passes of three barriers, whatever the candidates.
+// Calls of contiguous buckets, us with that and with this: fp32 [1, 32768] k=8 k_mult=2 9.4 and 5.8, fp16 [16, 32768] k=32
+// k_mult=2 8.7 and 6.5, [256, 32768] k=64 k_mult=2 12.0 and 10.6, [2000, 32768] 38.6 and 34.9, fp32 [16, 32768] k=100 k_mult=2 8.4 and
+// 7.7.  Every candidate is compared with every other: many rows with longer ones lose ([16384, 8192] of 100 candidates
+// 120 and 114, of 128 73 and 74, of 200 134 and 156).
+constexpr uint32_t kRankMax = 256;
+constexpr int64_t kRankWork = 1 << 27;  // comparisons
+
+template <typename E, int WAVES>
+__global__ __launch_bounds__(256) void rank_select_kernel(const typename E::raw_t* __restrict__ cand_values,
+                                                          const int64_t* __restrict__ cand_indices, uint32_t rows,
+                                                          uint32_t k0, uint32_t k,
+                                                          typename E::raw_t* __restrict__ values,
+                                                          const IndexOut indices) {
+  using raw_t = typename E::raw_t;
+  constexpr uint32_t kThreads = WAVES * select::kWave, kRows = 256 / kThreads;
+  __shared__ __align__(16) uint64_t words[256];
+  __shared__ uint32_t kept_of[4];
+  const uint32_t t = threadIdx.x % kThreads, lane = threadIdx.x % select::kWave;
+  const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x / select::kWave), first = wave / WAVES * WAVES;
+  const uint32_t row = blockIdx.x * kRows + wave / WAVES;
+  const bool real = row < rows && t < k0;
+  raw_t raw{};
+  uint32_t index = 0;
+  uint64_t mine = 0;
+  if (real) {
+    const int64_t at = (int64_t)row * k0 + t;
+    raw = cand_values[at];
+    index = (uint32_t)cand_indices[at];
+    mine = ((uint64_t)E::key(raw) << 32) | (uint32_t)~index;
+  }
+  words[threadIdx.x] = mine;  // (0 past the row's end: above no candidate)
+  __syncthreads();
+  const uint64_t* of_row = words + first * select::kWave;
+  uint32_t better = 0;
+#pragma unroll 4
+  for (uint32_t i = 0; i < k0; i += 2) {
+    const ulonglong2 two = *reinterpret_cast<const ulonglong2*>(&of_row[i]);
+    better += (two.x > mine ? 1u : 0u) + (two.y > mine ? 1u : 0u);
+  }
+  const uint64_t mask = __ballot(real && better < k);
+  uint32_t o = select::rank_in(mask);
+  if constexpr (WAVES > 1) {
+    if (lane == 0) kept_of[wave] = (uint32_t)__popcll(mask);
+    __syncthreads();
+    for (uint32_t w = first; w < wave; ++w) o += kept_of[w];
+  }
+  if (real && better < k && o < k) {
+    const int64_t to = (int64_t)row * k + o;
+    if (values != nullptr) values[to] = raw;
+    indices.put(to, (int64_t)index);
+  }
+}
+
+// Whether the kernel above takes a call: words of 32-bit keys and indices, and a launch that can count its threads.
+// (Rows of 65 to 128 candidates take two waves, of more four; 64 candidates and fewer win whatever the rows.)
+bool ranks(int64_t rows, int64_t k0, int64_t index_bound, int dtype) {
+  if (k0 > kRankMax || elem_bytes(dtype) > 4 || index_bound > 0xffffffffll || rows > 0xffffff) return false;
+  const int64_t threads = k0 <= 64 ? 64 : k0 <= 128 ? 128 : 256;
+  return threads == 64 || rows * threads * threads <= kRankWork;
+}
+
 // LDS a workgroup may use for keys; the rest of the 160 KB of a gfx950 CU is
 // left to the static block above and to a second resident workgroup's needs.
 constexpr size_t kMaxKeyLds = 128 * 1024;
@@ -119,6 +185,22 @@ SplitPlan plan_split(int64_t rows, int64_t k0, int64_t k) {
   sp.counts_off = ((size_t)rows * sizeof(select::GlobalCut) + 255) / 256 * 256;
   sp.total = sp.counts_off + ((size_t)rows * kSegments * sizeof(uint32_t) + 255) / 256 * 256;
   return sp;
+}
+
+template <typename E>
+int launch_rank(const void* cand_values, const int64_t* cand_indices, int64_t rows, int64_t k0, int64_t k, void* values,
+                IndexOut indices, hipStream_t stream) {
+  if constexpr (sizeof(typename E::key_t) == 4) {
+    const int per_row = k0 <= 64 ? 1 : k0 <= 128 ? 2 : 4;
+    auto kern = per_row == 1 ? rank_select_kernel<E, 1> : per_row == 2 ? rank_select_kernel<E, 2> : rank_select_kernel<E, 4>;
+    const int64_t per_group = 4 / per_row;
+    hipLaunchKernelGGL(kern, dim3((unsigned)((rows + per_group - 1) / per_group)), dim3(256), 0, stream,
+                       (const typename E::raw_t*)cand_values, cand_indices, (uint32_t)rows, (uint32_t)k0, (uint32_t)k,
+                       (typename E::raw_t*)values, indices);
+    return hipGetLastError() == hipSuccess ? ATK_OK : ATK_ERR_LAUNCH;
+  } else {
+    return ATK_ERR_ARG;  // (never asked for: see ranks)
+  }
 }
 
 template <typename E>
@@ -179,7 +261,12 @@ size_t select_workspace_bytes(int64_t rows, int64_t k0, int64_t k, int dtype) {
 
 void describe_select(int64_t rows, int64_t k0, int64_t k, int64_t index_bound, int dtype, bool with_workspace,
                      std::string& out) {
-  (void)index_bound;
+  if (ranks(rows, k0, index_bound, dtype)) {
+    const int per_row = k0 <= 64 ? 1 : k0 <= 128 ? 2 : 4, per_group = 4 / per_row;
+    out += "rank_select_kernel<" + std::string(dtype_name(dtype)) + ", WAVES=" + std::to_string(per_row) + "> grid=" +
+           std::to_string((rows + per_group - 1) / per_group) + " block=256";
+    return;
+  }
   const int kb = elem_bytes(dtype) == 8 ? 8 : 4;  // bytes of an order key
   const bool in_lds = (size_t)k0 * kb <= kMaxKeyLds;
   int nt = 1024;
@@ -200,6 +287,12 @@ int launch_select(const void* cand_values, const int64_t* cand_indices, int64_t 
                   int64_t k0, int64_t k, int64_t index_bound, int dtype, void* values,
                   IndexOut indices, void* ws, size_t ws_bytes, hipStream_t stream) {
   if (k0 > 0x7fffffffll || rows > 0x7fffffffll) return ATK_ERR_TOO_LARGE;
+  if (ranks(rows, k0, index_bound, dtype)) {
+    int rc = ATK_ERR_DTYPE;
+    ATK_DTYPE_SWITCH(dtype, E, rc = ATK_ERR_DTYPE,
+                     rc = launch_rank<E>(cand_values, cand_indices, rows, k0, k, values, indices, stream));
+    return rc;
+  }
   int index_bits = 1;
   while (index_bits < 63 && (1ll << index_bits) < index_bound) ++index_bits;
   // without a workspace the one workgroup also writes the survivors

@@ -256,3 +256,21 @@ def test_one_launch_select_of_lists_of_every_length(k0, m):
 def test_one_launch_select_of_short_rows(dtype, rows, k0, k):
     kinds = ["ties", "equal", "steps"] if dtype == torch.uint8 else ["spread", "ties", "equal", "steps", "crowded"]
     _chain_case([kinds[r % len(kinds)] for r in range(rows)], k0, k, dtype, seed=k0 + k + rows)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.int32, torch.int8, torch.float64])
+@pytest.mark.parametrize("rows,k0,k", [(1, 2, 1), (5, 63, 1), (6, 64, 63), (7, 65, 30), (3, 127, 126), (8, 128, 64), (9, 129, 128),
+                                       (4, 255, 17), (5, 256, 255), (1001, 100, 50), (8193, 70, 9)])
+def test_select_of_rows_ranked_by_comparison(dtype, rows, k0, k):
+    # a wave, two and four to a row; rows that do not fill the last workgroup; ties, NaNs and zeros of both signs
+    g = torch.Generator().manual_seed(rows + k0)
+    cv = torch.randint(-9, 10, (rows, k0), generator=g)
+    if dtype.is_floating_point:
+        cv = cv / 4
+        cv[:, ::5] = -0.0
+        cv[0, 1::7] = float("nan")
+        cv[-1, :] = float("-inf")
+    cv = cv.to(dtype)
+    ci = torch.stack([torch.randperm(1 << 10, generator=g)[:k0] for _ in range(rows)])
+    v, i = _select(cv, ci, k, 1 << 10)
+    assert_same(v, i, *oracle.stage2(cv, ci, k), f"{dtype} {rows} {k0} {k}")
