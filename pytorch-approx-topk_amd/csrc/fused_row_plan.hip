@@ -263,10 +263,10 @@ constexpr double kOneKernelShare = 0.85;
 // selection, by the candidates of a lane and the waves that wait for one another.
 // The constants are a least-squares fit to 1415 launches of 620 calls (fp32 and fp16, 1-8192 rows of 2048-2^18 elements,
 // half of them of no round length, 32-8192 candidates, j 1, 2, 4, k_mult 2-8, up to 160 MiB; every width of load): off by
-// 10 % in the root mean square.  Among those calls, the choice by these estimates is 1.4 % slower than the best of two kernels
+// 10 % in the root mean square.  Among those calls, the choice by these estimates is 2.2 % slower than the best of two kernels
 // and one with each width; the rules of size with the usual width, which stood before, are 16 %.  (float32 [859, 2048]
-// k=64 j=4 k_mult=2 29.0 us by the rules, 10.4 with one column a lane; [1053, 19352] k=152 j=1 k_mult=2 35.5 in two kernels, 21.1
-// in one; fp16 [2048, 8192] k=100 j=2 k_mult=4 37.1 in two kernels, 18 in one.)
+// k=64 j=4 k_mult=2 29.1 us by the rules, 10.1 with one column a lane; [1053, 19352] k=152 j=1 k_mult=2 35.5 in two kernels, 21.4
+// in one; fp16 [2048, 8192] k=100 j=2 k_mult=4 37.5 in two kernels, 17.3 in one.)
 double estimate(const Plan& pl, int64_t rows, int64_t n, int j, int es) {
   constexpr double kBytes = 5.2e6;                                      // per us
   constexpr double kLaunch = 1.45, kTrip = 0.14, kShare = 0.51;         // us; kShare: a SIMD's wave beside others

@@ -140,8 +140,9 @@ Plan plan_with(int64_t rows, int64_t n, int64_t k0, int j, int layout, int dtype
   }
   // A launch of a few workgroups more than CUs gives those few CUs twice the work, with the others waiting: down to no
   // more workgroups than CUs (264 -> 242 workgroups bf16 [22, 546918] k=60 j=4 18.0 -> 14.2 us, 294 -> 252 fp32 [42, 632917]
-  // k=484 j=2 30.1 -> 24.6, 266 -> 252 fp16 [14, 4194304] k=16 j=2 k_mult=4 37.4 -> 29.1; of 24 such shapes 20 are up to a fifth
-  // faster, none with 240 workgroups and more left is slower by over 3 %; with one slab left, and no merge, some lose a third).
+  // k=484 j=2 30.1 -> 24.6, 266 -> 252 fp16 [14, 4194304] k=16 j=2 k_mult=4 37.4 -> 29.1; of 45 drawn shapes 38
+  // are 4 to 27 % faster, five within 3 %, and two slower: fp32 [1, 4331110] k=640 k_mult=2, 260 -> 240, by 6 %, int32 [3, 2^23]
+  // k=64 j=2, 258 -> 255, by 10 %.  Others cut from 258 to 255 gain; with one slab left, and no merge, some lose a third).
   const int64_t per_slab = rows * pl.col_tiles;  // workgroups
   const uint32_t slabs_asked = pl.slabs;
   if (pl.slabs > 1 && pl.slabs * per_slab > kCus && kCus / per_slab > 1) pl.slabs = (uint32_t)(kCus / per_slab);

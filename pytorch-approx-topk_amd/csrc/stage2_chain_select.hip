@@ -620,7 +620,7 @@ __global__ __launch_bounds__(kSoloThreads) void chain_solo_kernel(
           "v_addc_co_u32_e64 %0, %2, %0, %0, %2\n\t"
           "v_addc_co_u32_e32 %1, vcc, %1, %1, vcc"
           : "+v"(better), "+v"(members), "=&s"(mask)
-          : "v"(key[u]), "s"(above), "v"(key[u] - first), "s"(width1)
+          : "v"(key[u]), "v"(above), "v"(key[u] - first), "v"(width1)
           : "vcc");
     }
     uint32_t exist = ~0u;
