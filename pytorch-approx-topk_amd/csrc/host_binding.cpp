@@ -188,7 +188,7 @@ struct TopkWithGradient : torch::autograd::Function<TopkWithGradient> {
     ctx->saved_data["call"] = std::move(call);
     ctx->set_materialize_grads(false);
     ctx->save_for_backward({indices});
-    ctx->mark_non_differentiable({indices});
+    // (not marked as non-differentiable: integers are not anyway, and compiled autograd takes no node with marks)
     return {values, indices};
   }
 

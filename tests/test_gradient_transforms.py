@@ -176,3 +176,26 @@ def test_a_missing_gradient_of_the_values_counts_as_zeros():
         x = torch.randn(2, 64).to(dtype).requires_grad_()
         _Drops.apply(topk(x, 8, -1)[0]).backward()
         assert x.grad.dtype == dtype and x.grad.shape == x.shape and not x.grad.any()
+
+
+def _nodes():
+    """The wrapper's node in Python and the native one, which it takes for plain GPU tensors."""
+    from approx_topk import _native
+    from approx_topk.experimental import differentiable
+    yield differentiable._TopkWithGradient.apply
+    yield _native.host.differentiable_topk
+
+
+@pytest.mark.parametrize("wrapped", [False, True])
+def test_backward_under_compiled_autograd(wrapped):
+    # the forward runs eagerly, the backward through a graph that compiled autograd builds of its nodes
+    from torch._dynamo import compiled_autograd
+    for node in _nodes():
+        x = torch.randn(3, 64, generator=torch.Generator().manual_seed(2)).requires_grad_()
+        values, indices = node(x * 2 if wrapped else x, 8, -1, 2, 2, True, False)
+        assert values.requires_grad and not indices.requires_grad and indices.grad_fn is None
+        w = torch.randn(values.shape, generator=torch.Generator().manual_seed(4))
+        with compiled_autograd._enable(lambda graph: torch.compile(graph, backend="eager")):
+            (values * w).sum().backward()
+        want = torch.zeros(3, 64).scatter(-1, indices, w) * (2 if wrapped else 1)
+        assert torch.equal(x.grad, want)
