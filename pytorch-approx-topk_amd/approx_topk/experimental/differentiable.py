@@ -17,7 +17,7 @@ from __future__ import annotations
 
 import torch
 from torch import Tensor, is_grad_enabled
-from torch._C import _AutoDispatchBelowAutograd
+from torch._C import _AutoDispatchBelowAutograd, _is_torch_function_mode_enabled
 from torch._C._functorch import peek_interpreter_stack
 from torch.autograd import forward_ad
 from torch.compiler import is_compiling
@@ -36,6 +36,26 @@ def _autograd_has_work(grad_values: Tensor) -> bool:
             or peek_interpreter_stack() is not None or is_compiling())
 
 
+def _gradient(grad_values: Tensor | None, indices: Tensor, shape: torch.Size, dtype: torch.dtype, dim: int, k0: int,
+              j: int, interleaved: bool) -> Tensor:
+    """The gradient with respect to an input of `shape` and `dtype`, given that of the values."""
+    if grad_values is None:  # (not materialized: that would fill an int64 gradient of the indices as well)
+        return indices.new_zeros(shape, dtype=dtype)
+    if len(shape) and dim == len(shape) - 1 and indices.numel() and shape[-1] <= _native.MAX_GRAD_ROW:
+        if _autograd_has_work(grad_values):
+            return _topk_grad(grad_values, indices, shape[-1], k0, j, interleaved)
+        # the operator's autograd kernel would find nothing to do, in 6 us of host time
+        with _AutoDispatchBelowAutograd():
+            return _topk_grad(grad_values, indices, shape[-1], k0, j, interleaved)
+    if len(shape) == 0:
+        return grad_values.reshape(()) if indices.numel() else grad_values.new_zeros(())
+    return grad_values.new_zeros(shape).scatter(dim, indices, grad_values)
+
+
+if _native.host is not None:
+    _native.host.set_gradient(_gradient)
+
+
 class _TopkWithGradient(torch.autograd.Function):
     @staticmethod
     def forward(ctx, xs, k, dim, j, k_mult, interleaved, multithread_buckets):
@@ -51,19 +71,7 @@ class _TopkWithGradient(torch.autograd.Function):
     @staticmethod
     def backward(ctx, grad_values, _grad_indices):
         (indices,) = ctx.saved_tensors
-        shape = ctx.shape
-        if grad_values is None:  # (not materialized: that would fill an int64 gradient of the indices as well)
-            return indices.new_zeros(shape, dtype=ctx.dtype), None, None, None, None, None, None
-        if len(shape) and ctx.dim == len(shape) - 1 and indices.numel() and shape[-1] <= _native.MAX_GRAD_ROW:
-            if _autograd_has_work(grad_values):
-                grad_xs = _topk_grad(grad_values, indices, shape[-1], *ctx.buckets)
-            else:  # the operator's autograd kernel would find nothing to do, in 6 us of host time
-                with _AutoDispatchBelowAutograd():
-                    grad_xs = _topk_grad(grad_values, indices, shape[-1], *ctx.buckets)
-        elif len(shape) == 0:
-            grad_xs = grad_values.reshape(()) if indices.numel() else grad_values.new_zeros(())
-        else:
-            grad_xs = grad_values.new_zeros(shape).scatter(ctx.dim, indices, grad_values)
+        grad_xs = _gradient(grad_values, indices, ctx.shape, ctx.dtype, ctx.dim, *ctx.buckets)
         return grad_xs, None, None, None, None, None, None
 
 
@@ -77,9 +85,10 @@ def topk(
     multithread_buckets: bool | None = False,
 ) -> tuple[Tensor, Tensor]:
     """``approx_topk.topk`` whose values carry a gradient with respect to ``xs``."""
-    # Plain GPU tensors outside of every transform: the same node in native code (csrc/host_binding.cpp), whose
-    # backward leaves what is differentiated again to the operator's autograd kernel as the one above does.
+    # Plain GPU tensors outside of every transform and mode that would see the operator's call: the same node in
+    # native code (csrc/host_binding.cpp), whose backward leaves all but a plain gradient to `_gradient`.
     if (not is_compiling() and _native.host is not None and type(xs) in _PLAIN and xs.is_cuda
-            and peek_interpreter_stack() is None and forward_ad._current_level < 0):
+            and peek_interpreter_stack() is None and forward_ad._current_level < 0
+            and not _is_torch_function_mode_enabled()):
         return _native.host.differentiable_topk(xs, k, dim, j, k_mult, interleaved, multithread_buckets)
     return _TopkWithGradient.apply(xs, k, dim, j, k_mult, interleaved, multithread_buckets)

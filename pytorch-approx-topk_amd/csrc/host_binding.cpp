@@ -18,6 +18,9 @@
 
 #include <ATen/hip/impl/HIPGuardImplMasqueradingAsCUDA.h>
 #include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
+#include <ATen/PythonTorchFunctionTLS.h>
+#include <torch/csrc/Dtype.h>
+#include <torch/csrc/DynamicTypes.h>
 
 #include "../../include/approx_topk_hip.h"
 
@@ -39,6 +42,7 @@ decltype(&atk_topk_grad) g_topk_grad;
 // the Python functions that take what the fast paths do not (held until the process ends)
 PyObject* g_topk_any = nullptr;
 PyObject* g_topk_grad_any = nullptr;
+PyObject* g_gradient_any = nullptr;
 
 void check(int status) {
   if (status != ATK_OK) throw std::runtime_error(g_strerror(status));
@@ -201,19 +205,20 @@ struct TopkWithGradient : torch::autograd::Function<TopkWithGradient> {
     const at::IntArrayRef shape = at::IntArrayRef(call).slice(5);
     const Tensor& grad = grads[0];
     Tensor grad_xs;
-    if (!grad.defined()) {
-      grad_xs = at::zeros(shape, indices.options().dtype((at::ScalarType)call[4]));
-    } else if (!shape.empty() && dim == (int64_t)shape.size() - 1 && indices.numel() && shape.back() <= kMaxGradRow) {
-      if ((at::GradMode::is_enabled() && grad.requires_grad()) || !plain(grad) || grad._fw_grad(0).defined()) {
-        grad_xs = call_topk_grad(grad, indices, shape.back(), k0, j, interleaved);
-      } else {  // (the operator's autograd kernel would find nothing to do)
-        at::AutoDispatchBelowAutograd guard;
-        grad_xs = call_topk_grad(grad, indices, shape.back(), k0, j, interleaved);
-      }
-    } else if (shape.empty()) {
-      grad_xs = indices.numel() ? grad.reshape({}) : at::zeros({}, grad.options());
+    // a plain gradient whose own derivative nobody asks for: the operator's autograd kernel would find nothing to do
+    if (grad.defined() && !shape.empty() && dim == (int64_t)shape.size() - 1 && indices.numel() && shape.back() <= kMaxGradRow &&
+        plain(grad) && !(at::GradMode::is_enabled() && grad.requires_grad()) && !grad._fw_grad(0).defined() &&
+        !at::impl::torch_function_mode_enabled()) {
+      at::AutoDispatchBelowAutograd guard;
+      grad_xs = call_topk_grad(grad, indices, shape.back(), k0, j, interleaved);
     } else {
-      grad_xs = at::zeros(shape, grad.options()).scatter(dim, indices, grad);
+      py::gil_scoped_acquire gil;
+      py::tuple sizes(shape.size());
+      for (size_t d = 0; d < shape.size(); ++d) sizes[d] = shape[d];
+      const py::object dtype = py::reinterpret_borrow<py::object>((PyObject*)torch::getTHPDtype((at::ScalarType)call[4]));
+      grad_xs = py::reinterpret_borrow<py::object>(g_gradient_any)(grad.defined() ? py::cast(grad) : py::object(py::none()),
+                                                                   indices, sizes, dtype, dim, k0, j, interleaved)
+                    .cast<Tensor>();
     }
     return {grad_xs, Tensor(), Tensor(), Tensor(), Tensor(), Tensor(), Tensor()};
   }
@@ -230,6 +235,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     g_topk_any = topk_any.release().ptr();
     g_topk_grad_any = topk_grad_any.release().ptr();
   });
+  m.def("set_gradient", [](py::object gradient_any) { g_gradient_any = gradient_any.release().ptr(); });
   m.def("bind", [](const py::dict& addresses) {
     take(g_strerror, addresses, "atk_strerror");
     take(g_stage1_workspace, addresses, "atk_stage1_workspace_bytes");

@@ -162,6 +162,53 @@ def test_gradient_node_under_transforms():
         assert not topk(x, 16, -1)[0].requires_grad
 
 
+def test_function_modes_see_the_operators():
+    from torch.overrides import TorchFunctionMode
+    from approx_topk.experimental.differentiable import topk
+
+    class Seen(TorchFunctionMode):
+        def __init__(self):
+            super().__init__()
+            self.calls = []
+
+        def __torch_function__(self, func, types, args=(), kwargs=None):
+            self.calls.append(func)
+            return func(*args, **(kwargs or {}))
+
+    x = _pair().requires_grad_()
+    want = topk(x, 16, -1, j=2, k_mult=2)
+    for forward_too in (True, False):
+        mode = Seen()
+        if forward_too:
+            with mode:
+                values, indices = topk(x, 16, -1, j=2, k_mult=2)
+            assert torch.ops.approx_topk.topk.default in mode.calls
+            assert torch.equal(values, want[0]) and torch.equal(indices, want[1])
+        else:
+            values, indices = want
+        mode.calls.clear()
+        with mode:
+            torch.autograd.backward((values,), (torch.ones_like(values),))
+        assert torch.ops.approx_topk.topk_grad.default in mode.calls
+    assert torch.equal(x.grad, 2 * _expect(x, want[1], torch.ones_like(want[0])).detach())
+
+
+@pytest.mark.parametrize("node", ["native", "python"])
+def test_backward_under_compiled_autograd(node):
+    from torch._dynamo import compiled_autograd
+    from approx_topk.experimental import differentiable
+    x = _pair().requires_grad_()
+    if node == "native":
+        values, indices = differentiable.topk(x, 16, -1, j=2, k_mult=2)
+    else:
+        values, indices = differentiable._TopkWithGradient.apply(x, 16, -1, 2, 2, True, False)
+    assert not indices.requires_grad and indices.grad_fn is None
+    grad = _pair(values.shape, 1)
+    with compiled_autograd._enable(lambda graph: torch.compile(graph, backend="eager")):
+        (values * grad).sum().backward()
+    assert torch.equal(x.grad, _expect(x, indices, grad).detach())
+
+
 def test_threads_and_streams():
     from approx_topk import topk
     from approx_topk.experimental import differentiable

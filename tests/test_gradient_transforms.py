@@ -199,3 +199,24 @@ def test_backward_under_compiled_autograd(wrapped):
             (values * w).sum().backward()
         want = torch.zeros(3, 64).scatter(-1, indices, w) * (2 if wrapped else 1)
         assert torch.equal(x.grad, want)
+
+
+def test_function_modes_see_the_gradient_operator():
+    from torch.overrides import TorchFunctionMode
+
+    class Seen(TorchFunctionMode):
+        def __init__(self):
+            super().__init__()
+            self.calls = []
+
+        def __torch_function__(self, func, types, args=(), kwargs=None):
+            self.calls.append(func)
+            return func(*args, **(kwargs or {}))
+
+    for node in _nodes():
+        x = torch.randn(3, 64, generator=torch.Generator().manual_seed(2)).requires_grad_()
+        values, indices = node(x, 8, -1, 2, 2, True, False)
+        with Seen() as mode:
+            torch.autograd.backward((values,), (torch.ones(3, 8),))
+        assert torch.ops.approx_topk.topk_grad.default in mode.calls
+        assert torch.equal(x.grad, torch.zeros(3, 64).scatter(-1, indices, 1.0))
