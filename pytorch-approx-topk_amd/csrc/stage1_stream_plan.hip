@@ -15,6 +15,10 @@ constexpr int64_t kTargetWaves = 1024;
 constexpr int64_t kCus = 256;
 // Fewest bytes a wave reads, and most bytes of partial queues, of slabs that are cut to have a workgroup on every CU.
 constexpr int64_t kWaveBytes = 8 << 10, kRaisedBytes = 2 << 20;
+// Most partial queues of a row whose merge selects, with slabs that are cut to have a workgroup on every CU.
+constexpr int64_t kRaisedSelectQueues = 4096;
+// How much longer a slab may get to have no more workgroups than CUs.
+constexpr double kLongerFourWaves = 1.34, kLongerOneElement = 1.17;
 // Sub-rows worth giving to one wave before a row is also cut into slabs.
 constexpr int64_t kSlabRun = 16;
 // Fewest workgroups of a launch whose results take the trip through LDS.
@@ -45,8 +49,9 @@ constexpr double kLargeShare = 0.95;
 // Buckets from this length on are folded whatever the fold.
 constexpr int64_t kFoldAnyLength = 128;
 
-// The plan with 16-byte loads (`wide`) or with one-element loads.
-Plan plan_with(int64_t rows, int64_t n, int64_t k0, int j, int layout, int dtype, bool wide) {
+// The plan with 16-byte loads (`wide`) or with one-element loads.  `second_stage`: behind the candidates (without
+// one, rows are cut into as many slabs or more: the bound of the workspace).
+Plan plan_with(int64_t rows, int64_t n, int64_t k0, int j, int layout, int dtype, bool wide, bool second_stage) {
   Plan pl{};
   pl.ok = false;
   if (layout != ATK_INTERLEAVED && layout != ATK_INTERLEAVED_PADDED) return pl;
@@ -138,26 +143,45 @@ Plan plan_with(int64_t rows, int64_t n, int64_t k0, int j, int layout, int dtype
     if (slabs > longest) slabs = longest;
     if (slabs > (int64_t)pl.slabs) pl.slabs = (uint32_t)slabs;
   }
-  // A launch of a few workgroups more than CUs gives those few CUs twice the work, with the others waiting: down to no
-  // more workgroups than CUs (264 -> 242 workgroups bf16 [22, 546918] k=60 j=4 18.0 -> 14.2 us, 294 -> 252 fp32 [42, 632917]
-  // k=484 j=2 30.1 -> 24.6, 266 -> 252 fp16 [14, 4194304] k=16 j=2 k_mult=4 37.4 -> 29.1; of 45 drawn shapes 38
-  // are 4 to 27 % faster, five within 3 %, and two slower: fp32 [1, 4331110] k=640 k_mult=2, 260 -> 240, by 6 %, int32 [3, 2^23]
-  // k=64 j=2, 258 -> 255, by 10 %.  Others cut from 258 to 255 gain; with one slab left, and no merge, some lose a third).
+  // A launch of more workgroups than CUs gives some CUs twice the work, with the others waiting: down to no more
+  // workgroups than CUs, in fewer and longer slabs.  How much longer they may get lies with how well a CU's second
+  // workgroup hides behind the first.  519 launches (all types, 1-200 rows, 4-70 M elements), time cut over time as asked:
+  //   eight waves with 16-byte loads, or of eight-byte elements, each a CU's worth of instructions: 236 launches 0.80, of
+  //     them slabs a third to a half longer (three slabs to two: 172 to 200 workgroups) 51 launches 0.87, none over
+  //     1.03 (fp32 [42, 632917] k=484 j=2 294 -> 252 workgroups 30.1 -> 24.6 us, bf16 [89, 266666] k=23 267 -> 178 18.8 -> 15.8);
+  //   four waves: up to a third longer 59 launches 0.90 (one over 1.05), beyond, of 2-byte elements with three and four of
+  //     a bucket 66 launches 0.95, with two 35 launches 1.06 (fp16 [2, 45395679] b=75 j=2, 512 -> 256 workgroups, 51.0 ->
+  //     59.1 us) and of 4-byte ones 30 launches 1.26: those keep two workgroups a CU, but no more (513 -> 510, 20 launches 0.79);
+  //   one-element loads: up to a sixth longer 117 launches 0.94 (seven over 1.05, four of them fp32 [3, 2^24], 258 -> 255
+  //     workgroups), beyond 60 launches 1.04 and up to 1.32 (int8 [92, 1483801] b=2 j=2, 276 -> 184, 80.7 -> 106.5 us).
+  // (With one slab left, and no merge, some lose a third.)
   const int64_t per_slab = rows * pl.col_tiles;  // workgroups
   const uint32_t slabs_asked = pl.slabs;
-  if (pl.slabs > 1 && pl.slabs * per_slab > kCus && kCus / per_slab > 1) pl.slabs = (uint32_t)(kCus / per_slab);
+  const int64_t in_one_turn = kCus / per_slab;  // slabs
+  if (in_one_turn > 1 && (int64_t)pl.slabs > in_one_turn) {
+    const double longer = (double)pl.slabs / (double)in_one_turn;
+    const bool whole_cu = es == 8 || (pl.vec > 1 && w == 8), long_queues = w < 8 && es <= 2 && j >= 3;
+    if (whole_cu || long_queues || longer <= (w < 8 ? kLongerFourWaves : kLongerOneElement))
+      pl.slabs = (uint32_t)in_one_turn;
+    else if (w < 8 && (int64_t)pl.slabs > 2 * kCus / per_slab)
+      pl.slabs = (uint32_t)(2 * kCus / per_slab);
+  }
   // CUs left idle while every wave has a long way to go: up to a workgroup each, with what a wave reads at kWaveBytes or
   // more, and the second stage left in the merge where it is (132 -> 252 workgroups fp16 [7, 2^22] k=32 j=4 k_mult=2 28.8 ->
   // 24.0 us, 144 -> 252 bf16 [9, 2^22] k=512 j=4 32.9 -> 24.7, fp32 [2, 2^23] k=1024 j=4 k_mult=4 128 -> 256 37.2 -> 29.3; with 2-4 KB
   // a wave, f16 [3, 346950] k=324 j=2, 7.7 -> 8.3).  Small partial queues only: the workspace stays within what the call
-  // that cannot allocate has taken.
+  // that cannot allocate has taken.  One workgroup a row reads them all where the merge selects: up to
+  // kRaisedSelectQueues (107 launches up to there 0.92, of one to three elements a bucket and more queues 29 launches
+  // 1.03: bf16 [1, 11732747] k=16 k_mult=2, 179 -> 256 slabs, 14.4 -> 17.1 us).
   if (pl.slabs > 1 && pl.slabs * per_slab < kCus && rows * k0 * (es + 8) <= kRaisedBytes) {
-    int64_t slabs = kCus / per_slab;
+    int64_t slabs = in_one_turn;
     const int64_t by_wave = full * kWave * pl.vec * es / (w * kWaveBytes), by_queues = kRaisedBytes / (rows * k0 * (es + 4));
     if (slabs > by_wave) slabs = by_wave;
     if (slabs > by_queues) slabs = by_queues;
-    if (k0 <= kMergeSelectMax && k0 * (int64_t)pl.slabs <= kMergeSelectEntries && slabs > kMergeSelectEntries / k0)
-      slabs = kMergeSelectEntries / k0;
+    if (k0 <= kMergeSelectMax && k0 * (int64_t)pl.slabs <= kMergeSelectEntries) {
+      const int64_t most_queues = second_stage && es <= 4 ? kRaisedSelectQueues : kMergeSelectEntries / j;
+      if (slabs > most_queues / b) slabs = most_queues / b;
+    }
     if (slabs > (int64_t)pl.slabs) pl.slabs = (uint32_t)slabs;
   }
   pl.slab_len = (uint32_t)(full / pl.slabs);
@@ -264,12 +288,12 @@ double estimate(const Plan& pl, int64_t rows, int64_t n, int64_t k0, int j, int 
 }  // namespace
 
 Plan make_plan(int64_t rows, int64_t n, int64_t k0, int j, int layout, int dtype, int64_t select_bound) {
-  const Plan w = plan_with(rows, n, k0, j, layout, dtype, true);
+  const Plan w = plan_with(rows, n, k0, j, layout, dtype, true, select_bound > 0);
   if (!w.ok || w.vec == 1) return w;
   // whole-wave stores spare the lanes' entries most of what the estimate takes for them; with half of the lanes at work
   // they stay ahead (i8 [4475, 6579] b=320 j=2 42.8 us, 56.5 with one-element loads; bf16 [10470, 6399] b=136 j=4 163 and 114)
   if (w.wave_stores && 2 * w.width >= (int64_t)w.col_tiles * kWave * w.vec) return w;
-  const Plan v = plan_with(rows, n, k0, j, layout, dtype, false);
+  const Plan v = plan_with(rows, n, k0, j, layout, dtype, false, select_bound > 0);
   // (a launch's threads are counted in 32 bits)
   if (!v.ok || rows * (int64_t)v.slabs * v.col_tiles > 0xffffffffll / (kWave * v.waves)) return w;
   auto us = [&](const Plan& pl) {
@@ -298,8 +322,8 @@ bool selects_in_merge(const Plan& pl, int64_t k0, int64_t index_bound, int dtype
 
 size_t stage1_stream_workspace_bytes(int64_t rows, int64_t n, int64_t k0, int j, int layout, int dtype) {
   // (make_plan picks one of these)
-  const stream::Plan a = stream::plan_with(rows, n, k0, j, layout, dtype, true);
-  const stream::Plan u = stream::plan_with(rows, n, k0, j, layout, dtype, false);
+  const stream::Plan a = stream::plan_with(rows, n, k0, j, layout, dtype, true, false);
+  const stream::Plan u = stream::plan_with(rows, n, k0, j, layout, dtype, false, false);
   size_t need = 0;
   if (a.ok && a.ws_bytes > need) need = a.ws_bytes;
   if (u.ok && u.ws_bytes > need) need = u.ws_bytes;

@@ -443,3 +443,42 @@ def test_the_workspace_a_call_uses_stays_within_the_figure_at_its_address():
         buf = ctypes.create_string_buffer(1024)
         assert L.atk_describe(4096, *args, 4096, 4096, buf, 1024) == 0
         assert (used == 0) == buf.value.startswith(b"fused_"), (args, buf.value)
+
+
+def _plan(dtype, rows, n, k, j, k_mult=1):
+    from approx_topk import _native
+    buf = ctypes.create_string_buffer(1024)
+    code = _native.dtype_code(dtype)
+    assert _native.lib().atk_describe(4096, rows, n, n, k * k_mult, j, k, 0, code, 4096, 4096, buf, 1024) == 0
+    text = buf.value.decode()
+    found = re.search(r"V=(\d+), W=(\d+), .*? grid=(\d+) .* slabs=(\d+)", text)
+    return tuple(int(v) for v in found.groups()) + (text,)
+
+
+def test_slabs_are_cut_to_one_turn_of_the_cus_where_that_was_measured_faster():
+    f32, f16, i8, f64 = torch.float32, torch.float16, torch.int8, torch.float64
+    # 16-byte loads in eight waves, and eight-byte elements: no more workgroups than CUs, whatever a slab grows by
+    for dtype in (f32, f16, f64):
+        for rows in list(range(65, 128, 3)) + [85, 86, 127]:
+            vec, waves, grid, slabs, text = _plan(dtype, rows, 1 << 20, 64, 2)
+            if slabs > 1 and waves == 8 and (vec > 1 or dtype is f64):
+                assert grid <= 256 and grid > 128, text
+    assert _plan(f32, 86, 1 << 20, 64, 2)[:4] == (4, 8, 172, 2)
+    # four waves: two workgroups a CU stay, where a slab would get more than a third longer; no more than two
+    assert _plan(f16, 2, 45395679, 150, 2)[1:3] == (4, 512)
+    assert _plan(f16, 4, 1 << 25, 62, 2)[1:3] == (4, 512)
+    assert _plan(f16, 3, 1 << 25, 198, 2)[1:3] == (4, 510)
+    # (but queues of three and four of 2-byte elements)
+    assert _plan(f16, 1, 1 << 26, 4096, 4)[1:3] == (4, 256)
+    # one-element loads: two of three slabs stay three
+    for dtype in (i8, f16, f32):
+        for rows in range(86, 129):
+            vec, waves, grid, slabs, text = _plan(dtype, rows, 40001, 240, 1)
+            assert vec > 1 or slabs != 2 or waves < 8, text
+
+
+def test_merges_that_select_are_not_given_more_than_a_workgroup_reads_quickly():
+    # slabs raised to one workgroup a CU: with a merge that selects only up to 4096 partial queues
+    assert _plan(torch.bfloat16, 1, 11732747, 16, 1, 2)[3] == 179
+    assert _plan(torch.bfloat16, 1, 11732747, 32, 1)[3] == 256  # (no second stage)
+    assert _plan(torch.float16, 7, 1 << 22, 32, 4, 2)[3] == 36
