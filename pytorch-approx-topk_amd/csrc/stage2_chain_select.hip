@@ -464,6 +464,33 @@ constexpr int kSoloWaves = kSoloThreads / select::kWave;
 constexpr uint32_t kSoloRankDirect = 512;
 static_assert((uint32_t)kSoloThreads == kSoloSegment, "a thread's u-th candidate lies in segment u");
 
+// Whether twelve lanes and more have the digit of the first lane that counts (of candidates spread over 20 digits, few waves do).
+__device__ __forceinline__ bool crowded(uint32_t digit, bool counts) {
+  const uint64_t those = __ballot(counts);
+  if (those == 0) return false;
+  const int first = __builtin_amdgcn_readfirstlane((int)__ffsll((unsigned long long)those) - 1);
+  return __popcll(__ballot(counts && digit == (uint32_t)__builtin_amdgcn_readlane((int)digit, first))) >= 12;
+}
+
+// Adds a wave's digits to the histogram.  `gather`: lanes with the same digit, from eight on, as one add (an LDS counter
+// takes a lane at a time: 8192 candidates of one key added 10 us).
+__device__ __forceinline__ void count_digits(uint32_t* hist, uint32_t digit, bool counts, uint32_t lane, bool gather) {
+  if (gather) {
+#pragma unroll
+    for (int crowd = 0; crowd < 2; ++crowd) {
+      const uint64_t left = __ballot(counts);
+      if (left == 0) return;
+      const int first = __builtin_amdgcn_readfirstlane((int)__ffsll((unsigned long long)left) - 1);
+      const uint32_t lead = (uint32_t)__builtin_amdgcn_readlane((int)digit, first);
+      const uint32_t same = (uint32_t)__popcll(__ballot(counts && digit == lead));
+      if (same < 8u) break;
+      if (lane == (uint32_t)first) atomicAdd(&hist[lead], same);
+      counts = counts && digit != lead;
+    }
+  }
+  if (counts) atomicAdd(&hist[digit], 1u);
+}
+
 // FULL: the row has exactly NPT * 1024 candidates, so that every key a thread holds exists and
 // nothing has to say which do (32 wave-wide masks otherwise, which the kernel with 32 keys per
 // thread has no scalar registers for).
@@ -485,6 +512,10 @@ __global__ __launch_bounds__(kSoloThreads) void chain_solo_kernel(
   __shared__ uint64_t cut_word;
   uint64_t* words = reinterpret_cast<uint64_t*>(dyn_lds);
   uint32_t* ats = reinterpret_cast<uint32_t*>(dyn_lds + (size_t)(kListCap + 8) * sizeof(uint64_t));
+  // Members of the cut digit up to which they are listed.  With registers to spare a longer list is narrowed down, at
+  // about 1.5 us a level: ranking 512 by comparison takes 3, the radix select over 1536 took 10.
+  constexpr bool kSpare = NPT <= 16;
+  constexpr uint32_t kListed = TIES && kSpare ? kSoloRankDirect / 2 : kListCap;
   const uint32_t row = blockIdx.x / groups, g = blockIdx.x - row * groups;
   const uint32_t tid = threadIdx.x, lane = tid % select::kWave, wave = tid / select::kWave;
   const raw_t* cv = cand_values + (int64_t)row * k0;
@@ -522,9 +553,15 @@ __global__ __launch_bounds__(kSoloThreads) void chain_solo_kernel(
   uint32_t low, shift;
   regs::digit_from_folded<kSoloThreads>(folded, red, low, shift);  // (its barrier covers the clearing)
   ATK_TRACE_GROUP(1);
+  // (a wave looks at two of its keys for a digit that many of them share: looking at each was 0.4 us for eight of them)
+  const bool gather = kSpare && (crowded((key[0] - low) >> shift, valid(0)) || crowded((key[1] - low) >> shift, valid(1)));
+  if (gather) {
 #pragma unroll
-  for (int u = 0; u < NPT; ++u)
-    if (valid(u)) atomicAdd(&hist[(key[u] - low) >> shift], 1u);
+    for (int u = 0; u < NPT; ++u) count_digits(hist, (key[u] - low) >> shift, valid(u), lane, true);
+  } else {
+#pragma unroll
+    for (int u = 0; u < NPT; ++u) count_digits(hist, (key[u] - low) >> shift, valid(u), lane, false);
+  }
   __syncthreads();
   ATK_TRACE_GROUP(2);
   if (wave == 0) {
@@ -537,7 +574,7 @@ __global__ __launch_bounds__(kSoloThreads) void chain_solo_kernel(
   // The cut digit holds more candidates than the list: they are counted again by
   // the next bits of their offsets, which narrows the digit, until its members
   // fit or no bits are left.
-  if (f.need != f.count && f.count > kListCap && shift != 0) {
+  if (f.need != f.count && f.count > kListed && shift != 0) {
     // Members of one and the same key (a ReLU's zeros) are not told apart by any further level,
     // and every level would add them up in one counter, a lane at a time (16384 of them: 20 us
     // a level).  Found out first: some member leaves its key in LDS, and every thread compares
@@ -559,7 +596,7 @@ __global__ __launch_bounds__(kSoloThreads) void chain_solo_kernel(
       shift = 0;
     }
   }
-  while (f.need != f.count && f.count > kListCap && shift != 0) {
+  while (f.need != f.count && f.count > kListed && shift != 0) {
     const uint32_t finer = shift > (uint32_t)regs::kDigitBits ? shift - (uint32_t)regs::kDigitBits : 0u;
     const uint32_t mask = (1u << (shift - finer)) - 1u;
     __syncthreads();  // everyone has read `found`, wave 0 the histogram
@@ -568,7 +605,7 @@ __global__ __launch_bounds__(kSoloThreads) void chain_solo_kernel(
 #pragma unroll
     for (int u = 0; u < NPT; ++u) {
       const uint32_t off = key[u] - low;
-      if (valid(u) && (off >> shift) == f.digit) atomicAdd(&hist[(off >> finer) & mask], 1u);
+      count_digits(hist, (off >> finer) & mask, valid(u) && (off >> shift) == f.digit, lane, kSpare);
     }
     __syncthreads();
     if (wave == 0) {
@@ -583,15 +620,14 @@ __global__ __launch_bounds__(kSoloThreads) void chain_solo_kernel(
     shift = finer;
   }
   const bool cut_digit = f.need != f.count;  // else every member of B survives
-  // TIES: shift == 0 and still too many -- thousands of candidates of one key around the cut,
+  // TIES: shift == 0 and still too many -- hundreds of candidates of one key around the cut,
   // which is what stage 1 makes of saturated 8-bit data (the bucket maxima of uniform uint8 are
-  // all 255) -- and their indices decide.  Built for the 1-byte types only: the code costs the
-  // kernel 4-5 us whether it runs or not (it sits at its register limit).
-  const bool tie_mode = TIES && cut_digit && f.count > kListCap;
-  // The list in LDS holds kListCap entries: a cut digit with more members (which, without
-  // TIES, no bits are left to narrow) is not listed at all; the row then goes to the
-  // whole-row path below.
-  const bool list_it = cut_digit && f.count <= kListCap;
+  // all 255) and of a ReLU's zeros -- and their indices decide.  With 32 keys per thread built for the 1-byte
+  // types only: there the code costs the kernel 4-5 us whether it runs or not (it sits at its register limit).
+  const bool tie_mode = TIES && cut_digit && f.count > kListed;
+  // A cut digit with more members than are listed (which, without TIES, no bits are left to
+  // narrow) is not listed at all; the row then goes to the whole-row path below.
+  const bool list_it = cut_digit && f.count <= kListed;
   const uint32_t own = g * kSoloThreads + tid;  // this thread's candidate of segment g
   const bool own_valid = FULL || own < k0;
   // survivors above the cut digit (or in it, when it belongs whole) in the
@@ -644,7 +680,8 @@ __global__ __launch_bounds__(kSoloThreads) void chain_solo_kernel(
   if constexpr (TIES) {
     if (tie_mode) {
       // The members (all of one key) are counted by the leading bits of their inverted indices,
-      // 11 at a time, until the group that is cut fits the list.  Their indices are read eight
+      // 11 at a time from the first that an index has (those before it are set in all of them, and a histogram of one
+      // bin is slow), until the group that is cut fits the list.  Their indices are read eight
       // segments at a time (the low halves: the planner sends only indices below 2^31 here).
       const uint32_t* ci_low = reinterpret_cast<const uint32_t*>(ci);
       auto for_members = [&](auto&& fn) __attribute__((always_inline)) {
@@ -662,15 +699,16 @@ __global__ __launch_bounds__(kSoloThreads) void chain_solo_kernel(
             if ((members >> (c0 + e)) & 1u) fn((uint32_t)(c0 + e), ~iv[e]);
         }
       };
-      uint32_t ishift = 32, iprefix = 0;  // the group: inverted indices whose bits from ishift up are iprefix
-      while (need != count && count > kListCap && ishift != 0) {
+      // the group: inverted indices whose bits from ishift up are iprefix
+      uint32_t ishift = (uint32_t)(index_bits < 31 ? index_bits : 31), iprefix = ~0u >> ishift;
+      while (need != count && count > kListed && ishift != 0) {
         const uint32_t finer = ishift > (uint32_t)regs::kDigitBits ? ishift - (uint32_t)regs::kDigitBits : 0u;
         const uint32_t mask = (1u << (ishift - finer)) - 1u;
         __syncthreads();  // everyone has read `found`, wave 0 the histogram
         for (uint32_t i = tid; i < (uint32_t)regs::kBins; i += kSoloThreads) hist[i] = 0;
         __syncthreads();
         for_members([&](uint32_t, uint32_t inv) {
-          if (ishift == 32u || (inv >> ishift) == iprefix) atomicAdd(&hist[(inv >> finer) & mask], 1u);
+          if ((inv >> ishift) == iprefix) atomicAdd(&hist[(inv >> finer) & mask], 1u);
         });
         __syncthreads();
         if (wave == 0) {
@@ -684,7 +722,7 @@ __global__ __launch_bounds__(kSoloThreads) void chain_solo_kernel(
         need = f2.need;
         count = f2.count;
       }
-      if (ishift != 32u && (need == count || count <= kListCap)) {
+      if (need == count || count <= kListed) {
         const uint64_t key_word = (uint64_t)(low + f.digit) << 32;  // (shift == 0: the digit is the key's offset)
         for_members([&](uint32_t u, uint32_t inv) {
           const uint32_t group = inv >> ishift;
@@ -779,8 +817,8 @@ __global__ __launch_bounds__(kSoloThreads) void chain_solo_kernel(
       if (tid == 0) list_count = 0;
     }
   }
-  if (need != count && count > kListCap) {
-    // More than kListCap candidates of one key around the cut (TIES: of one key and
+  if (need != count && count > kListed) {
+    // More candidates of one key around the cut than are listed (TIES: of one key and
     // one index, which only a caller of the stand-alone select can hand over): the
     // row's first workgroup runs the block-wide radix select of stage2_select.h over
     // all of the row's candidates, read from global memory.
@@ -879,6 +917,10 @@ __global__ __launch_bounds__(kSoloThreads) void chain_solo_kernel(
 // row: 1 row of 4096 / 6144 / 8192 candidates 15.4 / 16.8 / 15.8 -> 12.6 / 10.8 / 10.1, 4 of 8192 16.9 -> 11.4, 16 of 2048 14.7 ->
 // 13.2, of 1536 15.5 -> 14.4, 20 of 8192 23.7 -> 18.4, 32 of 8192 29.0 -> 24.2, 64 of 4096 38.8 -> 36.5; of 1024 candidates 64 rows
 // 36.1 -> 34.6, fewer not measured (their slabs' merge takes the select along).
+// Candidates of few keys, which crowd one counter and one list, were the exception (atk_select alone, one workgroup per row
+// against this kernel before and with count_digits and the list of 256): half of them zeros, fp32 [1, 2048] 10.9 us, 15.8
+// and 9.5, [32, 8192] 19.6, 22.8 and 14.8, bf16 [128, 2048] 9.4, 16.4 and 10.8; all equal, fp32 [1, 8192] 18.9, 32.1 and 12.0,
+// uint8 [1, 2048] 7.5, 19.1 and 8.0, [4, 8192] 13.4, 31.5 and 11.8; what buckets leave of N(0, 1), fp32 [1, 8192] 11.7, 6.1 and 6.2.
 constexpr int64_t kSoloMinCandidates = 1536;
 constexpr int64_t kSoloMaxCandidates = 32 * kSoloThreads;
 constexpr int64_t kSoloMaxWorkgroups = 256;

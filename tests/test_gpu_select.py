@@ -274,3 +274,25 @@ def test_select_of_rows_ranked_by_comparison(dtype, rows, k0, k):
     ci = torch.stack([torch.randperm(1 << 10, generator=g)[:k0] for _ in range(rows)])
     v, i = _select(cv, ci, k, 1 << 10)
     assert_same(v, i, *oracle.stage2(cv, ci, k), f"{dtype} {rows} {k0} {k}")
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.uint8])
+@pytest.mark.parametrize("k0,bound", [(1536, 1 << 13), (2047, (1 << 31) - 1), (8192, 1 << 13), (8191, 1 << 24), (9000, 1 << 16),
+                                      (16384, (1 << 31) - 1)])
+@pytest.mark.parametrize("m", [255, 256, 257, 513, 1500])
+def test_one_launch_select_of_crowded_keys(dtype, k0, bound, m):
+    # m candidates of one key around the cut, listed up to 256 of them and told apart by their indices beyond;
+    # those above and below are spread, or of one key each (a wave adds eight of a digit and more at once)
+    g = torch.Generator().manual_seed(k0 + m)
+    cv = torch.randint(0, 100, (4, k0), generator=g)
+    cv = torch.where(cv >= 50, cv + 1, cv)
+    cv[1:3] = torch.where(cv[1:3] > 50, 100, 0)
+    for r in range(4):
+        cv[r, torch.randperm(k0, generator=g)[:m]] = 50
+    cv = cv.to(dtype)
+    ci = torch.stack([torch.randperm(min(bound, 1 << 20), generator=g)[:k0] for _ in range(4)])
+    ci[2:] += bound - min(bound, 1 << 20)  # the last ones that the bound allows
+    above = [int((cv[r] > 50).sum()) for r in range(4)]
+    for k in {above[0] + 1, above[0] + m // 2, above[1] + m - 1, min(above) + m}:
+        v, i = _select(cv, ci, k, bound)
+        assert_same(v, i, *oracle.stage2(cv, ci, k), f"{dtype} k0={k0} m={m} k={k}")
