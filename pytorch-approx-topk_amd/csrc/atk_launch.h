@@ -134,6 +134,10 @@ bool describe_stage1_contig(const void* x, int64_t rows, int64_t n, int64_t row_
 void describe_stage1_lane_per_bucket(int64_t rows, int64_t k0, int j, int dtype, std::string& out);
 bool describe_fused_row(const void* x, int64_t rows, int64_t n, int64_t row_stride, int64_t k0, int j, int64_t k,
                         int layout, int dtype, std::string& out);
+// Which kernel a select of its own would be (the estimate of stage1_stream_plan.hip goes by it).
+bool one_launch_select_takes(int64_t rows, int64_t k0, int64_t index_bound, int dtype);
+bool rank_select_takes(int64_t rows, int64_t k0, int64_t index_bound, int dtype);
+
 bool describe_multi_select(int64_t rows, int64_t k0, int64_t k, int64_t index_bound, int dtype, std::string& out);
 bool describe_chain_select(int64_t rows, int64_t k0, int64_t k, int64_t index_bound, int dtype, std::string& out);
 void describe_select(int64_t rows, int64_t k0, int64_t k, int64_t index_bound, int dtype, bool with_workspace,

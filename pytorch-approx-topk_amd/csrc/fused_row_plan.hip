@@ -254,8 +254,11 @@ bool taken_by_size(int64_t rows, int64_t n, int64_t k0, int j, int64_t k, int la
 namespace {
 // Rows and candidates up to which the estimates below were fitted.
 constexpr int64_t kEstimatedRow = 1 << 20, kEstimatedCandidates = 8192;
-// A call that the rules of size leave to two kernels takes one where its estimate is this share of theirs.
-constexpr double kOneKernelShare = 0.85;
+// A call that the rules of size leave to two kernels takes one where its estimate is this share of theirs.  On 1500 calls that
+// both take and neither estimate was fitted to, the choice (the rules of size included) is 1.2 % slower than the better of the
+// two, one kernel throughout 33 %, two 20 %; the share could be 1.0, but for rows whose cut falls among ties, which cost one
+// kernel more (of 43 such shapes four were over 10 % slower at 0.85).
+constexpr double kOneKernelShare = 0.9;
 
 // Estimated microseconds of the register kernel under a plan of elements of two or four bytes: the scan (memory, instructions
 // and the round trips of a wave's loads, which overlap: the root of the sum of their squares), and what every
@@ -263,7 +266,7 @@ constexpr double kOneKernelShare = 0.85;
 // selection, by the candidates of a lane and the waves that wait for one another.
 // The constants are a least-squares fit to 1415 launches of 620 calls (fp32 and fp16, 1-8192 rows of 2048-2^18 elements,
 // half of them of no round length, 32-8192 candidates, j 1, 2, 4, k_mult 2-8, up to 160 MiB; every width of load): off by
-// 10 % in the root mean square.  Among those calls, the choice by these estimates is 2.2 % slower than the best of two kernels
+// 10 % in the root mean square.  Among those calls, the choice by these estimates was 2.2 % slower than the best of two kernels
 // and one with each width; the rules of size with the usual width, which stood before, are 16 %.  (float32 [859, 2048]
 // k=64 j=4 k_mult=2 29.1 us by the rules, 10.1 with one column a lane; [1053, 19352] k=152 j=1 k_mult=2 35.5 in two kernels, 21.4
 // in one; fp16 [2048, 8192] k=100 j=2 k_mult=4 37.5 in two kernels, 17.3 in one.)

@@ -1837,8 +1837,8 @@ struct Plan {
 // against 67, one byte, uint8 [1024, 32768] k=2048 j=2 45.0 against 13.1.
 Plan make_plan(int64_t rows, int64_t n, int64_t k0, int j, int layout, int dtype, int64_t select_bound);
 
-// Estimated microseconds of a call with a second stage through these kernels and a select (interleaved buckets; what all plans
-// share is fitted to 620 such calls, see csrc/fused_row_plan.hip: off by 13 % in the root mean square).
+// Estimated microseconds of a call with a second stage through these kernels and a select (interleaved buckets; see
+// csrc/stage1_stream_plan.hip).
 double estimate_two_kernels(int64_t rows, int64_t n, int64_t k0, int j, int dtype);
 
 // One instance per element type, each in its own translation unit.

@@ -18,7 +18,7 @@ constexpr int64_t kWaveBytes = 8 << 10, kRaisedBytes = 2 << 20;
 // Most partial queues of a row whose merge selects, with slabs that are cut to have a workgroup on every CU.
 constexpr int64_t kRaisedSelectQueues = 4096;
 // How much longer a slab may get to have no more workgroups than CUs.
-constexpr double kLongerFourWaves = 1.34, kLongerOneElement = 1.17;
+constexpr double kLonger = 1.34, kLongerOneByte = 1.17;
 // Sub-rows worth giving to one wave before a row is also cut into slabs.
 constexpr int64_t kSlabRun = 16;
 // Fewest workgroups of a launch whose results take the trip through LDS.
@@ -145,15 +145,16 @@ Plan plan_with(int64_t rows, int64_t n, int64_t k0, int j, int layout, int dtype
   }
   // A launch of more workgroups than CUs gives some CUs twice the work, with the others waiting: down to no more
   // workgroups than CUs, in fewer and longer slabs.  How much longer they may get lies with how well a CU's second
-  // workgroup hides behind the first.  519 launches (all types, 1-200 rows, 4-70 M elements), time cut over time as asked:
+  // workgroup hides behind the first.  Time cut over time as asked, 960 launches (all types, 1-200 rows of 2^13 to 2^26):
   //   eight waves with 16-byte loads, or of eight-byte elements, each a CU's worth of instructions: 236 launches 0.80, of
   //     them slabs a third to a half longer (three slabs to two: 172 to 200 workgroups) 51 launches 0.87, none over
   //     1.03 (fp32 [42, 632917] k=484 j=2 294 -> 252 workgroups 30.1 -> 24.6 us, bf16 [89, 266666] k=23 267 -> 178 18.8 -> 15.8);
-  //   four waves: up to a third longer 59 launches 0.90 (one over 1.05), beyond, of 2-byte elements with three and four of
+  //   four waves: up to a third longer 59 launches 0.90 (one over 1.05); beyond, of 2-byte elements with three and four of
   //     a bucket 66 launches 0.95, with two 35 launches 1.06 (fp16 [2, 45395679] b=75 j=2, 512 -> 256 workgroups, 51.0 ->
   //     59.1 us) and of 4-byte ones 30 launches 1.26: those keep two workgroups a CU, but no more (513 -> 510, 20 launches 0.79);
-  //   one-element loads: up to a sixth longer 117 launches 0.94 (seven over 1.05, four of them fp32 [3, 2^24], 258 -> 255
-  //     workgroups), beyond 60 launches 1.04 and up to 1.32 (int8 [92, 1483801] b=2 j=2, 276 -> 184, 80.7 -> 106.5 us).
+  //   one-element loads, of the calls that are not faster with wider ones: 2- and 4-byte elements up to a third longer 95
+  //     launches 0.93 (three over 1.05, all of fp32 [3, 2^24], 258 -> 255 workgroups), beyond 28 launches 0.99 and up to
+  //     1.18; one byte up to a sixth longer 19 launches 0.94, beyond 20 launches 1.02 and up to 1.11.
   // (With one slab left, and no merge, some lose a third.)
   const int64_t per_slab = rows * pl.col_tiles;  // workgroups
   const uint32_t slabs_asked = pl.slabs;
@@ -161,7 +162,7 @@ Plan plan_with(int64_t rows, int64_t n, int64_t k0, int j, int layout, int dtype
   if (in_one_turn > 1 && (int64_t)pl.slabs > in_one_turn) {
     const double longer = (double)pl.slabs / (double)in_one_turn;
     const bool whole_cu = es == 8 || (pl.vec > 1 && w == 8), long_queues = w < 8 && es <= 2 && j >= 3;
-    if (whole_cu || long_queues || longer <= (w < 8 ? kLongerFourWaves : kLongerOneElement))
+    if (whole_cu || long_queues || longer <= (es == 1 ? kLongerOneByte : kLonger))
       pl.slabs = (uint32_t)in_one_turn;
     else if (w < 8 && (int64_t)pl.slabs > 2 * kCus / per_slab)
       pl.slabs = (uint32_t)(2 * kCus / per_slab);
@@ -220,30 +221,33 @@ Plan plan_with(int64_t rows, int64_t n, int64_t k0, int j, int layout, int dtype
 }  // namespace
 
 namespace {
-// Estimated microseconds of a plan (less what all plans of a call share), for the choice between 16-byte and
-// one-element loads where both are possible.  With one-element loads a lane owns one column instead of two to eight:
-// more workgroups, in rows cut into slabs fewer partial queues, and a shorter end of every workgroup, against fewer bytes
-// in flight, a load for every element and more waves to launch.  What a plan takes is
+// Estimated microseconds of a call, for the choice between 16-byte and one-element loads where both are possible, and
+// for that between these kernels and the one-kernel path.  With one-element loads a lane owns one column instead of two to
+// eight: more workgroups, in rows cut into slabs fewer partial queues, and a shorter end of every workgroup, against fewer
+// bytes in flight, a load for every element and more waves to launch.  What a plan takes is
 //   the scan: memory, instructions, the launch of the waves and the round trips of a wave's loads, which overlap
 //     (the root of the sum of their squares);
 //   a workgroup's end: the other waves' queues folded into the leading wave's, folded columns put together, and a
 //     lane's entries written, by one wave, next to the ends and scans of the workgroups that the CU holds with it;
-//   the launches behind it: the merge of the slabs, with or without the second stage, or the stand-alone select.
-// The constants are a least-squares fit to 2070 calls timed both ways (all nine types, 1-20000 rows of 37 to 2^24
-// elements, up to 128 MiB, j 1-4, k_mult 1-8, half of them few rows, most of them off 16 bytes).  Its choice is
-// 1.0 % slower than the better one of the two in the geometric mean (10 % and more in one call of 24), 16-byte loads
-// throughout 14 %, one-element loads throughout 6 %: fp32 [3, 2^21] b=128 j=4 k_mult=8 30.2 us wide, 17.9 narrow, int8
-// [1, 172601] b=1310 j=4 8.5 and 4.0, uint8 [39, 152696] b=201 j=4 14.7 and 8.6, fp64 [2, 310384] b=799 j=4 13.6 and
-// 11.1, fp16 [168, 298475] b=544 j=4 67.9 and 42.1, but int8 [51, 507136] b=2391 j=3 11.5 and 17.4, fp16 [21, 1426304]
-// b=8338 j=2 17.1 and 24.1.
-double estimate(const Plan& pl, int64_t rows, int64_t n, int64_t k0, int j, int dtype, bool second_stage,
-                bool selects) {
+//   the launches behind it: the merge of the slabs, with or without the second stage, or a select of its own.
+// The scan's and the end's constants are a least-squares fit to 2070 calls timed both ways (all nine types, 1-20000 rows
+// of 37 to 2^24 elements, up to 128 MiB, j 1-4, k_mult 1-8, half of them few rows, most of them off 16 bytes); those of the
+// launches behind them to 18500 launches of 8900 calls with the merge and the selects as they are (four partial queues
+// a thread; up to 512 MiB): off by 16 % in the root mean square.  On 3000 other calls the choice is 1.1 % slower than the better
+// one of the two in the geometric mean (10 % and more in one call of 26), 16-byte loads throughout 11 %, one-element loads
+// throughout 11 %: fp32 [3, 2^21] b=128 j=4 k_mult=8 30.2 us wide, 17.9 narrow, int8
+// [1, 172601] b=1310 j=4 8.3 and 4.0, uint8 [39, 152696] b=201 j=4 14.5 and 8.7, fp64 [2, 310384] b=799 j=4 12.3 and
+// 10.8, fp16 [168, 298475] b=544 j=4 67.9 and 42.1, but int8 [51, 507136] b=2391 j=3 11.2 and 16.9, fp16 [21, 1426304]
+// b=8338 j=2 16.8 and 23.5.
+double estimate(const Plan& pl, int64_t rows, int64_t n, int64_t k0, int j, int dtype, int64_t select_bound) {
   constexpr double kBytes = 5.1e6, kSlowFolds = 1.2, kWaveLaunch = 3.6e-4;  // per us; us
   constexpr double kTrip = 0.34, kLoad = 0.0087;          // us: a batch of loads, issuing one (a wave per SIMD)
   constexpr double kHandOver = 0.008, kEntry = 0.067;     // us an entry of a lane: handed over, written
   constexpr double kFold = 0.4, kFoldStep = 0.039;
-  constexpr double kMerge = 2.8, kMergeStep = 0.097;
-  constexpr double kMergeSelect = 4.5, kMergeSelectEntry = 3.1e-4, kSelect = 6.0, kSelectEntry = 6.6e-4;
+  constexpr double kLaunch = 2.42, kMerge = 2.49, kMergeStep = 0.107, kMergeSelect = 4.3, kMergeSelectEntry = 3.6e-4;
+  constexpr double kRank = 3.22, kRankEntry = 3.76e-3, kOneLaunch = 5.96, kOneLaunchEntry = 2.7e-4, kSelect = 6.49,
+                   kSelectEntry = 1.24e-3;
+  constexpr double kLastTurn = 0.37;
   struct Push { double column, entry; };                  // us per sub-row (a wave per SIMD): a column, and per entry kept
   const int es = elem_bytes(dtype);
   const Push push = es == 1 ? Push{0.0067, 0.001} : es == 8 ? Push{0.0026, 0.029} : es == 4 ? Push{0.021, 0.0036}
@@ -259,8 +263,12 @@ double estimate(const Plan& pl, int64_t rows, int64_t n, int64_t k0, int j, int 
   const bool slow_folds = es == 4 && j <= 2 && pl.vec > 1 && pl.fold > 1 && pl.slabs > 1;
   const double memory = bytes / kBytes * (slow_folds ? kSlowFolds : 1.0), launch = waves * kWaveLaunch;
   const double trips = kTrip * (1 + (run > loads ? run / loads : 1.0));
-  const double pushes = run * (kLoad + pl.vec * (push.column + j * push.entry)) * (waves > 1024 ? waves / 1024 : 1.0);
-  double us = std::sqrt(memory * memory + launch * launch + trips * trips + pushes * pushes);
+  // (slabs that were left with a few workgroups more than CUs: the CUs with one more take part of a turn longer)
+  double turns = groups / kCus;
+  if (pl.merge && pl.vec == 1 && es < 8 && turns > 1 && turns <= 4) turns += kLastTurn * (std::ceil(turns) - turns);
+  const double on_simd = turns * pl.waves / 4;
+  const double pushes = run * (kLoad + pl.vec * (push.column + j * push.entry)) * (on_simd > 1 ? on_simd : 1.0);
+  double us = kLaunch + std::sqrt(memory * memory + launch * launch + trips * trips + pushes * pushes);
   double end = (kHandOver * (pl.waves - 1) + kEntry) * j * pl.vec;
   if (pl.fold > 1) {
     uint32_t at_once = kWave;  // buckets (see fold_columns)
@@ -275,14 +283,20 @@ double estimate(const Plan& pl, int64_t rows, int64_t n, int64_t k0, int j, int 
   const double by_lds = 160 * 1024 / (hand > words ? hand : words), by_waves = (pl.vec > 1 ? 16.0 : 32.0) / pl.waves;
   const double held = by_lds < by_waves ? (by_lds > 1 ? by_lds : 1.0) : by_waves;
   us += end * (groups > 256 * held ? groups / (256 * held) : 1.0);
-  if (pl.merge && selects) {
+  const bool selects = select_bound > 0 && selects_in_merge(pl, k0, select_bound, dtype);
+  if (selects) {
     us += kMergeSelect + kMergeSelectEntry * (double)pl.slabs * (double)k0;
   } else if (pl.merge) {
     uint32_t at_once = kWave;  // buckets (as the launch chooses them)
     while (at_once > 1 && (at_once / 2 >= b || (int64_t)pl.slabs * at_once > kMergeQueues * kMergeThreads)) at_once /= 2;
     us += kMerge + kMergeStep * j * std::ceil((double)pl.slabs * at_once / kMergeThreads);
   }
-  if (second_stage && !selects) us += kSelect + kSelectEntry * (double)k0 * (rows > 256 ? rows / 256.0 : 1.0);
+  if (select_bound > 0 && !selects) {
+    const double many = rows > kCus ? (double)rows / kCus : 1.0;
+    if (rank_select_takes(rows, k0, select_bound, dtype)) us += kRank + kRankEntry * (double)k0 * many;
+    else if (one_launch_select_takes(rows, k0, select_bound, dtype)) us += kOneLaunch + kOneLaunchEntry * (double)k0;
+    else us += kSelect + kSelectEntry * (double)k0 * many;
+  }
   return us;
 }
 }  // namespace
@@ -296,10 +310,7 @@ Plan make_plan(int64_t rows, int64_t n, int64_t k0, int j, int layout, int dtype
   const Plan v = plan_with(rows, n, k0, j, layout, dtype, false, select_bound > 0);
   // (a launch's threads are counted in 32 bits)
   if (!v.ok || rows * (int64_t)v.slabs * v.col_tiles > 0xffffffffll / (kWave * v.waves)) return w;
-  auto us = [&](const Plan& pl) {
-    const bool second = select_bound > 0;
-    return estimate(pl, rows, n, k0, j, dtype, second, second && selects_in_merge(pl, k0, select_bound, dtype));
-  };
+  auto us = [&](const Plan& pl) { return estimate(pl, rows, n, k0, j, dtype, select_bound); };
   const int es = elem_bytes(dtype);
   const bool large = rows * n * es > (es == 8 ? kLargeEight : kLargeBytes);
   return us(v) < us(w) * (large ? kLargeShare : 1.0) ? v : w;
@@ -308,9 +319,7 @@ Plan make_plan(int64_t rows, int64_t n, int64_t k0, int j, int layout, int dtype
 double estimate_two_kernels(int64_t rows, int64_t n, int64_t k0, int j, int dtype) {
   const Plan pl = make_plan(rows, n, k0, j, ATK_INTERLEAVED, dtype, n);
   if (!pl.ok) return INFINITY;
-  const bool selects = selects_in_merge(pl, k0, n, dtype);
-  const double us = estimate(pl, rows, n, k0, j, dtype, true, selects);
-  return selects ? 2.66 + 0.962 * us : 1.68 + us;
+  return estimate(pl, rows, n, k0, j, dtype, n);
 }
 
 bool selects_in_merge(const Plan& pl, int64_t k0, int64_t index_bound, int dtype) {

@@ -1066,6 +1066,11 @@ size_t chain_select_workspace_bytes(int64_t rows, int64_t k0, int64_t k, int64_t
   return pl.use ? pl.total : 0;
 }
 
+bool one_launch_select_takes(int64_t rows, int64_t k0, int64_t index_bound, int dtype) {
+  const ChainPlan pl = plan_chain(rows, k0, 1, index_bound, dtype);
+  return pl.use && pl.solo;
+}
+
 bool describe_chain_select(int64_t rows, int64_t k0, int64_t k, int64_t index_bound, int dtype, std::string& out) {
   const ChainPlan pl = plan_chain(rows, k0, k, index_bound, dtype);
   if (!pl.use) return false;

@@ -259,6 +259,10 @@ size_t select_workspace_bytes(int64_t rows, int64_t k0, int64_t k, int dtype) {
   return sp.use ? sp.total : 0;
 }
 
+bool rank_select_takes(int64_t rows, int64_t k0, int64_t index_bound, int dtype) {
+  return ranks(rows, k0, index_bound, dtype);
+}
+
 void describe_select(int64_t rows, int64_t k0, int64_t k, int64_t index_bound, int dtype, bool with_workspace,
                      std::string& out) {
   if (ranks(rows, k0, index_bound, dtype)) {

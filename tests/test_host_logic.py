@@ -482,3 +482,20 @@ def test_merges_that_select_are_not_given_more_than_a_workgroup_reads_quickly():
     assert _plan(torch.bfloat16, 1, 11732747, 16, 1, 2)[3] == 179
     assert _plan(torch.bfloat16, 1, 11732747, 32, 1)[3] == 256  # (no second stage)
     assert _plan(torch.float16, 7, 1 << 22, 32, 4, 2)[3] == 36
+
+
+# (type, rows, n, k, j, k_mult): calls timed in one kernel and in two, at least 20 % apart: the planner takes the faster one
+ONE = [(torch.bfloat16, 4, 32768, 333, 3, 2), (torch.int32, 4, 65536, 433, 1, 2), (torch.int16, 26, 8192, 88, 4, 3),
+       (torch.float16, 134, 70338, 1292, 4, 2), (torch.int32, 86, 131072, 878, 2, 4), (torch.float32, 537, 32768, 32, 4, 8),
+       (torch.int16, 338, 28275, 300, 4, 2), (torch.float16, 20, 32768, 161, 1, 2)]
+TWO = [(torch.int32, 106, 8192, 44, 4, 2), (torch.float16, 617, 56648, 6, 1, 8), (torch.bfloat16, 723, 10369, 20, 4, 4),
+       (torch.float16, 3, 158368, 84, 2, 4), (torch.bfloat16, 2, 377089, 36, 1, 2), (torch.bfloat16, 73, 336227, 80, 1, 8)]
+
+
+@pytest.mark.parametrize("kernels,calls", [("fused_regs_kernel<", ONE), ("stream_kernel<", TWO)], ids=["one", "two"])
+def test_one_kernel_or_two_follows_the_faster_plan(kernels, calls):
+    from approx_topk import _native
+    for dtype, rows, n, k, j, k_mult in calls:
+        buf = ctypes.create_string_buffer(1024)
+        assert _native.lib().atk_describe(4096, rows, n, n, k * k_mult, j, k, 0, _native.dtype_code(dtype), 4096, 4096, buf, 1024) == 0
+        assert buf.value.decode().startswith(kernels), (dtype, rows, n, k, j, k_mult, buf.value)
