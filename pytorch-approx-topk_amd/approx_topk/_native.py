@@ -11,6 +11,7 @@ import ctypes
 import functools
 import importlib
 import os
+import sysconfig
 
 import torch
 
@@ -65,8 +66,25 @@ _SIGNATURES = {
 
 
 _HOST_PATH = os.path.join(os.path.dirname(os.path.abspath(__file__)), "_host.so")
+
+
+def _import_host():
+    """(_host.so, None), or (None, what is wrong with it).  It is linked against torch: one that was built for
+    another torch or Python is not loaded, and what needs no native code goes on without it."""
+    if not os.path.exists(_HOST_PATH):
+        return None, "is missing"
+    built_for = f"approx_topk for torch {torch.__version__}, {sysconfig.get_config_var('SOABI')};"
+    with open(_HOST_PATH, "rb") as f:
+        if built_for.encode() not in f.read():
+            return None, f"is not built for torch {torch.__version__} and this Python"
+    try:
+        return importlib.import_module("._host", __package__), None
+    except ImportError as e:
+        return None, f"cannot be loaded ({e})"
+
+
 # (imported with the package: it registers the operators' kernels for the GPU)
-host = importlib.import_module("._host", __package__) if os.path.exists(_HOST_PATH) else None
+host, _host_fault = _import_host()
 
 
 def library_path() -> str:
@@ -89,7 +107,7 @@ def lib() -> ctypes.CDLL:
         raise RuntimeError(f"approx_topk: {path} has ABI {handle.atk_version()}, expected {ABI_VERSION}")
     if host is None:
         raise RuntimeError(
-            f"approx_topk: {_HOST_PATH} is missing. Build it with `python pytorch-approx-topk_amd/build.py`; "
+            f"approx_topk: {_HOST_PATH} {_host_fault}. Build it with `python pytorch-approx-topk_amd/build.py`; "
             "there is no fallback path.")
     host.bind({name: ctypes.cast(getattr(handle, name), ctypes.c_void_p).value for name in _SIGNATURES})
     return handle

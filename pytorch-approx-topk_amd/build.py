@@ -6,7 +6,8 @@ Every .hip file under csrc/ is compiled to an object (in parallel) and linked
 into approx_topk/libapprox_topk_hip.so, next to the Python package that loads
 it.  Nothing of it is linked against libtorch: the library speaks a C ABI only.
 csrc/host_binding.cpp, which calls that library with torch's tensors, becomes the
-extension module approx_topk/_host.so.
+extension module approx_topk/_host.so.  That one is for the torch and the Python it was
+built with, whose names it holds: it is built again when either is another one.
 
 --trace builds a second library, approx_topk/libapprox_topk_hip_trace.so, whose long
 kernels stamp a clock at their phase boundaries (csrc/atk_trace.h); it is what
@@ -18,6 +19,7 @@ import concurrent.futures
 import glob
 import importlib.util
 import os
+import shutil
 import subprocess
 import sys
 import sysconfig
@@ -46,14 +48,44 @@ def _newer(target: str, deps: list[str]) -> bool:
     return all(os.path.getmtime(d) <= t for d in deps)
 
 
+def _rocm_include() -> str:
+    """The HIP headers of the ROCm that HIPCC belongs to; HIPCC may be a name on the PATH."""
+    hipcc = shutil.which(HIPCC) or HIPCC
+    roots = [os.environ.get("ROCM_PATH", ""), *(os.path.dirname(os.path.dirname(p)) for p in (hipcc, os.path.realpath(hipcc))),
+             "/opt/rocm"]
+    for include in (os.path.join(root, "include") for root in roots if root):
+        if os.path.exists(os.path.join(include, "hip", "hip_runtime_api.h")):
+            return include
+    raise RuntimeError(f"no HIP headers found beside {HIPCC}; set ROCM_PATH")
+
+
+def _torch_dir() -> str:
+    return importlib.util.find_spec("torch").submodule_search_locations[0]
+
+
+def _built_for() -> str:
+    """What _host.so is for (approx_topk/_native.py looks for the same text in it)."""
+    spec = importlib.util.spec_from_file_location("torch_version", os.path.join(_torch_dir(), "version.py"))
+    version = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(version)
+    return f"approx_topk for torch {version.__version__}, {sysconfig.get_config_var('SOABI')};"
+
+
+def _host_is_current(sources: list[str]) -> bool:
+    if not _newer(HOST, sources):
+        return False
+    with open(HOST, "rb") as f:
+        return _built_for().encode() in f.read()
+
+
 def _host_command(source: str) -> list[str]:
-    torch_dir = importlib.util.find_spec("torch").submodule_search_locations[0]
-    include, lib = os.path.join(torch_dir, "include"), os.path.join(torch_dir, "lib")
-    rocm = os.path.join(os.path.dirname(os.path.dirname(HIPCC)), "include")
+    include, lib = os.path.join(_torch_dir(), "include"), os.path.join(_torch_dir(), "lib")
     return [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden", "-Wall",
             "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1", "-DTORCH_API_INCLUDE_EXTENSION_H", "-DTORCH_EXTENSION_NAME=_host",
+            f'-DATK_BUILT_FOR="{_built_for()}"',
             # (the headers of others, whose warnings are theirs)
-            "-isystem", include, "-isystem", os.path.join(include, "torch", "csrc", "api", "include"), "-isystem", rocm,
+            "-isystem", include, "-isystem", os.path.join(include, "torch", "csrc", "api", "include"),
+            "-isystem", _rocm_include(),
             "-isystem", sysconfig.get_paths()["include"], source, "-L" + lib, "-Wl,-rpath," + lib,
             "-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch_hip", "-ltorch", "-ltorch_python", "-o", HOST]
 
@@ -92,7 +124,7 @@ def build(force: bool = False, verbose: bool = True, trace: bool = False) -> str
         return len(heavy)
     jobs.sort(key=weight)
     host = os.path.join(CSRC, "host_binding.cpp")
-    if not trace and (force or not _newer(HOST, [host, headers[-1]])):
+    if not trace and (force or not _host_is_current([host, headers[-1]])):
         jobs.append(_host_command(host))
     with concurrent.futures.ThreadPoolExecutor(max_workers=min(8, max(1, len(jobs)))) as ex:
         for cmd, r in ex.map(run, jobs):

@@ -231,6 +231,7 @@ template <typename F> void take(F& fn, const py::dict& addresses, const char* na
 }  // namespace
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
+  m.attr("built_for") = ATK_BUILT_FOR;
   m.def("set_general", [](py::object topk_any, py::object topk_grad_any) {
     g_topk_any = topk_any.release().ptr();
     g_topk_grad_any = topk_grad_any.release().ptr();
