@@ -12,6 +12,8 @@
 //
 // The native library is loaded by _native.py with the first call that needs it, which hands its entry points over as
 // addresses (`bind`); until then the Python functions take every call.
+#include <atomic>
+
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/autograd/custom_function.h>
 #include <torch/extension.h>
@@ -35,9 +37,12 @@ decltype(&atk_stage1_workspace_bytes) g_stage1_workspace;
 decltype(&atk_stage1) g_stage1;
 decltype(&atk_stage1_i32) g_stage1_i32;
 decltype(&atk_topk_workspace_bytes_used) g_topk_workspace;
-decltype(&atk_topk) g_topk = nullptr;  // set last
+decltype(&atk_topk) g_topk;
 decltype(&atk_topk_i32) g_topk_i32;
 decltype(&atk_topk_grad) g_topk_grad;
+std::atomic<bool> g_bound{false};  // set behind them, once (the kernels below run without the interpreter's lock)
+
+bool bound() { return g_bound.load(std::memory_order_acquire); }
 
 // the Python functions that take what the fast paths do not (held until the process ends)
 PyObject* g_topk_any = nullptr;
@@ -125,7 +130,7 @@ std::tuple<Tensor, Tensor> run_rows(const Tensor& xs, int64_t k0, int64_t j, int
 }
 
 bool rows_in_place(const Tensor& xs) {
-  return g_topk != nullptr && plain(xs) && xs.dim() > 0 && xs.numel() > 0 && xs.is_contiguous() && dtype_code(xs.scalar_type()) >= 0;
+  return bound() && plain(xs) && xs.dim() > 0 && xs.numel() > 0 && xs.is_contiguous() && dtype_code(xs.scalar_type()) >= 0;
 }
 
 // ---- approx_topk::topk on the GPU ----
@@ -145,7 +150,7 @@ std::tuple<Tensor, Tensor> topk(const Tensor& xs, int64_t k, int64_t dim, int64_
 constexpr int64_t kMaxGradRow = (int64_t(1) << 31) - 1;
 
 Tensor topk_grad(const Tensor& grad_values, const Tensor& indices, int64_t n, int64_t k0, int64_t j, bool interleaved) {
-  if (g_topk != nullptr && plain(grad_values) && plain(indices) && indices.scalar_type() == at::kLong && indices.dim() > 0 &&
+  if (bound() && plain(grad_values) && plain(indices) && indices.scalar_type() == at::kLong && indices.dim() > 0 &&
       indices.numel() > 0 && grad_values.sizes() == indices.sizes() && grad_values.device() == indices.device() &&
       dtype_code(grad_values.scalar_type()) >= 0) {
     const Tensor grad = grad_values.contiguous(), index = indices.contiguous();
@@ -238,6 +243,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   });
   m.def("set_gradient", [](py::object gradient_any) { g_gradient_any = gradient_any.release().ptr(); });
   m.def("bind", [](const py::dict& addresses) {
+    if (bound()) return;  // (the library stays the one that was loaded first)
     take(g_strerror, addresses, "atk_strerror");
     take(g_stage1_workspace, addresses, "atk_stage1_workspace_bytes");
     take(g_stage1, addresses, "atk_stage1");
@@ -246,6 +252,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     take(g_topk_i32, addresses, "atk_topk_i32");
     take(g_topk_grad, addresses, "atk_topk_grad");
     take(g_topk, addresses, "atk_topk");
+    g_bound.store(true, std::memory_order_release);
   });
   // None where the rows are not the common case
   m.def("run", [](const Tensor& xs, int64_t k0, int64_t j, int64_t k, int layout, bool narrow, bool want_values,
