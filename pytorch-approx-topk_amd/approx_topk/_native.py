@@ -173,7 +173,7 @@ def rows_view(xs: torch.Tensor) -> tuple[torch.Tensor, int, int, int]:
     """
     n = xs.shape[-1]
     rows = xs.numel() // n if n else 0
-    if xs.is_contiguous():  # the common case, without walking the strides
+    if xs.is_contiguous():  # without walking the strides
         return xs, rows, n, n
     if xs.ndim == 1:
         return (xs if xs.stride(0) == 1 or n <= 1 else xs.contiguous()), rows, n, n
@@ -190,9 +190,10 @@ def rows_view(xs: torch.Tensor) -> tuple[torch.Tensor, int, int, int]:
     return xs, rows, n, step
 
 
-# Per-call constants of a contiguous input, keyed by everything they depend on:
-# (rows, n, dtype code, output shape, bound entry point).  One dictionary lookup
-# replaces the shape arithmetic on the way to the native call.
+# Per-call constants of what the native host module hands on, keyed by everything they depend on:
+# (rows, n, dtype code, output shape, bound entry point).  Those calls are rows at a pitch of their own,
+# copies of what has none, tensors that are more than plain ones, empty ones, and a process's first call;
+# one dictionary lookup replaces the shape arithmetic on the way to the native call.
 _CALLS: dict = {}
 
 

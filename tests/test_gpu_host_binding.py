@@ -1,8 +1,6 @@
 """The native host path of the operators (csrc/host_binding.cpp) against the Python functions that take every
 other call: the forms it accepts and those it hands on, the errors, and the gradient's node under what
 autograd does to it."""
-import threading
-
 import pytest
 import torch
 from torch.autograd import forward_ad
@@ -210,11 +208,11 @@ def test_backward_under_compiled_autograd(node):
 
 
 def test_threads_and_streams():
+    from concurrent.futures import ThreadPoolExecutor
     from approx_topk import topk
     from approx_topk.experimental import differentiable
     want = topk(_pair((64, 4096), dtype=torch.float32), 64, -1, j=2, k_mult=2)
     torch.cuda.synchronize()
-    bad = []
 
     def work(seed):
         with torch.cuda.stream(torch.cuda.Stream()):
@@ -222,10 +220,8 @@ def test_threads_and_streams():
                 x = _pair((64, 4096), dtype=torch.float32).requires_grad_()
                 values, indices = differentiable.topk(x, 64, -1, j=2, k_mult=2)
                 (g,) = torch.autograd.grad(values.sum(), x)
-                if not (torch.equal(values, want[0]) and torch.equal(indices, want[1]) and int(g.sum()) == 64 * 64):
-                    bad.append(seed)
+                assert torch.equal(values, want[0]) and torch.equal(indices, want[1]) and int(g.sum()) == 64 * 64
+        return seed
 
-    threads = [threading.Thread(target=work, args=(s,)) for s in range(4)]
-    [t.start() for t in threads]
-    [t.join() for t in threads]
-    assert not bad
+    with ThreadPoolExecutor(4) as pool:  # (result() raises what a worker raised)
+        assert [f.result(timeout=100) for f in [pool.submit(work, s) for s in range(4)]] == [0, 1, 2, 3]
