@@ -190,29 +190,19 @@ def rows_view(xs: torch.Tensor) -> tuple[torch.Tensor, int, int, int]:
     return xs, rows, n, step
 
 
-# Per-call constants of what the native host module hands on, keyed by everything they depend on:
-# (rows, n, dtype code, output shape, bound entry point).  Those calls are rows at a pitch of their own,
-# copies of what has none, tensors that are more than plain ones, empty ones, and a process's first call;
-# one dictionary lookup replaces the shape arithmetic on the way to the native call.
-_CALLS: dict = {}
-
-
 def _call_constants(xs: torch.Tensor, k_out: int, two_stage: bool, index_dtype: torch.dtype):
-    key = (xs.shape, xs.dtype, k_out, two_stage, index_dtype)
-    hit = _CALLS.get(key)
-    if hit is None:
-        L = lib()
-        n = xs.shape[-1]
-        rows = xs.numel() // n if n else 0
-        narrow = index_dtype != torch.int64
-        if two_stage:
-            entry = L.atk_topk_i32 if narrow else L.atk_topk
-        else:
-            entry = L.atk_stage1_i32 if narrow else L.atk_stage1
-        hit = (rows, n, dtype_code(xs.dtype), tuple(xs.shape[:-1]) + (k_out,), entry)
-        if len(_CALLS) < 4096:
-            _CALLS[key] = hit
-    return hit
+    """(rows, n, dtype code, output shape, entry point) of a call that the native host module hands on: rows at a pitch
+    of their own, copies of what has none, tensors that are more than plain ones, and a process's first call.
+    (Nothing is kept by the call's arguments: 8 and 8.0 are one key, and only one of them a size.)"""
+    L = lib()
+    n = xs.shape[-1]
+    rows = xs.numel() // n if n else 0
+    narrow = index_dtype != torch.int64
+    if two_stage:
+        entry = L.atk_topk_i32 if narrow else L.atk_topk
+    else:
+        entry = L.atk_stage1_i32 if narrow else L.atk_stage1
+    return rows, n, dtype_code(xs.dtype), (*xs.shape[:-1], k_out), entry
 
 
 def stage1(xs: torch.Tensor, k0: int, j: int, layout: int, index_dtype: torch.dtype = torch.int64,

@@ -499,3 +499,12 @@ def test_one_kernel_or_two_follows_the_faster_plan(kernels, calls):
         buf = ctypes.create_string_buffer(1024)
         assert _native.lib().atk_describe(4096, rows, n, n, k * k_mult, j, k, 0, _native.dtype_code(dtype), 4096, 4096, buf, 1024) == 0
         assert buf.value.decode().startswith(kernels), (dtype, rows, n, k, j, k_mult, buf.value)
+
+
+def test_a_refused_size_leaves_nothing_behind_for_the_next_call():
+    # (8.0 and 8 are one key of a dictionary)
+    from approx_topk import _native
+    x = torch.zeros(3, 64)
+    for k in (8.0, 8):
+        shape = _native._call_constants(x, k, False, torch.int64)[3]
+        assert [type(size) for size in shape] == [int, type(k)]
