@@ -90,5 +90,7 @@ def topk(
     if (not is_compiling() and _native.host is not None and type(xs) in _PLAIN and xs.is_cuda
             and peek_interpreter_stack() is None and forward_ad._current_level < 0
             and not _is_torch_function_mode_enabled()):
-        return _native.host.differentiable_topk(xs, k, dim, j, k_mult, interleaved, multithread_buckets)
+        out = _native.host.differentiable_topk(xs, k, dim, j, k_mult, interleaved, multithread_buckets)
+        if out is not None:
+            return out
     return _TopkWithGradient.apply(xs, k, dim, j, k_mult, interleaved, multithread_buckets)

@@ -271,4 +271,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     auto out = TopkWithGradient::apply(xs, k, dim, j, k_mult, interleaved, multithread_buckets);
     return std::make_tuple(out[0], out[1]);
   });
+  // arguments of other types: None, for the Python function that accepts or refuses them
+  m.def("run", [](const py::args&) { return py::none(); });
+  m.def("differentiable_topk", [](const py::args&) { return py::none(); });
 }

@@ -89,6 +89,26 @@ def test_what_is_refused_stays_refused(args, kwargs, monkeypatch):
     assert outcome(topk) == _general(monkeypatch, lambda: outcome(_topk))
 
 
+@pytest.mark.parametrize("args", [(8.0, -1), ("8", -1), (8, -1.0), (1 << 70, -1), (8, -1, 1, 1, "no"), (8, -1, 1, None), (None, -1),
+                                  (8, -1, True, True, 1, None), (torch.tensor(8), -1)], ids=str)
+def test_arguments_of_other_types_as_in_python(args, monkeypatch):
+    from approx_topk.experimental import bucketed_argmax, compact_indices, differentiable
+    x = torch.randn(3, 64).cuda()
+
+    def outcome(fn):
+        try:
+            values, indices = fn()
+            return values.cpu().tolist(), indices.cpu().tolist()
+        except Exception as e:
+            return type(e), str(e).splitlines()[0]
+
+    calls = [lambda: differentiable.topk(x, *args), lambda: compact_indices.topk(x, *args)]
+    if len(args) == 2:
+        calls.append(lambda: bucketed_argmax.topk_triton(x, *args, True))
+    for call in calls:
+        assert outcome(call) == _general(monkeypatch, lambda: outcome(call))
+
+
 def test_other_dtypes_and_devices_are_refused():
     from approx_topk import topk
     with pytest.raises(RuntimeError, match="unsupported dtype"):
