@@ -46,3 +46,24 @@ def test_narrow_tiles(dtype, shape):
     only = compact_indices.topk_indices(xd, k, -1, j=j, k_mult=k_mult)
     assert torch.equal(only.cpu().long(), want[1]), plan
 
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16], ids=lambda d: str(d).split(".")[-1])
+@pytest.mark.parametrize("shape", [
+    (5, 5000, 320, 1, 2, 5008, 0),     # a wave per tile; rows on 16 bytes, some of them
+    (129, 3002, 98, 1, 2, 3003, 1),    # rows anywhere
+    (64, 20480, 512, 2, 2, 20484, 3),  # eight tiles of one column a lane
+    (300, 7505, 142, 4, 4, 7600, 5),   # waves that share a tile
+])
+def test_narrow_tiles_of_rows_at_a_pitch(dtype, shape):
+    from approx_topk import _native, topk
+    rows, n, k, j, k_mult, pitch, first = shape
+    g = torch.Generator().manual_seed(n + pitch)
+    whole = (torch.randint(-30000, 30000, (rows, pitch), generator=g) / 64).to(dtype)
+    whole[rows // 2, first + 7:first + n:997] = float("nan")
+    whole[:, :first] = whole[:, first + n:] = float("inf")  # (between the rows: not theirs)
+    x = whole[:, first:first + n]
+    xd = whole.cuda()[:, first:first + n]
+    plan = _native.describe(xd, k * k_mult, j, k)
+    assert plan.startswith("fused_regs_kernel") and any(f"V={v}," in plan for v in (1, 2)), plan
+    assert_same(*topk(xd, k, -1, j=j, k_mult=k_mult), *oracle.topk(x.contiguous(), k, -1, j=j, k_mult=k_mult), plan)
