@@ -513,9 +513,13 @@ __global__ __launch_bounds__(kSoloThreads) void chain_solo_kernel(
   uint64_t* words = reinterpret_cast<uint64_t*>(dyn_lds);
   uint32_t* ats = reinterpret_cast<uint32_t*>(dyn_lds + (size_t)(kListCap + 8) * sizeof(uint64_t));
   // Members of the cut digit up to which they are listed.  With registers to spare a longer list is narrowed down, at
-  // about 1.5 us a level: ranking 512 by comparison takes 3, the radix select over 1536 took 10.
+  // about 1.5 us a level: ranking 300 by comparison takes 4 us more than 200, 500 another 3, the radix select over
+  // 1536 took 10.  Members of one key are told apart in trips to memory for their indices, which grow with the row: of
+  // up to 8192 candidates 300 are faster narrowed down (fp32 [1, 8192] 11.3 us, listed 12.9), of 16384 listed (15.8 us, 17.1),
+  // and 500 are not (19.2 us, 17.1).  (bf16 [1, 2^23] k=8192 k_mult=2, 281 members: the call 22.8 us with 256 for all, 19.6 now.)
   constexpr bool kSpare = NPT <= 16;
   constexpr uint32_t kListed = TIES && kSpare ? kSoloRankDirect / 2 : kListCap;
+  constexpr uint32_t kTied = TIES && NPT == 16 ? 384 : kListed;
   const uint32_t row = blockIdx.x / groups, g = blockIdx.x - row * groups;
   const uint32_t tid = threadIdx.x, lane = tid % select::kWave, wave = tid / select::kWave;
   const raw_t* cv = cand_values + (int64_t)row * k0;
@@ -624,10 +628,10 @@ __global__ __launch_bounds__(kSoloThreads) void chain_solo_kernel(
   // which is what stage 1 makes of saturated 8-bit data (the bucket maxima of uniform uint8 are
   // all 255) and of a ReLU's zeros -- and their indices decide.  With 32 keys per thread built for the 1-byte
   // types only: there the code costs the kernel 4-5 us whether it runs or not (it sits at its register limit).
-  const bool tie_mode = TIES && cut_digit && f.count > kListed;
+  const bool tie_mode = TIES && cut_digit && f.count > kTied;
   // A cut digit with more members than are listed (which, without TIES, no bits are left to
   // narrow) is not listed at all; the row then goes to the whole-row path below.
-  const bool list_it = cut_digit && f.count <= kListed;
+  const bool list_it = cut_digit && f.count <= kTied;
   const uint32_t own = g * kSoloThreads + tid;  // this thread's candidate of segment g
   const bool own_valid = FULL || own < k0;
   // survivors above the cut digit (or in it, when it belongs whole) in the
@@ -701,7 +705,7 @@ __global__ __launch_bounds__(kSoloThreads) void chain_solo_kernel(
       };
       // the group: inverted indices whose bits from ishift up are iprefix
       uint32_t ishift = (uint32_t)(index_bits < 31 ? index_bits : 31), iprefix = ~0u >> ishift;
-      while (need != count && count > kListed && ishift != 0) {
+      while (need != count && count > kTied && ishift != 0) {
         const uint32_t finer = ishift > (uint32_t)regs::kDigitBits ? ishift - (uint32_t)regs::kDigitBits : 0u;
         const uint32_t mask = (1u << (ishift - finer)) - 1u;
         __syncthreads();  // everyone has read `found`, wave 0 the histogram
@@ -722,7 +726,7 @@ __global__ __launch_bounds__(kSoloThreads) void chain_solo_kernel(
         need = f2.need;
         count = f2.count;
       }
-      if (need == count || count <= kListed) {
+      if (need == count || count <= kTied) {
         const uint64_t key_word = (uint64_t)(low + f.digit) << 32;  // (shift == 0: the digit is the key's offset)
         for_members([&](uint32_t u, uint32_t inv) {
           const uint32_t group = inv >> ishift;
@@ -817,7 +821,7 @@ __global__ __launch_bounds__(kSoloThreads) void chain_solo_kernel(
       if (tid == 0) list_count = 0;
     }
   }
-  if (need != count && count > kListed) {
+  if (need != count && count > kTied) {
     // More candidates of one key around the cut than are listed (TIES: of one key and
     // one index, which only a caller of the stand-alone select can hand over): the
     // row's first workgroup runs the block-wide radix select of stage2_select.h over

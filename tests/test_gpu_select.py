@@ -279,9 +279,9 @@ def test_select_of_rows_ranked_by_comparison(dtype, rows, k0, k):
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.uint8])
 @pytest.mark.parametrize("k0,bound", [(1536, 1 << 13), (2047, (1 << 31) - 1), (8192, 1 << 13), (8191, 1 << 24), (9000, 1 << 16),
                                       (16384, (1 << 31) - 1)])
-@pytest.mark.parametrize("m", [255, 256, 257, 513, 1500])
+@pytest.mark.parametrize("m", [256, 257, 384, 385, 513, 1500])
 def test_one_launch_select_of_crowded_keys(dtype, k0, bound, m):
-    # m candidates of one key around the cut, listed up to 256 of them and told apart by their indices beyond;
+    # m candidates of one key around the cut, listed up to 256 of them (384 in rows of more than 8192) and told apart by their indices beyond;
     # those above and below are spread, or of one key each (a wave adds eight of a digit and more at once)
     g = torch.Generator().manual_seed(k0 + m)
     cv = torch.randint(0, 100, (4, k0), generator=g)
