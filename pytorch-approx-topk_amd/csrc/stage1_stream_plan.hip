@@ -17,6 +17,12 @@ constexpr int64_t kCus = 256;
 constexpr int64_t kWaveBytes = 8 << 10, kRaisedBytes = 2 << 20;
 // Most partial queues of a row whose merge selects, with slabs that are cut to have a workgroup on every CU.
 constexpr int64_t kRaisedSelectQueues = 4096;
+// Workgroups from which calls of up to kRaisedEnoughBytes are left as they are with 16-byte loads (see plan_with).
+constexpr int64_t kRaisedEnough = 96, kRaisedEnoughBytes = 32 << 20;
+// Bytes of which a slab that is cut must not be nearly a multiple (4-byte elements, one-element loads).
+constexpr int64_t kStep = 128 << 10;
+// Partial queues of a row above which slabs of one-element loads are not cut to have the merge select.
+constexpr int64_t kCutSelectQueues = 8192;
 // How much longer a slab may get to have no more workgroups than CUs.
 constexpr double kLonger = 1.34, kLongerOneByte = 1.17;
 // Sub-rows worth giving to one wave before a row is also cut into slabs.
@@ -153,13 +159,25 @@ Plan plan_with(int64_t rows, int64_t n, int64_t k0, int j, int layout, int dtype
   //     a bucket 66 launches 0.95, with two 35 launches 1.06 (fp16 [2, 45395679] b=75 j=2, 512 -> 256 workgroups, 51.0 ->
   //     59.1 us) and of 4-byte ones 30 launches 1.26: those keep two workgroups a CU, but no more (513 -> 510, 20 launches 0.79);
   //   one-element loads, of the calls that are not faster with wider ones: 2- and 4-byte elements up to a third longer 95
-  //     launches 0.93 (three over 1.05, all of fp32 [3, 2^24], 258 -> 255 workgroups), beyond 28 launches 0.99 and up to
-  //     1.18; one byte up to a sixth longer 19 launches 0.94, beyond 20 launches 1.02 and up to 1.11.
-  // (With one slab left, and no merge, some lose a third.)
+  //     launches 0.93, beyond 28 launches 0.99 and up to 1.18; one byte up to a sixth longer 19 launches 0.94, beyond 20
+  //     launches 1.02 and up to 1.11.  Of 4-byte elements not where a slab would get up to a twentieth longer and 1 to 4 KiB
+  //     off a multiple of 128 KiB, as slabs of a 255th of 2^k elements are (read in step from the same parts of memory, it
+  //     seems): 109 launches 1.15, 104 of them over 1.03, against 599 launches 0.98 with four over 1.03 at other lengths
+  //     (int32 [3, 2^23] k=64 j=2, 258 -> 255 workgroups, 25.6 -> 27.2 us).
+  // (With one slab left, and no merge, some lose a third.)  One-element loads keep their slabs where fewer of them would
+  // have the merge select, of a row with more than kCutSelectQueues: 15 launches 1.10 (bf16 [1, 3212725] k=24 k_mult=8, 258 ->
+  // 255 workgroups and 16320 queues in one of them, 12.7 -> 15.9 us; with fewer queues, or 16-byte loads, 18 launches 0.90).
   const int64_t per_slab = rows * pl.col_tiles;  // workgroups
   const uint32_t slabs_asked = pl.slabs;
   const int64_t in_one_turn = kCus / per_slab;  // slabs
-  if (in_one_turn > 1 && (int64_t)pl.slabs > in_one_turn) {
+  const bool may_select = second_stage && es <= 4 && k0 <= kMergeSelectMax;
+  const bool long_select = pl.vec == 1 && may_select && k0 * (int64_t)pl.slabs > kMergeSelectEntries &&
+                           k0 * in_one_turn <= kMergeSelectEntries && b * in_one_turn > kCutSelectQueues;
+  const int64_t off_step = in_one_turn > 0 ? full / in_one_turn * width * es % kStep : 0;
+  const bool in_step = es == 4 && pl.vec == 1 && 20 * (int64_t)pl.slabs <= 21 * in_one_turn &&
+                       ((off_step >= 1024 && off_step <= 4096) ||
+                        (kStep - off_step >= 1024 && kStep - off_step <= 4096));
+  if (in_one_turn > 1 && (int64_t)pl.slabs > in_one_turn && !long_select && !in_step) {
     const double longer = (double)pl.slabs / (double)in_one_turn;
     const bool whole_cu = es == 8 || (pl.vec > 1 && w == 8), long_queues = w < 8 && es <= 2 && j >= 3;
     if (whole_cu || long_queues || longer <= (es == 1 ? kLongerOneByte : kLonger))
@@ -174,6 +192,10 @@ Plan plan_with(int64_t rows, int64_t n, int64_t k0, int j, int layout, int dtype
   // that cannot allocate has taken.  One workgroup a row reads them all where the merge selects: up to
   // kRaisedSelectQueues (107 launches up to there 0.92, of one to three elements a bucket and more queues 29 launches
   // 1.03: bf16 [1, 11732747] k=16 k_mult=2, 179 -> 256 slabs, 14.4 -> 17.1 us).
+  // Not with 16-byte loads from kRaisedEnough workgroups on in calls of up to kRaisedEnoughBytes, which have the memory
+  // busy for a few microseconds as they are: of 4-byte elements 310 launches 1.01 (83 over 1.03: fp32 [1, 3091105] k=24 j=4
+  // 191 -> 256 workgroups 14.5 -> 20.4 us, [8, 2^20] k=72 j=3 k_mult=2 128 -> 256 19.1 -> 22.0), of 1- and 2-byte ones raised by less
+  // than half 242 launches 1.00 (by more 547 launches 0.96); all others 2647 launches 0.94.
   if (pl.slabs > 1 && pl.slabs * per_slab < kCus && rows * k0 * (es + 8) <= kRaisedBytes) {
     int64_t slabs = in_one_turn;
     const int64_t by_wave = full * kWave * pl.vec * es / (w * kWaveBytes), by_queues = kRaisedBytes / (rows * k0 * (es + 4));
@@ -183,7 +205,9 @@ Plan plan_with(int64_t rows, int64_t n, int64_t k0, int j, int layout, int dtype
       const int64_t most_queues = second_stage && es <= 4 ? kRaisedSelectQueues : kMergeSelectEntries / j;
       if (slabs > most_queues / b) slabs = most_queues / b;
     }
-    if (slabs > (int64_t)pl.slabs) pl.slabs = (uint32_t)slabs;
+    const bool enough = pl.vec > 1 && pl.slabs * per_slab >= kRaisedEnough && rows * n * es <= kRaisedEnoughBytes &&
+                        (es == 4 || (es <= 2 && 2 * slabs < 3 * (int64_t)pl.slabs));
+    if (slabs > (int64_t)pl.slabs && !enough) pl.slabs = (uint32_t)slabs;
   }
   pl.slab_len = (uint32_t)(full / pl.slabs);
   // every wave scans exactly 4 or 8 sub-rows: straight-line kernels exist for that

@@ -22,9 +22,9 @@ CUT = [
 ]
 RAISED = [
     (F64, 1, 577600, 132, 4, 2, 64, 68), (F64, 15, 129856, 744, 3, 1, 3, 4), (F32, 3, 1205184, 2220, 3, 1, 4, 6),
-    (F64, 1, 1121152, 96, 4, 1, 72, 145), (F64, 24, 163615, 36, 3, 2, 6, 10), (F32, 38, 162112, 36, 1, 1, 5, 6),
+    (F64, 1, 1121152, 96, 4, 1, 72, 145), (F64, 24, 163615, 36, 3, 2, 6, 10), (BF16, 64, 143862, 24, 2, 2, 2, 4), (F16, 41, 285696, 36, 2, 2, 4, 6),
     (I32, 6, 550208, 144, 4, 1, 34, 42), (F32, 70, 61376, 24, 4, 2, 2, 3), (F32, 11, 209437, 408, 1, 2, 2, 4),
-    (F16, 27, 188992, 168, 1, 4, 2, 4), (I32, 2, 1448512, 72, 4, 2, 89, 113), (I32, 25, 117312, 744, 4, 2, 4, 5),
+    (F16, 27, 188992, 168, 1, 4, 2, 4), (I32, 2, 6448512, 72, 4, 2, 89, 128), (I32, 25, 417312, 744, 4, 2, 4, 5),
 ]
 
 

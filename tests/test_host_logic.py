@@ -478,10 +478,29 @@ def test_slabs_are_cut_to_one_turn_of_the_cus_where_that_was_measured_faster():
 
 
 def test_merges_that_select_are_not_given_more_than_a_workgroup_reads_quickly():
-    # slabs raised to one workgroup a CU: with a merge that selects only up to 4096 partial queues
-    assert _plan(torch.bfloat16, 1, 11732747, 16, 1, 2)[3] == 179
-    assert _plan(torch.bfloat16, 1, 11732747, 32, 1)[3] == 256  # (no second stage)
-    assert _plan(torch.float16, 7, 1 << 22, 32, 4, 2)[3] == 36
+    # one-element loads keep a slab more where one fewer would have the merge select from more than 8192 queues
+    assert _plan(torch.bfloat16, 1, 3212725, 24, 1, 8)[::3] == (1, 86)
+    assert _plan(torch.float16, 1, 2581297, 24, 1, 8)[::3] == (1, 86)
+    # ... and are cut as ever with fewer
+    assert _plan(torch.float16, 2, 1319472, 444, 2, 2)[::3] == (1, 18)
+
+
+def test_slabs_are_raised_to_a_workgroup_a_cu_only_where_that_was_measured_faster():
+    f32, f16, bf16 = torch.float32, torch.float16, torch.bfloat16
+    assert _plan(f16, 7, 1 << 22, 32, 4, 2)[2:4] == (252, 36) and _plan(f32, 2, 1 << 23, 1024, 4, 4)[2] == 256
+    # up to 32 MiB with 16-byte loads: 4-byte elements from 96 workgroups on not, shorter ones by half and more
+    assert _plan(f32, 8, 1 << 20, 72, 3, 2)[:4] == (4, 8, 128, 16)
+    assert _plan(bf16, 1, 11732747, 16, 1, 2)[3] == _plan(bf16, 1, 11732747, 32, 1)[3] == 179
+    assert _plan(f16, 41, 285696, 36, 2, 2)[3] == 6
+
+
+def test_slabs_of_four_byte_elements_do_not_all_start_in_step():
+    # 85 slabs of 2^23 elements are 1.5 KiB off a multiple of 128 KiB
+    for dtype in (torch.float32, torch.int32):
+        for k in (16, 32, 64, 128, 256, 1024):
+            vec, _, grid, _, text = _plan(dtype, 3, 1 << 23, k, 2)
+            assert vec > 1 or grid != 255, text
+    assert _plan(torch.int32, 3, 1 << 22, 64, 2)[:4] == (1, 8, 255, 85)
 
 
 # (type, rows, n, k, j, k_mult): calls timed in one kernel and in two, at least 20 % apart: the planner takes the faster one
